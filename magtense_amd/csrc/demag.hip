@@ -115,6 +115,24 @@ __device__ inline void lds_dma16_nt(const void* src, uint32_t lds) {
       : "memory");
 }
 
+// Three such transfers of consecutive KiB (the instruction's offset applies to
+// the global and to the LDS address), one M0 set-up for all of them.
+__device__ inline void lds_dma16x3(const void* src, uint32_t lds) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "global_load_lds_dwordx4 %1, off offset:1024\n\t"
+      "global_load_lds_dwordx4 %1, off offset:2048\n\t"
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0"
+      : "=&s"(saved)
+      : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds))
+      : "memory");
+}
+
 __device__ inline uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
@@ -925,29 +943,14 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
     const int ne = ix < 2 ? 4 : 1;  // entries this step is the first to use
     for (int k = 0; k < ne; ++k) {
       const int e = e0 + 2 * k;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const int f = wave * 3 + q;
-        lds_dma16(Kt + ((islab + e) * 12 + f) * 64 + lane, lds_addr(&ent[e & 7][f][0]));
-      }
+      lds_dma16x3(Kt + ((islab + e) * 12 + wave * 3) * 64 + lane, lds_addr(&ent[e & 7][wave * 3][0]));
     }
     const int64_t J = iJ0 + ix;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int f = wave * 3 + q;
-      lds_dma16(Mp + (J * 12 + f) * 64 + lane, lds_addr(&bst[g & 1][f][0]));
-    }
+    lds_dma16x3(Mp + (J * 12 + wave * 3) * 64 + lane, lds_addr(&bst[g & 1][wave * 3][0]));
     if (++ix == cpr) {
       ix = 0;
       if (++is < sb1) row_setup();
     }
-  };
-  auto fetch = [&](int x1c, int g, uint4 (&ra)[12], uint4 (&rb)[12]) {
-    const int slot = (cpr - 1 - x1c + 2 * wave) & 7;
-#pragma unroll
-    for (int q = 0; q < 12; ++q) ra[q] = ent[slot][q][lane];
-#pragma unroll
-    for (int q = 0; q < 12; ++q) rb[q] = bst[g & 1][q][lane];
   };
   floatx16 acc[2][3];
 #pragma unroll
@@ -956,38 +959,75 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
     for (int a = 0; a < 3; ++a)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[sb][a][r] = 0.0f;
-  auto mfmas = [&](const uint4 (&ra)[12], const uint4 (&rb)[12]) {
-    const int comp[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
-#pragma unroll
-    for (int beta = 0; beta < 3; ++beta)
-#pragma unroll
-      for (int t = 0; t < 3; ++t)  // hi*hi, hi*lo, lo*hi
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-          for (int sb = 0; sb < 2; ++sb) {
-            const int c = comp[a][beta];
-            const bf16x8 kf = as_bf16x8(ra[2 * c + (t == 2 ? 1 : 0)]);
-            const bf16x8 mf = as_bf16x8(rb[(beta * 2 + sb) * 2 + (t == 1 ? 1 : 0)]);
-            acc[sb][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, mf, acc[sb][a], 0, 0, 0);
-          }
-  };
-  // step g: wait for my step-g DMA and my step-(g-1) LDS reads, then for
-  // everyone's; read step g's fragments, DMA step g+1 (into slots step g does
-  // not read) and run step g's MFMAs (the compiler waits for each fragment
-  // just before its first use)
+  // the step's fragments: ra[2c + part] the tensor's, rb[(beta*2 + sb)*2 + part] the states'
   uint4 ra[12], rb[12];
+  auto entry_slot = [&](int x1c) { return (cpr - 1 - x1c + 2 * wave) & 7; };
+  auto read_a = [&](int slot, int c) {
+    ra[2 * c] = ent[slot][2 * c][lane];
+    ra[2 * c + 1] = ent[slot][2 * c + 1][lane];
+  };
+  auto read_b = [&](int g, int beta) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) rb[4 * beta + q] = bst[g & 1][4 * beta + q][lane];
+  };
+  // the three split products (hi*hi, hi*lo, lo*hi, in this order) of component
+  // c against source component beta, into output components a0 .. a0 + na - 1
+  // (cc: their tensor components); every accumulator sees beta 0, 1, 2
+  auto mfmas = [&](int a0, int na, const int* cc, int beta) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+      for (int a = 0; a < na; ++a)
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb) {
+          const bf16x8 kf = as_bf16x8(ra[2 * cc[a0 + a] + (t == 2 ? 1 : 0)]);
+          const bf16x8 mf = as_bf16x8(rb[(beta * 2 + sb) * 2 + (t == 1 ? 1 : 0)]);
+          acc[sb][a0 + a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, mf, acc[sb][a0 + a], 0, 0, 0);
+        }
+  };
+  const int c0[3] = {0, 1, 2}, c1[3] = {1, 3, 4}, c2[3] = {2, 4, 5};
+  // The barrier that hands over step g + 1 stands two thirds into step g: its
+  // DMA (issued in step g - 1) has landed, and all of step g's LDS reads are
+  // done.  Behind it the first fragments of step g + 1 are read, and the DMA
+  // of step g + 2 runs, under the last third of step g's MFMAs; the rest of a
+  // step's fragments are read under its first third.  So no MFMA waits for an
+  // LDS read that was not issued 12 or more MFMAs earlier.
   if (G > 0) {
     issue(0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (G > 1) issue(1);
     int x1c = 0;  // chunk of step g within its source row
+    read_a(entry_slot(0), 0);
+    read_a(entry_slot(0), 1);
+    read_b(0, 0);
     for (int g = 0; g < G; ++g) {
-      __builtin_amdgcn_s_waitcnt(0);
-      __builtin_amdgcn_s_barrier();
+      const int slot = entry_slot(x1c);
+      read_a(slot, 2);
+      read_a(slot, 3);
+      read_b(g, 1);
+      read_a(slot, 4);
+      read_a(slot, 5);
+      read_b(g, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0, 2, c0, 0);
+      mfmas(2, 1, c0, 0);
+      mfmas(0, 3, c1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(0);  // my DMA of step g + 1, my LDS reads of step g
+      __builtin_amdgcn_s_barrier();   // everyone's
       asm volatile("" ::: "memory");
-      fetch(x1c, g, ra, rb);
-      if (g + 1 < G) issue(g + 1);
-      mfmas(ra, rb);
       if (++x1c == cpr) x1c = 0;
+      if (g + 1 < G) {
+        const int next = entry_slot(x1c);
+        read_a(next, 0);
+        read_a(next, 1);
+        read_b(g + 1, 0);
+      }
+      if (g + 2 < G) issue(g + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(0, 3, c2, 2);
     }
     __builtin_amdgcn_s_waitcnt(0);  // no LDS write may outlive the workgroup
   }
