@@ -27,7 +27,9 @@ __device__ inline uint16_t bf16_bits(float v) {
 __device__ inline float bf16_value(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
 // FP32 states [s][3n] -> split BF16 B-fragments (columns s < nstates <= 64)
-__global__ void pack_bf16_kernel(const float* __restrict__ m, int n, int nstates, uint8_t* __restrict__ packed) {
+// (nonfinite, if any: set when a value is not finite in BF16)
+__global__ void pack_bf16_kernel(const float* __restrict__ m, int n, int nstates, uint8_t* __restrict__ packed,
+                                 int* __restrict__ nonfinite) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t total = (int64_t)nstates * 3 * n;
   if (t >= total) return;
@@ -44,6 +46,7 @@ __global__ void pack_bf16_kernel(const float* __restrict__ m, int n, int nstates
   uint16_t* p = reinterpret_cast<uint16_t*>(packed + frag * kFragBytes + lane * 16) + (j % 8);
   p[0] = hi;
   p[kFragBytes / 2] = lo;
+  if (nonfinite && !(fabsf(f) <= kBf16Max)) *nonfinite = 1;
 }
 
 // FP32 states [s][3n] -> FP32 B-fragments of the block-sparse FP32 product
@@ -289,7 +292,8 @@ int mt_toeplitz_tensor(int nx, int ny, int nz, double Lx, double Ly, double Lz, 
 extern "C++" {
 namespace mt {
 namespace {
-__global__ void zero16_kernel(uint4* __restrict__ p, int64_t n16) {
+__global__ void zero16_kernel(uint4* __restrict__ p, int64_t n16, int* __restrict__ flag) {
+  if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n16; t += (int64_t)gridDim.x * blockDim.x)
     p[t] = make_uint4(0u, 0u, 0u, 0u);
 }
@@ -309,7 +313,8 @@ Bf16x2Work bf16x2_work(int n, int nrows, int nx, int ny, int nz, int nstates, in
 // nrows < n only for a row block of the dense tensor (h holds 3 nrows per state).
 // `ws` holds w.bytes() of device memory.
 int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, const float* m, float* h, int nstates,
-                    float pref, const Bf16x2Work& w, uint8_t* ws, const BlockSparseView* bsv, bool f32) {
+                    float pref, const Bf16x2Work& w, uint8_t* ws, int* nonfinite, const BlockSparseView* bsv,
+                    bool f32) {
   int rc = kOk;
   const int64_t n3 = (int64_t)3 * n;
   const int64_t r3 = (int64_t)3 * nrows;
@@ -320,7 +325,7 @@ int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, con
   for (int s0 = 0; s0 < nstates && rc == kOk; s0 += kMaxCols) {
     int S = nstates - s0 < kMaxCols ? nstates - s0 : kMaxCols;
     hipLaunchKernelGGL(zero16_kernel, dim3((unsigned)std::min<int64_t>((n16 + 255) / 256, 4096)), dim3(256), 0,
-                       nullptr, reinterpret_cast<uint4*>(packed), n16);
+                       nullptr, reinterpret_cast<uint4*>(packed), n16, nonfinite);
     MT_HIP(hipGetLastError());
     int64_t tot = (int64_t)S * n3;
     if (f32)
@@ -328,7 +333,7 @@ int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, con
                          m + s0 * n3, n, S, packed);
     else
       hipLaunchKernelGGL(pack_bf16_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, nullptr, m + s0 * n3,
-                         n, S, packed);
+                         n, S, packed, nonfinite);
     MT_HIP(hipGetLastError());
     if (bsv)
       rc = launch_gemm_bsr((const uint8_t*)K, *bsv, f32, packed, n, part, n3, (int64_t)cols * n3, S, ks, nullptr);
@@ -336,7 +341,7 @@ int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, con
       rc = launch_gemm_f32((const uint8_t*)K, packed, n, part, n3, (int64_t)cols * n3, S, ks, nullptr);
     else if (nx > 0)
       rc = launch_gemm_bf16x2_toeplitz((const uint8_t*)K, nx, ny, nz, packed, part, n3, (int64_t)cols * n3, S, ks,
-                                       nullptr);
+                                       nonfinite, nullptr);
     else if (nrows < n)
       rc = launch_gemm_bf16x2_rows((const uint8_t*)K, packed, n, nrows, part, r3, (int64_t)cols * r3, S, ks,
                                    nullptr);
@@ -356,9 +361,11 @@ namespace {
 int apply_bf16x2(const void* K, int n, int nrows, int nx, int ny, int nz, const float* m, float* h, int nstates,
                  float pref) {
   const Bf16x2Work w = bf16x2_work(n, nrows, nx, ny, nz, nstates);
+  const size_t flag_at = (size_t)round_up((int64_t)w.bytes(), 256);
   DevArr<uint8_t> ws;
-  MT_HIP(ws.alloc(w.bytes()));
-  return apply_bf16x2_in(K, n, nrows, nx, ny, nz, m, h, nstates, pref, w, ws.p);
+  MT_HIP(ws.alloc(flag_at + sizeof(int)));
+  return apply_bf16x2_in(K, n, nrows, nx, ny, nz, m, h, nstates, pref, w, ws.p,
+                         reinterpret_cast<int*>(ws.p + flag_at));
 }
 }  // namespace
 }  // namespace mt
@@ -387,7 +394,7 @@ int mt_demag_apply_f32_mfma(const void* frags, int n, const float* m, float* h, 
   const Bf16x2Work w = bf16x2_work(n, n, 0, 0, 0, nstates);
   DevArr<uint8_t> ws;
   MT_HIP(ws.alloc(w.bytes()));
-  return apply_bf16x2_in(frags, n, n, 0, 0, 0, m, h, nstates, pref, w, ws.p, nullptr, true);
+  return apply_bf16x2_in(frags, n, n, 0, 0, 0, m, h, nstates, pref, w, ws.p, nullptr, nullptr, true);
 }
 
 int mt_demag_near_correction(int nx, int ny, int nz, double Lx, double Ly, double Lz, int radius, const float* m,
@@ -620,7 +627,7 @@ int mt_demag_apply_sparse(void* h, const float* m, float* hout, int nstates, flo
       sp->ws_bytes = w.bytes();
     }
     const BlockSparseView v = b.view();
-    return apply_bf16x2_in(b.frags, b.n, b.n, 0, 0, 0, m, hout, nstates, pref, w, sp->ws, &v, b.f32);
+    return apply_bf16x2_in(b.frags, b.n, b.n, 0, 0, 0, m, hout, nstates, pref, w, sp->ws, nullptr, &v, b.f32);
   }
   const int64_t n3 = (int64_t)3 * sp->n;
   for (int s0 = 0; s0 < nstates; s0 += kMaxCols) {

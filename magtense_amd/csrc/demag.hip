@@ -727,7 +727,43 @@ int launch_gemm_f32(const uint8_t* Kf, const uint8_t* Mpack, int n, float* out, 
   return launch_reg<4, false, false, true>(Kf, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream);
 }
 
-// Four-tile kernel for the translation-invariant table: a workgroup of four
+// Work of block b of the table kernels (block b runs on XCD b % 8): k-split
+// ks of row-tile group `group` (group >= groups: none).  A k-split of up to
+// eight ranges goes to the XCDs in pairs (first, last), (second, last but
+// one), ...: an XCD runs the later range of its pair and then the earlier one,
+// so its resident workgroups share one range's state and table slabs in its
+// L2, and all XCDs have the same work although the ranges of the receivers'
+// own plane, the first ones, take 30 MFMAs a chunk instead of 54.  Otherwise
+// each XCD takes a contiguous range of work, all k-splits among it.
+__device__ inline void table_block(int ksplit, int groups, int& ks, int& group) {
+  const int x = (int)(blockIdx.x % 8), q = (int)(blockIdx.x / 8);
+  if (ksplit == 1) {
+    ks = 0;
+    group = (int)blockIdx.x;
+  } else if (ksplit <= 8 && 8 % ksplit == 0) {
+    const int pairs = ksplit / 2, nsub = 8 / pairs, per = (groups + nsub - 1) / nsub;
+    const int p = x % pairs;
+    ks = q < per ? ksplit - 1 - p : p;
+    group = x / pairs + nsub * (q < per ? q : q - per);
+  } else {
+    const int per_xcd = (groups * ksplit + 7) / 8;
+    const int lin = x * per_xcd + q;
+    ks = lin % ksplit;
+    group = lin < groups * ksplit ? lin / ksplit : groups;
+  }
+}
+// Grid of a launch with that mapping.
+int table_blocks(int ksplit, int groups) {
+  if (ksplit > 1 && ksplit <= 8 && 8 % ksplit == 0) {
+    const int nsub = 8 / (ksplit / 2);
+    return 8 * 2 * ((groups + nsub - 1) / nsub);
+  }
+  return (groups * ksplit + 7) / 8 * 8;
+}
+
+// Four-tile kernel for the translation-invariant table (nx % 128 != 0; with
+// the in-plane chunks at 30 MFMAs instead of 54, 96 x 9 x 1: 0.127 -> 0.089
+// ms, 64 x 30 x 4: 0.79 -> 0.69 ms per 64-state call): a workgroup of four
 // waves owns four 32-row tiles, each wave one tile and all 64 states (six
 // accumulators).  Tensor and state fragments of a k-chunk (48 + 12 KiB) are
 // DMA'd into a single LDS slot; each wave copies its 24 fragments of the chunk
@@ -740,7 +776,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
                                                                 const uint4* __restrict__ Mp, int64_t np,
                                                                 int ksplit, float* __restrict__ out, int n,
                                                                 int64_t col_stride, int64_t split_stride, int ncols,
-                                                                int gnx, int gny, int gnz) {
+                                                                int gnx, int gny, int gnz,
+                                                                const int* __restrict__ nonfinite) {
   constexpr int FR = 60;     // fragments per slot: 4 tiles x 12 + 12 state fragments
   __shared__ uint4 smem[1][FR][64];
   const int lane = threadIdx.x & 63;
@@ -748,26 +785,9 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
   const int nJ = (int)(np / kTileK);
   const int n_row_tiles = (int)(np / kTileM);
   const int groups = (n_row_tiles + 3) / 4;
-  // XCD-aware order (block b runs on XCD b % 8).  With a k-split dividing 8,
-  // XCD x takes k-split x % ksplit for every group: its resident workgroups
-  // then walk the same offset sequence (below) and share the table slabs in
-  // its L2.  Otherwise each XCD takes a contiguous range of work.
   int ks, group;
-  const bool by_ks = ksplit <= 8 && 8 % ksplit == 0;
-  if (by_ks) {
-    const int xpk = 8 / ksplit;  // XCDs per k-split
-    const int x = (int)(blockIdx.x % 8);
-    ks = x % ksplit;
-    group = (int)(blockIdx.x / 8) * xpk + x / ksplit;
-    if (group >= groups) return;  // whole workgroup, before any barrier
-  } else {
-    const int total = groups * ksplit;
-    const int per_xcd = (total + 7) / 8;
-    const int lin = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-    if (lin >= total) return;
-    ks = lin % ksplit;
-    group = lin / ksplit;
-  }
+  table_block(ksplit, groups, ks, group);
+  if (group >= groups) return;  // whole workgroup, before any barrier
   const int jb = (int)((int64_t)nJ * ks / ksplit);
   const int je = (int)((int64_t)nJ * (ks + 1) / ksplit);
   const int64_t I = (int64_t)group * 4 + wave;
@@ -798,7 +818,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
     const int jy = (wy - r + gny) % gny, jz = (wz - sp + gnz) % gnz;
     return (jz * gny + jy) * cpr + x1c;
   };
-  auto issue = [&](int v, int slot) {
+  // full false: without the xz and yz fragments (4, 5, 8, 9)
+  auto issue = [&](auto full, int v, int slot) {
     const int J = chunk_of(v);
     const int jrow = J / cpr;
     const int x1c = J - jrow * cpr;
@@ -806,12 +827,10 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
     const int64_t base =
         (((int64_t)(tiz - jz + gnz - 1) * (2 * gny - 1) + (tiy - jy + gny - 1)) * U + (2 * tx0 - x1c + cpr - 1)) * 12;
 #pragma unroll
-    for (int q = 0; q < 12; ++q) lds_dma16(Kt + (base + q) * 64 + lane, lds_addr(&smem[slot][wave * 12 + q][0]));
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int f = wave * 3 + q;  // 0..11
-      lds_dma16(Mp + ((int64_t)J * 12 + f) * 64 + lane, lds_addr(&smem[slot][48 + f][0]));
-    }
+    for (int q = 0; q < 12; ++q)
+      if (full || q < 4 || q == 6 || q == 7 || q > 9)
+        lds_dma16(Kt + (base + q) * 64 + lane, lds_addr(&smem[slot][wave * 12 + q][0]));
+    lds_dma16x3(Mp + ((int64_t)J * 12 + wave * 3) * 64 + lane, lds_addr(&smem[slot][48 + wave * 3][0]));
   };
   floatx16 acc[2][3];
 #pragma unroll
@@ -822,7 +841,8 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
       for (int r = 0; r < 16; ++r) acc[sb][a][r] = 0.0f;
 
   uint4 ra[12], rb[12];
-  auto mfmas = [&]() {
+  auto mfmas = [&](auto full) {
+    constexpr bool FULL = decltype(full)::value;
     const int comp[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
 #pragma unroll
     for (int beta = 0; beta < 3; ++beta)
@@ -833,29 +853,47 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
 #pragma unroll
           for (int sb = 0; sb < 2; ++sb) {
             const int c = comp[a][beta];
+            if (!FULL && (c == 2 || c == 4)) continue;
             const bf16x8 kf = as_bf16x8(ra[2 * c + (t == 2 ? 1 : 0)]);
             const bf16x8 mf = as_bf16x8(rb[(beta * 2 + sb) * 2 + (t == 1 ? 1 : 0)]);
             acc[sb][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, mf, acc[sb][a], 0, 0, 0);
           }
   };
 
-  const int nchunks = je - jb;
-  if (nchunks > 0) {
-    issue(jb, 0);
-    for (int j = 0; j < nchunks; ++j) {
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // my loads of chunk j
+  // chunks [v0, v1), the DMA of v0 already issued; vn: the chunk after the last
+  auto chunks = [&](auto full, auto next_full, int v0, int v1, int vn) {
+    constexpr bool FULL = decltype(full)::value;
+    for (int v = v0; v < v1; ++v) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // my loads of chunk v
       __builtin_amdgcn_s_barrier();              // everyone's
       asm volatile("" ::: "memory");
 #pragma unroll
-      for (int q = 0; q < 12; ++q) ra[q] = smem[0][wave * 12 + q][lane];
+      for (int q = 0; q < 12; ++q)
+        if (FULL || q < 4 || q == 6 || q == 7 || q > 9) ra[q] = smem[0][wave * 12 + q][lane];
 #pragma unroll
       for (int q = 0; q < 12; ++q) rb[q] = smem[0][48 + q][lane];
       __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0): my reads done
       __builtin_amdgcn_s_barrier();              // everyone's: the slot is free
       asm volatile("" ::: "memory");
-      issue(jb + (j + 1 < nchunks ? j + 1 : j), 0);
-      if (tile_ok) mfmas();
+      if (v + 1 < v1) issue(full, v + 1, 0);
+      else issue(next_full, vn, 0);
+      if (tile_ok) mfmas(full);
     }
+  };
+  if (je > jb) {
+    // chunks v < ny cpr lie in the plane wz: the receivers' own where the
+    // group's tiles all do
+    const int last = group * 4 + 3 < n_row_tiles ? group * 4 + 3 : n_row_tiles - 1;
+    const bool one_plane = last / tpr / gny == wz && *nonfinite == 0;
+    int mid = one_plane ? gny * cpr : 0;
+    mid = mid < jb ? jb : (mid > je ? je : mid);
+    if (mid > jb) {
+      issue(std::false_type{}, jb, 0);
+      chunks(std::false_type{}, std::true_type{}, jb, mid, mid < je ? mid : je - 1);
+    } else {
+      issue(std::true_type{}, jb, 0);
+    }
+    chunks(std::true_type{}, std::true_type{}, mid, je, je - 1);
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no LDS write may outlive the workgroup
   }
   if (!tile_ok) return;
@@ -882,17 +920,21 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
 // four waves need cpr + 6 distinct entries where the four-tile kernel loads
 // 4 cpr.  Entries live in an eight-slot LDS ring (slot e mod 8): a step brings
 // one new entry (four at the first two chunks of a row) and one state chunk,
-// DMA'd one step ahead so that the transfer runs under the current step's
-// MFMAs; one barrier per step.  Slot safety (cpr % 8 == 0): the entries of
-// steps g and g+1 are eight consecutive values of e at most, so the DMA for
-// step g+1 (issued after the barrier that opens step g) writes only slots that
-// step g does not read, and the slots it overwrites were last read at step g-1,
-// whose reads every wave finished before that barrier.
+// DMA'd two steps ahead; one barrier per step, which stands inside the step
+// (below).  Slot safety (cpr % 8 == 0): the entries of steps g+1 and g+2 are
+// eight consecutive values of e at most, so the DMA for step g+2 (issued after
+// the barrier inside step g) writes only slots that step g+1 does not read,
+// and the slots it overwrites were last read at step g, whose reads every wave
+// finished before that barrier.
+// Bound by the matrix cores at the clock that their power leaves.  256 x 64 x
+// 2, 64 states, per call: 3.04 ms with the barrier at the step's start, 2.93
+// with it inside, 2.63 with the in-plane half of the chunks at 30 MFMAs
+// instead of 54 (nx x 2 planes; a single plane takes 30 throughout).
 __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __restrict__ Kt,
                                                                 const uint4* __restrict__ Mp, int ksplit,
                                                                 float* __restrict__ out, int n, int64_t col_stride,
                                                                 int64_t split_stride, int ncols, int gnx, int gny,
-                                                                int gnz) {
+                                                                int gnz, const int* __restrict__ nonfinite) {
   __shared__ uint4 ent[8][12][64];  // 96 KiB: table entries, slot e mod 8
   __shared__ uint4 bst[2][12][64];  // 24 KiB: state chunks, slot g mod 2
   const int lane = threadIdx.x & 63;
@@ -900,18 +942,8 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
   const int cpr = gnx / 16, tpr = gnx / 32, U = gnx / 8 - 2;
   const int rows = gny * gnz;
   const int groups = n / kTileM / 4;
-  // XCD-aware order as in the four-tile kernel (block b runs on XCD b % 8)
   int ks, group;
-  if (ksplit <= 8 && 8 % ksplit == 0) {
-    const int x = (int)(blockIdx.x % 8);
-    ks = x % ksplit;
-    group = (int)(blockIdx.x / 8) * (8 / ksplit) + x / ksplit;
-  } else {
-    const int per_xcd = (groups * ksplit + 7) / 8;
-    const int lin = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-    ks = lin % ksplit;
-    group = lin < groups * ksplit ? lin / ksplit : groups;
-  }
+  table_block(ksplit, groups, ks, group);
   if (group >= groups) return;  // whole workgroup, before any barrier
   const int sb0 = rows * ks / ksplit, sb1 = rows * (ks + 1) / ksplit;  // source rows of this split
   const int I0 = group * 4;
@@ -970,19 +1002,21 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
 #pragma unroll
     for (int q = 0; q < 4; ++q) rb[4 * beta + q] = bst[g & 1][4 * beta + q][lane];
   };
-  // the three split products (hi*hi, hi*lo, lo*hi, in this order) of component
-  // c against source component beta, into output components a0 .. a0 + na - 1
-  // (cc: their tensor components); every accumulator sees beta 0, 1, 2
-  auto mfmas = [&](int a0, int na, const int* cc, int beta) {
+  // the three split products (hi*hi, hi*lo, lo*hi, in this order) of the
+  // components cc against source component beta; every accumulator sees beta
+  // 0, 1, 2.  FULL false: the components xz and yz (2 and 4) are left out.
+  auto mfmas = [&](auto full, int a0, int a1, const int* cc, int beta) {
+    constexpr bool FULL = decltype(full)::value;
 #pragma unroll
     for (int t = 0; t < 3; ++t)
 #pragma unroll
-      for (int a = 0; a < na; ++a)
+      for (int a = a0; a < a1; ++a)
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb) {
-          const bf16x8 kf = as_bf16x8(ra[2 * cc[a0 + a] + (t == 2 ? 1 : 0)]);
+          if (!FULL && (cc[a] == 2 || cc[a] == 4)) continue;
+          const bf16x8 kf = as_bf16x8(ra[2 * cc[a] + (t == 2 ? 1 : 0)]);
           const bf16x8 mf = as_bf16x8(rb[(beta * 2 + sb) * 2 + (t == 1 ? 1 : 0)]);
-          acc[sb][a0 + a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, mf, acc[sb][a0 + a], 0, 0, 0);
+          acc[sb][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, mf, acc[sb][a], 0, 0, 0);
         }
   };
   const int c0[3] = {0, 1, 2}, c1[3] = {1, 3, 4}, c2[3] = {2, 4, 5};
@@ -991,29 +1025,22 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
   // done.  Behind it the first fragments of step g + 1 are read, and the DMA
   // of step g + 2 runs, under the last third of step g's MFMAs; the rest of a
   // step's fragments are read under its first third.  So no MFMA waits for an
-  // LDS read that was not issued 12 or more MFMAs earlier.
-  if (G > 0) {
-    issue(0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (G > 1) issue(1);
-    int x1c = 0;  // chunk of step g within its source row
-    read_a(entry_slot(0), 0);
-    read_a(entry_slot(0), 1);
-    read_b(0, 0);
-    for (int g = 0; g < G; ++g) {
+  // LDS read that was not issued several MFMAs earlier.
+  int x1c = 0;  // chunk of step g within its source row
+  auto steps = [&](auto full, int g0, int g1) {
+    constexpr bool FULL = decltype(full)::value;
+    for (int g = g0; g < g1; ++g) {
       const int slot = entry_slot(x1c);
-      read_a(slot, 2);
+      if (FULL) read_a(slot, 2);
       read_a(slot, 3);
       read_b(g, 1);
-      read_a(slot, 4);
+      if (FULL) read_a(slot, 4);
       read_a(slot, 5);
       read_b(g, 2);
       __builtin_amdgcn_sched_barrier(0);
-      mfmas(0, 2, c0, 0);
-      mfmas(2, 1, c0, 0);
-      mfmas(0, 3, c1, 1);
+      mfmas(full, 0, 2, c0, 0);
+      mfmas(full, 2, 3, c0, 0);
+      mfmas(full, 0, 3, c1, 1);
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0);  // my DMA of step g + 1, my LDS reads of step g
       __builtin_amdgcn_s_barrier();   // everyone's
@@ -1027,8 +1054,23 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __r
       }
       if (g + 2 < G) issue(g + 2);
       __builtin_amdgcn_sched_barrier(0);
-      mfmas(0, 3, c2, 2);
+      mfmas(full, 0, 3, c2, 2);
     }
+  };
+  if (G > 0) {
+    issue(0);
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (G > 1) issue(1);
+    read_a(entry_slot(0), 0);
+    read_a(entry_slot(0), 1);
+    read_b(0, 0);
+    // source rows s < ny are those of the receivers' own plane
+    const int own = sb0 < gny ? (sb1 < gny ? sb1 : gny) - sb0 : 0;
+    const int planar = *nonfinite ? 0 : own * cpr;
+    steps(std::false_type{}, 0, planar);
+    steps(std::true_type{}, planar, G);
     __builtin_amdgcn_s_waitcnt(0);  // no LDS write may outlive the workgroup
   }
   float* o = out + (int64_t)ks * split_stride;
@@ -1250,7 +1292,8 @@ int launch_gemm_bsr(const uint8_t* frags, const BlockSparseView& bs, bool f32, c
 }
 
 int launch_gemm_bf16x2_toeplitz(const uint8_t* Ktab, int nx, int ny, int nz, const uint8_t* Mpack, float* out,
-                                int64_t col_stride, int64_t split_stride, int ncols, int ksplit, hipStream_t stream) {
+                                int64_t col_stride, int64_t split_stride, int ncols, int ksplit,
+                                const int* nonfinite, hipStream_t stream) {
   if (nx % 32 != 0 || nx < 32 || ny < 1 || nz < 1) {
     set_error("the translation-invariant GEMM needs nx % 32 == 0");
     return kErrArg;
@@ -1258,10 +1301,9 @@ int launch_gemm_bf16x2_toeplitz(const uint8_t* Ktab, int nx, int ny, int nz, con
   const int n = nx * ny * nz;
   if (table_window_ok(nx, ny, nz, ksplit)) {
     const int groups = n / kTileM / 4;
-    const int blocks = (groups * ksplit + 7) / 8 * 8;
-    hipLaunchKernelGGL(gemm_bf16x2_tw_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
+    hipLaunchKernelGGL(gemm_bf16x2_tw_kernel, dim3((unsigned)table_blocks(ksplit, groups)), dim3(256), 0, stream,
                        reinterpret_cast<const uint4*>(Ktab), reinterpret_cast<const uint4*>(Mpack), ksplit, out, n,
-                       col_stride, split_stride, ncols, nx, ny, nz);
+                       col_stride, split_stride, ncols, nx, ny, nz, nonfinite);
     MT_HIP(hipGetLastError());
     return kOk;
   }
@@ -1272,10 +1314,9 @@ int launch_gemm_bf16x2_toeplitz(const uint8_t* Ktab, int nx, int ny, int nz, con
     // N = 32768, 64 states: 3.19 ms, against 3.31 ms for a two-stage version of
     // it and 3.50 ms for the two-tile four-stage kernel)
     const int groups4 = (n / kTileM + 3) / 4;
-    const int blocks4 = (groups4 * ksplit + 7) / 8 * 8;
-    hipLaunchKernelGGL(gemm_bf16x2_t4s_kernel, dim3((unsigned)blocks4), dim3(256), 0, stream,
+    hipLaunchKernelGGL(gemm_bf16x2_t4s_kernel, dim3((unsigned)table_blocks(ksplit, groups4)), dim3(256), 0, stream,
                        reinterpret_cast<const uint4*>(Ktab), reinterpret_cast<const uint4*>(Mpack), (int64_t)n,
-                       ksplit, out, n, col_stride, split_stride, ncols, nx, ny, nz);
+                       ksplit, out, n, col_stride, split_stride, ncols, nx, ny, nz, nonfinite);
     MT_HIP(hipGetLastError());
     return kOk;
   }

@@ -229,8 +229,14 @@ __global__ void __launch_bounds__(256) vec_kernel(const VecDesc* __restrict__ de
           *reinterpret_cast<float*>(pack.bf16 + f32_frag_offset(D.pack_col, c, j)) = (float)v[q];
         }
     } else {
+      bool bad = false;
 #pragma unroll
-      for (int q = 0; q < kVecE; ++q) tile[threadIdx.x + 256 * q] = (float)v[q];
+      for (int q = 0; q < kVecE; ++q) {
+        const float f = (float)v[q];
+        tile[threadIdx.x + 256 * q] = f;
+        bad |= !(fabsf(f) <= kBf16Max);
+      }
+      if (bad && pack.nonfinite) *pack.nonfinite = 1;
     }
   }
   switch (kind) {

@@ -69,9 +69,15 @@ int launch_gemm_bf16x2(const uint8_t* Ksplit, const uint8_t* Mpack, int n, float
 int launch_gemm_bf16x2_rows(const uint8_t* Krows, const uint8_t* Mpack, int n, int nrows, float* out,
                             int64_t col_stride, int64_t split_stride, int ncols, int ksplit, hipStream_t stream);
 // Same product with the tensor given as the translation-invariant fragment table of
-// an nx x ny x nz uniform grid (n = nx ny nz, nx % 32 == 0).
+// an nx x ny x nz uniform grid (n = nx ny nz, nx % 32 == 0).  Between cells of
+// one plane the components xz and yz of the table are exactly (+-)0, so their
+// products, which add +-0 to sums that are never -0, are left out there: the
+// same bits with 30 of 54 MFMAs.  That holds for finite states only (0 times
+// an infinity or a NaN is a NaN): *nonfinite (device; set by whoever packs
+// the states, sticky) brings all products back.
 int launch_gemm_bf16x2_toeplitz(const uint8_t* Ktab, int nx, int ny, int nz, const uint8_t* Mpack, float* out,
-                                int64_t col_stride, int64_t split_stride, int ncols, int ksplit, hipStream_t stream);
+                                int64_t col_stride, int64_t split_stride, int ncols, int ksplit,
+                                const int* nonfinite, hipStream_t stream);
 // Same product over a block-sparse tensor (fragment sets `frags`, structure
 // `bs`): split-BF16 fragments and states, or with f32 FP32 fragments and
 // states (the FP32 layouts of pack_f32_frag) on FP32 MFMAs.
@@ -127,9 +133,10 @@ Bf16x2Work bf16x2_work(int n, int nrows, int nx, int ny, int nz, int nstates, in
 // nx > 0: K is the translation-invariant table of an nx x ny x nz grid; nrows <
 // n: K is a row block of the dense tensor; bsv: K holds the fragments of a
 // block-sparse tensor (f32: its FP32 form, states packed as FP32 fragments).
+// nonfinite: the flag of launch_gemm_bf16x2_toeplitz (device, needed with nx > 0).
 int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, const float* m, float* h, int nstates,
-                    float pref, const Bf16x2Work& w, uint8_t* ws, const BlockSparseView* bsv = nullptr,
-                    bool f32 = false);
+                    float pref, const Bf16x2Work& w, uint8_t* ws, int* nonfinite = nullptr,
+                    const BlockSparseView* bsv = nullptr, bool f32 = false);
 int device_ok();
 
 struct SparseDemag {
@@ -327,7 +334,10 @@ struct PackSpec {
   float* f32;                // [col][3n]
   int64_t col_stride;
   uint8_t* bf16;             // fragment layout (split-BF16, or FP32 with kPackF32Frag)
+  int* nonfinite = nullptr;  // set to 1 when a packed value is not finite in BF16 (kPackBf16; may be null)
 };
+// largest finite BF16 value: a state beyond it packs to an infinity
+constexpr float kBf16Max = 3.3895313892515355e38f;
 
 int vec_blocks_per_state(int n3);
 // With one block per state (3n <= 2048) the vector kernel writes the

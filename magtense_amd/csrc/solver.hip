@@ -306,6 +306,7 @@ struct Solver {
   double* fout = nullptr;     // [B][n_h][nt][12n]
   float* packf = nullptr;     // [B][3n]
   uint8_t* packb = nullptr;   // fragment layout, 64 columns
+  int* nonfinite = nullptr;   // device flag: a packed state held a value that is not finite in BF16
   float* hbuf = nullptr;      // [ksplit][cols][3n]
   int ksplit = 1;
   int hcols = 0;
@@ -338,7 +339,7 @@ struct Solver {
       if (p) (void)hipFree(p);
     };
     f(K32); f(Ksplit); f(Kf32); f(Ktab); f(near_tab); f(jfact); f(kfact); f(aniso); f(ms32); f(pool); f(yout); f(fout); f(packf); f(packb);
-    f(hbuf); f(partials); f(results); f(arena_d); f(xs); f(xe); f(xc); f(xv);
+    f(hbuf); f(nonfinite); f(partials); f(results); f(arena_d); f(xs); f(xe); f(xc); f(xv);
     sparse.release();
     if (h_results) (void)hipHostFree(h_results);
     if (arena_h) (void)hipHostFree(arena_h);
@@ -347,7 +348,7 @@ struct Solver {
     if (stream) (void)hipStreamDestroy(stream);
     xs = xe = xc = nullptr; xv = nullptr;
     K32 = nullptr; Ksplit = nullptr; Kf32 = nullptr; Ktab = nullptr; near_tab = nullptr; jfact = kfact = aniso = nullptr; ms32 = nullptr; pool = yout = fout = nullptr;
-    packf = nullptr; packb = nullptr; hbuf = nullptr; partials = results = nullptr; arena_d = nullptr;
+    packf = nullptr; packb = nullptr; hbuf = nullptr; nonfinite = nullptr; partials = results = nullptr; arena_d = nullptr;
     h_results = nullptr; arena_h = nullptr; stream = nullptr;
     for (hipEvent_t& e : ev) e = nullptr;
   }
@@ -1150,7 +1151,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
       s.evals += 1;
     }
     PackSpec pk;
-    if (precision == MT_PREC_BF16X2) pk = PackSpec{kPackBf16, nullptr, 0, packb};
+    if (precision == MT_PREC_BF16X2) pk = PackSpec{kPackBf16, nullptr, 0, packb, nonfinite};
     else if (sparse.blocks || Kf32) pk = PackSpec{kPackF32Frag, nullptr, 0, packb};
     else pk = PackSpec{kPackF32, packf, (int64_t)N3, nullptr};
     if (timing) MT_HIP(hipEventRecord(ev[2], stream));
@@ -1187,7 +1188,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     if (precision == MT_PREC_BF16X2) {
       if (Ktab)
         rc = launch_gemm_bf16x2_toeplitz(Ktab, nx, ny, nz, packb, hbuf, (int64_t)N3, (int64_t)hcols * N3, S, ksplit,
-                                         stream);
+                                         nonfinite, stream);
       else if (sparse.blocks)
         rc = launch_gemm_bsr(sparse.blocks->frags, sparse.blocks->view(), false, packb, n, hbuf, (int64_t)N3,
                                     (int64_t)hcols * N3, S, ksplit, stream);
@@ -1656,6 +1657,8 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
                                                 : (P.Ktab ? gemm_ksplit_table(P.nx, P.ny, P.nz) : gemm_ksplit_dense(n, n)));
     MT_HIP(hipMalloc(&P.packb, (size_t)packed_m_bytes(n)));
     MT_HIP(hipMemsetAsync(P.packb, 0, (size_t)packed_m_bytes(n), P.stream));
+    MT_HIP(hipMalloc(&P.nonfinite, sizeof(int)));
+    MT_HIP(hipMemsetAsync(P.nonfinite, 0, sizeof(int), P.stream));
     // near-band correction of the split product (uniform grids: dense tensor,
     // table or block-sparse tiles): MT_NEAR_RADIUS cells (default 2, 0 switches it off)
     if (!unstructured) {
