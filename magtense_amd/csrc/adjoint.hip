@@ -22,6 +22,7 @@
 //   kbar1 = h/6 lam + h/2 mu2,  mu1 = vjp(Y1, kbar1)
 //   lam  <- lam + mu1 + mu2 + mu3 + mu4.
 
+#include <cfloat>
 #include <cstring>
 #include <memory>
 #include <string>
@@ -45,6 +46,8 @@ struct VjpDesc {
   double* mbar;         // out: direct part of the input cotangent
   double* hbar;         // out: field cotangent
   void* packed;         // out: (Ms * Hbar) for the transpose demag pass, FP32 or FP64
+  int cols, col;        // cols > 0: packed is the lattice product's layout of that many states, column col
+  int* nonfinite;       // its flag
   double* grad_ms;      // accumulate: per-cell Ms gradient
   double* hext_part;    // accumulate: per-block partial sums of -Hbar (3 per block)
   double hext[3];
@@ -113,7 +116,13 @@ __global__ void __launch_bounds__(256) vjp_kernel(const LlgGrid g, const VjpDesc
     for (int c = 0; c < 3; ++c) {
       D.mbar[(size_t)c * n + i] = -D.alpha * cxu[c] - hxc[c];
       D.hbar[(size_t)c * n + i] = hb[c];
-      static_cast<T*>(D.packed)[(size_t)c * n + i] = (T)(ms * hb[c]);
+      const T pk = (T)(ms * hb[c]);
+      if (D.cols > 0) {
+        static_cast<T*>(D.packed)[lattice_state_offset(n, D.cols, D.col, c, i)] = pk;
+        if (!(fabs((double)pk) <= FLT_MAX)) *D.nonfinite = 1;
+      } else {
+        static_cast<T*>(D.packed)[(size_t)c * n + i] = pk;
+      }
       gms += hb[c] * (hm[c] - hj[c] - hk[c]);
       hx_part[c] = -hb[c];
     }
@@ -138,6 +147,8 @@ struct FinishDesc {
   const double* mbar;   // direct part
   const double* hbar;   // field cotangent
   const void* T;        // K (Ms Hbar), FP32 or FP64
+  int nsplit;           // its partial-sum slots, added in order
+  int64_t split_stride;
   double* mu;           // out: vjp w.r.t. the stage input
 };
 
@@ -172,7 +183,9 @@ __global__ void __launch_bounds__(256) vjp_finish_kernel(const LlgGrid g, const 
       double lz = iz == 0 ? (w(i + sz) - wi) : (iz == g.nz - 1 ? (w(i - sz) - wi) : (w(i - sz) - 2.0 * wi + w(i + sz)));
       lap += lz * g.idz2;
     }
-    const double tv = (double)static_cast<const TT*>(D.T)[(size_t)c * n + i];
+    TT ts = static_cast<const TT*>(D.T)[(size_t)c * n + i];
+    for (int k = 1; k < D.nsplit; ++k) ts += static_cast<const TT*>(D.T)[(size_t)k * D.split_stride + (size_t)c * n + i];
+    const double tv = (double)ts;
     D.mu[(size_t)c * n + i] = D.mbar[(size_t)c * n + i] - 2.0 * lap - tv + ak[c];
   }
 }
@@ -195,6 +208,9 @@ struct Rk4 {
   size_t es = 4;           // bytes per demag element (4 or 8)
   float* K32 = nullptr;
   double* K64 = nullptr;
+  LatticeTable lattice;    // FP32: the distinct tensor entries instead of K32
+  int* nonfinite = nullptr;
+  int nsplit = 1;          // partial-sum slots of the product
   double *jfact = nullptr, *kfact = nullptr, *aniso = nullptr;
   float* ms32 = nullptr;
   double* ms64 = nullptr;
@@ -227,7 +243,7 @@ struct Rk4 {
     auto f = [](void* p) {
       if (p) (void)hipFree(p);
     };
-    f(K32); f(K64); f(jfact); f(kfact); f(aniso); f(ms32); f(ms64); f(packd); f(hbuf); f(ckpt); f(seg); f(segS);
+    f(K32); f(K64); f(nonfinite); f(jfact); f(kfact); f(aniso); f(ms32); f(ms64); f(packd); f(hbuf); f(ckpt); f(seg); f(segS);
     f(work);
     f(grad_ms); f(hext_part); f(desc_d); f(dcache_d);
     if (desc_h) (void)hipHostFree(desc_h);
@@ -238,13 +254,22 @@ struct Rk4 {
   void* hcol(void* base, int b) const { return static_cast<uint8_t*>(base) + (size_t)b * n3() * es; }
 
   // out (default hbuf) = K * packd for all B states, columns n3 apart
+  // (lattice: nsplit slots of partial sums, B n3 apart)
   int demag_pass(void* out = nullptr) {
     if (!out) out = hbuf;
+    if (lattice.v.a)
+      return launch_lattice_rows(lattice.v, static_cast<const float*>(packd), lattice_cols(B),
+                                 static_cast<float*>(out), (int64_t)B * n3(), (int64_t)n3(), B, nonfinite, stream);
     if (fp64)
       return launch_matvec_f64(K64, n, static_cast<const double*>(packd), (int64_t)n3(), static_cast<double*>(out),
                                (int64_t)n3(), B, stream);
     return launch_matvec_f32(K32, n, static_cast<const float*>(packd), (int64_t)n3(), static_cast<float*>(out),
-                             (int64_t)n3(), B, stream);
+                             (int64_t)n3(), B, 1.0f, stream);
+  }
+  PackSpec pack_spec() const {
+    if (fp64) return PackSpec{kPackNone, nullptr, 0, nullptr};
+    if (lattice.v.a) return PackSpec{kPackLattice, static_cast<float*>(packd), lattice_cols(B), nullptr, nonfinite};
+    return PackSpec{kPackF32, static_cast<float*>(packd), (int64_t)n3(), nullptr};
   }
   int nblocks() const { return (n + 255) / 256; }
 
@@ -292,7 +317,8 @@ struct Rk4 {
     if (rc) return rc;
     // recording: when the states' S_out columns are laid out like the demag
     // buffer's, the product is written there directly instead of copied
-    bool direct = S_out != nullptr;
+    // (the lattice product's partial sums are added, and recorded, by the LL kernel)
+    bool direct = S_out != nullptr && !lattice.v.a;
     for (int b = 1; b < B && direct; ++b)
       direct = static_cast<uint8_t*>(S_out[b]) == static_cast<uint8_t*>(S_out[0]) + (size_t)b * n3() * es;
     void* out = direct ? S_out[0] : hbuf;
@@ -316,8 +342,7 @@ struct Rk4 {
     const VecDesc* dvd = nullptr;
     int rc = upload(vd, &dvd, 0);
     if (rc) return rc;
-    PackSpec pk{fp64 ? kPackNone : kPackF32, fp64 ? nullptr : static_cast<float*>(packd), (int64_t)n3(), nullptr};
-    return launch_vec(dvd, B, n, nullptr, nullptr, pk, false, stream);
+    return launch_vec(dvd, B, n, nullptr, nullptr, pack_spec(), false, stream);
   }
 
   int llg(double* const* Y, double* const* k, void* const* S_out, void* sums) {
@@ -329,7 +354,9 @@ struct Rk4 {
       L.out = k[b];
       if (fp64) L.hpart64 = static_cast<const double*>(hcol(sums, b));
       else L.hpart = static_cast<const float*>(hcol(sums, b));
-      L.nsplit = 1;
+      L.nsplit = nsplit;
+      L.split_stride = (int64_t)B * n3();
+      if (S_out && lattice.v.a) L.sum_out = static_cast<float*>(S_out[b]);
       for (int c = 0; c < 3; ++c) L.hext[c] = hext[b * 3 + c];
       L.alpha = alpha;
       L.gamma = gamma;
@@ -339,7 +366,7 @@ struct Rk4 {
     if (rc) return rc;
     rc = launch_llg(grid, dl, B, stream);
     if (rc) return rc;
-    if (S_out)
+    if (S_out && !lattice.v.a)
       for (int b = 0; b < B; ++b)
         MT_HIP(hipMemcpyAsync(S_out[b], hcol(sums, b), n3() * es, hipMemcpyDeviceToDevice, stream));
     return kOk;
@@ -368,9 +395,8 @@ struct Rk4 {
     const VecDesc* dvd = nullptr;
     int rc = upload(vd, &dvd, 2);
     if (rc) return rc;
-    PackSpec pk{pack ? kPackF32 : kPackNone, pack ? static_cast<float*>(packd) : nullptr, pack ? (int64_t)n3() : 0,
-                nullptr};
-    return launch_vec(dvd, B, n, nullptr, nullptr, pk, false, stream);
+    const PackSpec none{kPackNone, nullptr, 0, nullptr};
+    return launch_vec(dvd, B, n, nullptr, nullptr, pack ? pack_spec() : none, false, stream);
   }
 
   // pointer tables
@@ -452,12 +478,16 @@ struct Rk4 {
     std::vector<VjpDesc> vd(B);
     for (int b = 0; b < B; ++b) {
       VjpDesc& d = vd[b];
+      std::memset(&d, 0, sizeof(d));  // the padding too: blocks are compared by their bytes
       d.m = Y[b];
       d.S = S[b];
       d.u = u[b];
       d.mbar = mbar[b];
       d.hbar = hbar[b];
-      d.packed = hcol(packd, b);
+      d.packed = lattice.v.a ? packd : hcol(packd, b);
+      d.cols = lattice.v.a ? lattice_cols(B) : 0;
+      d.col = b;
+      d.nonfinite = nonfinite;
       d.grad_ms = grad_ms + (size_t)b * n;
       d.hext_part = hext_part + (size_t)b * nblocks() * 3;
       for (int c = 0; c < 3; ++c) d.hext[c] = hext[b * 3 + c];
@@ -474,6 +504,9 @@ struct Rk4 {
     if (rc) return rc;
     std::vector<FinishDesc> fd(B);
     for (int b = 0; b < B; ++b) {
+      std::memset(&fd[b], 0, sizeof(fd[b]));
+      fd[b].nsplit = nsplit;
+      fd[b].split_stride = (int64_t)B * n3();
       fd[b].mbar = mbar[b];
       fd[b].hbar = hbar[b];
       fd[b].T = hcol(hbuf, b);
@@ -622,20 +655,43 @@ int mt_rk4_create(const mt_micromag_problem* q, double dt, long long nsteps, int
   MT_HIP(hipStreamCreateWithFlags(&P.stream, hipStreamNonBlocking));
   // tensor (FP32, receiver-major) from the assembly kernel or the caller
   const size_t nn = (size_t)n * n;
-  if (P.fp64) MT_HIP(hipMalloc(&P.K64, 6 * nn * sizeof(double)));
-  else MT_HIP(hipMalloc(&P.K32, 6 * nn * sizeof(float)));
+  std::vector<double> axes[3];
+  {
+    auto axis = [](int m, double L, double d, int i) { return m > 1 ? -L / 2 + i * d + d / 2 : 0.0; };
+    for (int i = 0; i < P.nx; ++i) axes[0].push_back(axis(P.nx, q->Lx, dx, i));
+    for (int i = 0; i < P.ny; ++i) axes[1].push_back(axis(P.ny, q->Ly, dy, i));
+    for (int i = 0; i < P.nz; ++i) axes[2].push_back(axis(P.nz, q->Lz, dz, i));
+  }
+  bool lattice = false;
+  if (!P.fp64 && !q->K_in && lattice_pays(n, P.B)) {
+    size_t free_b = 0, total_b = 0;
+    MT_HIP(hipMemGetInfo(&free_b, &total_b));
+    const double d[3] = {dx, dy, dz};
+    if (6.0 * nn * sizeof(float) < (double)total_b) {  // a problem too large for the device stays refused
+      int rc = P.lattice.build(P.nx, P.ny, P.nz, axes[0], axes[1], axes[2], d, P.stream, &lattice);
+      if (rc) return rc;
+    }
+  }
+  if (lattice) {
+    P.nsplit = lattice_nsplit(n);
+    MT_HIP(hipMalloc(&P.nonfinite, sizeof(int)));
+    MT_HIP(hipMemsetAsync(P.nonfinite, 0, sizeof(int), P.stream));
+  } else if (P.fp64) {
+    MT_HIP(hipMalloc(&P.K64, 6 * nn * sizeof(double)));
+  } else {
+    MT_HIP(hipMalloc(&P.K32, 6 * nn * sizeof(float)));
+  }
   if (q->K_in) {
     MT_HIP(hipMemcpyAsync(P.K32, q->K_in, 6 * nn * sizeof(float), hipMemcpyHostToDevice, P.stream));
-  } else {
+  } else if (!lattice) {
     std::vector<double> pts((size_t)n * 3);
-    auto axis = [](int m, double L, double d, int i) { return m > 1 ? -L / 2 + i * d + d / 2 : 0.0; };
     for (int k = 0; k < P.nz; ++k)
       for (int j = 0; j < P.ny; ++j)
         for (int i = 0; i < P.nx; ++i) {
           size_t ind = (size_t)i + (size_t)j * P.nx + (size_t)k * P.nx * P.ny;
-          pts[ind * 3] = axis(P.nx, q->Lx, dx, i);
-          pts[ind * 3 + 1] = axis(P.ny, q->Ly, dy, j);
-          pts[ind * 3 + 2] = axis(P.nz, q->Lz, dz, k);
+          pts[ind * 3] = axes[0][i];
+          pts[ind * 3 + 1] = axes[1][j];
+          pts[ind * 3 + 2] = axes[2][k];
         }
     double *dp = nullptr, *da = nullptr;
     double abc[3] = {dx, dy, dz};
@@ -682,8 +738,9 @@ int mt_rk4_create(const mt_micromag_problem* q, double dt, long long nsteps, int
   P.grid.jfact = P.jfact; P.grid.kfact = P.kfact; P.grid.ms32 = P.ms32; P.grid.ms64 = P.ms64;
   P.grid.aniso = P.aniso;
   P.nck = (int)((nsteps + P.ck - 1) / P.ck);
-  MT_HIP(hipMalloc(&P.packd, (size_t)P.B * N3 * P.es));
-  MT_HIP(hipMalloc(&P.hbuf, (size_t)P.B * N3 * P.es));
+  MT_HIP(hipMalloc(&P.packd, lattice ? (size_t)lattice_state_floats(n, lattice_cols(P.B)) * P.es
+                                     : (size_t)P.B * N3 * P.es));
+  MT_HIP(hipMalloc(&P.hbuf, (size_t)P.nsplit * P.B * N3 * P.es));
   MT_HIP(hipMalloc(&P.ckpt, (size_t)P.nck * P.B * N3 * sizeof(double)));
   MT_HIP(hipMalloc(&P.seg, (size_t)(P.ck + 1) * P.B * 5 * N3 * sizeof(double)));
   MT_HIP(hipMalloc(&P.segS, (size_t)P.ck * 4 * P.B * N3 * P.es));

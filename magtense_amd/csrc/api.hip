@@ -88,11 +88,6 @@ __global__ void transpose_kernel(const float* __restrict__ T, int n, float* __re
   }
 }
 
-__global__ void scale_kernel(float* __restrict__ h, int64_t total, float pref) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < total) h[t] *= pref;
-}
-
 // streaming kernels used to measure the achievable HBM bandwidth on the device
 // Streaming read: four independent 16-byte non-temporal loads per thread per
 // iteration (the fastest form measured on the MI355X: ~6.5-6.9 TB/s on 16 GiB
@@ -155,14 +150,7 @@ void set_error(const std::string& msg) { g_error = msg; }
 const char* last_error() { return g_error.c_str(); }
 
 int demag_apply_f32(const float* K32, int n, const float* m, float* h, int nstates, float pref, hipStream_t st) {
-  int rc = launch_matvec_f32(K32, n, m, (int64_t)3 * n, h, (int64_t)3 * n, nstates, st);
-  if (rc) return rc;
-  if (pref != 1.0f) {
-    int64_t total = (int64_t)nstates * 3 * n;
-    hipLaunchKernelGGL(scale_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, h, total, pref);
-    MT_HIP(hipGetLastError());
-  }
-  return kOk;
+  return launch_matvec_f32(K32, n, m, (int64_t)3 * n, h, (int64_t)3 * n, nstates, pref, st);
 }
 
 }  // namespace mt
@@ -502,7 +490,7 @@ int mt_ll_rhs(int nx, int ny, int nz, double Lx, double Ly, double Lz, const dou
   MT_HIP(hipMemcpy(dvd, vd.data(), nstates * sizeof(VecDesc), hipMemcpyHostToDevice));
   PackSpec pk{kPackF32, mf, n3, nullptr};
   rc = launch_vec(dvd, nstates, n, nullptr, nullptr, pk, false, nullptr);
-  if (rc == kOk) rc = launch_matvec_f32(K32, n, mf, n3, hb, n3, nstates, nullptr);
+  if (rc == kOk) rc = launch_matvec_f32(K32, n, mf, n3, hb, n3, nstates, 1.0f, nullptr);
   if (rc == kOk) {
     std::vector<LlgDesc> ld(nstates);
     for (int s = 0; s < nstates; ++s) {

@@ -1,0 +1,584 @@
+// FP32 demag product of a uniform grid from its distinct tensor entries.
+//
+// The dense FP32 tensor of an nx x ny x nz grid holds K(p_i - p_j) for every
+// pair of cells.  The differences repeat: along each axis there are 2n - 1
+// cell offsets, and the rounding of the cell centres gives each of them a few
+// FP64 values (4 on average on a 128-cell axis).  LatticeTable stores the
+// tensor once per distinct triple of differences, evaluated from the same FP64
+// arguments as the dense assembly, and index maps from cell pairs to entries:
+// the same FP32 entries in 4.4 MB instead of 402.7 MB for 128 x 32 x 1, 72 MB
+// instead of 25.8 GB for 256 x 64 x 2.
+//
+// Product: the sums of matvec_rows_f32 (matvec_rows.h), bit for bit.  There a
+// receiver row is summed by 256 threads, thread T taking the column quads
+// 4T + 1024 k in order of k ("chain" T; single columns T + 256 k when n % 4),
+// then a shuffle tree over each wave's 64 chains and the four waves in order.
+// Here a lane is a receiver and walks whole chains, so that the states' values
+// are wave-uniform (scalar loads) and the entries come from LDS.
+
+#include <algorithm>
+#include <cfloat>
+#include <type_traits>
+#include <vector>
+
+#include "matvec_rows.h"
+#include "mt_common.h"
+#include "mt_kernels.h"
+
+namespace mt {
+
+namespace {
+
+constexpr int kLatThreads = 1024;
+constexpr int kLatLds = 160 * 1024;   // LDS of a CU
+constexpr int kLatMaxRows = 4096;     // source rows x receiver rows of a tile
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// Asynchronous 16-byte-per-lane copy global -> LDS, lane l's bytes at lds +
+// 16 l (see the GEMM kernels, demag.hip); completion by vmcnt.
+__device__ inline void lat_dma16(const void* src, uint32_t lds) {
+  uint32_t saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0"
+      : "=&s"(saved)
+      : "v"(src), "s"(__builtin_amdgcn_readfirstlane(lds))
+      : "memory");
+}
+
+// Receiver tile of a workgroup: 64 lanes over one grid row (nx >= 64), or over
+// rr = 64 / nx whole rows.
+struct LatTile {
+  int rr, per_row, count;
+};
+__host__ __device__ inline LatTile lat_tiles(int nx, int rows) {
+  LatTile t;
+  t.rr = nx >= 64 ? 1 : 64 / nx;
+  t.per_row = nx >= 64 ? (nx + 63) / 64 : 1;
+  t.count = t.per_row * ((rows + t.rr - 1) / t.rr);
+  return t;
+}
+
+// LDS of a workgroup: the x map of its receivers, the table row of every
+// (receiver row, source row), nbuf buffers of table rows.  A step's columns
+// are one run of 256 (QC 4) or four of 64 (QC 1).
+struct LatLds {
+  int pmap, rowidx, touched, slabs, buf_a, buf, total;
+};
+__host__ __device__ inline LatLds lat_lds(const LatticeView& v, int qc, int nbuf) {
+  LatLds L;
+  const int rows = v.ny * v.nz;
+  const LatTile t = lat_tiles(v.nx, rows);
+  const int run = 64 * qc;
+  // grid rows that a run touches (it starts at a multiple of its length)
+  const int most = run % v.nx == 0 ? run / v.nx : (v.nx % run == 0 ? 1 : (run + v.nx - 2) / v.nx + 1);
+  L.touched = std::min(rows, most);
+  L.slabs = t.rr * L.touched * (4 / qc);
+  L.pmap = (v.nx + 3) / 4 * 512;
+  L.rowidx = (rows * t.rr * 4 + 15) / 16 * 16;
+  L.buf_a = L.slabs * v.ux * 16;
+  L.buf = L.buf_a + (v.b ? L.slabs * v.ux * 8 : 0);
+  L.total = L.pmap + L.rowidx + nbuf * L.buf;
+  return L;
+}
+
+// Workgroup (tile, w, state group): the chains 64 w .. 64 w + 63 of the tile's
+// receivers for SB states, lane = receiver.  Wave r takes the four chains r +
+// 16 c, which the shuffle tree joins first (lane xor 32, 16).  The columns go
+// in steps of 1024, four to a chain ("quad"): 4 T + q for chain T (QC 4), T +
+// 256 q (QC 1); the states lie quad by quad (lattice_state_offset).  Per step
+// the table rows of the workgroup's columns are copied to LDS one step ahead
+// (nbuf 2); a pair then costs a lane 2 bytes of the x map and 16 bytes (xx,
+// xy, yy, zz) of LDS reads, 8 more for (xz, yz) between planes.  Those are +-0
+// within a plane, where their products, which add +-0 to sums that are never
+// -0, are left out unless *nonfinite says that a state holds an infinity or a
+// NaN.
+template <int QC, bool HASB, bool ALIGNED, int SB>
+__global__ void __launch_bounds__(kLatThreads)
+    lattice_rows_kernel(const LatticeView v, const float* __restrict__ m, int cols, float* __restrict__ out,
+                        int64_t split_stride, int64_t col_stride, int nstates, int nbuf,
+                        const int* __restrict__ nonfinite) {
+  extern __shared__ __align__(16) uint8_t lat_smem[];
+  constexpr int kWaves = kLatThreads / 64, CH = 64 / kWaves;  // chains of a wave
+  static_assert(kWaves == 16 && CH == 4, "the order of the final sums");
+  const int lane = threadIdx.x & 63;
+  const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nx = v.nx, ny = v.ny, rows = v.ny * v.nz, n = nx * rows;
+  const LatTile T = lat_tiles(nx, rows);
+  const LatLds L = lat_lds(v, QC, nbuf);
+  const int tile = blockIdx.x, w = blockIdx.y, s0 = blockIdx.z * SB;
+  const int row0 = tile / T.per_row * T.rr, ix0 = tile % T.per_row * 64;
+  const int rho = nx >= 64 ? 0 : std::min(lane / nx, T.rr - 1);
+  const int ix = std::min(nx >= 64 ? ix0 + lane : lane - rho * nx, nx - 1);
+  const bool lane_ok = (nx >= 64 ? ix0 + lane < nx : lane < T.rr * nx) && row0 + rho < rows;
+  uint16_t* pmap = reinterpret_cast<uint16_t*>(lat_smem);  // [jx / 4][lane][jx % 4]
+  int* rowidx = reinterpret_cast<int*>(lat_smem + L.pmap);
+  uint8_t* bufs = lat_smem + L.pmap + L.rowidx;
+  const bool all = *nonfinite != 0;  // no product is left out
+
+  // source rows [plane_lo, plane_hi) lie in the one plane of the tile's receivers
+  const int plane0 = row0 / ny, plane1 = (std::min(row0 + T.rr, rows) - 1) / ny;
+  const int plane_lo = plane0 * ny, plane_hi = plane0 == plane1 ? plane_lo + ny : plane_lo;
+  constexpr int RUN = 64 * QC, NRUN = 4 / QC;
+  // first column of run g of the step at `base`
+  auto run_at = [&](int base, int g) { return base + RUN * w + (NRUN == 1 ? 0 : 256 * g); };
+  // every source row of the step against the tile: only xx, xy, yy, zz
+  auto flat_step = [&](int base) {
+    if (all) return false;
+    if (!HASB) return true;
+    const int lo = run_at(base, 0), hi = std::min(run_at(base, NRUN - 1) + RUN, n) - 1;
+    return lo / nx >= plane_lo && hi / nx < plane_hi;
+  };
+  // table row of receiver row q of the tile against source row j
+  auto table_row = [&](int q, int j) {
+    const int i = std::min(row0 + q, rows - 1);
+    return v.zmap[i / ny * v.nz + j / ny] * v.uy + v.ymap[i % ny * ny + j % ny];
+  };
+  // table rows of the step at `base` into buffer b; the first step looks them
+  // up itself, so that its copies run while the maps are filled
+  auto stage = [&](auto first, int base, int b) {
+    constexpr bool FIRST = decltype(first)::value;
+    uint8_t* A = bufs + (size_t)b * L.buf;
+    const uint32_t la = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)A;
+    const int pa = (v.ux + 63) / 64;
+    const int hx = v.ux / 2, pb = (hx + 63) / 64;  // (xz, yz): two entries per lane
+    const bool with_b = HASB && !flat_step(base);
+#pragma unroll
+    for (int g = 0; g < NRUN; ++g) {
+      const int c0 = run_at(base, g), c1 = std::min(c0 + RUN, n);
+      if (c0 >= n) break;
+      const int ra = c0 / nx, nr = (c1 - 1) / nx - ra + 1, slab0 = g * L.touched * T.rr;
+      for (int p = r; p < nr * T.rr * pa; p += kWaves) {
+        const int slab = p / pa, o = (p - slab * pa) * 64;  // slab = source row x rr + receiver row
+        const int sr = slab / T.rr, q = slab - sr * T.rr;
+        const int64_t src =
+            (int64_t)__builtin_amdgcn_readfirstlane(FIRST ? table_row(q, ra + sr) : rowidx[q * rows + ra + sr]) * v.ux +
+            o + lane;
+        if (o + lane < v.ux) lat_dma16(v.a + src * 4, la + (uint32_t)((slab0 + slab) * v.ux + o) * 16);
+      }
+      if (with_b)
+        for (int p = r; p < nr * T.rr * pb; p += kWaves) {
+          const int slab = p / pb, o = (p - slab * pb) * 64;
+          const int sr = slab / T.rr, q = slab - sr * T.rr;
+          const int64_t src =
+              (int64_t)__builtin_amdgcn_readfirstlane(FIRST ? table_row(q, ra + sr) : rowidx[q * rows + ra + sr]) * hx +
+              o + lane;
+          if (o + lane < hx)
+            lat_dma16(v.b + src * 4, la + (uint32_t)L.buf_a + (uint32_t)((slab0 + slab) * hx + o) * 16);
+        }
+    }
+  };
+
+  float acc[CH][SB][3];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int s = 0; s < SB; ++s) acc[c][s][0] = acc[c][s][1] = acc[c][s][2] = 0.0f;
+  // the states through the constant address space: uniform reads become scalar
+  // loads whatever the copies' memory clobbers
+  typedef const __attribute__((address_space(4))) float* const_floats;
+  const const_floats ms = (const_floats)(m + (size_t)s0 * 12);
+
+  struct Entries {
+    f32x4 a[4];
+    f32x2 b[4];
+  };
+  constexpr int SH = SB < 2 ? SB : 2;  // states in scalar registers at a time
+  struct States {
+    float x[SH][4], y[SH][4], z[SH][4];
+  };
+  // place of a quad's columns: x in their grid rows, first entry of the rows in the buffer
+  struct Place {
+    int jx[4], row[4];
+  };
+  auto advance = [&](Place& p) {  // to the wave's next chain
+#pragma unroll
+    for (int q = 0; q < (ALIGNED && QC == 4 ? 1 : 4); ++q) {
+      p.jx[q] += QC * kWaves;
+      while (p.jx[q] >= nx) {
+        p.jx[q] -= nx;
+        p.row[q] += T.rr * v.ux;
+      }
+    }
+  };
+  auto read_entries = [&](auto flat, Entries& k, const uint8_t* A, const Place& p, int have) {
+    constexpr bool FLAT = decltype(flat)::value;
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    u16x4 x4;
+    if (ALIGNED && QC == 4) x4 = *reinterpret_cast<const u16x4*>(pmap + (p.jx[0] >> 2) * 256 + lane * 4);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (QC == 1 && q >= have) continue;
+      int e;
+      if (ALIGNED && QC == 4) e = p.row[0] + rho * v.ux + x4[q];
+      else e = p.row[q] + rho * v.ux + pmap[(p.jx[q] >> 2) * 256 + lane * 4 + (p.jx[q] & 3)];
+      k.a[q] = *reinterpret_cast<const f32x4*>(A + (size_t)e * 16);
+      if (!FLAT) k.b[q] = HASB ? *reinterpret_cast<const f32x2*>(A + L.buf_a + (size_t)e * 8) : f32x2{0.0f, 0.0f};
+    }
+  };
+  auto read_states = [&](States& t, const_floats f) {
+#pragma unroll
+    for (int s = 0; s < SH; ++s)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        t.x[s][q] = f[s * 12 + q];
+        t.y[s][q] = f[s * 12 + 4 + q];
+        t.z[s][q] = f[s * 12 + 8 + q];
+      }
+  };
+  // states SH h .. SH h + SH - 1
+  auto add = [&](auto flat, float (&a)[SB][3], int h, const Entries& k, const States& t, int have) {
+    constexpr bool FLAT = decltype(flat)::value;
+#pragma unroll
+    for (int s = 0; s < SH; ++s) {
+      float(&as)[3] = a[SH * h + s];
+      if (QC == 4) {
+        if (FLAT) matvec_flat<4>(k.a, t.x[s], t.y[s], t.z[s], as);
+        else matvec_full<4>(k.a, k.b, t.x[s], t.y[s], t.z[s], as);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (q >= have) continue;
+          const f32x4 ka[1] = {k.a[q]};
+          const f32x2 kb[1] = {k.b[q]};
+          const float x[1] = {t.x[s][q]}, y[1] = {t.y[s][q]}, z[1] = {t.z[s][q]};
+          if (FLAT) matvec_flat<1>(ka, x, y, z, as);
+          else matvec_full<1>(ka, kb, x, y, z, as);
+        }
+      }
+    }
+  };
+  // the step at `base`: the entries of the next chain and the states of the
+  // next sums are read before a chain's (state pair's) sums
+  const int64_t chain_floats = (int64_t)kWaves * cols * 12;
+  auto compute = [&](auto flat, auto whole, int base, int b) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    const uint8_t* A = bufs + (size_t)b * L.buf;
+    Place p;
+#pragma unroll
+    for (int q = 0; q < (ALIGNED && QC == 4 ? 1 : 4); ++q) {
+      const int g = QC == 4 ? 0 : q;
+      const int c0 = run_at(base, g), ra = c0 / nx;
+      const int j = QC == 4 ? c0 + 4 * r + q : c0 + r;
+      const int row = j / nx;
+      p.jx[q] = j - row * nx;
+      p.row[q] = (g * L.touched + row - ra) * T.rr * v.ux;
+    }
+    const_floats f = ms + (int64_t)(base / 4 + 64 * w + r) * cols * 12;
+    if (WHOLE) {
+      Entries k[2];
+      States t[2];
+      read_entries(flat, k[0], A, p, 4);
+      read_states(t[0], f);
+#pragma unroll
+      for (int u = 0; u < CH * (SB / SH); ++u) {
+        const int c = u / (SB / SH), h = u % (SB / SH);
+        if (h == 0 && c + 1 < CH) {
+          advance(p);
+          read_entries(flat, k[(c + 1) & 1], A, p, 4);
+        }
+        if (u + 1 < CH * (SB / SH)) {
+          if (h + 1 == SB / SH) f += chain_floats - 12 * SH * (SB / SH - 1);
+          else f += 12 * SH;
+          read_states(t[(u + 1) & 1], f);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        add(flat, acc[c], h, k[c & 1], t[u & 1], 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        // QC 4: all of the quad's columns exist or none; QC 1: the first `have`
+        const int j = run_at(base, 0) + QC * (r + kWaves * c);
+        const int have = QC == 4 ? (j < n ? 4 : 0) : (j < n ? std::min(4, (n - 1 - j) / 256 + 1) : 0);
+        if (have > 0) {
+          Entries k;
+          read_entries(flat, k, A, p, have);
+#pragma unroll
+          for (int h = 0; h < SB / SH; ++h) {
+            States t;
+            read_states(t, f + 12 * SH * h);
+            add(flat, acc[c], h, k, t, have);
+          }
+        }
+        advance(p);
+        f += chain_floats;
+      }
+    }
+  };
+
+  stage(std::true_type{}, 0, 0);
+  for (int jx = r; jx < nx; jx += kWaves) pmap[(jx >> 2) * 256 + lane * 4 + (jx & 3)] = v.pmap[jx * nx + ix];
+  for (int e = threadIdx.x; e < rows * T.rr; e += kLatThreads) {
+    const int q = e / rows;
+    rowidx[e] = table_row(q, e - q * rows);
+  }
+  int b = 0;
+  for (int base = 0; run_at(base, 0) < n; base += 1024) {
+    if (nbuf == 1 && base > 0) {
+      __syncthreads();  // the previous step's reads
+      stage(std::false_type{}, base, 0);
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // my copies, my reads of the other buffer
+    __syncthreads();
+    if (nbuf == 2 && run_at(base + 1024, 0) < n) stage(std::false_type{}, base + 1024, b ^ 1);
+    const bool whole = run_at(base, NRUN - 1) + RUN <= n;
+    if (flat_step(base)) {
+      if (whole) compute(std::true_type{}, std::true_type{}, base, b);
+      else compute(std::true_type{}, std::false_type{}, base, b);
+    } else {
+      if (whole) compute(std::false_type{}, std::true_type{}, base, b);
+      else compute(std::false_type{}, std::false_type{}, base, b);
+    }
+    b ^= nbuf - 1;
+  }
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+
+  // chains r + 16 c of this wave in the shuffle tree's order (xor 32, 16), then
+  // the waves (xor 8, 4, 2, 1)
+  float* part = reinterpret_cast<float*>(bufs);  // [wave][s][component][lane]
+#pragma unroll
+  for (int s = 0; s < SB; ++s)
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      part[((r * SB + s) * 3 + a) * 64 + lane] =
+          (acc[0][s][a] + acc[2][s][a]) + (acc[1][s][a] + acc[3][s][a]);
+  __syncthreads();
+  for (int e = r; e < SB * 3; e += kWaves) {
+    const int s = e / 3, a = e - s * 3;
+    if (!lane_ok || s0 + s >= nstates) continue;
+    float t[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) t[q] = part[((q * SB + s) * 3 + a) * 64 + lane];
+#pragma unroll
+    for (int h = 8; h > 0; h >>= 1)
+#pragma unroll
+      for (int q = 0; q < h; ++q) t[q] += t[q + h];
+    out[(int64_t)w * split_stride + (int64_t)(s0 + s) * col_stride + (int64_t)a * n + (int64_t)(row0 + rho) * nx + ix] =
+        t[0];
+  }
+}
+
+// same[k] = 0 where x difference W + k (of offset owner[k]) and the commonest
+// one of its offset have different entries in some row: blocks (k, rows).
+__global__ void __launch_bounds__(256) lattice_same_kernel(const uint4* __restrict__ a, const uint2* __restrict__ b,
+                                                           int ux, int rows, int W, const int* __restrict__ owner,
+                                                           int* __restrict__ same) {
+  const int k = blockIdx.x, u = W + k, o = owner[k];
+  bool eq = true;
+  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
+    const uint4 p = a[(size_t)r * ux + u], q = a[(size_t)r * ux + o];
+    eq = eq && p.x == q.x && p.y == q.y && p.z == q.z && p.w == q.w;
+    if (b) {
+      const uint2 e = b[(size_t)r * ux + u], f = b[(size_t)r * ux + o];
+      eq = eq && e.x == f.x && e.y == f.y;
+    }
+  }
+  if (!eq) same[k] = 0;
+}
+
+// Distinct values of c[i] - c[j], the commonest value of each offset first:
+// value u < 2 m - 1 belongs to offset u - (m - 1), the others follow offset by
+// offset, so that the lanes of a row read neighbouring entries.  map[j * m + i]
+// is the value of the pair.
+void distinct_differences(const std::vector<double>& c, std::vector<double>& values, std::vector<int>& map) {
+  const int m = (int)c.size(), W = 2 * m - 1;
+  values.assign(W, 0.0);
+  map.assign((size_t)m * m, 0);
+  std::vector<double> seen;
+  std::vector<int> count, id;
+  for (int o = 0; o < W; ++o) {
+    const int d = o - (m - 1);  // i - j
+    const int j0 = std::max(0, -d), j1 = std::min(m, m - d);
+    seen.clear();
+    count.clear();
+    for (int j = j0; j < j1; ++j) {
+      const double x = c[j + d] - c[j];
+      size_t k = 0;
+      while (k < seen.size() && seen[k] != x) ++k;
+      if (k == seen.size()) {
+        seen.push_back(x);
+        count.push_back(0);
+      }
+      count[k] += 1;
+      map[(size_t)j * m + j + d] = (int)k;
+    }
+    const int top = (int)(std::max_element(count.begin(), count.end()) - count.begin());
+    id.assign(seen.size(), 0);
+    for (size_t k = 0; k < seen.size(); ++k) {
+      if ((int)k == top) {
+        id[k] = o;
+        values[o] = seen[k];
+      } else {
+        id[k] = (int)values.size();
+        values.push_back(seen[k]);
+      }
+    }
+    for (int j = j0; j < j1; ++j) map[(size_t)j * m + j + d] = id[map[(size_t)j * m + j + d]];
+  }
+}
+
+template <int QC, bool HASB, bool ALIGNED>
+int launch_rows(const LatticeView& v, const float* m, int cols, float* out, int64_t split_stride, int64_t col_stride,
+                int nstates, const int* nonfinite, hipStream_t stream) {
+  const int nbuf = lat_lds(v, QC, 2).total <= kLatLds ? 2 : 1;
+  const LatTile T = lat_tiles(v.nx, v.ny * v.nz);
+  const int nw = lattice_nsplit(v.nx * v.ny * v.nz);
+  auto go = [&](auto sb) {
+    constexpr int SB = decltype(sb)::value;
+    const size_t lds = std::max<size_t>(lat_lds(v, QC, nbuf).total,
+                                        lat_lds(v, QC, 0).total + (size_t)kLatThreads * SB * 3 * sizeof(float));
+    const dim3 grid((unsigned)T.count, (unsigned)nw, (unsigned)((nstates + SB - 1) / SB));
+    hipLaunchKernelGGL((lattice_rows_kernel<QC, HASB, ALIGNED, SB>), grid, dim3(kLatThreads), lds, stream, v, m, cols,
+                       out, split_stride, col_stride, nstates, nbuf, nonfinite);
+  };
+  if (nstates == 1) go(std::integral_constant<int, 1>{});
+  else if (nstates == 2) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
+  MT_HIP(hipGetLastError());
+  return kOk;
+}
+
+}  // namespace
+
+int lattice_nsplit(int n) {
+  const int width = n % 4 == 0 ? 256 : 64;
+  return std::min(4, (n + width - 1) / width);
+}
+
+void LatticeTable::release() {
+  auto f = [](void* p) {
+    if (p) (void)hipFree(p);
+  };
+  f(a); f(b); f(pmap); f(ymap); f(zmap);
+  a = b = nullptr;
+  pmap = nullptr;
+  ymap = zmap = nullptr;
+  v = LatticeView{};
+}
+
+int LatticeTable::build(int nx, int ny, int nz, const std::vector<double>& cx, const std::vector<double>& cy,
+                        const std::vector<double>& cz, const double d[3], hipStream_t stream, bool* fits) {
+  release();
+  *fits = false;
+  if (nx < 16 || nx > 1024 || (int64_t)ny * nz * lat_tiles(nx, ny * nz).rr > kLatMaxRows) return kOk;
+  std::vector<double> val[3];
+  std::vector<int> map[3];
+  distinct_differences(cx, val[0], map[0]);
+  if (val[0].size() % 2) {  // rows of whole 16-byte pieces; an entry that no pair has
+    val[0].push_back(val[0][0]);
+  }
+  if (val[0].size() > 65535) return kOk;
+  LatticeView q{};
+  q.nx = nx; q.ny = ny; q.nz = nz;
+  q.ux = (int)val[0].size();
+  if (nz > 1) q.b = reinterpret_cast<const float*>(sizeof(float));  // any non-null: the layout with (xz, yz)
+  if (lat_lds(q, nx * ny * nz % 4 == 0 ? 4 : 1, 1).total > kLatLds) return kOk;
+  distinct_differences(cy, val[1], map[1]);
+  distinct_differences(cz, val[2], map[2]);
+  q.uy = (int)val[1].size();
+  const int64_t entries = (int64_t)val[0].size() * val[1].size() * val[2].size();
+  const int64_t n = (int64_t)nx * ny * nz;
+  if (entries > n * n / 8) return kOk;
+  // the kernel looks rows up by receiver, then source
+  auto by_receiver = [](const std::vector<int>& t, int m) {
+    std::vector<int> o(t.size());
+    for (int j = 0; j < m; ++j)
+      for (int i = 0; i < m; ++i) o[(size_t)i * m + j] = t[(size_t)j * m + i];
+    return o;
+  };
+  const std::vector<int> ym = by_receiver(map[1], ny), zm = by_receiver(map[2], nz);
+  const int W = 2 * nx - 1, extra = (int)val[0].size() - W;
+  DevArr<double> dv[3];
+  for (int k = 0; k < 3; ++k) {
+    MT_HIP(dv[k].alloc(val[k].size()));
+    MT_HIP(hipMemcpyAsync(dv[k].p, val[k].data(), val[k].size() * sizeof(double), hipMemcpyHostToDevice, stream));
+  }
+  auto entries_of = [&](const std::vector<double>& x) -> int {
+    const int64_t cnt = (int64_t)x.size() * val[1].size() * val[2].size();
+    MT_HIP(hipMalloc(&a, (size_t)cnt * 4 * sizeof(float)));
+    if (nz > 1) MT_HIP(hipMalloc(&b, (size_t)cnt * 2 * sizeof(float)));
+    return launch_lattice_entries(dv[0].p, (int)x.size(), dv[1].p, (int)val[1].size(), dv[2].p, (int)val[2].size(), d,
+                                  a, b, stream);
+  };
+  int rc = entries_of(val[0]);
+  if (rc) return rc;
+  // x differences whose entries all equal those of their offset's commonest
+  // one are the same column of the table: 997 -> 316 columns at 128 x 32 x 1
+  std::vector<int> owner(std::max(extra, 1), 0), same(std::max(extra, 1), 1);
+  for (int j = 0; j < nx; ++j)
+    for (int i = 0; i < nx; ++i) {
+      const int u = map[0][(size_t)j * nx + i];
+      if (u >= W) owner[u - W] = i - j + nx - 1;
+    }
+  if (extra > 0) {
+    DevArr<int> downer, dsame;
+    MT_HIP(downer.alloc(extra));
+    MT_HIP(dsame.alloc(extra));
+    MT_HIP(hipMemcpyAsync(downer.p, owner.data(), extra * sizeof(int), hipMemcpyHostToDevice, stream));
+    MT_HIP(hipMemcpyAsync(dsame.p, same.data(), extra * sizeof(int), hipMemcpyHostToDevice, stream));
+    hipLaunchKernelGGL(lattice_same_kernel, dim3((unsigned)extra), dim3(256), 0, stream,
+                       reinterpret_cast<const uint4*>(a), reinterpret_cast<const uint2*>(b), q.ux,
+                       (int)(val[1].size() * val[2].size()), W, downer.p, dsame.p);
+    MT_HIP(hipGetLastError());
+    MT_HIP(hipMemcpyAsync(same.data(), dsame.p, extra * sizeof(int), hipMemcpyDeviceToHost, stream));
+    MT_HIP(hipStreamSynchronize(stream));
+    std::vector<double> x(val[0].begin(), val[0].begin() + W);
+    std::vector<int> to(extra);
+    for (int k = 0; k < extra; ++k) {
+      to[k] = same[k] ? owner[k] : (int)x.size();
+      if (!same[k]) x.push_back(val[0][W + k]);
+    }
+    if (x.size() % 2) x.push_back(x[0]);
+    if (x.size() < val[0].size()) {
+      for (int& u : map[0])
+        if (u >= W) u = to[u - W];
+      release();
+      q.ux = (int)x.size();
+      MT_HIP(hipMemcpyAsync(dv[0].p, x.data(), x.size() * sizeof(double), hipMemcpyHostToDevice, stream));
+      rc = entries_of(x);
+      if (rc) return rc;
+      MT_HIP(hipStreamSynchronize(stream));  // x leaves scope
+    }
+  }
+  const std::vector<uint16_t> pm(map[0].begin(), map[0].end());
+  MT_HIP(hipMalloc(&pmap, pm.size() * sizeof(uint16_t)));
+  MT_HIP(hipMalloc(&ymap, ym.size() * sizeof(int)));
+  MT_HIP(hipMalloc(&zmap, zm.size() * sizeof(int)));
+  MT_HIP(hipMemcpyAsync(pmap, pm.data(), pm.size() * sizeof(uint16_t), hipMemcpyHostToDevice, stream));
+  MT_HIP(hipMemcpyAsync(ymap, ym.data(), ym.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+  MT_HIP(hipMemcpyAsync(zmap, zm.data(), zm.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+  MT_HIP(hipStreamSynchronize(stream));
+  q.a = a; q.b = b; q.pmap = pmap; q.ymap = ymap; q.zmap = zmap;
+  v = q;
+  *fits = true;
+  return kOk;
+}
+
+int launch_lattice_rows(const LatticeView& v, const float* m, int cols, float* out, int64_t split_stride,
+                        int64_t col_stride, int nstates, const int* nonfinite, hipStream_t stream) {
+  const int n = v.nx * v.ny * v.nz;
+  if (nstates < 1 || nstates > 65535 || !v.a || cols % 4 || cols < nstates) {
+    set_error("lattice product: no table, states outside 1..65535, or a state layout of the wrong width");
+    return kErrArg;
+  }
+  auto by_b = [&](auto qc, auto aligned) {
+    constexpr int QC = decltype(qc)::value;
+    constexpr bool AL = decltype(aligned)::value;
+    return v.b ? launch_rows<QC, true, AL>(v, m, cols, out, split_stride, col_stride, nstates, nonfinite, stream)
+               : launch_rows<QC, false, AL>(v, m, cols, out, split_stride, col_stride, nstates, nonfinite, stream);
+  };
+  if (n % 4) return by_b(std::integral_constant<int, 1>{}, std::true_type{});
+  if (v.nx % 4 == 0) return by_b(std::integral_constant<int, 4>{}, std::true_type{});
+  return by_b(std::integral_constant<int, 4>{}, std::false_type{});
+}
+
+}  // namespace mt

@@ -17,6 +17,10 @@
 
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
+#include <cfloat>
+#include <type_traits>
+
 #include "llg_cell.h"
 #include "matvec_rows.h"
 #include "mt_common.h"
@@ -55,24 +59,28 @@ __global__ void __launch_bounds__(256) llg_kernel(const LlgGrid g, const LlgDesc
 }
 
 // The FP32 dense path's demag rows and LL right-hand side in one launch:
-// block = kFusedRows receiver rows of state blockIdx.y (the sums of
-// matvec_rows_f32), then one thread per row evaluates llg_cell with them.
-template <bool INL, bool VEC4, int RB>
+// block = RB receiver rows of S states, from s0 on (the sums of matvec_rows_f32),
+// then one thread per row and state evaluates llg_cell with them.
+template <bool INL, bool VEC4, int RB, int S, bool ONE>
 __global__ void __launch_bounds__(256) demag_llg_f32_kernel(const float* __restrict__ K, const LlgGrid g,
                                                             const LlgDesc* __restrict__ descs, LlgDescsInline inl,
-                                                            const float* __restrict__ m32, int64_t m_stride) {
-  const int s = blockIdx.y;
-  const int i0 = blockIdx.x * RB;
-  __shared__ float red[4][RB * 3];
-  __shared__ float sums[RB * 3];
-  matvec_rows_f32<RB, VEC4>(K, g.n, m32 + s * m_stride, i0, red, sums);
-  const int r = threadIdx.x;
-  if (r >= RB || i0 + r >= g.n) return;
-  const LlgDesc& D = INL ? inl.d[s] : descs[s];
+                                                            const float* __restrict__ m32, int64_t m_stride, int s0,
+                                                            int nstates, int groups) {
+  int rows = blockIdx.x, group = 0;
+  if (!ONE) matvec_block(blockIdx.x, groups, rows, group);
+  const int sb = s0 + group * S;
+  const int i0 = rows * RB;
+  if (i0 >= g.n) return;
+  __shared__ float red[4][RB * S * 3];
+  __shared__ float sums[RB * S * 3];
+  matvec_rows_f32<RB, VEC4, S, ONE>(K, g.n, m32 + sb * m_stride, m_stride, nstates - sb, i0, red, sums);
+  const int r = threadIdx.x % RB, s = threadIdx.x / RB;
+  if (s >= S || sb + s >= nstates || i0 + r >= g.n) return;
+  const LlgDesc& D = INL ? inl.d[sb + s] : descs[sb + s];
   // one partial-sum slot: S = 0 + row sum, as the LL kernel forms it
   llg_cell(g, D, i0 + r, [&](int c) {
     float v = 0.0f;
-    v += sums[r * 3 + c];
+    v += sums[(s * RB + r) * 3 + c];
     return v;
   });
 }
@@ -129,7 +137,7 @@ __global__ void __launch_bounds__(256) stage_demag_llg_f32_kernel(const float* _
   }
   __shared__ float red[4][RB * 3];
   __shared__ float sums[RB * 3];
-  matvec_rows_f32<RB, VEC4>(K, n, m32, i0, red, sums);
+  matvec_rows_f32<RB, VEC4, 1>(K, n, m32, 0, 1, i0, red, sums);
   const int r = threadIdx.x;
   if (r >= RB || i0 + r >= n) return;
   LlgDesc D = inl.d[s];
@@ -221,6 +229,17 @@ __global__ void __launch_bounds__(256) vec_kernel(const VecDesc* __restrict__ de
 #pragma unroll
       for (int q = 0; q < kVecE; ++q)
         if (ok[q]) pack.f32[(int64_t)D.pack_col * pack.col_stride + e0 + 256 * q] = (float)v[q];
+    } else if (pack.mode == kPackLattice) {
+      bool bad = false;
+#pragma unroll
+      for (int q = 0; q < kVecE; ++q)
+        if (ok[q]) {
+          const int e = e0 + 256 * q, c = e / n;
+          const float f = (float)v[q];
+          pack.f32[lattice_state_offset(n, (int)pack.col_stride, D.pack_col, c, e - c * n)] = f;
+          bad |= !(fabsf(f) <= FLT_MAX);
+        }
+      if (bad) *pack.nonfinite = 1;
     } else if (pack.mode == kPackF32Frag) {
 #pragma unroll
       for (int q = 0; q < kVecE; ++q)
@@ -478,26 +497,23 @@ int launch_llg_inline(const LlgGrid& g, const LlgDesc* h_descs, int nstates, hip
 }
 
 namespace {
-template <int RB>
-int launch_demag_llg_rb(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDescsInline& inl,
-                        const float* m32, int64_t m_stride, int nstates, hipStream_t stream) {
-  dim3 grid((unsigned)((g.n + RB - 1) / RB), (unsigned)nstates);
+template <int S>
+int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDescsInline& inl,
+                       const float* m32, int64_t m_stride, int s0, int nstates, int groups,
+                       hipStream_t stream) {
+  constexpr int RB = matvec_block_rows(S);
+  const dim3 grid(matvec_blocks((g.n + RB - 1) / RB, groups));
   const bool vec4 = (g.n % 4) == 0 && (m_stride % 4) == 0;
-  if (d_descs) {
-    if (vec4)
-      hipLaunchKernelGGL((demag_llg_f32_kernel<false, true, RB>), grid, dim3(256), 0, stream, K, g, d_descs, inl, m32,
-                         m_stride);
-    else
-      hipLaunchKernelGGL((demag_llg_f32_kernel<false, false, RB>), grid, dim3(256), 0, stream, K, g, d_descs, inl,
-                         m32, m_stride);
-  } else {
-    if (vec4)
-      hipLaunchKernelGGL((demag_llg_f32_kernel<true, true, RB>), grid, dim3(256), 0, stream, K, g, nullptr, inl, m32,
-                         m_stride);
-    else
-      hipLaunchKernelGGL((demag_llg_f32_kernel<true, false, RB>), grid, dim3(256), 0, stream, K, g, nullptr, inl, m32,
-                         m_stride);
-  }
+  auto go = [&](auto by_value, auto v4, auto one) {
+    hipLaunchKernelGGL((demag_llg_f32_kernel<decltype(by_value)::value, decltype(v4)::value, RB, S,
+                                             decltype(one)::value>),
+                       grid, dim3(256), 0, stream, K, g, d_descs, inl, m32, m_stride, s0, nstates, groups);
+  };
+  const std::true_type yes;
+  const std::false_type no;
+  if (!d_descs) vec4 ? go(yes, yes, yes) : go(yes, no, yes);  // by value: one group at a time
+  else if (groups == 1) vec4 ? go(no, yes, yes) : go(no, no, yes);
+  else vec4 ? go(no, yes, no) : go(no, no, no);
   MT_HIP(hipGetLastError());
   return kOk;
 }
@@ -513,9 +529,17 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
     }
     for (int s = 0; s < nstates; ++s) inl.d[s] = h_descs[s];
   }
-  // four receiver rows per block (the 128 x 32 film's 402.7 MB tensor: 2 / 4 / 8
-  // rows -> 72.2 / 66.8 / 114.4 us per launch)
-  return launch_demag_llg_rb<4>(K, g, d_descs, inl, m32, m_stride, nstates, stream);
+  for (int s0 = 0; s0 < nstates;) {
+    const int S = matvec_group(nstates - s0), groups = S == 8 ? std::max(1, std::min((nstates - s0) / 8, 64)) : 1;
+    int rc = kOk;
+    if (S == 8) rc = launch_demag_llg_s<8>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, stream);
+    else if (S == 4) rc = launch_demag_llg_s<4>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
+    else if (S == 2) rc = launch_demag_llg_s<2>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
+    else rc = launch_demag_llg_s<1>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
+    if (rc) return rc;
+    s0 += S * groups;
+  }
+  return kOk;
 }
 
 static_assert(sizeof(StageDescsInline) + sizeof(LlgDescsInline) + sizeof(LlgGrid) + 256 <= 4096,

@@ -18,7 +18,7 @@ namespace mt {
 // returns the FP32 demag sum S_c = sum of the partials of (K m)_c at i (used
 // unless D.hpart64 holds FP64 sums).
 template <typename HS>
-__device__ inline void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, HS hsum) {
+__device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, HS hsum) {
   const int n = g.n;
   const double* m = D.m;
   const int ix = i % g.nx;
@@ -75,6 +75,7 @@ __device__ inline void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, HS hs
   } else {
     for (int c = 0; c < 3; ++c) {
       const float s = hsum(c);
+      if (D.sum_out) D.sum_out[(int64_t)c * n + i] = s;
       float h = (-s) * g.ms32[i];
       hm[c] = (double)h;
     }

@@ -32,10 +32,16 @@ int launch_assemble_tetra(const double* pts, const double* nodes, const int* ele
 int launch_toeplitz_assemble(int nx, int ny, int nz, double Lx, double Ly, double Lz, uint8_t* out,
                              hipStream_t stream);
 
+// Entries of a uniform grid's FP32 tensor at every triple of the given
+// differences (lattice.hip), xfastest: a = (xx, xy, yy, zz), b = (xz, yz, or
+// null), prism edges d.  The values of the dense assembly at those offsets.
+int launch_lattice_entries(const double* x, int ux, const double* y, int uy, const double* z, int uz, const double d[3],
+                           float* a, float* b, hipStream_t stream);
+
 // ---- (b) demag product ------------------------------------------------------------
-// out[s*out_stride + c*n + i] = sum_j K_c.(i,j) m_s,.(j)   (positive K m)
+// out[s*out_stride + c*n + i] = pref * sum_j K_c.(i,j) m_s,.(j)
 int launch_matvec_f32(const float* K, int n, const float* m, int64_t m_stride, float* out, int64_t out_stride,
-                      int nstates, hipStream_t stream);
+                      int nstates, float pref, hipStream_t stream);
 // FP64 form of the same product (FP64 tensor planes and states)
 int launch_matvec_f64(const double* K, int n, const double* m, int64_t m_stride, double* out, int64_t out_stride,
                       int nstates, hipStream_t stream);
@@ -139,6 +145,52 @@ int apply_bf16x2_in(const void* K, int n, int nrows, int nx, int ny, int nz, con
                     const BlockSparseView* bsv = nullptr, bool f32 = false);
 int device_ok();
 
+// FP32 product of a uniform grid from its distinct tensor entries
+// (lattice.hip): the row sums of launch_matvec_f32 over the dense tensor of
+// the same grid, bit for bit.
+struct LatticeView {
+  int nx, ny, nz;
+  int ux, uy;            // distinct x differences (padded to an even number), y differences
+  const float* a;        // entries (xx, xy, yy, zz) at ((uz * uy_count + uy) * ux + x)
+  const float* b;        // (xz, yz); null with one plane, where they are +-0
+  const uint16_t* pmap;  // [jx * nx + ix]: x difference of a pair
+  const int* ymap;       // [iy * ny + jy]
+  const int* zmap;       // [iz * nz + jz]
+};
+struct LatticeTable {
+  LatticeView v{};
+  float *a = nullptr, *b = nullptr;
+  uint16_t* pmap = nullptr;
+  int *ymap = nullptr, *zmap = nullptr;
+  LatticeTable() = default;
+  LatticeTable(const LatticeTable&) = delete;
+  LatticeTable& operator=(const LatticeTable&) = delete;
+  // Builds the table of the grid with cell centres cx, cy, cz and edges d.
+  // *fits: false (and nothing built) where the kernel does not take the grid.
+  int build(int nx, int ny, int nz, const std::vector<double>& cx, const std::vector<double>& cy,
+            const std::vector<double>& cz, const double d[3], hipStream_t stream, bool* fits);
+  void release();
+  ~LatticeTable() { release(); }
+};
+// Whether the product from the table beats the one over the dense tensor.
+inline bool lattice_pays(int n, int nstates) { return n > 1024 || nstates > 4; }
+int lattice_nsplit(int n);  // partial-sum slots of launch_lattice_rows
+// Layout of its states, cols of them (a multiple of 4): the columns in steps of
+// 1024, of which chain T of the row sums takes four, 4 T + q, or T + 256 q
+// where n % 4; per chain and step 12 floats a state, x, y, z of those four.
+__host__ __device__ inline int64_t lattice_state_offset(int n, int cols, int s, int c, int j) {
+  const int quad = n % 4 == 0 ? j >> 2 : (j >> 10) * 256 + (j & 255);
+  const int q = n % 4 == 0 ? j & 3 : (j >> 8) & 3;
+  return ((int64_t)quad * cols + s) * 12 + c * 4 + q;
+}
+inline int lattice_cols(int nstates) { return (nstates + 3) / 4 * 4; }
+inline int64_t lattice_state_floats(int n, int cols) { return round_up(n, 1024) / 4 * cols * 12; }
+// out[w*split_stride + s*col_stride + c*n + i], w < lattice_nsplit(n): the four
+// waves' partial sums of a row of launch_matvec_f32, to be added in order of
+// w.  *nonfinite (device): as in launch_gemm_bf16x2_toeplitz.
+int launch_lattice_rows(const LatticeView& v, const float* m, int cols, float* out, int64_t split_stride,
+                        int64_t col_stride, int nstates, const int* nonfinite, hipStream_t stream);
+
 struct SparseDemag {
   int n = 0;
   float threshold = 0.0f;
@@ -193,6 +245,7 @@ struct LlgDesc {
   double hext[3];            // applied field (A/m) at the stage time
   double alpha, gamma;
   double* fields;            // optional 12n: H_exc, H_ext, H_dem, H_ani (negated, SoA)
+  float* sum_out;            // optional 3n: the FP32 demag sums over the partials
 };
 
 int launch_llg(const LlgGrid& g, const LlgDesc* d_descs, int nstates, hipStream_t stream);
@@ -316,7 +369,7 @@ struct VecDesc {
   int rslot;                 // the reduction's four results go to results[4*rslot .. 4*rslot+3]
 };
 
-enum PackMode { kPackNone = 0, kPackF32 = 1, kPackBf16 = 2, kPackF32Frag = 3 };
+enum PackMode { kPackNone = 0, kPackF32 = 1, kPackBf16 = 2, kPackF32Frag = 3, kPackLattice = 4 };
 
 // Byte offset of state column col's component c at source j in the FP32
 // B-fragment layout of the block-sparse FP32 product (same 12 KiB per 16-source
@@ -331,10 +384,10 @@ __host__ __device__ inline int64_t f32_frag_offset(int col, int c, int j) {
 
 struct PackSpec {
   int mode;
-  float* f32;                // [col][3n]
-  int64_t col_stride;
+  float* f32;                // kPackF32: [col][3n]; kPackLattice: lattice_state_offset
+  int64_t col_stride;        // kPackLattice: the layout's cols
   uint8_t* bf16;             // fragment layout (split-BF16, or FP32 with kPackF32Frag)
-  int* nonfinite = nullptr;  // set to 1 when a packed value is not finite in BF16 (kPackBf16; may be null)
+  int* nonfinite = nullptr;  // set to 1 when a packed value is not finite (kPackBf16: in BF16; kPackLattice; may be null)
 };
 // largest finite BF16 value: a state beyond it packs to an infinity
 constexpr float kBf16Max = 3.3895313892515355e38f;

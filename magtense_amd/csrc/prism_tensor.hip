@@ -717,6 +717,33 @@ int launch_assemble_avg(const double* pts, const double* abc, int n, const int n
   return kOk;
 }
 
+namespace {
+// Tensor entries of a uniform grid per distinct difference of cell centres
+// (lattice.hip): one thread per entry, consecutive threads along x.
+__global__ void __launch_bounds__(256) lattice_entries_kernel(const double* __restrict__ x, int ux,
+                                                              const double* __restrict__ y, int uy,
+                                                              const double* __restrict__ z, int64_t total, double dx,
+                                                              double dy, double dz, float4* __restrict__ a,
+                                                              float2* __restrict__ b) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= total) return;
+  const int64_t row = e / ux;
+  double k6[6];
+  prism_k6(dx, dy, dz, x[e - row * ux], y[row % uy], z[row / uy], k6);
+  a[e] = make_float4((float)k6[0], (float)k6[1], (float)k6[3], (float)k6[5]);
+  if (b) b[e] = make_float2((float)k6[2], (float)k6[4]);
+}
+}  // namespace
+
+int launch_lattice_entries(const double* x, int ux, const double* y, int uy, const double* z, int uz, const double d[3],
+                           float* a, float* b, hipStream_t stream) {
+  const int64_t total = (int64_t)ux * uy * uz;
+  hipLaunchKernelGGL(lattice_entries_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, x, ux, y, uy,
+                     z, total, d[0], d[1], d[2], reinterpret_cast<float4*>(a), reinterpret_cast<float2*>(b));
+  MT_HIP(hipGetLastError());
+  return kOk;
+}
+
 int launch_toeplitz_assemble(int nx, int ny, int nz, double Lx, double Ly, double Lz, uint8_t* out,
                              hipStream_t stream) {
   if (nx % 32 != 0) {

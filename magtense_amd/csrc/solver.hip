@@ -292,6 +292,7 @@ struct Solver {
   double* xv = nullptr;
   long long exch_nnz_host = 0;
   uint8_t* Ktab = nullptr;    // translation-invariant fragment table (bf16x2 on uniform grids)
+  LatticeTable lattice;       // FP32 dense product on uniform grids: the distinct tensor entries
   bool defer_early = false;   // read the early error estimate with stage 8's (cheap right-hand sides)
   bool stage_fusion = true;   // small FP32 dense problems: stage argument formed in the demag + LL launch
   bool near_llg = true;       // split product: the LL right-hand side evaluated by the near-band kernel
@@ -341,6 +342,7 @@ struct Solver {
     f(K32); f(Ksplit); f(Kf32); f(Ktab); f(near_tab); f(jfact); f(kfact); f(aniso); f(ms32); f(pool); f(yout); f(fout); f(packf); f(packb);
     f(hbuf); f(nonfinite); f(partials); f(results); f(arena_d); f(xs); f(xe); f(xc); f(xv);
     sparse.release();
+    lattice.release();
     if (h_results) (void)hipHostFree(h_results);
     if (arena_h) (void)hipHostFree(arena_h);
     for (hipEvent_t& e : ev)
@@ -1144,7 +1146,8 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
       L.fields = s.op.fields;
       L.hpart = hbuf + (size_t)k * N3;
       L.split_stride = (int64_t)hcols * N3;
-      L.nsplit = precision == MT_PREC_BF16X2 ? ksplit + (near_r > 0 ? 1 : 0) : (sparse.blocks || Kf32 ? ksplit : 1);
+      L.nsplit = precision == MT_PREC_BF16X2 ? ksplit + (near_r > 0 ? 1 : 0)
+                                             : (sparse.blocks || Kf32 || lattice.v.a ? ksplit : 1);
       hext_at(s, s.op.t, L.hext);
       L.alpha = alpha_at(s.op.t);
       L.gamma = gamma;
@@ -1153,6 +1156,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     PackSpec pk;
     if (precision == MT_PREC_BF16X2) pk = PackSpec{kPackBf16, nullptr, 0, packb, nonfinite};
     else if (sparse.blocks || Kf32) pk = PackSpec{kPackF32Frag, nullptr, 0, packb};
+    else if (lattice.v.a) pk = PackSpec{kPackLattice, packf, lattice_cols(std::min(B, kMaxCols)), nullptr, nonfinite};
     else pk = PackSpec{kPackF32, packf, (int64_t)N3, nullptr};
     if (timing) MT_HIP(hipEventRecord(ev[2], stream));
     // Small groups pass their descriptors by value; otherwise the group's
@@ -1160,7 +1164,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     // reads the LL descriptors from device memory)
     const bool inl = S <= kInlineStates && !(precision == MT_PREC_BF16X2 && near_r > 0);
     // the FP32 dense path runs its demag rows and the LL right-hand side in one kernel
-    const bool fused = precision == MT_PREC_FP32 && demag_approx == MT_DEMAG_DENSE;
+    const bool fused = precision == MT_PREC_FP32 && demag_approx == MT_DEMAG_DENSE && !lattice.v.a;
     // and on small problems forms the stage argument in that kernel as well
     const bool stage_fused = fused && inl && !pre_red && stage_fusion && n <= kStageFusedMaxCells;
     // the split product's near-band kernel evaluates the LL right-hand side
@@ -1206,6 +1210,9 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     } else if (sparse.blocks) {
       rc = launch_gemm_bsr(sparse.blocks->frags, sparse.blocks->view(), true, packb, n, hbuf, (int64_t)N3,
                            (int64_t)hcols * N3, S, ksplit, stream);
+    } else if (lattice.v.a) {
+      rc = launch_lattice_rows(lattice.v, packf, (int)pk.col_stride, hbuf, (int64_t)hcols * N3, (int64_t)N3, S,
+                               nonfinite, stream);
     } else if (demag_approx != MT_DEMAG_DENSE) {
       rc = sparse.apply(packf, (int64_t)N3, S, 1.0f, hbuf, stream);
     } else if (stage_fused) {
@@ -1456,12 +1463,26 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
            "the translation-invariant tensor needs a uniform grid, precision bf16x2, nx % 32 == 0 and no K_in");
   const bool use_toep = can_toep && q->toeplitz >= 0;
   const bool needsplit = P.precision == MT_PREC_BF16X2 && !use_toep && approx == MT_DEMAG_DENSE;
+  // FP32 on a uniform grid: the product from the distinct tensor entries, the
+  // same sums as over the dense tensor, which is held only where the caller
+  // gives it or asks for it, or on grids that the kernel does not take
+  bool lattice = false;
+  if (P.precision == MT_PREC_FP32 && approx == MT_DEMAG_DENSE && !unstructured && !q->K_in && !q->K_out &&
+      !q->keep_fp32_tensor && lattice_pays(n, P.B)) {
+    size_t free_b = 0, total_b = 0;
+    MT_HIP(hipMemGetInfo(&free_b, &total_b));
+    const double d[3] = {P.dx, P.dy, P.dz};
+    if (6.0 * nn * sizeof(float) < (double)total_b) {  // a problem too large for the device stays refused
+      int rc = P.lattice.build(P.nx, P.ny, P.nz, xs, ys, zs, d, P.stream, &lattice);
+      if (rc) return rc;
+    }
+  }
   if (use_toep) {
     MT_HIP(hipMalloc(&P.Ktab, (size_t)toeplitz_tensor_bytes(P.nx, P.ny, P.nz)));
     int rc = launch_toeplitz_assemble(P.nx, P.ny, P.nz, q->Lx, q->Ly, q->Lz, P.Ktab, P.stream);
     if (rc) return rc;
   }
-  if (need32) MT_HIP(hipMalloc(&P.K32, 6 * nn * sizeof(float)));
+  if (need32 && !lattice) MT_HIP(hipMalloc(&P.K32, 6 * nn * sizeof(float)));
   if (needsplit) MT_HIP(hipMalloc(&P.Ksplit, (size_t)split_tensor_bytes(n)));
   if (q->K_in) {
     DevArr<float> tmp;
@@ -1705,10 +1726,16 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
     MT_HIP(hipMemsetAsync(P.packb, 0, (size_t)packed_m_bytes(n), P.stream));
     MT_HIP(hipMalloc(&P.hbuf, (size_t)P.ksplit * P.hcols * n3 * sizeof(float)));
   } else {
-    P.ksplit = 1;
-    P.hcols = P.B;
-    MT_HIP(hipMalloc(&P.packf, (size_t)P.B * n3 * sizeof(float)));
-    MT_HIP(hipMalloc(&P.hbuf, (size_t)P.B * n3 * sizeof(float)));
+    P.ksplit = lattice ? lattice_nsplit(n) : 1;
+    P.hcols = lattice ? std::min(P.B, kMaxCols) : P.B;
+    const size_t packed = lattice ? (size_t)lattice_state_floats(n, lattice_cols(std::min(P.B, kMaxCols)))
+                                  : (size_t)P.B * n3;
+    MT_HIP(hipMalloc(&P.packf, packed * sizeof(float)));
+    MT_HIP(hipMalloc(&P.hbuf, (size_t)P.ksplit * P.hcols * n3 * sizeof(float)));
+    if (lattice) {
+      MT_HIP(hipMalloc(&P.nonfinite, sizeof(int)));
+      MT_HIP(hipMemsetAsync(P.nonfinite, 0, sizeof(int), P.stream));
+    }
   }
   const int bps = vec_blocks_per_state((int)n3);
   MT_HIP(hipMalloc(&P.partials, (size_t)3 * P.B * bps * 4 * sizeof(double)));
