@@ -1238,12 +1238,16 @@ __global__ void __launch_bounds__(256) near_corr_kernel(const uint32_t* __restri
   const int64_t i = ix + (int64_t)iy * nx + (int64_t)iz * nx * ny;
   if (LLG) {
     const LlgDesc& D = descs[s];
-    llg_cell(g, D, (int)i, [&](int c) {
-      float v = 0.0f;
-      for (int k = 0; k + 1 < D.nsplit; ++k) v += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * n + i];
-      v += acc[c];
-      return v;
-    });
+    double dm[3];
+    llg_cell(
+        g, D, (int)i,
+        [&](int c) {
+          float v = 0.0f;
+          for (int k = 0; k + 1 < D.nsplit; ++k) v += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * n + i];
+          v += acc[c];
+          return v;
+        },
+        dm);
     return;
   }
   float* o = out + (int64_t)s * col_stride + i;

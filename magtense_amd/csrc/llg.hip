@@ -40,32 +40,43 @@ __device__ inline float bf16_value(uint16_t b) { return __uint_as_float((uint32_
 // block b runs on XCD b % 8, and XCD x takes the contiguous x-th eighth of the
 // (state, cell block) range, so the exchange stencil's neighbour rows and
 // planes are read through the L2 that already holds them.  INL: descriptors
-// by value (inl) instead of from descs.
-template <bool INL>
+// by value (inl) instead of from descs.  NEXT: also the next stage argument.
+template <bool INL, bool NEXT>
 __global__ void __launch_bounds__(256) llg_kernel(const LlgGrid g, const LlgDesc* __restrict__ descs,
-                                                  LlgDescsInline inl, int cell_blocks, int nstates) {
+                                                  LlgDescsInline inl, int cell_blocks, int nstates,
+                                                  const StageDesc* __restrict__ nexts, StageDescsInline inext,
+                                                  PackSpec pack) {
   const int total = cell_blocks * nstates;
   const int per_xcd = (int)(gridDim.x / 8);
   const int w = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
   if (w >= total) return;
-  const LlgDesc& D = INL ? inl.d[w / cell_blocks] : descs[w / cell_blocks];
+  const int st = w / cell_blocks;
+  const LlgDesc& D = INL ? inl.d[st] : descs[st];
   const int i = (w % cell_blocks) * blockDim.x + threadIdx.x;
   if (i >= g.n) return;
-  llg_cell(g, D, i, [&](int c) {
-    float s = 0.0f;
-    for (int k = 0; k < D.nsplit; ++k) s += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * g.n + i];
-    return s;
-  });
+  double dm[3];
+  llg_cell(
+      g, D, i,
+      [&](int c) {
+        float s = 0.0f;
+        for (int k = 0; k < D.nsplit; ++k) s += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * g.n + i];
+        return s;
+      },
+      dm);
+  if (NEXT) next_stage_cell(INL ? inext.d[st] : nexts[st], D, g.n, i, dm, pack, st);
 }
 
 // The FP32 dense path's demag rows and LL right-hand side in one launch:
 // block = RB receiver rows of S states, from s0 on (the sums of matvec_rows_f32),
-// then one thread per row and state evaluates llg_cell with them.
-template <bool INL, bool VEC4, int RB, int S, bool ONE>
+// then one thread per row and state evaluates llg_cell with them (NEXT: and the
+// next stage argument of the cell).
+template <bool INL, bool VEC4, int RB, int S, bool ONE, bool NEXT>
 __global__ void __launch_bounds__(256) demag_llg_f32_kernel(const float* __restrict__ K, const LlgGrid g,
                                                             const LlgDesc* __restrict__ descs, LlgDescsInline inl,
                                                             const float* __restrict__ m32, int64_t m_stride, int s0,
-                                                            int nstates, int groups) {
+                                                            int nstates, int groups,
+                                                            const StageDesc* __restrict__ nexts,
+                                                            StageDescsInline inext, PackSpec pack) {
   int rows = blockIdx.x, group = 0;
   if (!ONE) matvec_block(blockIdx.x, groups, rows, group);
   const int sb = s0 + group * S;
@@ -78,34 +89,27 @@ __global__ void __launch_bounds__(256) demag_llg_f32_kernel(const float* __restr
   if (s >= S || sb + s >= nstates || i0 + r >= g.n) return;
   const LlgDesc& D = INL ? inl.d[sb + s] : descs[sb + s];
   // one partial-sum slot: S = 0 + row sum, as the LL kernel forms it
-  llg_cell(g, D, i0 + r, [&](int c) {
-    float v = 0.0f;
-    v += sums[(s * RB + r) * 3 + c];
-    return v;
-  });
+  double dm[3];
+  llg_cell(
+      g, D, i0 + r,
+      [&](int c) {
+        float v = 0.0f;
+        v += sums[(s * RB + r) * 3 + c];
+        return v;
+      },
+      dm);
+  if (NEXT) next_stage_cell(INL ? inext.d[sb + s] : nexts[sb + s], D, g.n, i0 + r, dm, pack, sb + s);
 }
-
-// Stage combination of a small problem, carried by value into the fused launch.
-struct StageDesc {
-  double* dst;
-  const double* base;
-  double bcoef, bconst, post_scale;
-  int nterm;
-  const double* src[kMaxTerms];
-  double coef[kMaxTerms];
-};
-struct StageDescsInline {
-  StageDesc d[kInlineStates];
-};
 
 // Stage argument + FP32 demag rows + LL right-hand side (launch_stage_demag_llg_f32).
 // Block = RB receiver rows of state blockIdx.y.  The whole stage vector goes to
 // LDS (3n FP64, then its FP32 rounding); each element sums bconst, bcoef*base
 // and the terms in the vector kernel's order, all of its operands loaded
 // before the sum (an index past nterm reloads operand 0, which is not used).
-template <bool VEC4, int RB>
+template <bool VEC4, int RB, bool NEXT>
 __global__ void __launch_bounds__(256) stage_demag_llg_f32_kernel(const float* __restrict__ K, const LlgGrid g,
-                                                                  StageDescsInline sd, LlgDescsInline inl) {
+                                                                  StageDescsInline sd, LlgDescsInline inl,
+                                                                  StageDescsInline inext, PackSpec pack) {
   extern __shared__ double stage_lds[];
   const int n = g.n, n3 = 3 * n;
   const int s = blockIdx.y;
@@ -142,11 +146,16 @@ __global__ void __launch_bounds__(256) stage_demag_llg_f32_kernel(const float* _
   if (r >= RB || i0 + r >= n) return;
   LlgDesc D = inl.d[s];
   D.m = m64;  // the stage argument from LDS (other blocks write its global copy)
-  llg_cell(g, D, i0 + r, [&](int c) {
-    float v = 0.0f;
-    v += sums[r * 3 + c];
-    return v;
-  });
+  double dm[3];
+  llg_cell(
+      g, D, i0 + r,
+      [&](int c) {
+        float v = 0.0f;
+        v += sums[r * 3 + c];
+        return v;
+      },
+      dm);
+  if (NEXT) next_stage_cell(inext.d[s], D, n, i0 + r, dm, pack, s);
 }
 
 __device__ inline double nan_to_inf(double v) { return isnan(v) ? INFINITY : v; }
@@ -446,11 +455,20 @@ __global__ void finalize_kernel(const VecDesc* __restrict__ descs, VecDescsInlin
 
 // kernel arguments are limited to 4 KiB
 static_assert(sizeof(VecDescsInline) + 256 <= 4096, "vector kernel arguments exceed 4 KiB");
-static_assert(sizeof(LlgDescsInline) + sizeof(LlgGrid) + 256 <= 4096, "LL kernel arguments exceed 4 KiB");
+static_assert(sizeof(LlgDescsInline) + sizeof(StageDescsInline) + sizeof(LlgGrid) + 256 <= 4096,
+              "LL kernel arguments exceed 4 KiB");
 
 namespace {
+StageDescsInline inline_next(const NextStage& next, int nstates) {
+  StageDescsInline d{};
+  if (next.h_descs)
+    for (int s = 0; s < nstates; ++s) d.d[s] = next.h_descs[s];
+  return d;
+}
+
 template <bool INL>
-int launch_llg_t(const LlgGrid& g, const LlgDesc* descs, const LlgDescsInline& inl, int nstates, hipStream_t stream) {
+int launch_llg_t(const LlgGrid& g, const LlgDesc* descs, const LlgDescsInline& inl, int nstates,
+                 const NextStage& next, hipStream_t stream) {
   const int cell_blocks = (g.n + 255) / 256;
   const int64_t total = (int64_t)cell_blocks * nstates;
   const int64_t blocks = (total + 7) / 8 * 8;
@@ -458,8 +476,13 @@ int launch_llg_t(const LlgGrid& g, const LlgDesc* descs, const LlgDescsInline& i
     set_error("LL kernel: too many cells x states for one launch");
     return kErrArg;
   }
-  hipLaunchKernelGGL(llg_kernel<INL>, dim3((unsigned)blocks), dim3(256), 0, stream, g, descs, inl, cell_blocks,
-                     nstates);
+  const StageDescsInline nx = inline_next(next, INL ? nstates : 0);
+  if (next.on())
+    hipLaunchKernelGGL((llg_kernel<INL, true>), dim3((unsigned)blocks), dim3(256), 0, stream, g, descs, inl,
+                       cell_blocks, nstates, next.d_descs, nx, next.pack);
+  else
+    hipLaunchKernelGGL((llg_kernel<INL, false>), dim3((unsigned)blocks), dim3(256), 0, stream, g, descs, inl,
+                       cell_blocks, nstates, next.d_descs, nx, next.pack);
   MT_HIP(hipGetLastError());
   return kOk;
 }
@@ -482,32 +505,38 @@ int launch_vec_t(const VecDesc* descs, const VecDescsInline& inl, int nstates, i
 }
 }  // namespace
 
-int launch_llg(const LlgGrid& g, const LlgDesc* d_descs, int nstates, hipStream_t stream) {
-  return launch_llg_t<false>(g, d_descs, LlgDescsInline{}, nstates, stream);
+int launch_llg(const LlgGrid& g, const LlgDesc* d_descs, int nstates, hipStream_t stream, const NextStage& next) {
+  return launch_llg_t<false>(g, d_descs, LlgDescsInline{}, nstates, next, stream);
 }
 
-int launch_llg_inline(const LlgGrid& g, const LlgDesc* h_descs, int nstates, hipStream_t stream) {
+int launch_llg_inline(const LlgGrid& g, const LlgDesc* h_descs, int nstates, hipStream_t stream,
+                      const NextStage& next) {
   if (nstates < 1 || nstates > kInlineStates) {
     set_error("LL kernel: descriptors by value hold at most kInlineStates states");
     return kErrArg;
   }
   LlgDescsInline inl{};
   for (int s = 0; s < nstates; ++s) inl.d[s] = h_descs[s];
-  return launch_llg_t<true>(g, nullptr, inl, nstates, stream);
+  return launch_llg_t<true>(g, nullptr, inl, nstates, next, stream);
 }
 
 namespace {
 template <int S>
 int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDescsInline& inl,
-                       const float* m32, int64_t m_stride, int s0, int nstates, int groups,
+                       const float* m32, int64_t m_stride, int s0, int nstates, int groups, const NextStage& next,
                        hipStream_t stream) {
   constexpr int RB = matvec_block_rows(S);
   const dim3 grid(matvec_blocks((g.n + RB - 1) / RB, groups));
   const bool vec4 = (g.n % 4) == 0 && (m_stride % 4) == 0;
-  auto go = [&](auto by_value, auto v4, auto one) {
+  const StageDescsInline nx = inline_next(next, d_descs ? 0 : nstates);
+  auto launch = [&](auto by_value, auto v4, auto one, auto with_next) {
     hipLaunchKernelGGL((demag_llg_f32_kernel<decltype(by_value)::value, decltype(v4)::value, RB, S,
-                                             decltype(one)::value>),
-                       grid, dim3(256), 0, stream, K, g, d_descs, inl, m32, m_stride, s0, nstates, groups);
+                                             decltype(one)::value, decltype(with_next)::value>),
+                       grid, dim3(256), 0, stream, K, g, d_descs, inl, m32, m_stride, s0, nstates, groups,
+                       next.d_descs, nx, next.pack);
+  };
+  auto go = [&](auto by_value, auto v4, auto one) {
+    next.on() ? launch(by_value, v4, one, std::true_type{}) : launch(by_value, v4, one, std::false_type{});
   };
   const std::true_type yes;
   const std::false_type no;
@@ -520,7 +549,7 @@ int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs,
 }  // namespace
 
 int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDesc* h_descs,
-                         const float* m32, int64_t m_stride, int nstates, hipStream_t stream) {
+                         const float* m32, int64_t m_stride, int nstates, hipStream_t stream, const NextStage& next) {
   LlgDescsInline inl{};
   if (!d_descs) {
     if (nstates < 1 || nstates > kInlineStates) {
@@ -532,21 +561,21 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
   for (int s0 = 0; s0 < nstates;) {
     const int S = matvec_group(nstates - s0), groups = S == 8 ? std::max(1, std::min((nstates - s0) / 8, 64)) : 1;
     int rc = kOk;
-    if (S == 8) rc = launch_demag_llg_s<8>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, stream);
-    else if (S == 4) rc = launch_demag_llg_s<4>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
-    else if (S == 2) rc = launch_demag_llg_s<2>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
-    else rc = launch_demag_llg_s<1>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, stream);
+    if (S == 8) rc = launch_demag_llg_s<8>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, next, stream);
+    else if (S == 4) rc = launch_demag_llg_s<4>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);
+    else if (S == 2) rc = launch_demag_llg_s<2>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);
+    else rc = launch_demag_llg_s<1>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);
     if (rc) return rc;
     s0 += S * groups;
   }
   return kOk;
 }
 
-static_assert(sizeof(StageDescsInline) + sizeof(LlgDescsInline) + sizeof(LlgGrid) + 256 <= 4096,
+static_assert(2 * sizeof(StageDescsInline) + sizeof(LlgDescsInline) + sizeof(LlgGrid) + 256 <= 4096,
               "stage + demag + LL kernel arguments exceed 4 KiB");
 
 int launch_stage_demag_llg_f32(const float* K, const LlgGrid& g, const VecDesc* h_pre, const LlgDesc* h_descs,
-                               int nstates, hipStream_t stream) {
+                               int nstates, hipStream_t stream, const NextStage& next) {
   if (nstates < 1 || nstates > kInlineStates || g.n < 1 || g.n > kStageFusedMaxCells) {
     set_error("stage + demag + LL kernel: 1..kInlineStates states, 1..kStageFusedMaxCells cells");
     return kErrArg;
@@ -554,31 +583,22 @@ int launch_stage_demag_llg_f32(const float* K, const LlgGrid& g, const VecDesc* 
   StageDescsInline sd{};
   LlgDescsInline inl{};
   for (int s = 0; s < nstates; ++s) {
-    const VecDesc& v = h_pre[s];
-    if (!v.dst || v.rkind != kRedNone || v.nterm < 0 || v.nterm > kMaxTerms) {
+    if (!stage_of(h_pre[s], sd.d[s])) {
       set_error("stage + demag + LL kernel: a stage combination with a destination and no reduction");
       return kErrArg;
-    }
-    StageDesc& d = sd.d[s];
-    d.dst = v.dst;
-    d.base = v.base;
-    d.bcoef = v.bcoef;
-    d.bconst = v.bconst;
-    d.post_scale = v.post_scale;
-    d.nterm = v.nterm;
-    for (int k = 0; k < v.nterm; ++k) {
-      d.src[k] = v.src[k];
-      d.coef[k] = v.coef[k];
     }
     inl.d[s] = h_descs[s];
   }
   constexpr int RB = 4;
   const dim3 grid((unsigned)((g.n + RB - 1) / RB), (unsigned)nstates);
   const size_t lds = (size_t)3 * g.n * (sizeof(double) + sizeof(float));
-  if (g.n % 4 == 0)
-    hipLaunchKernelGGL((stage_demag_llg_f32_kernel<true, RB>), grid, dim3(256), lds, stream, K, g, sd, inl);
-  else
-    hipLaunchKernelGGL((stage_demag_llg_f32_kernel<false, RB>), grid, dim3(256), lds, stream, K, g, sd, inl);
+  const StageDescsInline nx = inline_next(next, nstates);
+  auto go = [&](auto v4, auto with_next) {
+    hipLaunchKernelGGL((stage_demag_llg_f32_kernel<decltype(v4)::value, RB, decltype(with_next)::value>), grid,
+                       dim3(256), lds, stream, K, g, sd, inl, nx, next.pack);
+  };
+  if (g.n % 4 == 0) next.on() ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  else next.on() ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
   MT_HIP(hipGetLastError());
   return kOk;
 }

@@ -9,6 +9,8 @@
 // are kept negated as in the reference; the API's alpha is alpha_LL * gamma.
 #pragma once
 
+#include <cfloat>
+
 #include "mt_common.h"
 #include "mt_kernels.h"
 
@@ -16,9 +18,9 @@ namespace mt {
 
 // LL right-hand side of cell i for the state of descriptor D.  hsum(c)
 // returns the FP32 demag sum S_c = sum of the partials of (K m)_c at i (used
-// unless D.hpart64 holds FP64 sums).
+// unless D.hpart64 holds FP64 sums).  dm: dm/dt, which goes to D.out as well.
 template <typename HS>
-__device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, HS hsum) {
+__device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, HS hsum, double (&dm)[3]) {
   const int n = g.n;
   const double* m = D.m;
   const int ix = i % g.nx;
@@ -98,10 +100,13 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
   double dx = mc[1] * cz - mc[2] * cy;
   double dy = mc[2] * cx - mc[0] * cz;
   double dz = mc[0] * cy - mc[1] * cx;
+  dm[0] = -D.gamma * cx - D.alpha * dx;
+  dm[1] = -D.gamma * cy - D.alpha * dy;
+  dm[2] = -D.gamma * cz - D.alpha * dz;
   if (D.out) {
-    D.out[i] = -D.gamma * cx - D.alpha * dx;
-    D.out[n + i] = -D.gamma * cy - D.alpha * dy;
-    D.out[2 * n + i] = -D.gamma * cz - D.alpha * dz;
+    D.out[i] = dm[0];
+    D.out[n + i] = dm[1];
+    D.out[2 * n + i] = dm[2];
   }
   if (D.fields) {
     double* F = D.fields;
@@ -112,6 +117,52 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
       F[(size_t)(9 + c) * n + i] = hk[c];
     }
   }
+}
+
+// The next stage argument at cell i, straight after its right-hand side: the
+// vector kernel's combination (same order, same roundings) over the cell's
+// three components, with dm/dt taken from registers, and its demag input
+// packed into column col.  Only the cell's own values are read, so the launch
+// that evaluates dm/dt can write the next stage's argument as long as that is
+// not a vector it reads at other cells.
+__device__ __forceinline__ void next_stage_cell(const StageDesc& S, const LlgDesc& D, int n, int i,
+                                                const double (&dm)[3], const PackSpec& pack, int col) {
+  double v[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) v[c] = S.bconst;
+  const size_t at[3] = {(size_t)i, (size_t)n + i, 2 * (size_t)n + i};
+  if (S.base) {
+    double x[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) x[c] = S.base[at[c]];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] = __builtin_fma(S.bcoef, x[c], v[c]);
+  }
+  double x[kMaxTerms][3];
+#pragma unroll
+  for (int k = 0; k < kMaxTerms; ++k)
+    if (k < S.nterm && S.src[k] != D.out) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) x[k][c] = S.src[k][at[c]];
+    }
+#pragma unroll
+  for (int k = 0; k < kMaxTerms; ++k)
+    if (k < S.nterm) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[c] = __builtin_fma(S.coef[k], S.src[k] != D.out ? x[k][c] : dm[c], v[c]);
+    }
+  bool bad = false;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    v[c] = S.post_scale * v[c];
+    S.dst[at[c]] = v[c];
+    const float f = (float)v[c];
+    if (pack.mode == kPackF32) pack.f32[(int64_t)col * pack.col_stride + (int64_t)at[c]] = f;
+    else if (pack.mode == kPackLattice) pack.f32[lattice_state_offset(n, (int)pack.col_stride, col, c, i)] = f;
+    else if (pack.mode == kPackF32Frag) *reinterpret_cast<float*>(pack.bf16 + f32_frag_offset(col, c, i)) = f;
+    bad |= !(fabsf(f) <= FLT_MAX);
+  }
+  if (bad && pack.nonfinite) *pack.nonfinite = 1;
 }
 
 }  // namespace mt

@@ -248,26 +248,6 @@ struct LlgDesc {
   float* sum_out;            // optional 3n: the FP32 demag sums over the partials
 };
 
-int launch_llg(const LlgGrid& g, const LlgDesc* d_descs, int nstates, hipStream_t stream);
-
-// Small batches (up to kInlineStates states) pass their descriptors by value
-// in the launch arguments: no host -> device copy, and so no copy kernel, in
-// front of the launch (a tick of a small problem is a few kernels of a few
-// microseconds each).
-constexpr int kInlineStates = 4;
-struct LlgDescsInline {
-  LlgDesc d[kInlineStates];
-};
-int launch_llg_inline(const LlgGrid& g, const LlgDesc* h_descs, int nstates, hipStream_t stream);
-// Plain FP32 demag rows and the LL right-hand side in one launch (the FP32
-// dense path): the rows of matvec_f32 for each state, then the LL kernel's
-// arithmetic for the block's cells with those sums (bit-identical to
-// launch_matvec_f32 + launch_llg with one partial-sum slot).  Descriptors from
-// d_descs, or by value from h_descs when d_descs is null (nstates <=
-// kInlineStates); m32 + s * m_stride is state s's FP32 demag input.
-int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDesc* h_descs,
-                         const float* m32, int64_t m_stride, int nstates, hipStream_t stream);
-
 // Near-band correction of the split-BF16 product on a uniform nx x ny x nz
 // grid: the FP32 product's difference from the three split products, summed
 // over the sources within R cells in x and y and min(R, nz - 1) layers in z.
@@ -369,6 +349,32 @@ struct VecDesc {
   int rslot;                 // the reduction's four results go to results[4*rslot .. 4*rslot+3]
 };
 
+// A combination without a reduction: dst = post_scale * (bconst + bcoef*base + sum coef*src).
+struct StageDesc {
+  double* dst;
+  const double* base;
+  double bcoef, bconst, post_scale;
+  int nterm;
+  const double* src[kMaxTerms];
+  double coef[kMaxTerms];
+};
+
+// stage combination of a vector operation; false where it has none, or a reduction
+inline bool stage_of(const VecDesc& v, StageDesc& d) {
+  if (!v.dst || v.rkind != kRedNone || v.nterm < 0 || v.nterm > kMaxTerms) return false;
+  d.dst = v.dst;
+  d.base = v.base;
+  d.bcoef = v.bcoef;
+  d.bconst = v.bconst;
+  d.post_scale = v.post_scale;
+  d.nterm = v.nterm;
+  for (int k = 0; k < kMaxTerms; ++k) {
+    d.src[k] = k < v.nterm ? v.src[k] : nullptr;
+    d.coef[k] = k < v.nterm ? v.coef[k] : 0.0;
+  }
+  return true;
+}
+
 enum PackMode { kPackNone = 0, kPackF32 = 1, kPackBf16 = 2, kPackF32Frag = 3, kPackLattice = 4 };
 
 // Byte offset of state column col's component c at source j in the FP32
@@ -391,6 +397,42 @@ struct PackSpec {
 };
 // largest finite BF16 value: a state beyond it packs to an infinity
 constexpr float kBf16Max = 3.3895313892515355e38f;
+
+// Small batches (up to kInlineStates states) pass their descriptors by value
+// in the launch arguments: no host -> device copy, and so no copy kernel, in
+// front of the launch (a tick of a small problem is a few kernels of a few
+// microseconds each).
+constexpr int kInlineStates = 4;
+struct LlgDescsInline {
+  LlgDesc d[kInlineStates];
+};
+struct StageDescsInline {
+  StageDesc d[kInlineStates];
+};
+// The next stage arguments, formed by the launch that evaluates dm/dt: one
+// combination per state (device, or by value with descriptors by value) and
+// where their demag input goes (column = state).  No dst may be a vector or a
+// demag input that the launch itself reads.
+struct NextStage {
+  const StageDesc* d_descs = nullptr;
+  const StageDesc* h_descs = nullptr;
+  PackSpec pack{};
+  bool on() const { return d_descs || h_descs; }
+};
+
+int launch_llg(const LlgGrid& g, const LlgDesc* d_descs, int nstates, hipStream_t stream,
+               const NextStage& next = NextStage{});
+int launch_llg_inline(const LlgGrid& g, const LlgDesc* h_descs, int nstates, hipStream_t stream,
+                      const NextStage& next = NextStage{});
+// Plain FP32 demag rows and the LL right-hand side in one launch (the FP32
+// dense path): the rows of matvec_f32 for each state, then the LL kernel's
+// arithmetic for the block's cells with those sums (bit-identical to
+// launch_matvec_f32 + launch_llg with one partial-sum slot).  Descriptors from
+// d_descs, or by value from h_descs when d_descs is null (nstates <=
+// kInlineStates); m32 + s * m_stride is state s's FP32 demag input.
+int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDesc* h_descs,
+                         const float* m32, int64_t m_stride, int nstates, hipStream_t stream,
+                         const NextStage& next = NextStage{});
 
 int vec_blocks_per_state(int n3);
 // With one block per state (3n <= 2048) the vector kernel writes the
@@ -415,6 +457,6 @@ int launch_vec_inline(const VecDesc* h_descs, int nstates, int n, double* partia
 // no reduction in h_pre.
 constexpr int kStageFusedMaxCells = 1024;
 int launch_stage_demag_llg_f32(const float* K, const LlgGrid& g, const VecDesc* h_pre, const LlgDesc* h_descs,
-                               int nstates, hipStream_t stream);
+                               int nstates, hipStream_t stream, const NextStage& next = NextStage{});
 
 }  // namespace mt

@@ -109,7 +109,7 @@ struct Sim {
   bool at_t_start = true, at_t_end = false, chkeff = false, phase2 = true;
   int st_range = -1, st_interp = -1;
   // device vectors (3n doubles each); stage[1..7]; p[1..5]
-  double *y = nullptr, *yp = nullptr, *y_old = nullptr, *scratch = nullptr, *errest = nullptr, *weights = nullptr;
+  double *y = nullptr, *yp = nullptr, *y_old = nullptr, *scratch = nullptr, *alt = nullptr, *errest = nullptr, *weights = nullptr;
   double* stage[8] = {};
   double *xstage = nullptr, *ytemp = nullptr, *arg = nullptr, *y_step = nullptr, *y_last = nullptr;
   double* p[6] = {};
@@ -305,7 +305,8 @@ struct Solver {
   double* pool = nullptr;     // state vectors
   double* yout = nullptr;     // [B][n_h][nt][3n]
   double* fout = nullptr;     // [B][n_h][nt][12n]
-  float* packf = nullptr;     // [B][3n]
+  float* packf = nullptr;     // [B][3n], or the lattice product's layout
+  float* packf2 = nullptr;    // the same again: the next stage's, written while packf is read
   uint8_t* packb = nullptr;   // fragment layout, 64 columns
   int* nonfinite = nullptr;   // device flag: a packed state held a value that is not finite in BF16
   float* hbuf = nullptr;      // [ksplit][cols][3n]
@@ -339,7 +340,7 @@ struct Solver {
     auto f = [](void* p) {
       if (p) (void)hipFree(p);
     };
-    f(K32); f(Ksplit); f(Kf32); f(Ktab); f(near_tab); f(jfact); f(kfact); f(aniso); f(ms32); f(pool); f(yout); f(fout); f(packf); f(packb);
+    f(K32); f(Ksplit); f(Kf32); f(Ktab); f(near_tab); f(jfact); f(kfact); f(aniso); f(ms32); f(pool); f(yout); f(fout); f(packf); f(packf2); f(packb);
     f(hbuf); f(nonfinite); f(partials); f(results); f(arena_d); f(xs); f(xe); f(xc); f(xv);
     sparse.release();
     lattice.release();
@@ -350,7 +351,7 @@ struct Solver {
     if (stream) (void)hipStreamDestroy(stream);
     xs = xe = xc = nullptr; xv = nullptr;
     K32 = nullptr; Ksplit = nullptr; Kf32 = nullptr; Ktab = nullptr; near_tab = nullptr; jfact = kfact = aniso = nullptr; ms32 = nullptr; pool = yout = fout = nullptr;
-    packf = nullptr; packb = nullptr; hbuf = nullptr; nonfinite = nullptr; partials = results = nullptr; arena_d = nullptr;
+    packf = packf2 = nullptr; packb = nullptr; hbuf = nullptr; nonfinite = nullptr; partials = results = nullptr; arena_d = nullptr;
     h_results = nullptr; arena_h = nullptr; stream = nullptr;
     for (hipEvent_t& e : ev) e = nullptr;
   }
@@ -549,6 +550,9 @@ struct Solver {
       bool restart = false;
       for (int i = 2; i <= 8; ++i) {
         VecDesc pre = blank();
+        // consecutive stage arguments alternate between two vectors: the launch
+        // that evaluates a stage may already write the next one's argument
+        std::swap(s.scratch, s.alt);
         pre.dst = s.scratch;  // y_new
         pre.base = s.y;
         add_term(pre, s.yp, htry * T.A[i][1]);
@@ -1075,9 +1079,65 @@ struct Solver {
   }
 
   // ---- scheduler ----------------------------------------------------------------
+  // Right-hand sides whose results nobody waits for are launched one tick late:
+  // by then the states' next stage arguments are known, and where those are
+  // plain combinations the launch that evaluates dm/dt forms them too (no
+  // vector launch between two stages).  FP32 products, one demag pass a tick.
+  struct Pending {
+    std::vector<Sim*> sims;
+    std::vector<LlgDesc> ld;
+    std::vector<VecDesc> pre;   // stage arguments that the launch forms itself (small problems), or empty
+    bool dense = false;         // the demag rows run in the LL launch
+    bool inl = false;
+  } pending;
+  int flush_pending(const std::vector<VecDesc>* next);
+  PackSpec pack_f32(bool other) const {
+    float* p = other ? packf2 : packf;
+    if (lattice.v.a) return PackSpec{kPackLattice, p, lattice_cols(std::min(B, kMaxCols)), nullptr, nonfinite};
+    return PackSpec{kPackF32, p, (int64_t)n3(), nullptr};
+  }
   int run_until_idle();
   int execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs);
 };
+
+// Launches the pending right-hand sides; next: the stage arguments to form with
+// them (the demag input then goes to the other buffer, which becomes packf).
+int Solver::flush_pending(const std::vector<VecDesc>* next) {
+  Pending& p = pending;
+  if (p.sims.empty()) return kOk;
+  const int S = (int)p.sims.size();
+  const size_t N3 = n3();
+  std::vector<StageDesc> stages;
+  if (next) {
+    stages.resize(S);
+    for (int k = 0; k < S; ++k)
+      if (!stage_of((*next)[k], stages[k])) {
+        set_error("next stage: not a plain combination");
+        return kErrState;
+      }
+  }
+  NextStage nx;
+  if (next) nx.pack = pack_f32(true);
+  const LlgDesc* dl = nullptr;
+  if (p.inl) {
+    nx.h_descs = next ? stages.data() : nullptr;
+  } else {
+    int rc = stage_reserve(2 * 256 + (size_t)S * (sizeof(StageDesc) + sizeof(LlgDesc)));
+    if (rc) return rc;
+    dl = stage_put(p.ld);
+    if (next) nx.d_descs = stage_put(stages);
+    rc = stage_flush();
+    if (rc) return rc;
+  }
+  int rc;
+  if (!p.pre.empty()) rc = launch_stage_demag_llg_f32(K32, grid, p.pre.data(), p.ld.data(), S, stream, nx);
+  else if (p.dense) rc = launch_demag_llg_f32(K32, grid, dl, p.ld.data(), packf, (int64_t)N3, S, stream, nx);
+  else if (p.inl) rc = launch_llg_inline(grid, p.ld.data(), S, stream, nx);
+  else rc = launch_llg(grid, dl, S, stream, nx);
+  if (next) std::swap(packf, packf2);
+  p.sims.clear();
+  return rc;
+}
 
 int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
   const size_t N3 = n3();
@@ -1088,6 +1148,22 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
   double* res_pre = results + nres;
   double* res_post = results + 2 * nres;
   PackSpec nopack{kPackNone, nullptr, 0, nullptr};
+  // the last tick's right-hand sides, with this tick's stage arguments where
+  // the same states follow with plain combinations into other vectors
+  bool formed = false;
+  if (!pending.sims.empty()) {
+    bool follow = vecs.empty() && evals.size() == pending.sims.size();
+    std::vector<VecDesc> next(follow ? evals.size() : 0);
+    for (size_t k = 0; k < evals.size() && follow; ++k) {
+      next[k] = evals[k]->op.pre;
+      StageDesc unused;
+      follow = evals[k] == pending.sims[k] && stage_of(next[k], unused) && next[k].dst != pending.ld[k].m &&
+               next[k].dst != pending.ld[k].out;
+    }
+    int rc = flush_pending(follow ? &next : nullptr);
+    if (rc) return rc;
+    formed = follow;
+  }
   // vector-only operations of this tick
   bool vec_reduce = false;
   if (!vecs.empty()) {
@@ -1156,8 +1232,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     PackSpec pk;
     if (precision == MT_PREC_BF16X2) pk = PackSpec{kPackBf16, nullptr, 0, packb, nonfinite};
     else if (sparse.blocks || Kf32) pk = PackSpec{kPackF32Frag, nullptr, 0, packb};
-    else if (lattice.v.a) pk = PackSpec{kPackLattice, packf, lattice_cols(std::min(B, kMaxCols)), nullptr, nonfinite};
-    else pk = PackSpec{kPackF32, packf, (int64_t)N3, nullptr};
+    else pk = pack_f32(false);
     if (timing) MT_HIP(hipEventRecord(ev[2], stream));
     // Small groups pass their descriptors by value; otherwise the group's
     // three descriptor arrays go over in one copy (the near-band correction
@@ -1166,24 +1241,27 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     // the FP32 dense path runs its demag rows and the LL right-hand side in one kernel
     const bool fused = precision == MT_PREC_FP32 && demag_approx == MT_DEMAG_DENSE && !lattice.v.a;
     // and on small problems forms the stage argument in that kernel as well
-    const bool stage_fused = fused && inl && !pre_red && stage_fusion && n <= kStageFusedMaxCells;
+    const bool stage_fused = fused && inl && !pre_red && stage_fusion && n <= kStageFusedMaxCells && !formed;
+    // nobody waits for these right-hand sides: left to the next tick
+    bool late = (fused || lattice.v.a) && !timing && !post_red && evals.size() <= (size_t)kMaxCols && !pre_sync;
+    for (int k = 0; k < S && late; ++k) late = !ld[k].fields && ld[k].out;
     // the split product's near-band kernel evaluates the LL right-hand side
     const bool llg_in_near = precision == MT_PREC_BF16X2 && near_r > 0 && near_llg;
     const VecDesc* dpre = nullptr;
     const LlgDesc* dl = nullptr;
     const VecDesc* dpost = nullptr;
     int rc;
-    if (!inl) {
+    if (!inl && !(late && formed)) {
       rc = stage_reserve(3 * 256 + (size_t)S * (2 * sizeof(VecDesc) + sizeof(LlgDesc)));
       if (rc) return rc;
-      dpre = stage_put(pre);
-      dl = stage_put(ld);
+      if (!formed) dpre = stage_put(pre);
+      if (!late) dl = stage_put(ld);
       dpost = post_red ? stage_put(post) : nullptr;
       rc = stage_flush();
       if (rc) return rc;
     }
     double* pre_parts = partials + (size_t)B * vec_blocks_per_state((int)N3) * 4;
-    if (!stage_fused) {
+    if (!stage_fused && !formed) {
       rc = inl ? launch_vec_inline(pre.data(), S, n, pre_parts, res_pre, pk, pre_red, stream)
                : launch_vec(dpre, S, n, pre_parts, res_pre, pk, pre_red, stream);
       if (rc) return rc;
@@ -1215,6 +1293,8 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
                                nonfinite, stream);
     } else if (demag_approx != MT_DEMAG_DENSE) {
       rc = sparse.apply(packf, (int64_t)N3, S, 1.0f, hbuf, stream);
+    } else if (late) {
+      rc = kOk;  // rows and LL right-hand side with the next tick
     } else if (stage_fused) {
       rc = launch_stage_demag_llg_f32(K32, grid, pre.data(), ld.data(), S, stream);
     } else {
@@ -1223,7 +1303,13 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     if (rc) return rc;
     if (timing) MT_HIP(hipEventRecord(ev[4], stream));
     demag_passes += 1;
-    if (!fused && !llg_in_near) {
+    if (late) {
+      for (int k = 0; k < S; ++k) pending.sims.push_back(evals[g0 + k]);
+      pending.ld = ld;
+      pending.pre = stage_fused ? pre : std::vector<VecDesc>();
+      pending.dense = fused;
+      pending.inl = inl;
+    } else if (!fused && !llg_in_near) {
       rc = inl ? launch_llg_inline(grid, ld.data(), S, stream) : launch_llg(grid, dl, S, stream);
       if (rc) return rc;
     }
@@ -1328,6 +1414,8 @@ int Solver::run_until_idle() {
     int rc = execute_tick(evals, vecs);
     if (rc) return rc;
   }
+  int rc = flush_pending(nullptr);
+  if (rc) return rc;
   MT_HIP(hipStreamSynchronize(stream));
   arena_off = 0;
   return kOk;
@@ -1645,8 +1733,8 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
     }
     P.grid.xs = P.xs; P.grid.xe = P.xe; P.grid.xc = P.xc; P.grid.xv = P.xv;
   }
-  // state vectors: 23 per state
-  constexpr int kSlots = 23;
+  // state vectors: 24 per state
+  constexpr int kSlots = 24;
   const size_t slot = (size_t)round_up((int64_t)n3, 64);
   MT_HIP(hipMalloc(&P.pool, (size_t)P.B * kSlots * slot * sizeof(double)));
   MT_HIP(hipMemsetAsync(P.pool, 0, (size_t)P.B * kSlots * slot * sizeof(double), P.stream));
@@ -1731,6 +1819,7 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
     const size_t packed = lattice ? (size_t)lattice_state_floats(n, lattice_cols(std::min(P.B, kMaxCols)))
                                   : (size_t)P.B * n3;
     MT_HIP(hipMalloc(&P.packf, packed * sizeof(float)));
+    MT_HIP(hipMalloc(&P.packf2, packed * sizeof(float)));
     MT_HIP(hipMalloc(&P.hbuf, (size_t)P.ksplit * P.hcols * n3 * sizeof(float)));
     if (lattice) {
       MT_HIP(hipMalloc(&P.nonfinite, sizeof(int)));
@@ -1756,7 +1845,7 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
     double* base = P.pool + (size_t)b * kSlots * slot;
     int k = 0;
     auto next = [&]() { return base + (size_t)(k++) * slot; };
-    s.y = next(); s.yp = next(); s.y_old = next(); s.scratch = next(); s.errest = next(); s.weights = next();
+    s.y = next(); s.yp = next(); s.y_old = next(); s.scratch = next(); s.alt = next(); s.errest = next(); s.weights = next();
     for (int j = 1; j <= 7; ++j) s.stage[j] = next();
     s.xstage = next(); s.ytemp = next(); s.arg = next(); s.y_step = next(); s.y_last = next();
     for (int j = 1; j <= 5; ++j) s.p[j] = next();
