@@ -658,11 +658,12 @@ void rotation_matrices(const double ang[3], double* R, double* Ri) {
 }
 
 // Fortran-ordered (n,3) host arrays -> device tile records of kTileRec doubles.
-int tile_records(const mt_tiles* t, bool need_m, std::vector<double>& rec) {
+int tile_records(const mt_tiles* t, bool need_m, std::vector<double>& rec, TileKind* kind) {
   MT_CHECK(t && t->n_tiles > 0 && t->size && t->offset, "mt_tiles needs n_tiles > 0, size and offset");
   MT_CHECK(!need_m || t->M, "mt_tiles_h_field needs the tile magnetisation M");
   const int nt = t->n_tiles;
   rec.assign((size_t)nt * kTileRec, 0.0);
+  int prisms = 0, tetras = 0;
   for (int i = 0; i < nt; ++i) {
     const int type = t->tile_type ? t->tile_type[i] : 2;
     if (type != 2 && type != 5) {
@@ -695,7 +696,9 @@ int tile_records(const mt_tiles* t, bool need_m, std::vector<double>& rec) {
     rotation_matrices(ang, r + 6, r + 15);
     for (int a = 0; a < 3; ++a) r[24 + a] = r[6 + 3 * a] * M[0] + r[7 + 3 * a] * M[1] + r[8 + 3 * a] * M[2];
     r[30] = (t->use_sym && t->use_sym[i] == 1) ? 1.0 : 0.0;
+    if (r[30] == 0.0) (type == 2 ? prisms : tetras) += 1;
   }
+  *kind = prisms == nt ? TileKind::kPrism : (tetras == nt ? TileKind::kTetra : TileKind::kAny);
   return kOk;
 }
 
@@ -708,7 +711,8 @@ int mt_tiles_demag_tensor(const mt_tiles* tiles, int n_pts, const double* pts, d
   if (rc) return rc;
   MT_CHECK(n_pts > 0 && pts && N, "invalid points or output");
   std::vector<double> rec;
-  rc = tile_records(tiles, false, rec);
+  TileKind kind = TileKind::kAny;
+  rc = tile_records(tiles, false, rec, &kind);
   if (rc) return rc;
   const int nt = tiles->n_tiles;
   const size_t nN = (size_t)nt * n_pts * 9;
@@ -718,7 +722,7 @@ int mt_tiles_demag_tensor(const mt_tiles* tiles, int n_pts, const double* pts, d
   MT_HIP(dN.alloc(nN));
   MT_HIP(hipMemcpy(drec.p, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice));
   MT_HIP(hipMemcpy(dpts.p, pts, (size_t)n_pts * 3 * sizeof(double), hipMemcpyHostToDevice));
-  rc = launch_tiles_tensor(drec.p, nt, dpts.p, n_pts, dN.p, nullptr);
+  rc = launch_tiles_tensor(drec.p, nt, kind, dpts.p, n_pts, dN.p, nullptr);
   if (rc) return rc;
   MT_HIP(hipMemcpy(N, dN.p, nN * sizeof(double), hipMemcpyDeviceToHost));
   return kOk;
@@ -729,13 +733,14 @@ int mt_tiles_h_field(const mt_tiles* tiles, int n_pts, const double* pts, const 
   if (rc) return rc;
   MT_CHECK(n_pts > 0 && pts && H, "invalid points or output");
   std::vector<double> rec;
-  rc = tile_records(tiles, true, rec);
+  TileKind kind = TileKind::kAny;
+  rc = tile_records(tiles, true, rec, &kind);
   if (rc) return rc;
   const int nt = tiles->n_tiles;
   DevArr<double> drec, dpts, dN, dH;
   MT_HIP(drec.alloc(rec.size()));
   MT_HIP(dpts.alloc((size_t)n_pts * 3));
-  MT_HIP(dH.alloc((size_t)n_pts * 3));
+  MT_HIP(dH.alloc((size_t)tiles_field_plan(nt, n_pts).parts * n_pts * 3));
   MT_HIP(hipMemcpy(drec.p, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice));
   MT_HIP(hipMemcpy(dpts.p, pts, (size_t)n_pts * 3 * sizeof(double), hipMemcpyHostToDevice));
   if (N) {
@@ -743,7 +748,7 @@ int mt_tiles_h_field(const mt_tiles* tiles, int n_pts, const double* pts, const 
     MT_HIP(dN.alloc(nN));
     MT_HIP(hipMemcpy(dN.p, N, nN * sizeof(double), hipMemcpyHostToDevice));
   }
-  rc = launch_tiles_field(drec.p, nt, dpts.p, n_pts, dN.p, dH.p, nullptr);
+  rc = launch_tiles_field(drec.p, nt, kind, dpts.p, n_pts, dN.p, dH.p, nullptr);
   if (rc) return rc;
   MT_HIP(hipMemcpy(H, dH.p, (size_t)n_pts * 3 * sizeof(double), hipMemcpyDeviceToHost));
   return kOk;

@@ -13,9 +13,17 @@ int launch_assemble(const double* src, const double* abc, int abc_stride, const 
 // Magnetostatic tiles: records of kTileRec doubles (abc, offset, R, Rinv, R*M,
 // symmetry ops, symmetry flag, tile type 2 / 5, tetrahedron vertices); points
 // Fortran-ordered (npt,3); record size kTileRec (mt_common.h).
-int launch_tiles_tensor(const double* tiles, int nt, const double* pts, int npt, double* out, hipStream_t stream);
-int launch_tiles_field(const double* tiles, int nt, const double* pts, int npt, const double* Nin, double* H,
-                       hipStream_t stream);
+// kind: every tile a prism (type 2) or every tile a tetrahedron (type 5), without symmetry.
+enum class TileKind { kAny, kPrism, kTetra };
+int launch_tiles_tensor(const double* tiles, int nt, TileKind kind, const double* pts, int npt, double* out,
+                        hipStream_t stream);
+// H holds tiles_field_plan(nt, npt).parts x 3 npt doubles; the field is left in the first 3 npt.
+struct TilesFieldPlan {
+  int width, blocks, parts;
+};
+TilesFieldPlan tiles_field_plan(int nt, int npt);
+int launch_tiles_field(const double* tiles, int nt, TileKind kind, const double* pts, int npt, const double* Nin,
+                       double* H, hipStream_t stream);
 int launch_split(const float* K, int n, uint8_t* split, hipStream_t stream);
 // FP32 planes -> the dense tensor as FP32 MFMA fragments (split_tensor_bytes(n) bytes)
 int launch_f32_fragments(const float* K, int n, uint8_t* frags, hipStream_t stream);

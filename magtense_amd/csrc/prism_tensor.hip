@@ -7,12 +7,11 @@
 // and the per-pair loop of LandauLifshitzEquationSolver.f90:935-984 /
 // DemagFieldGetSolution.f90:685-730 (identity rotation: offset = p_i - c_j).
 //
-// GPU form: one thread evaluates eight consecutive source columns j of one
-// receiver row i, entirely in FP64 (the eight-term arctangent sums and the
-// logarithm ratios cancel catastrophically in the far field, so FP64 is kept
-// for every pair; the FP64 pipe of gfx950 makes this cheap relative to one
-// integration step).  The eight corner distances are shared by all six
-// components.  Results are written in up to three layouts in the same pass:
+// GPU form: everything in FP64 (the eight-term arctangent sums and the
+// logarithm ratios cancel catastrophically in the far field); the eight corner
+// distances are shared by all six components.  What bounds every kernel here is
+// the issue of FP64 instructions, so that the count of them per pair is what
+// there is to save.  Results are written in up to three layouts:
 //   * FP32 receiver-major planes K[c][i*N + j]   (the plain per-state path),
 //   * FP64 receiver-major planes                 (validation),
 //   * split BF16 hi/lo MFMA A-fragments           (the batched MFMA path).
@@ -20,6 +19,9 @@
 // serial restatement of the reference formula.
 
 #include <hip/hip_bf16.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "mt_common.h"
 #include "mt_kernels.h"
@@ -33,6 +35,28 @@ constexpr double kPi = 3.141592653589793;
 constexpr double kSclH = 1.0001, kSclL = 0.9999;
 
 __device__ inline double sq(double v) { return v * v; }
+
+// a / b and sqrt(a), rounded to nearest as the operators give them, without the
+// scaling and the special cases around the same Newton steps (8 operations for
+// 11, 13 for 19): for arguments and results in FP64's normal range, which the
+// unit of length of prism_k6 sees to; root(0) = 0.
+__device__ inline double quotient(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(y, fma(-b, y, 1.0), y);
+  y = fma(y, fma(-b, y, 1.0), y);
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+__device__ inline double root(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double s = a * y, h = 0.5 * y;
+  const double r = fma(-h, s, 0.5);
+  h = fma(h, r, h);
+  s = fma(s, r, s);
+  s = fma(fma(-s, s, a), h, s);
+  s = fma(fma(-s, s, a), h, s);
+  return a == 0.0 ? 0.0 : s;
+}
 
 // One guarded arctangent argument f/g/h: numerator p*q, denominator d*R, with
 // the "d == 0" limit rule of TileRectangularPrismTensor.f90:53-61 (the
@@ -85,68 +109,158 @@ __device__ inline void corner_terms(double a, double b, double c, double x, doub
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int k = 0; k < 2; ++k) R[i][j][k] = sqrt(sq(hx[i]) + sq(hy[j]) + sq(hz[k]));
+      for (int k = 0; k < 2; ++k) R[i][j][k] = root(sq(hx[i]) + sq(hy[j]) + sq(hz[k]));
 }
 
-__device__ inline double off_diagonal(double a, double b, double c, double x, double y, double z, int which,
-                                      double nom, double den) {
-  double v;
-  if (den == 0.0 || nom == 0.0) {
-    // getF_limit (TileRectangularPrismTensor.f90:7-38): all three coordinates scaled
-    double hx[2], hy[2], hz[2], R[2][2][2];
-    double nl, dl, nh, dh;
-    corner_terms(a, b, c, x * kSclL, y * kSclL, z * kSclL, hx, hy, hz, R);
-    log_products(hx, hy, hz, R, which, nl, dl);
-    corner_terms(a, b, c, x * kSclH, y * kSclH, z * kSclH, hx, hy, hz, R);
-    log_products(hx, hy, hz, R, which, nh, dh);
-    double lim = (0.5 * (nl + nh)) / (0.5 * (dl + dh));
-    v = -1. / (4. * kPi) * log(lim);
-  } else {
-    v = -1. / (4. * kPi) * log(nom / den);
+// getF_limit (TileRectangularPrismTensor.f90:7-38): all three coordinates scaled.
+__device__ inline double limit_ratio(double a, double b, double c, double x, double y, double z, int which) {
+  double nom = 0.0, den = 0.0;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const double f = pass == 0 ? kSclL : kSclH;
+    double hx[2], hy[2], hz[2], R[2][2][2], n, d;
+    corner_terms(a, b, c, x * f, y * f, z * f, hx, hy, hz, R);
+    log_products(hx, hy, hz, R, which, n, d);
+    nom += n;
+    den += d;
   }
-  if (fabs((nom - den) / den) < 10. * 2.220446049250313e-16) v = 0.0;
-  return v;
+  return (0.5 * nom) / (0.5 * den);
+}
+
+// The three arctangent sums term by term, each with its guard, for a point in
+// the plane of a face (some half edge - s is zero).
+__device__ inline void face_sums(const double edge[3], const double s[3], const double hx[2], const double hy[2],
+                                 const double hz[2], double sum[3]) {
+  // sign combinations in the order of TileNComponents.f90:647-649, bit q of each word:
+  // (x,y,z) (-x,y,z) (x,-y,z) (x,y,-z) (-x,-y,z) (x,-y,-z) (-x,y,-z) (-x,-y,-z)
+  sum[0] = sum[1] = sum[2] = -0.0;  // -0 + t is t, of either sign
+#pragma unroll 1
+  for (int q = 0; q < 8; ++q) {
+    const bool i = (0xd2 >> q) & 1, j = (0xb4 >> q) & 1, k = (0xe8 >> q) & 1;
+    const double u = i ? hx[1] : hx[0], v = j ? hy[1] : hy[0], w = k ? hz[1] : hz[0];
+    const double r = sqrt(sq(u) + sq(v) + sq(w));
+    sum[0] += atan(guarded_ratio(edge[0] / 2., i ? -s[0] : s[0], v, w, u, r, 0));
+    sum[1] += atan(guarded_ratio(edge[1] / 2., j ? -s[1] : s[1], u, w, v, r, 1));
+    sum[2] += atan(guarded_ratio(edge[2] / 2., k ? -s[2] : s[2], u, v, w, r, 2));
+  }
+}
+
+// An angle in (-2 pi, 2 pi) as the direction (re, im) and the whole turns that
+// the direction leaves out: angle = atan2(im, re) + 2 pi turns.
+struct Turned {
+  double re, im, turns;
+};
+
+__device__ inline Turned plus(const Turned& s, const Turned& t) {
+  Turned o;
+  o.re = fma(s.re, t.re, -(s.im * t.im));
+  o.im = fma(s.re, t.im, s.im * t.re) + 0.0;  // -0 -> +0: a half turn is +pi
+  o.turns = s.turns + t.turns;
+  // two angles of (0, pi] that pass pi, or two of (-pi, 0) that pass -pi: there the
+  // imaginary part is a sum of like signs, so that its sign is the sine's
+  const bool sp = s.im > 0.0 || (s.im == 0.0 && s.re < 0.0), tp = t.im > 0.0 || (t.im == 0.0 && t.re < 0.0);
+  if (sp && tp && (o.im < 0.0 || (o.im == 0.0 && o.re > 0.0))) o.turns += 1.0;
+  if (s.im < 0.0 && t.im < 0.0 && o.im >= 0.0) o.turns -= 1.0;
+  return o;
+}
+
+// sum over the eight corners of atan(p q / (d R)): the arguments of the numbers
+// |d| R + i p q (in (-pi/2, pi/2)) add up in their product, so that one
+// arctangent and no division take the place of eight of each.  d: the two face
+// distances along the axis; p, q along the others; r[i][j][k] with i along d.
+// The error is that of the products, about as many roundings as the eight
+// arctangents and their sum had (measured: at prism_k6).
+__device__ inline double corner_angle(const double d[2], const double p[2], const double q[2],
+                                      const double r[2][2][2]) {
+  Turned side[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const double m = fabs(d[i]);
+    auto pair = [&](int j) {  // two arguments: in (-pi, pi), no turn to count
+      const double re0 = m * r[i][j][0], im0 = p[j] * q[0], re1 = m * r[i][j][1], im1 = p[j] * q[1];
+      return Turned{fma(re0, re1, -(im0 * im1)), fma(re0, im1, im0 * re1), 0.0};
+    };
+    side[i] = plus(pair(0), pair(1));
+    if (d[i] < 0.0) {  // atan is odd; a half turn (im == 0, re < 0) becomes -pi
+      if (side[i].im == 0.0 && side[i].re < 0.0) side[i].turns += 1.0;
+      side[i].turns = -side[i].turns;
+      side[i].im = 0.0 - side[i].im;
+    }
+  }
+  const Turned t = plus(side[0], side[1]);
+  return atan2(t.im, t.re) + 2. * kPi * t.turns;
 }
 
 }  // namespace
 
 // K = -N_standard for a prism with full edges (a,b,c) at offset (x,y,z) from
-// its centre.  out: xx, xy, xz, yy, yz, zz.
+// its centre.  out: xx, xy, xz, yy, yz, zz.  Two forms of the diagonal:
+//   PRODUCT = false: the reference's eight arctangents each, in its order.  The
+//     assembled tensors use it: a far diagonal entry is what is left of angles
+//     of order one, so that any other rounding (a better one too) changes the
+//     last FP32 bit of 0.1 % (a film) to 10 % (300 cells away) of the entries,
+//     and with them every result computed from a tensor.
+//   PRODUCT = true: corner_angle.  Against 80-bit arithmetic over cells, films,
+//     plates, needles, points inside, near and on faces and 1e6 edges away its
+//     largest error is 0.4 to 0.9 of the other form's and its root mean square
+//     half (2e-18 to 3e-17 against 1e-17 to 6e-17).
+template <bool PRODUCT>
 __device__ void prism_k6(double a, double b, double c, double x, double y, double z, double out[6]) {
+  // The tensor has no unit of length, and a power of two leaves every rounding
+  // as it is: the largest length comes to [1/2, 1), where no square, quotient or
+  // product of corner terms leaves FP64's normal range.
+  const double largest = fmax(fmax(fmax(fabs(a), fabs(b)), fmax(fabs(c), fabs(x))), fmax(fabs(y), fabs(z)));
+  const double unit = ldexp(1.0, -max(__builtin_amdgcn_frexp_exp(largest), -1000));
+  a *= unit; b *= unit; c *= unit; x *= unit; y *= unit; z *= unit;
   double hx[2], hy[2], hz[2], R[2][2][2];
   corner_terms(a, b, c, x, y, z, hx, hy, hz, R);
-  double sx[2] = {x, -x}, sy[2] = {y, -y}, sz[2] = {z, -z};
-  // sign combinations in the order of TileNComponents.f90:647-649:
-  // (x,y,z) (-x,y,z) (x,-y,z) (x,y,-z) (-x,-y,z) (x,-y,-z) (-x,y,-z) (-x,-y,-z)
-  const int cmb[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 0}, {0, 1, 1}, {1, 0, 1}, {1, 1, 1}};
-  double sxx = 0.0, syy = 0.0, szz = 0.0;
+  double sum[3];
+  if (hx[0] == 0.0 || hx[1] == 0.0 || hy[0] == 0.0 || hy[1] == 0.0 || hz[0] == 0.0 || hz[1] == 0.0) {
+    const double edge[3] = {a, b, c}, s[3] = {x, y, z};
+    face_sums(edge, s, hx, hy, hz, sum);
+  } else if constexpr (PRODUCT) {
+    double ry[2][2][2], rz[2][2][2];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    int i = cmb[q][0], j = cmb[q][1], k = cmb[q][2];
-    double r = R[i][j][k];
-    double fx = guarded_ratio(a / 2., sx[i], hy[j], hz[k], hx[i], r, 0);
-    double fy = guarded_ratio(b / 2., sy[j], hx[i], hz[k], hy[j], r, 1);
-    double fz = guarded_ratio(c / 2., sz[k], hx[i], hy[j], hz[k], r, 2);
-    sxx = (q == 0) ? atan(fx) : sxx + atan(fx);
-    syy = (q == 0) ? atan(fy) : syy + atan(fy);
-    szz = (q == 0) ? atan(fz) : szz + atan(fz);
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          ry[j][i][k] = R[i][j][k];
+          rz[k][i][j] = R[i][j][k];
+        }
+    sum[0] = corner_angle(hx, hy, hz, R);
+    sum[1] = corner_angle(hy, hx, hz, ry);
+    sum[2] = corner_angle(hz, hx, hy, rz);
+  } else {
+    // in the order of face_sums
+    const int cmb[8][3] = {{0, 0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 0}, {0, 1, 1}, {1, 0, 1}, {1, 1, 1}};
+    sum[0] = sum[1] = sum[2] = -0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = cmb[q][0], j = cmb[q][1], k = cmb[q][2];
+      const double r = R[i][j][k];
+      sum[0] += atan(quotient(hy[j] * hz[k], hx[i] * r));
+      sum[1] += atan(quotient(hx[i] * hz[k], hy[j] * r));
+      sum[2] += atan(quotient(hx[i] * hy[j], hz[k] * r));
+    }
   }
-  double nxx = 1. / (4. * kPi) * sxx;
-  double nyy = 1. / (4. * kPi) * syy;
-  double nzz = 1. / (4. * kPi) * szz;
-  double nm, dn;
-  log_products(hx, hy, hz, R, 0, nm, dn);
-  double nxy = off_diagonal(a, b, c, x, y, z, 0, nm, dn);
-  log_products(hx, hy, hz, R, 1, nm, dn);
-  double nyz = off_diagonal(a, b, c, x, y, z, 1, nm, dn);
-  log_products(hx, hy, hz, R, 2, nm, dn);
-  double nxz = off_diagonal(a, b, c, x, y, z, 2, nm, dn);
-  out[0] = -nxx;
-  out[1] = -nxy;
-  out[2] = -nxz;
-  out[3] = -nyy;
-  out[4] = -nyz;
-  out[5] = -nzz;
+  double off[3];
+#pragma unroll
+  for (int which = 0; which < 3; ++which) {
+    double nom, den;
+    log_products(hx, hy, hz, R, which, nom, den);
+    double ratio = quotient(nom, den);
+    if (den == 0.0 || nom == 0.0) ratio = limit_ratio(a, b, c, x, y, z, which);
+    off[which] = -1. / (4. * kPi) * log(ratio);
+    if (fabs(nom - den) < 10. * 2.220446049250313e-16 * fabs(den)) off[which] = 0.0;
+  }
+  out[0] = -(1. / (4. * kPi) * sum[0]);
+  out[1] = -off[0];
+  out[2] = -off[2];
+  out[3] = -(1. / (4. * kPi) * sum[1]);
+  out[4] = -off[1];
+  out[5] = -(1. / (4. * kPi) * sum[2]);
 }
 
 namespace {
@@ -170,43 +284,69 @@ __device__ inline int64_t frag_offset(int64_t np, int64_t i, int64_t j, int c, i
   return frag * kFragBytes + (int64_t)lane * 16;
 }
 
+// Offset of point p from prism j, in the prism's axes: diffPos = rotMat (p - offset),
+// DemagFieldGetSolution.f90:705-709.
+__device__ inline void prism_offset(const double* __restrict__ src, const double* __restrict__ rot, int64_t j,
+                                    const double p[3], double d[3]) {
+  const double* s = src + j * 3;
+  const double dx = p[0] - s[0], dy = p[1] - s[1], dz = p[2] - s[2];
+  d[0] = dx; d[1] = dy; d[2] = dz;
+  if (rot) {
+    const double* R = rot + j * 9;
+    for (int r = 0; r < 3; ++r) d[r] = R[3 * r] * dx + R[3 * r + 1] * dy + R[3 * r + 2] * dz;
+  }
+}
+
+// Receiver-major planes alone: one thread per pair, the lanes along j, so that
+// every store is one line.  16384 x 16384 pairs to FP32: 14.8 ms, where eight
+// columns to a thread, a branch around each of the 24 quotients and the scaled
+// forms of quotient and root took 17.3 (122 registers for 200, no scratch).
+__global__ void __launch_bounds__(256) assemble_planes_kernel(const double* __restrict__ src,
+                                                              const double* __restrict__ abc, int abc_stride,
+                                                              const double* __restrict__ rot,
+                                                              const double* __restrict__ pts, int n_src, int n_pts,
+                                                              int64_t first, float* __restrict__ out32,
+                                                              double* __restrict__ out64) {
+  const int64_t pair = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = pair / n_src, j = pair - i * n_src;
+  if (i >= n_pts) return;
+  double d[3], k6[6];
+  prism_offset(src, rot, j, pts + i * 3, d);
+  const double* e = abc + j * abc_stride;
+  prism_k6<false>(e[0], e[1], e[2], d[0], d[1], d[2], k6);
+  const size_t plane = (size_t)n_pts * n_src;
+  for (int c = 0; c < 6; ++c) {
+    if (out32) out32[c * plane + pair] = (float)k6[c];
+    if (out64) out64[c * plane + pair] = k6[c];
+  }
+}
+
 __global__ void __launch_bounds__(256) assemble_kernel(const double* __restrict__ src, const double* __restrict__ abc,
                                                        int abc_stride, const double* __restrict__ rot,
                                                        const double* __restrict__ pts, int n_src,
                                                        int n_pts, int64_t np, float* __restrict__ out32,
                                                        double* __restrict__ out64, uint8_t* __restrict__ split) {
-  // Thread -> (row i, 8 columns starting at j0); for the split layout the grid
-  // covers the padded rows x padded sources (np = round_up(n_src, 32)).
-  int64_t groups_per_row = (split ? np : round_up(n_src, 8)) / 8;
+  // Thread -> (row i, 8 columns starting at j0) over the padded rows x padded
+  // sources (np = round_up(n_src, 32)) of the split layout.
+  int64_t groups_per_row = np / 8;
   int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t i = tid / groups_per_row;
   int64_t j0 = (tid % groups_per_row) * 8;
-  int64_t rows = split ? round_up(n_pts, kTileM) : n_pts;
-  if (i >= rows) return;
+  if (i >= round_up(n_pts, kTileM)) return;
   float v32[6][8];
   bool row_ok = i < n_pts;
-  double px = 0, py = 0, pz = 0;
-  if (row_ok) {
-    px = pts[i * 3 + 0];
-    py = pts[i * 3 + 1];
-    pz = pts[i * 3 + 2];
-  }
+  double p[3] = {0, 0, 0};
+  if (row_ok)
+    for (int r = 0; r < 3; ++r) p[r] = pts[i * 3 + r];
   for (int e = 0; e < 8; ++e) {
     int64_t j = j0 + e;
     double k6[6] = {0, 0, 0, 0, 0, 0};
     bool ok = row_ok && j < n_src;
     if (ok) {
-      const double* s = src + j * 3;
       const double* d = abc + j * abc_stride;
-      double dx = px - s[0], dy = py - s[1], dz = pz - s[2];
-      if (rot) {  // diffPos = rotMat (p - offset), DemagFieldGetSolution.f90:705-709
-        const double* R = rot + j * 9;
-        double rx = R[0] * dx + R[1] * dy + R[2] * dz;
-        double ry = R[3] * dx + R[4] * dy + R[5] * dz;
-        double rz = R[6] * dx + R[7] * dy + R[8] * dz;
-        dx = rx; dy = ry; dz = rz;
-      }
-      prism_k6(d[0], d[1], d[2], dx, dy, dz, k6);
+      double off[3];
+      prism_offset(src, rot, j, p, off);
+      prism_k6<false>(d[0], d[1], d[2], off[0], off[1], off[2], k6);
       if (out64) {
         size_t plane = (size_t)n_pts * n_src;
         for (int c = 0; c < 6; ++c) out64[c * plane + (size_t)i * n_src + j] = k6[c];
@@ -220,21 +360,19 @@ __global__ void __launch_bounds__(256) assemble_kernel(const double* __restrict_
       for (int e = 0; e < 8; ++e)
         if (j0 + e < n_src) out32[c * plane + (size_t)i * n_src + j0 + e] = v32[c][e];
   }
-  if (split) {
-    for (int c = 0; c < 6; ++c) {
-      uint16_t hi[8], lo[8];
-      for (int e = 0; e < 8; ++e) {
-        hi[e] = bf16_bits(v32[c][e]);
-        lo[e] = bf16_bits(v32[c][e] - bf16_value(hi[e]));
-      }
-      uint4 h4, l4;
-      h4.x = hi[0] | ((uint32_t)hi[1] << 16); h4.y = hi[2] | ((uint32_t)hi[3] << 16);
-      h4.z = hi[4] | ((uint32_t)hi[5] << 16); h4.w = hi[6] | ((uint32_t)hi[7] << 16);
-      l4.x = lo[0] | ((uint32_t)lo[1] << 16); l4.y = lo[2] | ((uint32_t)lo[3] << 16);
-      l4.z = lo[4] | ((uint32_t)lo[5] << 16); l4.w = lo[6] | ((uint32_t)lo[7] << 16);
-      *reinterpret_cast<uint4*>(split + frag_offset(np, i, j0, c, 0)) = h4;
-      *reinterpret_cast<uint4*>(split + frag_offset(np, i, j0, c, 1)) = l4;
+  for (int c = 0; c < 6; ++c) {
+    uint16_t hi[8], lo[8];
+    for (int e = 0; e < 8; ++e) {
+      hi[e] = bf16_bits(v32[c][e]);
+      lo[e] = bf16_bits(v32[c][e] - bf16_value(hi[e]));
     }
+    uint4 h4, l4;
+    h4.x = hi[0] | ((uint32_t)hi[1] << 16); h4.y = hi[2] | ((uint32_t)hi[3] << 16);
+    h4.z = hi[4] | ((uint32_t)hi[5] << 16); h4.w = hi[6] | ((uint32_t)hi[7] << 16);
+    l4.x = lo[0] | ((uint32_t)lo[1] << 16); l4.y = lo[2] | ((uint32_t)lo[3] << 16);
+    l4.z = lo[4] | ((uint32_t)lo[5] << 16); l4.w = lo[6] | ((uint32_t)lo[7] << 16);
+    *reinterpret_cast<uint4*>(split + frag_offset(np, i, j0, c, 0)) = h4;
+    *reinterpret_cast<uint4*>(split + frag_offset(np, i, j0, c, 1)) = l4;
   }
 }
 
@@ -270,7 +408,7 @@ __global__ void __launch_bounds__(256) toeplitz_assemble_kernel(int nx, int ny, 
     const int iy = dyi > 0 ? dyi : 0, jy = dyi > 0 ? 0 : -dyi;
     const int iz = dzi > 0 ? dzi : 0, jz = dzi > 0 ? 0 : -dzi;
     double k6[6];
-    prism_k6(dx, dy, dz, centre(nx, Lx, dx, ix) - centre(nx, Lx, dx, jx), centre(ny, Ly, dy, iy) - centre(ny, Ly, dy, jy),
+    prism_k6<false>(dx, dy, dz, centre(nx, Lx, dx, ix) - centre(nx, Lx, dx, jx), centre(ny, Ly, dy, iy) - centre(ny, Ly, dy, jy),
              centre(nz, Lz, dz, iz) - centre(nz, Lz, dz, jz), k6);
     for (int c = 0; c < 6; ++c) v32[c][e] = (float)k6[c];
   }
@@ -503,7 +641,30 @@ __device__ bool tetra_n(const double* __restrict__ vert, const double r[3], doub
 // eight mirrored evaluations of getFieldFromTile_symm (:744-822).  The symmetry
 // matrices of getSymmOpMatrices (:833-896) are a signed identity (for M) and a
 // diagonal mirror (for H and the point), applied here as sign products.
+// KIND: every tile a prism, or every tile a tetrahedron, without symmetry (the
+// kernels for any tile hold both formulas: 260 registers, one wave per SIMD,
+// against 90 with prisms alone).
+template <TileKind KIND>
 __device__ void tile_tensor(const double* __restrict__ T, double px, double py, double pz, double N[9]) {
+  if constexpr (KIND != TileKind::kAny) {
+    const double* R = T + 6;
+    const double dx = px - T[3], dy = py - T[4], dz = pz - T[5];
+    const double rx = R[0] * dx + R[1] * dy + R[2] * dz;
+    const double ry = R[3] * dx + R[4] * dy + R[5] * dz;
+    const double rz = R[6] * dx + R[7] * dy + R[8] * dz;
+    if constexpr (KIND == TileKind::kTetra) {
+      const double r3[3] = {rx, ry, rz};
+      if (!tetra_n(T + 32, r3, N))
+        for (int q = 0; q < 9; ++q) N[q] = __builtin_nan("");
+    } else {
+      double k[6];
+      prism_k6<true>(T[0], T[1], T[2], rx, ry, rz, k);
+      N[0] = k[0]; N[1] = k[1]; N[2] = k[2];
+      N[3] = k[1]; N[4] = k[3]; N[5] = k[4];
+      N[6] = k[2]; N[7] = k[4]; N[8] = k[5];
+    }
+    return;
+  }
   const double* R = T + 6;
   const bool tetra = T[31] == 5.0;
   int sym = T[30] != 0.0;
@@ -529,7 +690,7 @@ __device__ void tile_tensor(const double* __restrict__ T, double px, double py, 
         for (int q = 0; q < 9; ++q) full[q] = __builtin_nan("");
     } else {
       double k[6];
-      prism_k6(T[0], T[1], T[2], rx, ry, rz, k);
+      prism_k6<true>(T[0], T[1], T[2], rx, ry, rz, k);
       full[0] = k[0]; full[1] = k[1]; full[2] = k[2];
       full[3] = k[1]; full[4] = k[3]; full[5] = k[4];
       full[6] = k[2]; full[7] = k[4]; full[8] = k[5];
@@ -545,39 +706,50 @@ __device__ void tile_tensor(const double* __restrict__ T, double px, double py, 
 }
 
 // out: N(n_tiles, n_pts, 3, 3) in Fortran order, (i,p,a,b) at i + nt*(p + np*(a + 3b)).
+// One thread per (tile, point) pair, tiles fastest: full waves whatever the
+// number of tiles, and stores of consecutive values.  20 prisms at 400 points:
+// 7 us (10 with a block per 256 tiles and point).
+template <TileKind KIND>
 __global__ void __launch_bounds__(256) tiles_tensor_kernel(const double* __restrict__ tiles, int nt,
                                                            const double* __restrict__ pts, int npt,
                                                            double* __restrict__ out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nt) return;
-  const double* T = tiles + (size_t)i * kTileRec;
-  for (int p = blockIdx.y; p < npt; p += gridDim.y) {
-    double N[9];
-    tile_tensor(T, pts[p], pts[p + (size_t)npt], pts[p + 2 * (size_t)npt], N);
-    for (int a = 0; a < 3; ++a)
-      for (int b = 0; b < 3; ++b) out[i + (size_t)nt * (p + (size_t)npt * (a + 3 * b))] = N[a * 3 + b];
-  }
+  const int64_t pairs = (int64_t)nt * npt;
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= pairs) return;
+  const int p = (int)(e / nt), i = (int)(e - (int64_t)p * nt);
+  double N[9];
+  tile_tensor<KIND>(tiles + (size_t)i * kTileRec, pts[p], pts[p + (size_t)npt], pts[p + 2 * (size_t)npt], N);
+  for (int a = 0; a < 3; ++a)
+    for (int b = 0; b < 3; ++b) out[e + pairs * (a + 3 * b)] = N[a * 3 + b];
 }
 
 // H(p) = sum_i Rinv_i (N_ip (R_i M_i)) (getDotProd, :909-918, and the
-// back-rotation, :721-726).  One block per point, threads stride over tiles,
-// fixed-order tree reduction.  Nin (Fortran-ordered as above) replaces the
-// tensor evaluation when given (useStoredN).
-__global__ void __launch_bounds__(256) tiles_field_kernel(const double* __restrict__ tiles, int nt,
-                                                          const double* __restrict__ pts, int npt,
-                                                          const double* __restrict__ Nin, double* __restrict__ H) {
+// back-rotation, :721-726).  A block holds 256 / width points; width threads
+// (a power of two) stride over a point's tiles i = z * width + t, z from
+// blockIdx.y in steps of gridDim.y, and add up in a fixed tree: part z goes to
+// H + z * 3 * npt.  Nin (Fortran-ordered as above) replaces the tensor
+// evaluation when given (useStoredN).
+//
+// 6000 prisms at 5000 points: 1.1 ms (FP64 issue; 135 registers, three waves per
+// SIMD), 3.6 with both formulas in one kernel and 24 arctangents per prism.
+template <TileKind KIND>
+__global__ void __launch_bounds__(256, KIND == TileKind::kPrism ? 3 : 1)
+    tiles_field_kernel(const double* __restrict__ tiles, int nt, const double* __restrict__ pts, int npt, int width,
+                       const double* __restrict__ Nin, double* __restrict__ H) {
   __shared__ double red[3][256];
-  for (int p = blockIdx.x; p < npt; p += gridDim.x) {
-    double px = pts[p], py = pts[p + (size_t)npt], pz = pts[p + 2 * (size_t)npt];
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) {
+  const int t = threadIdx.x % width;
+  const int p = blockIdx.x * (256 / width) + threadIdx.x / width;
+  double acc[3] = {0.0, 0.0, 0.0};
+  if (p < npt) {
+    const double px = pts[p], py = pts[p + (size_t)npt], pz = pts[p + 2 * (size_t)npt];
+    for (int64_t i = (int64_t)blockIdx.y * width + t; i < nt; i += (int64_t)gridDim.y * width) {
       const double* T = tiles + (size_t)i * kTileRec;
       double N[9];
       if (Nin) {
         for (int a = 0; a < 3; ++a)
           for (int b = 0; b < 3; ++b) N[a * 3 + b] = Nin[i + (size_t)nt * (p + (size_t)npt * (a + 3 * b))];
       } else {
-        tile_tensor(T, px, py, pz, N);
+        tile_tensor<KIND>(T, px, py, pz, N);
       }
       const double* Ri = T + 15;
       const double* RM = T + 24;
@@ -588,47 +760,99 @@ __global__ void __launch_bounds__(256) tiles_field_kernel(const double* __restri
       acc[1] += Ri[3] * d0 + Ri[4] * d1 + Ri[5] * d2;
       acc[2] += Ri[6] * d0 + Ri[7] * d1 + Ri[8] * d2;
     }
-    for (int a = 0; a < 3; ++a) red[a][threadIdx.x] = acc[a];
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w)
-        for (int a = 0; a < 3; ++a) red[a][threadIdx.x] += red[a][threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0)
-      for (int a = 0; a < 3; ++a) H[p + (size_t)npt * a] = red[a][0];
+  }
+  for (int a = 0; a < 3; ++a) red[a][threadIdx.x] = acc[a];
+  __syncthreads();
+  for (int w = width / 2; w > 0; w >>= 1) {
+    if (t < w)
+      for (int a = 0; a < 3; ++a) red[a][threadIdx.x] += red[a][threadIdx.x + w];
     __syncthreads();
   }
+  if (t == 0 && p < npt)
+    for (int a = 0; a < 3; ++a) H[(size_t)blockIdx.y * 3 * npt + p + (size_t)npt * a] = red[a][threadIdx.x];
+}
+
+// H[e] = sum over the parts, in order (in place in part 0)
+__global__ void __launch_bounds__(256) tiles_field_sum_kernel(double* __restrict__ H, int parts, int64_t total) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= total) return;
+  double s = H[e];
+  for (int z = 1; z < parts; ++z) s += H[(int64_t)z * total + e];
+  H[e] = s;
 }
 
 }  // namespace
 
 // Host launchers -------------------------------------------------------------
 
-int launch_tiles_tensor(const double* tiles, int nt, const double* pts, int npt, double* out, hipStream_t stream) {
+namespace {
+template <class F>
+void by_kind(TileKind kind, F&& go) {
+  switch (kind) {
+    case TileKind::kPrism: go(std::integral_constant<TileKind, TileKind::kPrism>{}); break;
+    case TileKind::kTetra: go(std::integral_constant<TileKind, TileKind::kTetra>{}); break;
+    default: go(std::integral_constant<TileKind, TileKind::kAny>{}); break;
+  }
+}
+}  // namespace
+
+int launch_tiles_tensor(const double* tiles, int nt, TileKind kind, const double* pts, int npt, double* out,
+                        hipStream_t stream) {
   if (nt <= 0 || npt <= 0) return kOk;
-  dim3 grid((unsigned)((nt + 255) / 256), (unsigned)(npt < 65535 ? npt : 65535));
-  hipLaunchKernelGGL(tiles_tensor_kernel, grid, dim3(256), 0, stream, tiles, nt, pts, npt, out);
+  const dim3 grid((unsigned)(((int64_t)nt * npt + 255) / 256));
+  by_kind(kind, [&](auto k) {
+    hipLaunchKernelGGL(tiles_tensor_kernel<decltype(k)::value>, grid, dim3(256), 0, stream, tiles, nt, pts, npt, out);
+  });
   MT_HIP(hipGetLastError());
   return kOk;
 }
 
-int launch_tiles_field(const double* tiles, int nt, const double* pts, int npt, const double* Nin, double* H,
-                       hipStream_t stream) {
+// Threads of a point: the tiles, up to a block.  Parts of a point's tiles: as
+// many as give the chip 2048 blocks (256 CUs, two or three of these blocks on
+// each, several rounds), while every thread keeps a tile.
+TilesFieldPlan tiles_field_plan(int nt, int npt) {
+  TilesFieldPlan q;
+  q.width = 1;
+  while (q.width < 256 && q.width < nt) q.width *= 2;
+  q.blocks = (int)(((int64_t)npt * q.width + 255) / 256);
+  const int64_t most = (nt + q.width - 1) / q.width;
+  q.parts = (int)std::max<int64_t>(1, std::min<int64_t>(most, 2048 / std::max(q.blocks, 1)));
+  return q;
+}
+
+int launch_tiles_field(const double* tiles, int nt, TileKind kind, const double* pts, int npt, const double* Nin,
+                       double* H, hipStream_t stream) {
   if (npt <= 0) return kOk;
-  unsigned blocks = (unsigned)(npt < 65535 ? npt : 65535);
-  hipLaunchKernelGGL(tiles_field_kernel, dim3(blocks), dim3(256), 0, stream, tiles, nt, pts, npt, Nin, H);
+  const TilesFieldPlan q = tiles_field_plan(nt, npt);
+  const dim3 grid((unsigned)q.blocks, (unsigned)q.parts);
+  by_kind(kind, [&](auto k) {
+    hipLaunchKernelGGL(tiles_field_kernel<decltype(k)::value>, grid, dim3(256), 0, stream, tiles, nt, pts, npt, q.width,
+                       Nin, H);
+  });
   MT_HIP(hipGetLastError());
+  if (q.parts > 1) {
+    const int64_t total = (int64_t)3 * npt;
+    hipLaunchKernelGGL(tiles_field_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, H, q.parts,
+                       total);
+    MT_HIP(hipGetLastError());
+  }
   return kOk;
 }
 
 int launch_assemble(const double* src, const double* abc, int abc_stride, const double* rot, const double* pts,
                     int n_src, int n_pts, float* out32, double* out64, uint8_t* split, hipStream_t stream) {
-  int64_t np = round_up(n_src, kTileM);
-  int64_t groups_per_row = (split ? np : round_up(n_src, 8)) / 8;
-  int64_t rows = split ? round_up(n_pts, kTileM) : n_pts;
-  int64_t threads = rows * groups_per_row;
-  int64_t blocks = (threads + 255) / 256;
+  if (!split) {
+    const int64_t pairs = (int64_t)n_pts * n_src, most = 1ll << 31;  // a grid holds fewer than 2^32 threads
+    for (int64_t first = 0; first < pairs; first += most) {
+      const int64_t blocks = (std::min(pairs - first, most) + 255) / 256;
+      hipLaunchKernelGGL(assemble_planes_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, src, abc, abc_stride,
+                         rot, pts, n_src, n_pts, first, out32, out64);
+      MT_HIP(hipGetLastError());
+    }
+    return kOk;
+  }
+  const int64_t np = round_up(n_src, kTileM);
+  const int64_t blocks = (round_up(n_pts, kTileM) * (np / 8) + 255) / 256;
   hipLaunchKernelGGL(assemble_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, src, abc, abc_stride, rot, pts,
                      n_src, n_pts, np, out32, out64, split);
   MT_HIP(hipGetLastError());
@@ -660,7 +884,7 @@ __global__ void __launch_bounds__(256) assemble_avg_kernel(const double* __restr
       for (int ia = 1; ia <= nax; ++ia) {
         const double px = bx + dx * ia, py = by + dy * ja, pz = bz + dz * ka;
         double k6[6];
-        prism_k6(a[0], a[1], a[2], px - cx, py - cy, pz - cz, k6);
+        prism_k6<false>(a[0], a[1], a[2], px - cx, py - cy, pz - cz, k6);
         for (int c = 0; c < 6; ++c) acc[c] += k6[c];
       }
   const double cnt = (double)(nax * nay * naz);
@@ -729,7 +953,7 @@ __global__ void __launch_bounds__(256) lattice_entries_kernel(const double* __re
   if (e >= total) return;
   const int64_t row = e / ux;
   double k6[6];
-  prism_k6(dx, dy, dz, x[e - row * ux], y[row % uy], z[row / uy], k6);
+  prism_k6<false>(dx, dy, dz, x[e - row * ux], y[row % uy], z[row / uy], k6);
   a[e] = make_float4((float)k6[0], (float)k6[1], (float)k6[3], (float)k6[5]);
   if (b) b[e] = make_float2((float)k6[2], (float)k6[4]);
 }
@@ -779,7 +1003,7 @@ __global__ void near_table_kernel(int nx, int ny, int nz, double Lx, double Ly, 
   const int iy = oy > 0 ? oy : 0, jy = oy > 0 ? 0 : -oy;
   const int iz = oz > 0 ? oz : 0, jz = oz > 0 ? 0 : -oz;
   double k6[6];
-  prism_k6(dx, dy, dz, centre(nx, Lx, dx, ix) - centre(nx, Lx, dx, jx), centre(ny, Ly, dy, iy) - centre(ny, Ly, dy, jy),
+  prism_k6<false>(dx, dy, dz, centre(nx, Lx, dx, ix) - centre(nx, Lx, dx, jx), centre(ny, Ly, dy, iy) - centre(ny, Ly, dy, jy),
            centre(nz, Lz, dz, iz) - centre(nz, Lz, dz, jz), k6);
   float k32[6];
   for (int c = 0; c < 6; ++c) {
