@@ -92,12 +92,15 @@ __device__ __forceinline__ float wave_tree_sum(float v) {
   return add_row_ror<1>(v);
 }
 
+constexpr int kRowThreads = 256;  // of matvec_rows_f32
+
 // Rows i0 .. i0 + RB - 1 of (K m) for S states m + s * m_stride (x, then y, then
 // z of all cells) with a block of 256 threads: every thread sums its columns
 // over the six receiver-major planes, then a tree per wave and the four waves
 // in order; the tensor is read once for the S states, each of which sums as it
 // would alone.  On return (after a barrier) sums[(s * RB + r) * 3 + c] holds
-// component c of row i0 + r; red is the block's scratch.  States from `have` on
+// component c of row i0 + r; red is the block's scratch.  Two barriers, which
+// further waves of the block meet by themselves.  States from `have` on
 // repeat the last one.
 // NT: non-temporal tensor loads, for a tensor that the launch reads once, so that
 // it does not displace the state vectors from L2.
