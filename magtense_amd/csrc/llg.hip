@@ -292,12 +292,13 @@ __device__ __forceinline__ void accumulate(double (&acc)[E], int cnt, PF ptr, CF
   }
 }
 
-// INL: descriptors by value (inl) instead of from descs.  With one block
-// per state the block's reduction is the result (written to results).
+// INL: descriptors by value (inl) instead of from descs.  A block's reduction
+// goes to the host (lines), or to partials; with one block per state it is the
+// result (written to results).
 template <bool INL, int T, int E>
 __global__ void __launch_bounds__(T) vec_kernel(const VecDesc* __restrict__ descs, VecDescsInline inl, int n, int n3,
                                                 int blocks_per_state, double* __restrict__ partials,
-                                                double* __restrict__ results, PackSpec pack) {
+                                                double* __restrict__ results, ResultLines lines, PackSpec pack) {
   static_assert(T * E == 2048, "a block's elements");
   const VecDesc& D = INL ? inl.d[blockIdx.y] : descs[blockIdx.y];
   const int t0 = blockIdx.x * 2048;
@@ -524,7 +525,12 @@ __global__ void __launch_bounds__(T) vec_kernel(const VecDesc* __restrict__ desc
     int k = threadIdx.x;
     double x = red[0][k];
     for (int w = 1; w < T / 64; ++w) x = is_sum ? x + red[w][k] : fmax(x, red[w][k]);
-    if (blocks_per_state == 1 && results) results[D.rslot * 4 + k] = x;
+    if (lines.base) {
+      ResultLine* l = lines.base + (int64_t)D.rslot * lines.stride + blockIdx.x;
+      l->v[k] = x;
+      __threadfence_system();  // the four lanes' values before the number
+      if (k == 0) __hip_atomic_store(&l->seq, lines.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else if (blocks_per_state == 1 && results) results[D.rslot * 4 + k] = x;
     else partials[((int64_t)blockIdx.y * blocks_per_state + blockIdx.x) * 4 + k] = x;
   }
 }
@@ -592,18 +598,18 @@ constexpr int kVecWideBlocks = 256;
 
 template <bool INL>
 int launch_vec_t(const VecDesc* descs, const VecDescsInline& inl, int nstates, int n, double* partials,
-                 double* results, const PackSpec& pack, bool reduce, hipStream_t stream) {
+                 double* results, const PackSpec& pack, bool reduce, hipStream_t stream, const ResultLines& lines) {
   int n3 = 3 * n;
   int bps = vec_blocks_per_state(n3);
   dim3 grid((unsigned)bps, (unsigned)nstates);
   if ((int64_t)bps * nstates <= kVecWideBlocks)
     hipLaunchKernelGGL((vec_kernel<INL, 1024, 2>), grid, dim3(1024), 0, stream, descs, inl, n, n3, bps, partials,
-                       results, pack);
+                       results, lines, pack);
   else
     hipLaunchKernelGGL((vec_kernel<INL, 256, 8>), grid, dim3(256), 0, stream, descs, inl, n, n3, bps, partials, results,
-                       pack);
+                       lines, pack);
   MT_HIP(hipGetLastError());
-  if (reduce && bps > 1) {
+  if (reduce && bps > 1 && !lines.base) {
     int t = nstates * 4;
     hipLaunchKernelGGL(finalize_kernel<INL>, dim3((unsigned)((t + 127) / 128)), dim3(128), 0, stream, descs, inl,
                        nstates, bps, partials, results);
@@ -714,19 +720,19 @@ int launch_stage_demag_llg_f32(const float* K, const LlgGrid& g, const VecDesc* 
 int vec_blocks_per_state(int n3) { return (n3 + 256 * 8 - 1) / (256 * 8); }
 
 int launch_vec(const VecDesc* d_descs, int nstates, int n, double* partials, double* results, const PackSpec& pack,
-               bool reduce, hipStream_t stream) {
-  return launch_vec_t<false>(d_descs, VecDescsInline{}, nstates, n, partials, results, pack, reduce, stream);
+               bool reduce, hipStream_t stream, const ResultLines& lines) {
+  return launch_vec_t<false>(d_descs, VecDescsInline{}, nstates, n, partials, results, pack, reduce, stream, lines);
 }
 
 int launch_vec_inline(const VecDesc* h_descs, int nstates, int n, double* partials, double* results,
-                      const PackSpec& pack, bool reduce, hipStream_t stream) {
+                      const PackSpec& pack, bool reduce, hipStream_t stream, const ResultLines& lines) {
   if (nstates < 1 || nstates > kInlineStates) {
     set_error("vector kernel: descriptors by value hold at most kInlineStates states");
     return kErrArg;
   }
   VecDescsInline inl{};
   for (int s = 0; s < nstates; ++s) inl.d[s] = h_descs[s];
-  return launch_vec_t<true>(nullptr, inl, nstates, n, partials, results, pack, reduce, stream);
+  return launch_vec_t<true>(nullptr, inl, nstates, n, partials, results, pack, reduce, stream, lines);
 }
 
 }  // namespace mt

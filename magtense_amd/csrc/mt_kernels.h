@@ -454,17 +454,31 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
                          const NextStage& next = NextStage{});
 
 int vec_blocks_per_state(int n3);
+// One block's share of a reduction in host memory that the device writes: the
+// values first, then seq, released at system scope.
+struct alignas(64) ResultLine {
+  double v[4];
+  uint32_t seq;
+};
+// Where the reductions of a launch go as lines: [rslot][stride], stride >= the
+// blocks per state.  base null: to partials and results in device memory.
+struct ResultLines {
+  ResultLine* base = nullptr;
+  int stride = 0;
+  uint32_t seq = 0;
+};
+inline bool reduces(int rkind) { return rkind != kRedNone && rkind != kRedWeightsAvg; }
 // With one block per state (3n <= 2048) the vector kernel writes the
 // reductions' results itself (no combine launch).
 int launch_vec(const VecDesc* d_descs, int nstates, int n, double* partials, double* results, const PackSpec& pack,
-               bool reduce, hipStream_t stream);
+               bool reduce, hipStream_t stream, const ResultLines& lines = ResultLines{});
 
 struct VecDescsInline {
   VecDesc d[kInlineStates];
 };
 // launch_vec with the descriptors by value (nstates <= kInlineStates)
 int launch_vec_inline(const VecDesc* h_descs, int nstates, int n, double* partials, double* results,
-                      const PackSpec& pack, bool reduce, hipStream_t stream);
+                      const PackSpec& pack, bool reduce, hipStream_t stream, const ResultLines& lines = ResultLines{});
 
 // Small problems on the FP32 dense path: the stage argument formed in the
 // demag + LL launch.  Every workgroup evaluates the whole combination of
