@@ -643,21 +643,23 @@ int launch_matvec_f32(const float* K, int n, const float* m, int64_t m_stride, f
                       int nstates, float pref, hipStream_t stream) {
   const bool vec4 = (n % 4) == 0 && (m_stride % 4) == 0;
   auto go = [&](auto s, int s0, int groups) {
-    constexpr int S = decltype(s)::value, RB = matvec_block_rows(S);
-    const dim3 grid(matvec_blocks((n + RB - 1) / RB, groups));
+    constexpr int S = decltype(s)::value;
     const float* ms = m + (int64_t)s0 * m_stride;
     float* o = out + (int64_t)s0 * out_stride;
     auto kernel = [&](auto v4, auto one) {
+      constexpr int RB = matvec_block_rows(S, decltype(v4)::value);
+      const dim3 grid(matvec_blocks((n + RB - 1) / RB, groups));
       hipLaunchKernelGGL((matvec_f32_kernel<RB, decltype(v4)::value, S, decltype(one)::value>), grid, dim3(256), 0,
                          stream, K, n, ms, m_stride, o, out_stride, pref, nstates - s0, groups);
     };
-    if (groups == 1) vec4 ? kernel(std::true_type{}, std::true_type{}) : kernel(std::false_type{}, std::true_type{});
-    else vec4 ? kernel(std::true_type{}, std::false_type{}) : kernel(std::false_type{}, std::false_type{});
+    auto by_groups = [&](auto v4) { groups == 1 ? kernel(v4, std::true_type{}) : kernel(v4, std::false_type{}); };
+    if constexpr (S == 12) by_groups(std::false_type{});  // matvec_group: single columns
+    else vec4 ? by_groups(std::true_type{}) : by_groups(std::false_type{});
   };
   for (int s0 = 0; s0 < nstates;) {
-    const int S = matvec_group(nstates - s0);
-    const int groups = S == 8 ? std::max(1, std::min((nstates - s0) / 8, 64)) : 1;
+    const int S = matvec_group(nstates - s0, vec4), groups = matvec_groups(nstates - s0, S);
     switch (S) {
+      case 12: go(std::integral_constant<int, 12>{}, s0, groups); break;
       case 8: go(std::integral_constant<int, 8>{}, s0, groups); break;
       case 4: go(std::integral_constant<int, 4>{}, s0, groups); break;
       case 2: go(std::integral_constant<int, 2>{}, s0, groups); break;

@@ -639,11 +639,11 @@ template <int S>
 int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs, const LlgDescsInline& inl,
                        const float* m32, int64_t m_stride, int s0, int nstates, int groups, const NextStage& next,
                        hipStream_t stream) {
-  constexpr int RB = matvec_block_rows(S);
-  const dim3 grid(matvec_blocks((g.n + RB - 1) / RB, groups));
   const bool vec4 = (g.n % 4) == 0 && (m_stride % 4) == 0;
   const StageDescsInline nx = inline_next(next, d_descs ? 0 : nstates);
   auto launch = [&](auto by_value, auto v4, auto one, auto with_next) {
+    constexpr int RB = matvec_block_rows(S, decltype(v4)::value);
+    const dim3 grid(matvec_blocks((g.n + RB - 1) / RB, groups));
     hipLaunchKernelGGL((demag_llg_f32_kernel<decltype(by_value)::value, decltype(v4)::value, RB, S,
                                              decltype(one)::value, decltype(with_next)::value>),
                        grid, dim3(kDemagLlgThreads<S>), 0, stream, K, g, d_descs, inl, m32, m_stride, s0, nstates, groups,
@@ -654,9 +654,14 @@ int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs,
   };
   const std::true_type yes;
   const std::false_type no;
-  if (!d_descs) vec4 ? go(yes, yes, yes) : go(yes, no, yes);  // by value: one group at a time
-  else if (groups == 1) vec4 ? go(no, yes, yes) : go(no, no, yes);
-  else vec4 ? go(no, yes, no) : go(no, no, no);
+  auto by_columns = [&](auto v4) {
+    if constexpr (S <= kInlineStates) {
+      if (!d_descs) return go(yes, v4, yes);  // by value: one group
+    }
+    groups == 1 ? go(no, v4, yes) : go(no, v4, no);
+  };
+  if constexpr (S == 12) by_columns(no);  // matvec_group: single columns
+  else vec4 ? by_columns(yes) : by_columns(no);
   MT_HIP(hipGetLastError());
   return kOk;
 }
@@ -673,9 +678,11 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
     for (int s = 0; s < nstates; ++s) inl.d[s] = h_descs[s];
   }
   for (int s0 = 0; s0 < nstates;) {
-    const int S = matvec_group(nstates - s0), groups = S == 8 ? std::max(1, std::min((nstates - s0) / 8, 64)) : 1;
+    const int S = matvec_group(nstates - s0, g.n % 4 == 0 && m_stride % 4 == 0);
+    const int groups = matvec_groups(nstates - s0, S);
     int rc = kOk;
-    if (S == 8) rc = launch_demag_llg_s<8>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, next, stream);
+    if (S == 12) rc = launch_demag_llg_s<12>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, next, stream);
+    else if (S == 8) rc = launch_demag_llg_s<8>(K, g, d_descs, inl, m32, m_stride, s0, nstates, groups, next, stream);
     else if (S == 4) rc = launch_demag_llg_s<4>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);
     else if (S == 2) rc = launch_demag_llg_s<2>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);
     else rc = launch_demag_llg_s<1>(K, g, d_descs, inl, m32, m_stride, s0, nstates, 1, next, stream);

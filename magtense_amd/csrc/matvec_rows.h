@@ -3,6 +3,8 @@
 // same order.
 #pragma once
 
+#include <algorithm>
+
 #include "mt_common.h"
 
 namespace mt {
@@ -70,26 +72,49 @@ __device__ __forceinline__ void matvec_flat(const K4 (&k4)[QC], const float (&vx
   acc[2] += z;
 }
 
-template <int ROR>
-__device__ __forceinline__ float add_row_ror(float v) {
-  const int x = __builtin_bit_cast(int, v);
-  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, 0x120 | ROR, 0xF, 0xF, false));
+// Sums over the 64 lanes of N values, each by v + v(lane xor 32), then xor 16,
+// 8, 4, 2, 1, to dst[0 .. N-1].  The lanes that a step leaves with copies of a
+// sum take the next value's instead: two registers become one at every step, in
+// the vector pipe throughout.  144 values: 0.4 thousand instructions where a
+// tree to every lane for each takes 1.4, and 3 LDS writes for 144 (12 states of
+// 45 x 17 x 2: 29.8 us a right-hand side, 37.3 with trees; 8 of 90 x 70: 0.227 ms
+// a product, 0.234).
+template <int CTRL, int BANKS>
+__device__ __forceinline__ float dpp_into(float old, float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v),
+                                                               CTRL, 0xF, BANKS, false));
 }
-// Sum over the 64 lanes, v + v(lane xor 32), then xor 16, 8, 4, 2, 1; every lane
-// gets it.  Half and row exchanges and row rotations (once lanes xor 8 are
-// equal, a rotation by 4 in a row of 16 brings the value of lane xor 4) stay
-// in the vector pipe: 2 swaps and 6 additions instead of six LDS permutes.
-__device__ __forceinline__ float wave_tree_sum(float v) {
-  unsigned x = __builtin_bit_cast(unsigned, v);
-  const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-  x = __builtin_bit_cast(unsigned, v);
-  const auto w = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-  v = __uint_as_float(w[0]) + __uint_as_float(w[1]);
-  v = add_row_ror<8>(v);
-  v = add_row_ror<4>(v);
-  v = add_row_ror<2>(v);
-  return add_row_ror<1>(v);
+// a + a(lane xor BIT) where lane & BIT is 0, b + b(lane xor BIT) where it is not
+template <int BIT>
+__device__ __forceinline__ float fold_lanes(float a, float b, int lane) {
+  if constexpr (BIT == 32 || BIT == 16) {
+    const unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+    const auto h = BIT == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
+                             : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  } else if constexpr (BIT == 4) {  // rows of 16 lanes shifted left and right by 4, into alternate banks of 4
+    float o = dpp_into<0x104, 0x5>(0.0f, a);
+    o = dpp_into<0x114, 0xA>(o, b);
+    return (lane & 4 ? b : a) + o;
+  } else {  // row rotation by 8; quad permutations
+    const float keep = lane & BIT ? b : a, send = lane & BIT ? a : b;
+    return keep + dpp_into<BIT == 8 ? 0x128 : (BIT == 2 ? 0x4E : 0xB1), 0xF>(0.0f, send);
+  }
+}
+template <int TOTAL, int BIT = 32, int N>
+__device__ __forceinline__ void wave_tree_sums(const float (&v)[N], int lane, float* dst) {
+  constexpr int M = (N + 1) / 2;
+  float o[M];
+#pragma unroll
+  for (int i = 0; i < M; ++i) o[i] = fold_lanes<BIT>(v[2 * i], v[2 * i + 1 < N ? 2 * i + 1 : 2 * i], lane);
+  if constexpr (BIT > 1) {
+    wave_tree_sums<TOTAL, BIT / 2>(o, lane, dst);
+  } else {
+    const int first = (int)(__brev((unsigned)lane) >> 26);  // lane bit 5 chose value bit 0, and so on
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      if (first + 64 * i < TOTAL) dst[first + 64 * i] = o[i];
+  }
 }
 
 constexpr int kRowThreads = 256;  // of matvec_rows_f32
@@ -155,15 +180,14 @@ __device__ __forceinline__ void matvec_rows_f32(const float* __restrict__ K, int
     }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float v[RB * S * 3];
 #pragma unroll
   for (int s = 0; s < S; ++s)
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const float v = wave_tree_sum(acc[r][s][c]);
-        if (lane == 0) red[wave][(s * RB + r) * 3 + c] = v;
-      }
+      for (int c = 0; c < 3; ++c) v[(s * RB + r) * 3 + c] = acc[r][s][c];
+  wave_tree_sums<RB * S * 3>(v, lane, red[wave]);
   __syncthreads();
   if (threadIdx.x < RB * S * 3)
     sums[threadIdx.x] = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
@@ -185,11 +209,19 @@ inline unsigned matvec_blocks(int row_blocks, int G) {
 
 // States per block for the next `left` states: the narrowest kernel that takes
 // them in one pass, some of its states idle (90 x 70 cells: 1 / 2 / 4 / 8 states
-// 0.165 / 0.171 / 0.185 / 0.255 ms a pass, all HBM).
-inline int matvec_group(int left) { return left > 4 ? 8 : (left > 2 ? 4 : left); }
-// Receiver rows of its blocks: four (402.7 MB tensor, one state: 2 / 4 / 8 rows
-// -> 72.2 / 66.8 / 114.4 us per launch); two beside eight states, whose sums and
-// values take the registers.
-constexpr int matvec_block_rows(int S) { return S >= 8 ? 2 : 4; }
+// 0.164 / 0.170 / 0.182 / 0.227 ms a pass, HBM up to four).  With single columns
+// (n % 4 != 0) a thread holds a quarter of the values, and twelve states fit.
+inline int matvec_group(int left, bool vec4) {
+  if (left > 8 && !vec4) return 12;
+  return left > 4 ? 8 : (left > 2 ? 4 : left);
+}
+// Groups of S states of one launch.
+inline int matvec_groups(int left, int S) { return S >= 8 ? std::max(1, std::min(left / S, 64)) : 1; }
+// Receiver rows of its blocks: a value of a state is read from L2 once per block,
+// so that more rows are less traffic, until the sums take a wave's registers.
+// One state, 402.7 MB tensor: 2 / 4 / 8 rows -> 72.2 / 66.8 / 114.4 us per launch;
+// 8 states of 90 x 70: 2 / 3 rows -> 0.254 / 0.234 ms (4: 299 registers, one wave
+// per SIMD).
+constexpr int matvec_block_rows(int S, bool vec4) { return S >= 8 && vec4 ? 3 : 4; }
 
 }  // namespace mt
