@@ -1,6 +1,7 @@
 // Kernel descriptors and launchers shared by the host runtime.
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "mt_common.h"
@@ -216,11 +217,18 @@ struct SparseDemag {
   int64_t nnz[6] = {0, 0, 0, 0, 0, 0};
   int64_t* rowptr = nullptr;  // 6 x (n+1), per component
   int64_t* coff = nullptr;    // 6 component offsets into cols/vals (device)
-  int* cols = nullptr;
+  void* cols = nullptr;       // uint16_t up to 65536 cells, int above
   float* vals = nullptr;
-  float* mT = nullptr;        // transposed staging for the many-state product
-  float* hT = nullptr;
-  int tcols = 0;
+  size_t col_bytes() const { return n <= 65536 ? sizeof(uint16_t) : sizeof(int); }
+  template <typename F>
+  auto by_columns(F&& f) {
+    if (n <= 65536) return f(static_cast<uint16_t*>(cols));
+    return f(static_cast<int*>(cols));
+  }
+  float* mT = nullptr;        // states interleaved or transposed, 64 at most; made with the matrix, or
+  float* hT = nullptr;        // by the first product that needs it
+  std::mutex launch;          // one product's launches on them at a time (all on one stream)
+  int scratch();
   BlockSparse* blocks = nullptr;  // split-BF16 block-sparse form (precision bf16x2) instead of the CSR
   uint8_t* ws = nullptr;          // the block-sparse product's workspace, kept between calls
   size_t ws_bytes = 0;

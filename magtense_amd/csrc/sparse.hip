@@ -8,8 +8,8 @@
 // (MagTenseCudaBlas.cu:106-297).
 //
 // Layout: six CSR matrices (xx, xy, xz, yy, yz, zz), rows = receiver cells,
-// columns ascending, 64-bit row pointers, 32-bit columns, FP32 values.  An
-// entry is kept when |K| > threshold (FP32 comparison).  The threshold for a
+// columns ascending, 64-bit row pointers, 16-bit columns up to 65536 cells (32-bit
+// above), FP32 values.  An entry is kept when |K| > threshold (FP32 comparison).  The threshold for a
 // fraction is found by the reference's FP32 bisection over the positive
 // entries, with the counts formed on the device.
 //
@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include <hip/hip_bf16.h>
@@ -80,9 +81,10 @@ __global__ void __launch_bounds__(1024) csr_scan_kernel(int64_t* __restrict__ ro
 }
 
 // ordered compaction of one row: tiles of 256 entries, block-wide exclusive scan
+template <typename C>
 __global__ void __launch_bounds__(256) csr_fill_kernel(const float* __restrict__ K, int n, float thr,
                                                        const int64_t* __restrict__ rowptr, const int64_t* coff,
-                                                       int* __restrict__ cols, float* __restrict__ vals) {
+                                                       C* __restrict__ cols, float* __restrict__ vals) {
   const int i = blockIdx.x, c = blockIdx.y;
   const float* row = K + (size_t)c * n * n + (size_t)i * n;
   int64_t pos = coff[c] + rowptr[(size_t)c * (n + 1) + i];
@@ -102,7 +104,7 @@ __global__ void __launch_bounds__(256) csr_fill_kernel(const float* __restrict__
       total += wsum[w];
     }
     if (keep) {
-      cols[pos + off + before] = j;
+      cols[pos + off + before] = (C)j;
       vals[pos + off + before] = v;
     }
     pos += total;
@@ -160,10 +162,11 @@ __global__ void transpose_f32_kernel(const float* __restrict__ in, int rows, int
   }
 }
 
+template <typename C>
 struct CsrView {
   const int64_t* rowptr;  // 6 x (n+1), relative to the component's base
   const int64_t* coff;    // 6 component bases into cols/vals
-  const int* cols;
+  const C* cols;
   const float* vals;
 };
 
@@ -174,7 +177,8 @@ struct CsrView {
 // entries per unrolled group keep sixteen independent gathers in flight
 // (measured: eight 12.3 ms, sixteen 10.2 ms, thirty-two 10.6 ms per product on
 // the 32768-cell film); the sums still run over the entries in CSR order.
-__global__ void __launch_bounds__(256) spmm_rows_kernel(CsrView A, int n, int S, const float* __restrict__ mT,
+template <typename C>
+__global__ void __launch_bounds__(256) spmm_rows_kernel(CsrView<C> A, int n, int S, const float* __restrict__ mT,
                                                         float pref, float* __restrict__ hT) {
   const int lane = threadIdx.x & 63;
   // wave-uniform row: the CSR walk runs on scalar registers
@@ -220,10 +224,29 @@ __global__ void __launch_bounds__(256) spmm_rows_kernel(CsrView A, int n, int S,
     for (int a = 0; a < 3; ++a) hT[((size_t)a * n + i) * S + lane] = pref * acc[a];
 }
 
-// few states (S <= 4): wave per receiver row, lanes split the entries; m, h are [S][3n]
-template <int S>
-__global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView A, int n, const float* __restrict__ m, int64_t ld,
+// [S][3n] -> [ceil(S / W)][3n][W], zeros beyond S: the states of one gather
+template <int W>
+__global__ void __launch_bounds__(256) interleave_kernel(const float* __restrict__ m, int64_t ld, int S, int n3,
+                                                         float* __restrict__ out) {
+  const int e = blockIdx.x * 256 + threadIdx.x, s0 = blockIdx.y * W;
+  if (e >= n3) return;
+  float v[W];
+#pragma unroll
+  for (int s = 0; s < W; ++s) v[s] = s0 + s < S ? m[(s0 + s) * ld + e] : 0.0f;
+  float* o = out + ((int64_t)blockIdx.y * n3 + e) * W;
+#pragma unroll
+  for (int s = 0; s < W; ++s) o[s] = v[s];
+}
+
+// few states (S <= 8): wave per receiver row, lanes split the entries, h is
+// [S][3n], m the states interleaved by W.  Bound by the gathers of m through L1:
+// a lane takes W states of a source with one load, and the matrix is read once
+// (6 bytes an entry, 8 with 32-bit columns).  @@
+template <int S, int W, typename C>
+__global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, const float* __restrict__ m, int64_t ld,
                                                         float pref, float* __restrict__ h) {
+  typedef float vecw __attribute__((ext_vector_type(W)));
+  constexpr int G = (S + W - 1) / W;
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= n) return;
@@ -243,9 +266,22 @@ __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView A, int n, const 
     for (int64_t q = q0 + lane; q < q1; q += 64) {
       const int j = A.cols[q];
       const float v = A.vals[q];
-      for (int s = 0; s < S; ++s) {
-        acc[a][s] += v * m[s * ld + (size_t)b * n + j];
-        if (a != b) acc[b][s] += v * m[s * ld + (size_t)a * n + j];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float* f = m + (int64_t)g * 3 * n * W + (int64_t)j * W;
+        if constexpr (W == 1) {
+          acc[a][g] += v * f[(int64_t)b * n];
+          if (a != b) acc[b][g] += v * f[(int64_t)a * n];
+        } else {
+          const vecw x = *reinterpret_cast<const vecw*>(f + (int64_t)b * n * W);
+#pragma unroll
+          for (int s = 0; s < W && g * W + s < S; ++s) acc[a][g * W + s] += v * x[s];
+          if (a != b) {
+            const vecw y = *reinterpret_cast<const vecw*>(f + (int64_t)a * n * W);
+#pragma unroll
+            for (int s = 0; s < W && g * W + s < S; ++s) acc[b][g * W + s] += v * y[s];
+          }
+        }
       }
     }
   }
@@ -545,7 +581,7 @@ void SparseDemag::release() {
   if (mT) (void)hipFree(mT);
   if (hT) (void)hipFree(hT);
   rowptr = nullptr; cols = nullptr; vals = nullptr; coff = nullptr; mT = nullptr; hT = nullptr;
-  n = 0; tcols = 0;
+  n = 0;
   for (int c = 0; c < 6; ++c) nnz[c] = 0;
 }
 
@@ -628,11 +664,19 @@ int SparseDemag::build(const float* K32, int n_, float thr, hipStream_t st) {
   }
   MT_HIP(hipMalloc(&coff, sizeof(off)));
   MT_HIP(hipMemcpyAsync(coff, off, sizeof(off), hipMemcpyHostToDevice, st));
-  MT_HIP(hipMalloc(&cols, (size_t)(tot > 0 ? tot : 1) * sizeof(int)));
+  MT_HIP(hipMalloc(&cols, (size_t)(tot > 0 ? tot : 1) * col_bytes()));
   MT_HIP(hipMalloc(&vals, (size_t)(tot > 0 ? tot : 1) * sizeof(float)));
-  hipLaunchKernelGGL(csr_fill_kernel, dim3((unsigned)n, 6), dim3(256), 0, st, K32, n, thr, rowptr, coff, cols, vals);
+  by_columns([&](auto* c) {
+    hipLaunchKernelGGL(csr_fill_kernel, dim3((unsigned)n, 6), dim3(256), 0, st, K32, n, thr, rowptr, coff, c, vals);
+  });
   MT_HIP(hipGetLastError());
   MT_HIP(hipStreamSynchronize(st));
+  return scratch();
+}
+
+int SparseDemag::scratch() {
+  if (!mT) MT_HIP(hipMalloc(&mT, (size_t)3 * n * kMaxCols * sizeof(float)));
+  if (!hT) MT_HIP(hipMalloc(&hT, (size_t)3 * n * kMaxCols * sizeof(float)));
   return kOk;
 }
 
@@ -668,12 +712,20 @@ int SparseDemag::load_component(int c, int n_, int nnz_c, const float* values, c
   if (cols) (void)hipFree(cols);
   if (vals) (void)hipFree(vals);
   if (!coff) MT_HIP(hipMalloc(&coff, sizeof(off)));
-  MT_HIP(hipMalloc(&cols, (size_t)(tot > 0 ? tot : 1) * sizeof(int)));
+  MT_HIP(hipMalloc(&cols, (size_t)(tot > 0 ? tot : 1) * col_bytes()));
   MT_HIP(hipMalloc(&vals, (size_t)(tot > 0 ? tot : 1) * sizeof(float)));
   MT_HIP(hipMemcpyAsync(coff, off, sizeof(off), hipMemcpyHostToDevice, st));
   for (int k = 0; k < 6; ++k) {
     if (!nnz[k]) continue;
-    MT_HIP(hipMemcpyAsync(cols + off[k], host_cols[k].data(), nnz[k] * sizeof(int), hipMemcpyHostToDevice, st));
+    // 32-bit on the host; narrowed before the copy, which ends before c goes
+    const int rc = by_columns([&](auto* d) -> int {
+      typedef std::remove_pointer_t<decltype(d)> C;
+      const std::vector<C> c(host_cols[k].begin(), host_cols[k].end());
+      MT_HIP(hipMemcpyAsync(d + off[k], c.data(), nnz[k] * sizeof(C), hipMemcpyHostToDevice, st));
+      MT_HIP(hipStreamSynchronize(st));
+      return kOk;
+    });
+    if (rc) return rc;
     MT_HIP(hipMemcpyAsync(vals + off[k], host_vals[k].data(), nnz[k] * sizeof(float), hipMemcpyHostToDevice, st));
   }
   MT_HIP(hipStreamSynchronize(st));
@@ -683,42 +735,67 @@ int SparseDemag::load_component(int c, int n_, int nnz_c, const float* values, c
 // h[s*ld + a*n + i] = pref * sum K_a.(i,:) m_s,.  for s < S (m, h: [S][3n], row stride ld)
 int SparseDemag::apply(const float* m, int64_t ld, int S, float pref, float* h, hipStream_t st) {
   MT_CHECK(rowptr && cols && vals && coff, "sparse demag tensor not built");
-  CsrView A{rowptr, coff, cols, vals};
   const unsigned blocks = (unsigned)((n + 3) / 4);
   const int n3 = 3 * n;
-  // up to 16 states: the few-state kernel on groups of at most four (the
-  // 32768-cell film at 8 % density: 0.95 / 1.23 / 1.76 ms for 1 / 2 / 4
-  // states; the many-state kernel takes 8.4-9.8 ms from 5 to 32 states)
+  std::lock_guard<std::mutex> lock(launch);
+  // up to 16 states: the few-state kernel on groups of at most eight (8192 cells,
+  // 71 M entries: 122 / 145 / 173 / 257 / 497 us for 1 / 2 / 4 / 8 / 16 states; the
+  // many-state kernel takes 1.33 to 1.48 ms)
   if (S <= 16) {
-    for (int s0 = 0; s0 < S; s0 += 4) {
-      const int g = S - s0 < 4 ? S - s0 : 4;
+    for (int s0 = 0; s0 < S;) {
+      const int g = std::min(S - s0, 8);
       const float* mg = m + (int64_t)s0 * ld;
       float* hg = h + (int64_t)s0 * ld;
-      switch (g) {
-        case 1: hipLaunchKernelGGL(spmv_rows_kernel<1>, dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg); break;
-        case 2: hipLaunchKernelGGL(spmv_rows_kernel<2>, dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg); break;
-        case 3: hipLaunchKernelGGL(spmv_rows_kernel<3>, dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg); break;
-        default: hipLaunchKernelGGL(spmv_rows_kernel<4>, dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg); break;
+      if (g > 1) {
+        int rc = scratch();
+        if (rc) return rc;
+        const unsigned eb = (unsigned)((n3 + 255) / 256);
+        if (g == 2)
+          hipLaunchKernelGGL(interleave_kernel<2>, dim3(eb), dim3(256), 0, st, mg, ld, g, n3, mT);
+        else
+          hipLaunchKernelGGL(interleave_kernel<4>, dim3(eb, (unsigned)((g + 3) / 4)), dim3(256), 0, st, mg, ld, g, n3,
+                             mT);
+        MT_HIP(hipGetLastError());
+        mg = mT;
       }
+      by_columns([&](auto* c) {
+        typedef std::remove_pointer_t<decltype(c)> C;
+        const CsrView<C> A{rowptr, coff, c, vals};
+        auto go = [&](auto w) {
+          constexpr int G = decltype(w)::value, W = G < 3 ? G : 4;
+          hipLaunchKernelGGL((spmv_rows_kernel<G, W, C>), dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg);
+        };
+        switch (g) {
+          case 1: go(std::integral_constant<int, 1>{}); break;
+          case 2: go(std::integral_constant<int, 2>{}); break;
+          case 3: go(std::integral_constant<int, 3>{}); break;
+          case 4: go(std::integral_constant<int, 4>{}); break;
+          case 5: go(std::integral_constant<int, 5>{}); break;
+          case 6: go(std::integral_constant<int, 6>{}); break;
+          case 7: go(std::integral_constant<int, 7>{}); break;
+          default: go(std::integral_constant<int, 8>{}); break;
+        }
+      });
       MT_HIP(hipGetLastError());
+      s0 += g;
     }
     return kOk;
   }
   MT_CHECK(S <= kMaxCols, "at most 64 states per sparse product");
   MT_CHECK((n3 + 31) / 32 <= 65535, "sparse product supports up to 699040 cells");
-  if (tcols < S) {
-    if (mT) (void)hipFree(mT);
-    if (hT) (void)hipFree(hT);
-    mT = hT = nullptr;
-    MT_HIP(hipMalloc(&mT, (size_t)n3 * kMaxCols * sizeof(float)));
-    MT_HIP(hipMalloc(&hT, (size_t)n3 * kMaxCols * sizeof(float)));
-    tcols = kMaxCols;
+  {
+    int rc = scratch();
+    if (rc) return rc;
   }
   // [S][3n] -> [3n][S]
   hipLaunchKernelGGL(transpose_f32_kernel, dim3((unsigned)((n3 + 31) / 32), (unsigned)((S + 31) / 32)), dim3(32, 8), 0,
                      st, m, S, n3, ld, mT, (int64_t)S);
   MT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(spmm_rows_kernel, dim3(blocks), dim3(256), 0, st, A, n, S, mT, pref, hT);
+  by_columns([&](auto* c) {
+    typedef std::remove_pointer_t<decltype(c)> C;
+    hipLaunchKernelGGL(spmm_rows_kernel<C>, dim3(blocks), dim3(256), 0, st, CsrView<C>{rowptr, coff, c, vals}, n, S, mT,
+                       pref, hT);
+  });
   MT_HIP(hipGetLastError());
   // [3n][S] -> [S][3n]
   hipLaunchKernelGGL(transpose_f32_kernel, dim3((unsigned)((S + 31) / 32), (unsigned)((n3 + 31) / 32)), dim3(32, 8), 0,
