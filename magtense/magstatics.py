@@ -19,6 +19,7 @@ and a sequence of ``n`` rows replaces the whole array.
 """
 
 import ctypes as C
+import struct
 from typing import List, Optional, Tuple, Union
 
 import numpy as np
@@ -381,6 +382,9 @@ def grid_config(spots: Union[List, np.ndarray], area: Union[List, np.ndarray], f
 
 # ---- GPU evaluation -------------------------------------------------------------
 
+_TILES_FIELDS = struct.Struct("@i8P")  # MtTiles
+
+
 def _tiles_struct(tiles: Tiles, with_m: bool):
     """Fortran-ordered copies of the tile arrays and the mt_tiles struct over them."""
     n = tiles.n
@@ -400,16 +404,11 @@ def _tiles_struct(tiles: Tiles, with_m: bool):
         "sym_ops": np.asfortranarray(np.asarray(tiles.sym_op, dtype=np.float64).reshape(n, 3)),
         "vertices": np.asfortranarray(np.asarray(tiles.vertices, dtype=np.float64).reshape(n, 3, 4)),
     }
-    dp = C.POINTER(C.c_double)
-    ip = C.POINTER(C.c_int)
-    st = _lib.MtTiles()
-    st.n_tiles = n
-    for k in ("size", "offset", "rot", "sym_ops"):
-        setattr(st, k, keep[k].ctypes.data_as(dp))
-    st.M = keep["M"].ctypes.data_as(dp) if with_m else None
-    st.tile_type = keep["tile_type"].ctypes.data_as(ip)
-    st.use_sym = keep["use_sym"].ctypes.data_as(ip)
-    st.vertices = keep["vertices"].ctypes.data_as(dp)
+    addr = {k: a.__array_interface__["data"][0] for k, a in keep.items()}
+    # the struct's fields in order, as addresses: half the time of a pointer object each
+    st = _lib.MtTiles.from_buffer_copy(_TILES_FIELDS.pack(
+        n, addr["size"], addr["offset"], addr["rot"], addr["M"] if with_m else 0, addr["tile_type"], addr["use_sym"],
+        addr["sym_ops"], addr["vertices"]))
     return st, keep
 
 

@@ -632,38 +632,69 @@ void mt_demag_sparse_destroy(void* h) { delete static_cast<SparseDemag*>(h); }
 // ---- magnetostatic prism tiles (getNFromTiles / getHFromTiles) ---------------
 }  // extern "C"
 
-#pragma clang fp contract(off)
-
 namespace {
 
-void mat3_mul(const double* A, const double* B, double* C) {
-  for (int r = 0; r < 3; ++r)
-    for (int c = 0; c < 3; ++c) C[3 * r + c] = A[3 * r] * B[c] + A[3 * r + 1] * B[3 + c] + A[3 * r + 2] * B[6 + c];
-}
+// Pinned host memory that a call's input is packed into and its output written
+// to, both by the kernels themselves: a copy of a few KB through the runtime takes
+// 12-14 us, of 100 KB from pageable memory up to 180, and a call of 20 tiles needed
+// three.  Blocks of kHostBlock bytes; a call takes one for its duration, at most
+// kHostBlocksKept wait for the next call of any thread.
+constexpr size_t kHostBlock = 2u << 20, kHostBlocksKept = 4;
+std::mutex g_host_mutex;
+std::vector<void*> g_host_blocks;
 
-// getRotationMatrices (DemagFieldGetSolution.f90:925-948): R = Rz(-t3) Ry(-t2)
-// Rx(-t1), Rinv = Rx^T Ry^T Rz^T; row-major.
-void rotation_matrices(const double ang[3], double* R, double* Ri) {
-  double ax = -ang[0], ay = -ang[1], az = -ang[2];
-  const double X[9] = {1, 0, 0, 0, std::cos(ax), -std::sin(ax), 0, std::sin(ax), std::cos(ax)};
-  const double Y[9] = {std::cos(ay), 0, std::sin(ay), 0, 1, 0, -std::sin(ay), 0, std::cos(ay)};
-  const double Z[9] = {std::cos(az), -std::sin(az), 0, std::sin(az), std::cos(az), 0, 0, 0, 1};
-  double ZY[9], Xt[9], Yt[9], Zt[9], XtYt[9];
-  mat3_mul(Z, Y, ZY);
-  mat3_mul(ZY, X, R);
-  for (int r = 0; r < 3; ++r)
-    for (int c = 0; c < 3; ++c) { Xt[3 * r + c] = X[3 * c + r]; Yt[3 * r + c] = Y[3 * c + r]; Zt[3 * r + c] = Z[3 * c + r]; }
-  mat3_mul(Xt, Yt, XtYt);
-  mat3_mul(XtYt, Zt, Ri);
-}
+class HostBlock {
+ public:
+  HostBlock() {
+    {
+      std::lock_guard<std::mutex> lock(g_host_mutex);
+      if (!g_host_blocks.empty()) {
+        p_ = g_host_blocks.back();
+        g_host_blocks.pop_back();
+      }
+    }
+    constexpr unsigned flags = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+    if (!p_ && hipHostMalloc(&p_, kHostBlock, flags) != hipSuccess) {
+      (void)hipGetLastError();
+      p_ = nullptr;
+    }
+    if (p_ && hipHostGetDevicePointer(&d_, p_, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      d_ = nullptr;
+    }
+  }
+  // the kernels that use it have ended: every path out of a call waits for them
+  ~HostBlock() {
+    if (!p_) return;
+    (void)hipStreamSynchronize(nullptr);
+    std::lock_guard<std::mutex> lock(g_host_mutex);
+    if (g_host_blocks.size() < kHostBlocksKept) g_host_blocks.push_back(p_);
+    else (void)hipHostFree(p_);
+  }
+  HostBlock(const HostBlock&) = delete;
+  HostBlock& operator=(const HostBlock&) = delete;
+  // room for n more doubles: host and device address, or false
+  bool take(size_t n, double** host, double** dev) {
+    const size_t bytes = (n * sizeof(double) + 255) / 256 * 256;
+    if (!d_ || used_ + bytes > kHostBlock) return false;
+    *host = reinterpret_cast<double*>(static_cast<char*>(p_) + used_);
+    *dev = reinterpret_cast<double*>(static_cast<char*>(d_) + used_);
+    used_ += bytes;
+    return true;
+  }
 
-// Fortran-ordered (n,3) host arrays -> device tile records of kTileRec doubles.
-int tile_records(const mt_tiles* t, bool need_m, std::vector<double>& rec, TileKind* kind) {
+ private:
+  void *p_ = nullptr, *d_ = nullptr;
+  size_t used_ = 0;
+};
+
+// Checks the tiles; *vertices: some tile is a tetrahedron.
+int check_tiles(const mt_tiles* t, bool need_m, TileKind* kind, bool* vertices) {
   MT_CHECK(t && t->n_tiles > 0 && t->size && t->offset, "mt_tiles needs n_tiles > 0, size and offset");
   MT_CHECK(!need_m || t->M, "mt_tiles_h_field needs the tile magnetisation M");
   const int nt = t->n_tiles;
-  rec.assign((size_t)nt * kTileRec, 0.0);
   int prisms = 0, tetras = 0;
+  *vertices = false;
   for (int i = 0; i < nt; ++i) {
     const int type = t->tile_type ? t->tile_type[i] : 2;
     if (type != 2 && type != 5) {
@@ -672,33 +703,85 @@ int tile_records(const mt_tiles* t, bool need_m, std::vector<double>& rec, TileK
       return kErrUnsupported;
     }
     MT_CHECK(type != 5 || t->vertices, "tetrahedron tiles (tile_type 5) need the vertices");
-    double* r = rec.data() + (size_t)i * kTileRec;
-    r[31] = type;
     if (type == 5) {  // vertices (n,3,4) Fortran order: component c of vertex k at i + n*(c + 3k)
-      for (int k = 0; k < 4; ++k)
-        for (int c = 0; c < 3; ++c) r[32 + 3 * k + c] = t->vertices[i + (size_t)nt * (c + 3 * (size_t)k)];
+      *vertices = true;
       double e[3][3];
       for (int k = 0; k < 3; ++k)
-        for (int c = 0; c < 3; ++c) e[k][c] = r[35 + 3 * k + c] - r[32 + c];
+        for (int c = 0; c < 3; ++c)
+          e[k][c] = t->vertices[i + (size_t)nt * (c + 3 * (size_t)(k + 1))] - t->vertices[i + (size_t)nt * c];
       const double vol = e[0][0] * (e[1][1] * e[2][2] - e[1][2] * e[2][1]) -
                          e[0][1] * (e[1][0] * e[2][2] - e[1][2] * e[2][0]) +
                          e[0][2] * (e[1][0] * e[2][1] - e[1][1] * e[2][0]);
       MT_CHECK(vol != 0.0, "tetrahedron tile " + std::to_string(i) + " is degenerate (zero volume)");
     }
-    double ang[3], M[3];
-    for (int k = 0; k < 3; ++k) {
-      r[k] = t->size[i + (size_t)nt * k];
-      r[3 + k] = t->offset[i + (size_t)nt * k];
-      ang[k] = t->rot ? t->rot[i + (size_t)nt * k] : 0.0;
-      M[k] = t->M ? t->M[i + (size_t)nt * k] : 0.0;
-      r[27 + k] = t->sym_ops ? t->sym_ops[i + (size_t)nt * k] : 1.0;
-    }
-    rotation_matrices(ang, r + 6, r + 15);
-    for (int a = 0; a < 3; ++a) r[24 + a] = r[6 + 3 * a] * M[0] + r[7 + 3 * a] * M[1] + r[8 + 3 * a] * M[2];
-    r[30] = (t->use_sym && t->use_sym[i] == 1) ? 1.0 : 0.0;
-    if (r[30] == 0.0) (type == 2 ? prisms : tetras) += 1;
+    if (!(t->use_sym && t->use_sym[i] == 1)) (type == 2 ? prisms : tetras) += 1;
   }
   *kind = prisms == nt ? TileKind::kPrism : (tetras == nt ? TileKind::kTetra : TileKind::kAny);
+  return kOk;
+}
+
+size_t tiles_raw_doubles(int nt, bool vertices, int n_pts) {
+  return (size_t)nt * (vertices ? kTileRaw + 12 : kTileRaw) + (size_t)3 * n_pts;
+}
+// The packed input of launch_tile_records.
+void pack_tiles(const mt_tiles* t, bool vertices, int n_pts, const double* pts, double* raw) {
+  const size_t nt = t->n_tiles;
+  auto rows = [&](const double* from, size_t count, double missing) {
+    if (from) std::memcpy(raw, from, count * nt * sizeof(double));
+    else std::fill(raw, raw + count * nt, missing);
+    raw += count * nt;
+  };
+  rows(t->size, 3, 0.0);
+  rows(t->offset, 3, 0.0);
+  for (size_t e = 0; e < 3 * nt; ++e) {
+    const double a = t->rot ? -t->rot[e] : 0.0;
+    raw[e] = std::cos(a);
+    raw[3 * nt + e] = std::sin(a);
+  }
+  raw += 6 * nt;
+  rows(t->M, 3, 0.0);
+  rows(t->sym_ops, 3, 1.0);
+  for (size_t i = 0; i < nt; ++i)
+    raw[i] = (t->tile_type ? t->tile_type[i] : 2) + (t->use_sym && t->use_sym[i] == 1 ? 8.0 : 0.0);
+  raw += nt;
+  if (vertices) rows(t->vertices, 12, 0.0);
+  std::memcpy(raw, pts, (size_t)3 * n_pts * sizeof(double));
+}
+
+// A call on tiles and points in host memory: their records and points on the
+// device, then run(tiles, pts, out), which writes n_out doubles to device address
+// out, which end in dst.
+template <class F>
+int on_tiles(const mt_tiles* t, bool vertices, int n_pts, const double* pts, size_t n_out, double* dst, F&& run) {
+  const int nt = t->n_tiles;
+  const size_t n_raw = tiles_raw_doubles(nt, vertices, n_pts);
+  HostBlock block;
+  DevArr<double> work, draw, dout;
+  MT_HIP(work.alloc((size_t)nt * kTileRec + (size_t)3 * n_pts));
+  double *raw_h = nullptr, *raw_d = nullptr, *out_h = nullptr, *out_d = nullptr;
+  if (block.take(n_raw, &raw_h, &raw_d)) {
+    pack_tiles(t, vertices, n_pts, pts, raw_h);
+  } else {
+    std::vector<double> raw(n_raw);
+    pack_tiles(t, vertices, n_pts, pts, raw.data());
+    MT_HIP(draw.alloc(n_raw));
+    MT_HIP(hipMemcpy(draw.p, raw.data(), n_raw * sizeof(double), hipMemcpyHostToDevice));
+    raw_d = draw.p;
+  }
+  if (!block.take(n_out, &out_h, &out_d)) {
+    MT_HIP(dout.alloc(n_out));
+    out_d = dout.p;
+  }
+  double *recs = work.p, *points = work.p + (size_t)nt * kTileRec;
+  int rc = launch_tile_records(raw_d, nt, vertices, n_pts, recs, points, nullptr);
+  if (rc == kOk) rc = run(recs, points, out_d);
+  if (rc) return rc;
+  if (out_h) {
+    MT_HIP(hipStreamSynchronize(nullptr));
+    std::memcpy(dst, out_h, n_out * sizeof(double));
+  } else {
+    MT_HIP(hipMemcpy(dst, out_d, n_out * sizeof(double), hipMemcpyDeviceToHost));
+  }
   return kOk;
 }
 
@@ -710,48 +793,35 @@ int mt_tiles_demag_tensor(const mt_tiles* tiles, int n_pts, const double* pts, d
   int rc = device_ok();
   if (rc) return rc;
   MT_CHECK(n_pts > 0 && pts && N, "invalid points or output");
-  std::vector<double> rec;
   TileKind kind = TileKind::kAny;
-  rc = tile_records(tiles, false, rec, &kind);
+  bool vertices = false;
+  rc = check_tiles(tiles, false, &kind, &vertices);
   if (rc) return rc;
   const int nt = tiles->n_tiles;
-  const size_t nN = (size_t)nt * n_pts * 9;
-  DevArr<double> drec, dpts, dN;
-  MT_HIP(drec.alloc(rec.size()));
-  MT_HIP(dpts.alloc((size_t)n_pts * 3));
-  MT_HIP(dN.alloc(nN));
-  MT_HIP(hipMemcpy(drec.p, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice));
-  MT_HIP(hipMemcpy(dpts.p, pts, (size_t)n_pts * 3 * sizeof(double), hipMemcpyHostToDevice));
-  rc = launch_tiles_tensor(drec.p, nt, kind, dpts.p, n_pts, dN.p, nullptr);
-  if (rc) return rc;
-  MT_HIP(hipMemcpy(N, dN.p, nN * sizeof(double), hipMemcpyDeviceToHost));
-  return kOk;
+  return on_tiles(tiles, vertices, n_pts, pts, (size_t)nt * n_pts * 9, N, [&](double* recs, double* p, double* out) {
+    return launch_tiles_tensor(recs, nt, kind, p, n_pts, out, nullptr);
+  });
 }
 
 int mt_tiles_h_field(const mt_tiles* tiles, int n_pts, const double* pts, const double* N, double* H) {
   int rc = device_ok();
   if (rc) return rc;
   MT_CHECK(n_pts > 0 && pts && H, "invalid points or output");
-  std::vector<double> rec;
   TileKind kind = TileKind::kAny;
-  rc = tile_records(tiles, true, rec, &kind);
+  bool vertices = false;
+  rc = check_tiles(tiles, true, &kind, &vertices);
   if (rc) return rc;
-  const int nt = tiles->n_tiles;
-  DevArr<double> drec, dpts, dN, dH;
-  MT_HIP(drec.alloc(rec.size()));
-  MT_HIP(dpts.alloc((size_t)n_pts * 3));
-  MT_HIP(dH.alloc((size_t)tiles_field_plan(nt, n_pts).parts * n_pts * 3));
-  MT_HIP(hipMemcpy(drec.p, rec.data(), rec.size() * sizeof(double), hipMemcpyHostToDevice));
-  MT_HIP(hipMemcpy(dpts.p, pts, (size_t)n_pts * 3 * sizeof(double), hipMemcpyHostToDevice));
+  const int nt = tiles->n_tiles, parts = tiles_field_plan(nt, n_pts).parts;
+  DevArr<double> dN, part;
+  if (parts > 1) MT_HIP(part.alloc((size_t)parts * n_pts * 3));
   if (N) {
     const size_t nN = (size_t)nt * n_pts * 9;
     MT_HIP(dN.alloc(nN));
     MT_HIP(hipMemcpy(dN.p, N, nN * sizeof(double), hipMemcpyHostToDevice));
   }
-  rc = launch_tiles_field(drec.p, nt, kind, dpts.p, n_pts, dN.p, dH.p, nullptr);
-  if (rc) return rc;
-  MT_HIP(hipMemcpy(H, dH.p, (size_t)n_pts * 3 * sizeof(double), hipMemcpyDeviceToHost));
-  return kOk;
+  return on_tiles(tiles, vertices, n_pts, pts, (size_t)n_pts * 3, H, [&](double* recs, double* p, double* out) {
+    return launch_tiles_field(recs, nt, kind, p, n_pts, dN.p, part.p, out, nullptr);
+  });
 }
 
 // ---- reference plug-in ABI: one global instance, host arrays, PCIe per call ----

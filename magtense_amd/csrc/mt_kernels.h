@@ -18,13 +18,20 @@ int launch_assemble(const double* src, const double* abc, int abc_stride, const 
 enum class TileKind { kAny, kPrism, kTetra };
 int launch_tiles_tensor(const double* tiles, int nt, TileKind kind, const double* pts, int npt, double* out,
                         hipStream_t stream);
-// H holds tiles_field_plan(nt, npt).parts x 3 npt doubles; the field is left in the first 3 npt.
+// The records and the points from the packed input of a call: size, offset,
+// cosines and sines of the negated rotation angles, M, symmetry operations (three
+// rows each), type + 8 * symmetric, twelve rows of vertices where there are any, all
+// [row][nt]; then the points.
+constexpr int kTileRaw = 19;
+int launch_tile_records(const double* raw, int nt, bool vertices, int npt, double* tiles, double* pts,
+                        hipStream_t stream);
+// part holds tiles_field_plan(nt, npt).parts x 3 npt doubles (unused with one part), H the field.
 struct TilesFieldPlan {
   int width, blocks, parts;
 };
 TilesFieldPlan tiles_field_plan(int nt, int npt);
 int launch_tiles_field(const double* tiles, int nt, TileKind kind, const double* pts, int npt, const double* Nin,
-                       double* H, hipStream_t stream);
+                       double* part, double* H, hipStream_t stream);
 int launch_split(const float* K, int n, uint8_t* split, hipStream_t stream);
 // FP32 planes -> the dense tensor as FP32 MFMA fragments (split_tensor_bytes(n) bytes)
 int launch_f32_fragments(const float* K, int n, uint8_t* frags, hipStream_t stream);

@@ -772,18 +772,86 @@ __global__ void __launch_bounds__(256, KIND == TileKind::kPrism ? 3 : 1)
     for (int a = 0; a < 3; ++a) H[(size_t)blockIdx.y * 3 * npt + p + (size_t)npt * a] = red[a][threadIdx.x];
 }
 
-// H[e] = sum over the parts, in order (in place in part 0)
-__global__ void __launch_bounds__(256) tiles_field_sum_kernel(double* __restrict__ H, int parts, int64_t total) {
+// H[e] = sum over the parts, in order
+__global__ void __launch_bounds__(256) tiles_field_sum_kernel(const double* __restrict__ part, int parts,
+                                                              int64_t total, double* __restrict__ H) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= total) return;
-  double s = H[e];
-  for (int z = 1; z < parts; ++z) s += H[(int64_t)z * total + e];
+  double s = part[e];
+#pragma unroll 8
+  for (int z = 1; z < parts; ++z) s += part[(int64_t)z * total + e];
   H[e] = s;
 }
 
 }  // namespace
 
 // Host launchers -------------------------------------------------------------
+
+namespace {
+// The 3 x 3 product A B, row-major.
+__device__ void mat3_mul(const double* A, const double* B, double* C) {
+  for (int r = 0; r < 3; ++r)
+    for (int c = 0; c < 3; ++c) C[3 * r + c] = A[3 * r] * B[c] + A[3 * r + 1] * B[3 + c] + A[3 * r + 2] * B[6 + c];
+}
+
+// Tile records and the points from the packed input of a call, which may lie in
+// host memory: every value is read once.  Rotations by getRotationMatrices
+// (DemagFieldGetSolution.f90:925-948): R = Rz(-t3) Ry(-t2) Rx(-t1), Rinv = Rx^T
+// Ry^T Rz^T; row-major.  The input holds the host's cosines and sines of -t: near
+// an edge an entry is thousands of times as sensitive to the point as elsewhere,
+// and the last bit of a rotation shows (2e-13 of a tensor entry, 7e-10 of a field
+// of 6000 prisms).
+__global__ void __launch_bounds__(64) tile_records_kernel(const double* __restrict__ raw, int nt, int vertices,
+                                                          int64_t npt3, double* __restrict__ tiles,
+                                                          double* __restrict__ pts) {
+  const int64_t t = (int64_t)blockIdx.x * 64 + threadIdx.x, stride = (int64_t)gridDim.x * 64;
+  const double* p = raw + (int64_t)nt * (vertices ? kTileRaw + 12 : kTileRaw);
+  for (int64_t e = t; e < npt3; e += stride) pts[e] = p[e];
+  for (int64_t i = t; i < nt; i += stride) {
+    double v[kTileRaw];
+    for (int k = 0; k < kTileRaw; ++k) v[k] = raw[(int64_t)k * nt + i];
+    double* r = tiles + i * kTileRec;
+    for (int k = 0; k < 6; ++k) r[k] = v[k];
+    const double *co = v + 6, *si = v + 9;
+    const double X[9] = {1, 0, 0, 0, co[0], -si[0], 0, si[0], co[0]};
+    const double Y[9] = {co[1], 0, si[1], 0, 1, 0, -si[1], 0, co[1]};
+    const double Z[9] = {co[2], -si[2], 0, si[2], co[2], 0, 0, 0, 1};
+    double A[9], B[9], Rm[9], Xt[9], Yt[9], Zt[9];
+    mat3_mul(Z, Y, A);
+    mat3_mul(A, X, Rm);
+    for (int a = 0; a < 3; ++a)
+      for (int c = 0; c < 3; ++c) {
+        Xt[3 * a + c] = X[3 * c + a];
+        Yt[3 * a + c] = Y[3 * c + a];
+        Zt[3 * a + c] = Z[3 * c + a];
+      }
+    mat3_mul(Xt, Yt, A);
+    mat3_mul(A, Zt, B);
+    for (int k = 0; k < 9; ++k) {
+      r[6 + k] = Rm[k];
+      r[15 + k] = B[k];
+    }
+    for (int a = 0; a < 3; ++a) {
+      r[24 + a] = Rm[3 * a] * v[12] + Rm[3 * a + 1] * v[13] + Rm[3 * a + 2] * v[14];
+      r[27 + a] = v[15 + a];
+    }
+    r[30] = v[18] >= 8.0 ? 1.0 : 0.0;
+    r[31] = v[18] >= 8.0 ? v[18] - 8.0 : v[18];
+    if (vertices)
+      for (int k = 0; k < 12; ++k) r[32 + k] = raw[(int64_t)(kTileRaw + k) * nt + i];
+  }
+}
+}  // namespace
+
+int launch_tile_records(const double* raw, int nt, bool vertices, int npt, double* tiles, double* pts,
+                        hipStream_t stream) {
+  const int64_t most = std::max<int64_t>(nt, (int64_t)3 * npt);
+  const unsigned blocks = (unsigned)std::min<int64_t>((most + 63) / 64, 4096);
+  hipLaunchKernelGGL(tile_records_kernel, dim3(blocks), dim3(64), 0, stream, raw, nt, vertices ? 1 : 0,
+                     (int64_t)3 * npt, tiles, pts);
+  MT_HIP(hipGetLastError());
+  return kOk;
+}
 
 namespace {
 template <class F>
@@ -821,19 +889,20 @@ TilesFieldPlan tiles_field_plan(int nt, int npt) {
 }
 
 int launch_tiles_field(const double* tiles, int nt, TileKind kind, const double* pts, int npt, const double* Nin,
-                       double* H, hipStream_t stream) {
+                       double* part, double* H, hipStream_t stream) {
   if (npt <= 0) return kOk;
   const TilesFieldPlan q = tiles_field_plan(nt, npt);
+  double* first = q.parts > 1 ? part : H;
   const dim3 grid((unsigned)q.blocks, (unsigned)q.parts);
   by_kind(kind, [&](auto k) {
     hipLaunchKernelGGL(tiles_field_kernel<decltype(k)::value>, grid, dim3(256), 0, stream, tiles, nt, pts, npt, q.width,
-                       Nin, H);
+                       Nin, first);
   });
   MT_HIP(hipGetLastError());
   if (q.parts > 1) {
     const int64_t total = (int64_t)3 * npt;
-    hipLaunchKernelGGL(tiles_field_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, H, q.parts,
-                       total);
+    hipLaunchKernelGGL(tiles_field_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, part,
+                       q.parts, total, H);
     MT_HIP(hipGetLastError());
   }
   return kOk;
