@@ -347,7 +347,14 @@ constexpr int kTableChainChunks = 256;  // longest partial sum of the entry-reus
 // float q), A = K_c(row l % 32, k = 2s + l / 32) and, for the states, B =
 // m_beta(k = 2s + l / 32, column l % 32 of the half) — eight FP32 MFMAs per
 // block instead of three split products.
-template <int D, bool TOEP, bool BSR = false, bool F32 = false>
+// HALVES: column halves of 32 states.  The loads of a later chunk go between the
+// MFMAs of this one, one every few; issued together they held the wave, and with
+// it the matrix pipe, until the memory pipe had taken all fifteen.  FP32, 8192
+// cells: 355 us a product up to 32 states and 652 up to 64, 440 and 695 before (of
+// 255 for the tensor at 6.3 TB/s, and 250 and 500 for the MFMAs); BF16, 20000
+// cells, 64 states: 2.03 ms, 2.31 before.  With two halves three chunks of ring fit
+// the registers, with one four.
+template <int D, bool TOEP, bool BSR, bool F32, int HALVES>
 __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __restrict__ Kt,
                                                                  const uint4* __restrict__ Mp, int64_t np,
                                                                  int ksplit, float* __restrict__ out, int n,
@@ -422,7 +429,6 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __
                            : (TOEP ? 0 : Il * nJ * 12 * 64);
   const u32x4* A = reinterpret_cast<const u32x4*>(Kt) + aoff + lane;
   const u32x4* B = reinterpret_cast<const u32x4*>(Mp) + threadIdx.x;
-  const bool two_halves = ncols > 32;
   // translation-invariant lookup: this wave's tile (x0 tile, iy, iz) and the
   // group's first tile row (wy, wz), which sets the shared chunk order
   const int cpr = gnx / 16, tpr = gnx / 32, U = gnx / 8 - 2;
@@ -443,9 +449,9 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __
   // acc sums at most kFlushChunks chunks before it is added into sum and
   // restarted: two-level FP32 summation, so a long row's partial sum does not
   // swallow the rounding of thousands of additions
-  floatx16 acc[2][3], sum[2][3];
+  floatx16 acc[HALVES][3], sum[HALVES][3];
 #pragma unroll
-  for (int h = 0; h < 2; ++h)
+  for (int h = 0; h < HALVES; ++h)
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -475,56 +481,61 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __
     _Pragma("unroll") for (int q = 0; q < 3; ++q) br[slot][q] = b_[q * 256];                              \
   } while (0)
 
-  // chunk j -> LDS slot j & 1, barrier, MFMAs from register slot `slot`
-#define MT_REG_CONSUME(j, slot)                                                                         \
+  // chunk j -> LDS slot j & 1, barrier; `ahead` (the loads of a later chunk); MFMAs
+  // from register slot `slot`.  A wave past the last tile sums its group's first
+  // tile, which is not stored: no branch between the loads and the MFMAs.
+#define MT_REG_CONSUME(j, slot, ahead)                                                                   \
   do {                                                                                                   \
     u32x4* dst_ = &bs[(j) & 1][0][0] + threadIdx.x;                                                      \
-    _Pragma("unroll") for (int q = 0; q < 3; ++q) dst_[q * 256] = br[slot][q];                          \
+    _Pragma("unroll") for (int q = 0; q < 3; ++q) dst_[q * 256] = br[slot][q];                           \
     __syncthreads();                                                                                     \
-    if (tile_ok) {                                                                                       \
-      if (F32) {                                                                                         \
-        f32x4 b0[3][2], b1[3][2];                                                                        \
-        _Pragma("unroll") for (int beta = 0; beta < 3; ++beta)                                           \
-        _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                  \
-          b0[beta][h] = __builtin_bit_cast(f32x4, bs[(j) & 1][(beta * 2 + h) * 2 + 0][lane]);            \
-          b1[beta][h] = __builtin_bit_cast(f32x4, bs[(j) & 1][(beta * 2 + h) * 2 + 1][lane]);            \
-        }                                                                                                \
-        _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                  \
-          if (h == 1 && !two_halves) break;                                                              \
-          _Pragma("unroll") for (int a = 0; a < 3; ++a)                                                  \
-          _Pragma("unroll") for (int beta = 0; beta < 3; ++beta) {                                       \
-            const int c = (a == 0 ? beta : (a == 1 ? (beta == 0 ? 1 : 2 + beta) : (beta == 0 ? 2 : 3 + beta))); \
-            const f32x4 k0 = __builtin_bit_cast(f32x4, ar[slot][2 * c]);                                 \
-            const f32x4 k1 = __builtin_bit_cast(f32x4, ar[slot][2 * c + 1]);                             \
-            _Pragma("unroll") for (int q = 0; q < 4; ++q)                                                \
-              acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x2f32(k0[q], b0[beta][h][q], acc[h][a], 0, 0, 0); \
-            _Pragma("unroll") for (int q = 0; q < 4; ++q)                                                \
-              acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x2f32(k1[q], b1[beta][h][q], acc[h][a], 0, 0, 0); \
-          }                                                                                              \
-        }                                                                                                \
-      } else {                                                                                           \
-        bf16x8 bh[3][2], bl[3][2];                                                                       \
-        _Pragma("unroll") for (int beta = 0; beta < 3; ++beta)                                           \
-        _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                  \
-          bh[beta][h] = __builtin_bit_cast(bf16x8, bs[(j) & 1][(beta * 2 + h) * 2 + 0][lane]);           \
-          bl[beta][h] = __builtin_bit_cast(bf16x8, bs[(j) & 1][(beta * 2 + h) * 2 + 1][lane]);           \
-        }                                                                                                \
-        _Pragma("unroll") for (int h = 0; h < 2; ++h) {                                                  \
-          if (h == 1 && !two_halves) break;                                                              \
-          _Pragma("unroll") for (int a = 0; a < 3; ++a)                                                  \
-          _Pragma("unroll") for (int beta = 0; beta < 3; ++beta) {                                       \
-            const int c = (a == 0 ? beta : (a == 1 ? (beta == 0 ? 1 : 2 + beta) : (beta == 0 ? 2 : 3 + beta))); \
-            const bf16x8 khi = __builtin_bit_cast(bf16x8, ar[slot][2 * c]);                              \
-            const bf16x8 klo = __builtin_bit_cast(bf16x8, ar[slot][2 * c + 1]);                          \
-            acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(khi, bh[beta][h], acc[h][a], 0, 0, 0);   \
-            acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(khi, bl[beta][h], acc[h][a], 0, 0, 0);   \
-            acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(klo, bh[beta][h], acc[h][a], 0, 0, 0);   \
-          }                                                                                              \
+    ahead;                                                                                               \
+    /* steps outermost: consecutive MFMAs go to other accumulators, each of which sums in its order */   \
+    _Pragma("unroll") for (int beta = 0; beta < 3; ++beta) {                                             \
+      u32x4 b0[HALVES], b1[HALVES];                                                                      \
+      _Pragma("unroll") for (int h = 0; h < HALVES; ++h) {                                               \
+        b0[h] = bs[(j) & 1][(beta * 2 + h) * 2 + 0][lane];                                               \
+        b1[h] = bs[(j) & 1][(beta * 2 + h) * 2 + 1][lane];                                               \
+      }                                                                                                  \
+      _Pragma("unroll") for (int q = 0; q < (F32 ? 8 : 3); ++q)                                          \
+      _Pragma("unroll") for (int h = 0; h < HALVES; ++h)                                                 \
+      _Pragma("unroll") for (int a = 0; a < 3; ++a) {                                                    \
+        const int c = (a == 0 ? beta : (a == 1 ? (beta == 0 ? 1 : 2 + beta) : (beta == 0 ? 2 : 3 + beta)));\
+        if (F32) {                                                                                       \
+          const f32x4 k = __builtin_bit_cast(f32x4, ar[slot][2 * c + q / 4]);                            \
+          const f32x4 b = __builtin_bit_cast(f32x4, q < 4 ? b0[h] : b1[h]);                              \
+          acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[q % 4], b[q % 4], acc[h][a], 0, 0, 0);      \
+        } else { /* hi hi, hi lo, lo hi */                                                               \
+          const bf16x8 k = __builtin_bit_cast(bf16x8, ar[slot][2 * c + q / 2]);                          \
+          const bf16x8 b = __builtin_bit_cast(bf16x8, q == 1 ? b1[h] : b0[h]);                           \
+          acc[h][a] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k, b, acc[h][a], 0, 0, 0);                 \
         }                                                                                                \
       }                                                                                                  \
     }                                                                                                    \
+    /* a load every few MFMAs: fifteen at once hold the wave while the memory pipe takes them */         \
+    constexpr int kMfma_ = (F32 ? 24 : 9) * HALVES / 5;                                                  \
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * HALVES, 0); /* LDS read */                           \
+    _Pragma("unroll") for (int beta_ = 0; beta_ < 3; ++beta_) {                                          \
+      _Pragma("unroll") for (int q_ = 0; q_ < 5; ++q_) {                                                 \
+        __builtin_amdgcn_sched_group_barrier(0x008, kMfma_, 0); /* MFMA */                               \
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);      /* global load */                        \
+        if (q_ == 3 && beta_ < 2) __builtin_amdgcn_sched_group_barrier(0x100, 2 * HALVES, 0);            \
+      }                                                                                                  \
+      __builtin_amdgcn_sched_group_barrier(0x008, (F32 ? 24 : 9) * HALVES - 5 * kMfma_, 0);              \
+    }                                                                                                    \
   } while (0)
 
+  auto flush = [&](int j) {
+    if ((j + 1) % (F32 ? kFlushChunksF32 : kFlushChunks) != 0) return;
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        sum[h][a] += acc[h][a];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[h][a][r] = 0.0f;
+      }
+  };
   if (nchunks > 0) {
     // chunk j0 + s always sits in register slot s: no branch inside the main
     // loop, so every slot keeps one register assignment around the loop
@@ -534,32 +545,25 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __
     for (; j0 + D <= nchunks; j0 += D) {
 #pragma unroll
       for (int s = 0; s < D; ++s) {
-        MT_REG_ISSUE(j0 + s + D - 1, (s + D - 1) % D);
-        MT_REG_CONSUME(j0 + s, s);
-      }
-      if ((j0 + D) % (F32 ? kFlushChunksF32 : kFlushChunks) == 0) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            sum[h][a] += acc[h][a];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[h][a][r] = 0.0f;
-          }
+        MT_REG_CONSUME(j0 + s, s, MT_REG_ISSUE(j0 + s + D - 1, (s + D - 1) % D));
+        flush(j0 + s);
       }
     }
     // fewer than D chunks left, all already issued into slots 0 .. rem - 1
     const int rem = nchunks - j0;
 #pragma unroll
     for (int s = 0; s < D - 1; ++s)
-      if (s < rem) MT_REG_CONSUME(j0 + s, s);
+      if (s < rem) {
+        MT_REG_CONSUME(j0 + s, s, (void)0);
+        flush(j0 + s);
+      }
   }
 #undef MT_REG_CONSUME
 #undef MT_REG_ISSUE
   if (tile_ok) {
     float* o = out + (int64_t)ks * split_stride;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < HALVES; ++h) {
       const int col = 32 * h + (lane & 31);
       if (col >= ncols) break;
 #pragma unroll
@@ -574,7 +578,7 @@ __global__ void __launch_bounds__(256, 1) gemm_bf16x2_reg_kernel(const uint4* __
   }  // segments
 }
 
-template <int D, bool TOEP = false, bool BSR = false, bool F32 = false>
+template <bool TOEP = false, bool BSR = false, bool F32 = false>
 int launch_reg(const uint8_t* K, const uint8_t* Mpack, int n, int nrows, float* out, int64_t col_stride,
                int64_t split_stride, int ncols, int ksplit, hipStream_t stream, int gnx = 0, int gny = 1,
                int gnz = 1, BlockSparseView bs = BlockSparseView{}) {
@@ -585,9 +589,15 @@ int launch_reg(const uint8_t* K, const uint8_t* Mpack, int n, int nrows, float* 
   if (BSR) blocks = bs.nwg;  // the balanced schedule's ranges
   if (blocks == 0) return kOk;
   const size_t lds = BSR ? (size_t)bs.seg_max * sizeof(int) : 0;
-  hipLaunchKernelGGL((gemm_bf16x2_reg_kernel<D, TOEP, BSR, F32>), dim3((unsigned)blocks), dim3(256), lds, stream,
-                     reinterpret_cast<const uint4*>(K), reinterpret_cast<const uint4*>(Mpack), np, ksplit, out, nrows,
-                     col_stride, split_stride, ncols, gnx, gny, gnz, bs, bs.chunks, bs.segs, bs.goff, bs.tiles);
+  auto go = [&](auto halves) {
+    constexpr int H = decltype(halves)::value, D = H == 2 ? 3 : 4;
+    hipLaunchKernelGGL((gemm_bf16x2_reg_kernel<D, TOEP, BSR, F32, H>), dim3((unsigned)blocks),
+                       dim3(256), lds, stream, reinterpret_cast<const uint4*>(K),
+                       reinterpret_cast<const uint4*>(Mpack), np, ksplit, out, nrows, col_stride, split_stride, ncols,
+                       gnx, gny, gnz, bs, bs.chunks, bs.segs, bs.goff, bs.tiles);
+  };
+  if (ncols > 32) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 1>{});
   MT_HIP(hipGetLastError());
   return kOk;
 }
@@ -732,7 +742,7 @@ int gemm_ksplit_dense(int n, int nrows) {
 int launch_gemm_bf16x2_rows(const uint8_t* Krows, const uint8_t* Mpack, int n, int nrows, float* out,
                             int64_t col_stride, int64_t split_stride, int ncols, int ksplit, hipStream_t stream) {
   if (gemm_variant() != 6)
-    return launch_reg<4>(Krows, Mpack, n, nrows, out, col_stride, split_stride, ncols, ksplit, stream);
+    return launch_reg<>(Krows, Mpack, n, nrows, out, col_stride, split_stride, ncols, ksplit, stream);
   // variant 6: the two-tile kernel with the four-stage LDS DMA ring
   const int64_t np = round_up(n, kTileM);
   const int groups2 = (int)((round_up(nrows, kTileM) / kTileM + 1) / 2);
@@ -750,7 +760,7 @@ int launch_gemm_bf16x2(const uint8_t* Ksplit, const uint8_t* Mpack, int n, float
 
 int launch_gemm_f32(const uint8_t* Kf, const uint8_t* Mpack, int n, float* out, int64_t col_stride,
                     int64_t split_stride, int ncols, int ksplit, hipStream_t stream) {
-  return launch_reg<4, false, false, true>(Kf, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream);
+  return launch_reg<false, false, true>(Kf, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream);
 }
 
 // Work of block b of the table kernels (block b runs on XCD b % 8): k-split
@@ -1315,9 +1325,9 @@ int launch_gemm_bsr(const uint8_t* frags, const BlockSparseView& bs, bool f32, c
     return kOk;
   }
   if (f32)
-    return launch_reg<4, false, true, true>(frags, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, 0,
+    return launch_reg<false, true, true>(frags, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, 0,
                                             1, 1, bs);
-  return launch_reg<4, false, true>(frags, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, 0, 1, 1,
+  return launch_reg<false, true>(frags, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, 0, 1, 1,
                                     bs);
 }
 
@@ -1338,7 +1348,7 @@ int launch_gemm_bf16x2_toeplitz(const uint8_t* Ktab, int nx, int ny, int nz, con
     return kOk;
   }
   if (gemm_variant() == 4)
-    return launch_reg<4, true>(Ktab, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, nx, ny, nz);
+    return launch_reg<true>(Ktab, Mpack, n, n, out, col_stride, split_stride, ncols, ksplit, stream, nx, ny, nz);
   if (gemm_variant() != 2) {
     // default: single-stage four-tile kernel, two workgroups per CU (measured at
     // N = 32768, 64 states: 3.19 ms, against 3.31 ms for a two-stage version of
