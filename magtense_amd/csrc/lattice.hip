@@ -99,6 +99,14 @@ __host__ __device__ inline LatLds lat_lds(const LatticeView& v, int qc, int nbuf
 // within a plane, where their products, which add +-0 to sums that are never
 // -0, are left out unless *nonfinite says that a state holds an infinity or a
 // NaN.
+//
+// Bound by LDS reads (one state, 256 x 64 x 2: their cycles and bank conflicts are
+// 0.6 of the launch's) and by what a wave waits for between them.  The next sums'
+// reads are issued after the last ones have arrived, the x map's values of a step
+// before its barrier, and a step's place in the grid is kept up by addition.
+// Before, with a wait per read, us a launch: one state 128 x 32 x 1 16.7 (17.7), 90
+// x 70 x 1 70 (81), 91 x 71 x 1 86 (119), 256 x 64 x 2 896 (1024), there four
+// states 1770 (1867).
 template <int QC, bool HASB, bool ALIGNED, int SB>
 __global__ void __launch_bounds__(kLatThreads)
     lattice_rows_kernel(const LatticeView v, const float* __restrict__ m, int cols, float* __restrict__ out,
@@ -107,6 +115,7 @@ __global__ void __launch_bounds__(kLatThreads)
   extern __shared__ __align__(16) uint8_t lat_smem[];
   constexpr int kWaves = kLatThreads / 64, CH = 64 / kWaves;  // chains of a wave
   static_assert(kWaves == 16 && CH == 4, "the order of the final sums");
+  constexpr bool AHEAD = QC == 4 || SB < 4;  // registers for the reads of the next sums
   const int lane = threadIdx.x & 63;
   const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nx = v.nx, ny = v.ny, rows = v.ny * v.nz, n = nx * rows;
@@ -128,35 +137,59 @@ __global__ void __launch_bounds__(kLatThreads)
   constexpr int RUN = 64 * QC, NRUN = 4 / QC;
   // first column of run g of the step at `base`
   auto run_at = [&](int base, int g) { return base + RUN * w + (NRUN == 1 ? 0 : 256 * g); };
+  // The grid rows and x of a step's run starts, kept up from step to step (no
+  // divisions by nx in the loop).
+  struct Cursor {
+    int row[NRUN], jx[NRUN];
+  };
+  const int step_rows = 1024 / nx, step_x = 1024 - step_rows * nx;
+  const int run_rows = (RUN - 1) / nx, run_x = RUN - 1 - run_rows * nx;
+  auto next_step = [&](Cursor& c) {
+#pragma unroll
+    for (int g = 0; g < NRUN; ++g) {
+      c.row[g] += step_rows;
+      c.jx[g] += step_x;
+      if (c.jx[g] >= nx) {
+        c.jx[g] -= nx;
+        c.row[g] += 1;
+      }
+    }
+  };
+  // last grid row of run g of the step at `base`, at cursor c
+  auto last_row = [&](const Cursor& c, int base, int g) {
+    const int left = n - run_at(base, g);
+    if (left < RUN) return rows - 1;
+    return c.row[g] + run_rows + (c.jx[g] + run_x >= nx ? 1 : 0);
+  };
   // every source row of the step against the tile: only xx, xy, yy, zz
-  auto flat_step = [&](int base) {
+  auto flat_step = [&](const Cursor& c, int base) {
     if (all) return false;
     if (!HASB) return true;
-    const int lo = run_at(base, 0), hi = std::min(run_at(base, NRUN - 1) + RUN, n) - 1;
-    return lo / nx >= plane_lo && hi / nx < plane_hi;
+    int g = NRUN - 1;  // the last run that has columns
+    while (g > 0 && run_at(base, g) >= n) --g;
+    return c.row[0] >= plane_lo && last_row(c, base, g) < plane_hi;
   };
   // table row of receiver row q of the tile against source row j
   auto table_row = [&](int q, int j) {
     const int i = std::min(row0 + q, rows - 1);
     return v.zmap[i / ny * v.nz + j / ny] * v.uy + v.ymap[i % ny * ny + j % ny];
   };
-  // table rows of the step at `base` into buffer b; the first step looks them
-  // up itself, so that its copies run while the maps are filled
-  auto stage = [&](auto first, int base, int b) {
+  // table rows of the step at `base` (cursor cur) into buffer b; the first step
+  // looks them up itself, so that its copies run while the maps are filled
+  auto stage = [&](auto first, const Cursor& cur, int base, int b) {
     constexpr bool FIRST = decltype(first)::value;
     uint8_t* A = bufs + (size_t)b * L.buf;
     const uint32_t la = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)A;
     const int pa = (v.ux + 63) / 64;
     const int hx = v.ux / 2, pb = (hx + 63) / 64;  // (xz, yz): two entries per lane
-    const bool with_b = HASB && !flat_step(base);
+    const bool with_b = HASB && !flat_step(cur, base);
 #pragma unroll
     for (int g = 0; g < NRUN; ++g) {
-      const int c0 = run_at(base, g), c1 = std::min(c0 + RUN, n);
-      if (c0 >= n) break;
-      const int ra = c0 / nx, nr = (c1 - 1) / nx - ra + 1, slab0 = g * L.touched * T.rr;
+      if (run_at(base, g) >= n) break;
+      const int ra = cur.row[g], nr = last_row(cur, base, g) - ra + 1, slab0 = g * L.touched * T.rr;
       for (int p = r; p < nr * T.rr * pa; p += kWaves) {
         const int slab = p / pa, o = (p - slab * pa) * 64;  // slab = source row x rr + receiver row
-        const int sr = slab / T.rr, q = slab - sr * T.rr;
+        const int sr = T.rr == 1 ? slab : slab / T.rr, q = slab - sr * T.rr;
         const int64_t src =
             (int64_t)__builtin_amdgcn_readfirstlane(FIRST ? table_row(q, ra + sr) : rowidx[q * rows + ra + sr]) * v.ux +
             o + lane;
@@ -165,7 +198,7 @@ __global__ void __launch_bounds__(kLatThreads)
       if (with_b)
         for (int p = r; p < nr * T.rr * pb; p += kWaves) {
           const int slab = p / pb, o = (p - slab * pb) * 64;
-          const int sr = slab / T.rr, q = slab - sr * T.rr;
+          const int sr = T.rr == 1 ? slab : slab / T.rr, q = slab - sr * T.rr;
           const int64_t src =
               (int64_t)__builtin_amdgcn_readfirstlane(FIRST ? table_row(q, ra + sr) : rowidx[q * rows + ra + sr]) * hx +
               o + lane;
@@ -193,31 +226,58 @@ __global__ void __launch_bounds__(kLatThreads)
   struct States {
     float x[SH][4], y[SH][4], z[SH][4];
   };
-  // place of a quad's columns: x in their grid rows, first entry of the rows in the buffer
-  struct Place {
-    int jx[4], row[4];
+  Cursor here;  // of the step that is computed
+  // Places of the wave's chains: the x map's values of their columns, read for
+  // all of them before the step's barrier (the map does not change), and the first
+  // entries of the columns' grid rows in the step's buffer.
+  constexpr int COLS = ALIGNED && QC == 4 ? 1 : 4;  // columns of a chain in rows of their own
+  typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+  struct Places {
+    u16x4 x[CH];
+    int row[CH][COLS];
   };
-  auto advance = [&](Place& p) {  // to the wave's next chain
+  auto places = [&](Places& P, const Cursor& cur, int base) {
+    int jx[COLS], row[COLS];
 #pragma unroll
-    for (int q = 0; q < (ALIGNED && QC == 4 ? 1 : 4); ++q) {
-      p.jx[q] += QC * kWaves;
-      while (p.jx[q] >= nx) {
-        p.jx[q] -= nx;
-        p.row[q] += T.rr * v.ux;
+    for (int q = 0; q < COLS; ++q) {
+      jx[q] = cur.jx[QC == 4 ? 0 : q] + (QC == 4 ? 4 * r + q : r);
+      row[q] = (QC == 4 ? 0 : q) * L.touched * T.rr * v.ux;
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int q = 0; q < COLS; ++q) {
+        while (jx[q] >= nx) {
+          jx[q] -= nx;
+          row[q] += T.rr * v.ux;
+        }
+        const uint16_t* m4 = pmap + (jx[q] >> 2) * 256 + lane * 4;
+        if constexpr (COLS == 1) P.x[c] = *reinterpret_cast<const u16x4*>(m4);
+        else P.x[c][q] = m4[jx[q] & 3];
+        P.row[c][q] = row[q];
+        jx[q] += QC * kWaves;
       }
+  };
+  // the same one chain at a time (QC 1); jx, row: where the last call stopped
+  auto place_of = [&](Places& P, int c, int (&jx)[4], int (&row)[4]) {
+#pragma unroll
+    for (int q = 0; q < COLS; ++q) {
+      jx[q] = c == 0 ? here.jx[q % NRUN] + r : jx[q] + kWaves;
+      if (c == 0) row[q] = q * L.touched * T.rr * v.ux;
+      while (jx[q] >= nx) {
+        jx[q] -= nx;
+        row[q] += T.rr * v.ux;
+      }
+      P.x[c][q] = pmap[(jx[q] >> 2) * 256 + lane * 4 + (jx[q] & 3)];
+      P.row[c][q] = row[q];
     }
   };
-  auto read_entries = [&](auto flat, Entries& k, const uint8_t* A, const Place& p, int have) {
+  auto read_entries = [&](auto flat, Entries& k, const uint8_t* A, const Places& P, int c, int have) {
     constexpr bool FLAT = decltype(flat)::value;
-    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
-    u16x4 x4;
-    if (ALIGNED && QC == 4) x4 = *reinterpret_cast<const u16x4*>(pmap + (p.jx[0] >> 2) * 256 + lane * 4);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (QC == 1 && q >= have) continue;
-      int e;
-      if (ALIGNED && QC == 4) e = p.row[0] + rho * v.ux + x4[q];
-      else e = p.row[q] + rho * v.ux + pmap[(p.jx[q] >> 2) * 256 + lane * 4 + (p.jx[q] & 3)];
+      const int e = P.row[c][COLS == 1 ? 0 : q] + rho * v.ux + P.x[c][q];
       k.a[q] = *reinterpret_cast<const f32x4*>(A + (size_t)e * 16);
       if (!FLAT) k.b[q] = HASB ? *reinterpret_cast<const f32x2*>(A + L.buf_a + (size_t)e * 8) : f32x2{0.0f, 0.0f};
     }
@@ -254,35 +314,27 @@ __global__ void __launch_bounds__(kLatThreads)
       }
     }
   };
-  // the step at `base`: the entries of the next chain and the states of the
-  // next sums are read before a chain's (state pair's) sums
+  // the step at `base`: the entries of the next chain and the states of the next
+  // sums are read before a chain's (state pair's) sums, and after everything read
+  // before has arrived: scalar loads return in any order, so that a wait for one
+  // is a wait for all that are out.
   const int64_t chain_floats = (int64_t)kWaves * cols * 12;
-  auto compute = [&](auto flat, auto whole, int base, int b) {
+  auto states_at = [&](int base) { return ms + (int64_t)(base / 4 + 64 * w + r) * cols * 12; };
+  auto arrived = [&] { __builtin_amdgcn_s_waitcnt(0xC07F); };  // lgkmcnt(0)
+  States t[2];
+  auto compute = [&](auto flat, auto whole, Places& P, int base, int b) {
     constexpr bool WHOLE = decltype(whole)::value;
     const uint8_t* A = bufs + (size_t)b * L.buf;
-    Place p;
-#pragma unroll
-    for (int q = 0; q < (ALIGNED && QC == 4 ? 1 : 4); ++q) {
-      const int g = QC == 4 ? 0 : q;
-      const int c0 = run_at(base, g), ra = c0 / nx;
-      const int j = QC == 4 ? c0 + 4 * r + q : c0 + r;
-      const int row = j / nx;
-      p.jx[q] = j - row * nx;
-      p.row[q] = (g * L.touched + row - ra) * T.rr * v.ux;
-    }
-    const_floats f = ms + (int64_t)(base / 4 + 64 * w + r) * cols * 12;
+    const_floats f = states_at(base);
     if (WHOLE) {
       Entries k[2];
-      States t[2];
-      read_entries(flat, k[0], A, p, 4);
-      read_states(t[0], f);
+      read_entries(flat, k[0], A, P, 0, 4);
 #pragma unroll
       for (int u = 0; u < CH * (SB / SH); ++u) {
         const int c = u / (SB / SH), h = u % (SB / SH);
-        if (h == 0 && c + 1 < CH) {
-          advance(p);
-          read_entries(flat, k[(c + 1) & 1], A, p, 4);
-        }
+        arrived();
+        __builtin_amdgcn_sched_barrier(0);
+        if (h == 0 && c + 1 < CH) read_entries(flat, k[(c + 1) & 1], A, P, c + 1, 4);
         if (u + 1 < CH * (SB / SH)) {
           if (h + 1 == SB / SH) f += chain_floats - 12 * SH * (SB / SH - 1);
           else f += 12 * SH;
@@ -293,49 +345,62 @@ __global__ void __launch_bounds__(kLatThreads)
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
+      int jx[4], row[4];
 #pragma unroll
       for (int c = 0; c < CH; ++c) {
+        if constexpr (!AHEAD) place_of(P, c, jx, row);
         // QC 4: all of the quad's columns exist or none; QC 1: the first `have`
         const int j = run_at(base, 0) + QC * (r + kWaves * c);
         const int have = QC == 4 ? (j < n ? 4 : 0) : (j < n ? std::min(4, (n - 1 - j) / 256 + 1) : 0);
         if (have > 0) {
           Entries k;
-          read_entries(flat, k, A, p, have);
+          read_entries(flat, k, A, P, c, have);
 #pragma unroll
           for (int h = 0; h < SB / SH; ++h) {
-            States t;
-            read_states(t, f + 12 * SH * h);
-            add(flat, acc[c], h, k, t, have);
+            States t1;
+            read_states(t1, f + 12 * SH * h);
+            add(flat, acc[c], h, k, t1, have);
           }
         }
-        advance(p);
         f += chain_floats;
       }
     }
   };
 
-  stage(std::true_type{}, 0, 0);
+  Cursor cur;
+#pragma unroll
+  for (int g = 0; g < NRUN; ++g) {
+    cur.row[g] = run_at(0, g) / nx;
+    cur.jx[g] = run_at(0, g) - cur.row[g] * nx;
+  }
+  if (run_at(0, 0) < n) stage(std::true_type{}, cur, 0, 0);
   for (int jx = r; jx < nx; jx += kWaves) pmap[(jx >> 2) * 256 + lane * 4 + (jx & 3)] = v.pmap[jx * nx + ix];
   for (int e = threadIdx.x; e < rows * T.rr; e += kLatThreads) {
     const int q = e / rows;
     rowidx[e] = table_row(q, e - q * rows);
   }
+  __syncthreads();  // the maps
   int b = 0;
   for (int base = 0; run_at(base, 0) < n; base += 1024) {
     if (nbuf == 1 && base > 0) {
       __syncthreads();  // the previous step's reads
-      stage(std::false_type{}, base, 0);
+      stage(std::false_type{}, cur, base, 0);
     }
+    const bool whole = AHEAD && run_at(base, NRUN - 1) + RUN <= n;
+    Places P;
+    if constexpr (AHEAD) places(P, cur, base);
+    if (whole) read_states(t[0], states_at(base));
     __builtin_amdgcn_s_waitcnt(0);  // my copies, my reads of the other buffer
     __syncthreads();
-    if (nbuf == 2 && run_at(base + 1024, 0) < n) stage(std::false_type{}, base + 1024, b ^ 1);
-    const bool whole = run_at(base, NRUN - 1) + RUN <= n;
-    if (flat_step(base)) {
-      if (whole) compute(std::true_type{}, std::true_type{}, base, b);
-      else compute(std::true_type{}, std::false_type{}, base, b);
+    here = cur;
+    next_step(cur);
+    if (nbuf == 2 && run_at(base + 1024, 0) < n) stage(std::false_type{}, cur, base + 1024, b ^ 1);
+    if (flat_step(here, base)) {
+      if (whole) compute(std::true_type{}, std::bool_constant<AHEAD>{}, P, base, b);
+      else compute(std::true_type{}, std::false_type{}, P, base, b);
     } else {
-      if (whole) compute(std::false_type{}, std::true_type{}, base, b);
-      else compute(std::false_type{}, std::false_type{}, base, b);
+      if (whole) compute(std::false_type{}, std::bool_constant<AHEAD>{}, P, base, b);
+      else compute(std::false_type{}, std::false_type{}, P, base, b);
     }
     b ^= nbuf - 1;
   }

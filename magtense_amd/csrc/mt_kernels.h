@@ -191,12 +191,12 @@ struct LatticeTable {
 // Whether the product from the table and the LL kernel (7 us) beat the one launch
 // over the dense tensor.  us per right-hand side, table + LL / dense:
 //   one state  32 x 40: 20 / 14, 44 x 40: 20 / 17, 96 x 24: 22 / 27, 64 x 64: 25 / 71
-//   8 states   30 x 30 x 2: 41 / 38, 44 x 40: 34 / 33, 96 x 24: 41 / 50
-//   12         32 x 40: 28 / 40, 64 x 30: 39 / 58
-//   16         32 x 16: 21 / 15, 20 x 20 x 2 (24 states): 40 / 30
+//   8 states   30 x 30 x 2: 41 / 33, 44 x 40: 34 / 28, 96 x 24: 43 / 39
+//   12         32 x 40: 33 / 30, 64 x 30: 40 / 51
+//   16         32 x 16: 21 / 15, 20 x 20 x 2 (24 states): 40 / 27
 // With n % 4 != 0 a chain's four columns lie in four places of the grid:
-//   one state  45 x 17 x 2: 30 / 16, 77 x 33: 48 / 30, 63 x 67: 61 / 87, 91 x 71: 127 / 188
-//   8 or more  45 x 17 x 2 (12): 60 / 37, 77 x 33 (12): 110 / 74, 63 x 67: 120 / 141
+//   one state  45 x 17 x 2: 30 / 16, 77 x 33: 48 / 30, 63 x 67: 47 / 84, 91 x 71: 93 / 184
+//   8 or more  45 x 17 x 2 (12): 60 / 30, 77 x 33 (12): 110 / 66, 63 x 67: 114 / 123
 inline bool lattice_pays(int n, int nstates) {
   if (n % 4) return n > 3500;
   return n > 2000 || (n > 1024 && nstates > 8);
