@@ -26,6 +26,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -39,10 +40,17 @@ namespace {
 
 constexpr double kMu0 = 4.0 * 3.141592653589793 * 1e-7;
 
+// Descriptors of up to kInlineStates states by value
+template <typename D>
+struct Inline {
+  D d[kInlineStates];
+};
+
 struct VjpDesc {
   const double* m;      // stage input Y
   const void* S;        // K Y (positive demag sums), FP32 or FP64
-  const double* u;      // cotangent of k = f(Y)
+  const double* u[2];   // cotangent of k = f(Y): c[0] u[0] + c[1] u[1] (u[1] may be null)
+  double c[2];
   double* mbar;         // out: direct part of the input cotangent
   double* hbar;         // out: field cotangent
   void* packed;         // out: (Ms * Hbar) for the transpose demag pass, FP32 or FP64
@@ -69,18 +77,22 @@ __device__ inline double lap_at(const double* v, int i, int ix, int iy, int iz, 
 
 // T: demag precision (float: the reference's FP32 product and FP32 Ms scaling;
 // double: FP64 tensor, product and Ms)
-template <typename T>
-__global__ void __launch_bounds__(256) vjp_kernel(const LlgGrid g, const VjpDesc* __restrict__ descs) {
-  const VjpDesc& D = descs[blockIdx.y];
+// INL: descriptors by value (inl) instead of from descs
+template <typename T, bool INL>
+__global__ void __launch_bounds__(256) vjp_kernel(const LlgGrid g, const VjpDesc* __restrict__ descs,
+                                                  Inline<VjpDesc> inl) {
+  const VjpDesc& D = INL ? inl.d[blockIdx.y] : descs[blockIdx.y];
   const int n = g.n;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double hx_part[3] = {0.0, 0.0, 0.0};
   if (i < n) {
     const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
     double m[3], u[3], hj[3], hm[3], hk[3], H[3];
+    const double gms0 = D.grad_ms[i];
     for (int c = 0; c < 3; ++c) {
       m[c] = D.m[(size_t)c * n + i];
-      u[c] = D.u[(size_t)c * n + i];
+      u[c] = __builtin_fma(D.c[0], D.u[0][(size_t)c * n + i], 0.0);
+      if (D.u[1]) u[c] = __builtin_fma(D.c[1], D.u[1][(size_t)c * n + i], u[c]);
       hj[c] = (-2.0 * lap_at(D.m + (size_t)c * n, i, ix, iy, iz, g)) * g.jfact[i];
       const T sv = static_cast<const T*>(D.S)[(size_t)c * n + i];
       if constexpr (sizeof(T) == 8) {
@@ -126,7 +138,7 @@ __global__ void __launch_bounds__(256) vjp_kernel(const LlgGrid g, const VjpDesc
       gms += hb[c] * (hm[c] - hj[c] - hk[c]);
       hx_part[c] = -hb[c];
     }
-    D.grad_ms[i] += gms / ms;
+    D.grad_ms[i] = gms0 + gms / ms;
   }
   // block partial of -sum Hbar for the applied-field gradient
   __shared__ double red[4][3];
@@ -150,17 +162,53 @@ struct FinishDesc {
   int nsplit;           // its partial-sum slots, added in order
   int64_t split_stride;
   double* mu;           // out: vjp w.r.t. the stage input
+  double* lam;          // of a step's last stage: lam += mu + later[0] + later[1] + later[2] (else null)
+  const double* later[3];
 };
 
-template <typename TT>
-__global__ void __launch_bounds__(256) vjp_finish_kernel(const LlgGrid g, const FinishDesc* __restrict__ descs) {
-  const FinishDesc& D = descs[blockIdx.y];
+// Every read of the cell before its first store: a launch of a few thousand cells
+// is its round trips to memory (128 x 32 x 1: 5 us, 8 with the components in turn).
+template <typename TT, bool INL>
+__global__ void __launch_bounds__(256) vjp_finish_kernel(const LlgGrid g, const FinishDesc* __restrict__ descs,
+                                                         Inline<FinishDesc> inl) {
+  const FinishDesc& D = INL ? inl.d[blockIdx.y] : descs[blockIdx.y];
   const int n = g.n;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
-  double hb[3];
-  for (int c = 0; c < 3; ++c) hb[c] = D.hbar[(size_t)c * n + i];
+  double hb[3], mb[3], lam[3], later[3][3];
+  TT part[4][3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const size_t at = (size_t)c * n + i;
+    hb[c] = D.hbar[at];
+    mb[c] = D.mbar[at];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (k < D.nsplit) part[k][c] = static_cast<const TT*>(D.T)[(size_t)k * D.split_stride + at];
+    if (D.lam) {
+      lam[c] = D.lam[at];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) later[k][c] = D.later[k][at];
+    }
+  }
+  // exchange transpose: -2 Lap(Jfact * Hbar); the weighted field is formed on the fly
+  const double* jf = g.jfact;
+  const int sy = g.nx, sz = g.nx * g.ny;
+  double lap[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double* h = D.hbar + (size_t)c * n;
+    auto w = [&](int k) { return jf[k] * h[k]; };
+    double wi = w(i);
+    double lx = ix == 0 ? (w(i + 1) - wi) : (ix == g.nx - 1 ? (w(i - 1) - wi) : (w(i - 1) - 2.0 * wi + w(i + 1)));
+    double ly = iy == 0 ? (w(i + sy) - wi) : (iy == g.ny - 1 ? (w(i - sy) - wi) : (w(i - sy) - 2.0 * wi + w(i + sy)));
+    lap[c] = lx * g.idx2 + ly * g.idy2;
+    if (g.nz > 1) {
+      double lz = iz == 0 ? (w(i + sz) - wi) : (iz == g.nz - 1 ? (w(i - sz) - wi) : (w(i - sz) - 2.0 * wi + w(i + sz)));
+      lap[c] += lz * g.idz2;
+    }
+  }
   double ak[3] = {0.0, 0.0, 0.0};
   if (g.aniso) {
     const double* A = g.aniso + (size_t)i * 6;
@@ -169,24 +217,23 @@ __global__ void __launch_bounds__(256) vjp_finish_kernel(const LlgGrid g, const 
     ak[1] = f * (A[1] * hb[0] + A[3] * hb[1] + A[4] * hb[2]);
     ak[2] = f * (A[2] * hb[0] + A[4] * hb[1] + A[5] * hb[2]);
   }
-  // exchange transpose: -2 Lap(Jfact * Hbar); the weighted field is formed on the fly
-  const double* jf = g.jfact;
+#pragma unroll
   for (int c = 0; c < 3; ++c) {
-    const double* h = D.hbar + (size_t)c * n;
-    auto w = [&](int k) { return jf[k] * h[k]; };
-    const int sy = g.nx, sz = g.nx * g.ny;
-    double wi = w(i);
-    double lx = ix == 0 ? (w(i + 1) - wi) : (ix == g.nx - 1 ? (w(i - 1) - wi) : (w(i - 1) - 2.0 * wi + w(i + 1)));
-    double ly = iy == 0 ? (w(i + sy) - wi) : (iy == g.ny - 1 ? (w(i - sy) - wi) : (w(i - sy) - 2.0 * wi + w(i + sy)));
-    double lap = lx * g.idx2 + ly * g.idy2;
-    if (g.nz > 1) {
-      double lz = iz == 0 ? (w(i + sz) - wi) : (iz == g.nz - 1 ? (w(i - sz) - wi) : (w(i - sz) - 2.0 * wi + w(i + sz)));
-      lap += lz * g.idz2;
-    }
-    TT ts = static_cast<const TT*>(D.T)[(size_t)c * n + i];
-    for (int k = 1; k < D.nsplit; ++k) ts += static_cast<const TT*>(D.T)[(size_t)k * D.split_stride + (size_t)c * n + i];
+    const size_t at = (size_t)c * n + i;
+    TT ts = part[0][c];
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+      if (k < D.nsplit) ts += part[k][c];
     const double tv = (double)ts;
-    D.mu[(size_t)c * n + i] = D.mbar[(size_t)c * n + i] - 2.0 * lap - tv + ak[c];
+    const double mu = mb[c] - 2.0 * lap[c] - tv + ak[c];
+    D.mu[at] = mu;
+    if (D.lam) {
+      double v = lam[c] + 0.0;
+      v += mu;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v += later[k][c];
+      D.lam[at] = v;
+    }
   }
 }
 
@@ -312,7 +359,9 @@ struct Rk4 {
   // k[b] = f(Y[b]) for every state; S (K Y) is written to S_out[b] when given.
   // packed: the FP32 demag input already holds Y (packed by the combination
   // that formed it).
-  int rhs(double* const* Y, double* const* k, void* const* S_out, bool packed = false) {
+  // next: a combination that the LL launch forms and packs as well.
+  int rhs(double* const* Y, double* const* k, void* const* S_out, bool packed,
+          const std::vector<StageDesc>& next) {
     int rc = packed && !fp64 ? kOk : pack_input(Y);
     if (rc) return rc;
     // recording: when the states' S_out columns are laid out like the demag
@@ -324,7 +373,7 @@ struct Rk4 {
     void* out = direct ? S_out[0] : hbuf;
     rc = demag_pass(out);
     if (rc) return rc;
-    return llg(Y, k, direct ? nullptr : S_out, out);
+    return llg(Y, k, direct ? nullptr : S_out, out, next);
   }
 
   int pack_input(double* const* Y) {
@@ -339,13 +388,18 @@ struct Rk4 {
       d.post_scale = 1.0;
       d.pack_col = fp64 ? -1 : b;
     }
+    return vec(vd, pack_spec());
+  }
+  // a small batch's descriptors go by value: no copy in front of the launch
+  int vec(const std::vector<VecDesc>& vd, const PackSpec& pack) {
+    if (B <= kInlineStates) return launch_vec_inline(vd.data(), B, n, nullptr, nullptr, pack, false, stream);
     const VecDesc* dvd = nullptr;
     int rc = upload(vd, &dvd, 0);
     if (rc) return rc;
-    return launch_vec(dvd, B, n, nullptr, nullptr, pack_spec(), false, stream);
+    return launch_vec(dvd, B, n, nullptr, nullptr, pack, false, stream);
   }
 
-  int llg(double* const* Y, double* const* k, void* const* S_out, void* sums) {
+  int llg(double* const* Y, double* const* k, void* const* S_out, void* sums, const std::vector<StageDesc>& next) {
     std::vector<LlgDesc> ld(B);
     for (int b = 0; b < B; ++b) {
       LlgDesc& L = ld[b];
@@ -361,10 +415,18 @@ struct Rk4 {
       L.alpha = alpha;
       L.gamma = gamma;
     }
-    const LlgDesc* dl = nullptr;
-    int rc = upload(ld, &dl, 1);
-    if (rc) return rc;
-    rc = launch_llg(grid, dl, B, stream);
+    NextStage nx;
+    nx.pack = pack_spec();
+    int rc;
+    if (B <= kInlineStates) {
+      nx.h_descs = next.data();
+      rc = launch_llg_inline(grid, ld.data(), B, stream, nx);
+    } else {
+      const LlgDesc* dl = nullptr;
+      rc = upload(ld, &dl, 1);
+      if (rc == kOk) rc = upload(next, &nx.d_descs, 5);
+      if (rc == kOk) rc = launch_llg(grid, dl, B, stream, nx);
+    }
     if (rc) return rc;
     if (S_out && !lattice.v.a)
       for (int b = 0; b < B; ++b)
@@ -372,31 +434,43 @@ struct Rk4 {
     return kOk;
   }
 
-  // dst[b] = base[b] + sum_k c_k src_k[b]; pack: also write dst into the FP32
-  // demag input (not in the FP64 mode, whose input is a plain copy)
-  int combine(double* const* dst, double* const* base, std::vector<std::pair<double* const*, double>> terms,
-              double bcoef = 1.0, bool pack = false) {
-    pack = pack && !fp64;
+  typedef std::vector<std::pair<double* const*, double>> Terms;
+  // dst[b] = base[b] + sum_k c_k src_k[b]
+  int combine(double* const* dst, double* const* base, const Terms& terms) {
     std::vector<VecDesc> vd(B);
     for (int b = 0; b < B; ++b) {
       VecDesc& d = vd[b];
       std::memset(&d, 0, sizeof(d));
       d.dst = dst[b];
       d.base = base ? base[b] : nullptr;
-      d.bcoef = bcoef;
+      d.bcoef = 1.0;
       d.post_scale = 1.0;
-      d.pack_col = pack ? b : -1;
+      d.pack_col = -1;
       for (auto& t : terms) {
         d.src[d.nterm] = t.first[b];
         d.coef[d.nterm] = t.second;
         d.nterm += 1;
       }
     }
-    const VecDesc* dvd = nullptr;
-    int rc = upload(vd, &dvd, 2);
-    if (rc) return rc;
-    const PackSpec none{kPackNone, nullptr, 0, nullptr};
-    return launch_vec(dvd, B, n, nullptr, nullptr, pack ? pack_spec() : none, false, stream);
+    return vec(vd, PackSpec{kPackNone, nullptr, 0, nullptr});
+  }
+  // the same as the next stage of an LL launch
+  std::vector<StageDesc> stage(double* const* dst, double* const* base, const Terms& terms) {
+    std::vector<StageDesc> sd(B);
+    for (int b = 0; b < B; ++b) {
+      StageDesc& d = sd[b];
+      std::memset(&d, 0, sizeof(d));  // the padding too: blocks are compared by their bytes
+      d.dst = dst[b];
+      d.base = base[b];
+      d.bcoef = 1.0;
+      d.post_scale = 1.0;
+      for (auto& t : terms) {
+        d.src[d.nterm] = t.first[b];
+        d.coef[d.nterm] = t.second;
+        d.nterm += 1;
+      }
+    }
+    return sd;
   }
 
   // pointer tables
@@ -410,8 +484,11 @@ struct Rk4 {
   double* seg_stage(long long j, int s) { return seg_y(j) + (size_t)(1 + s) * B * n3(); }    // stage input s
   uint8_t* seg_S(long long j, int s) { return segS + ((size_t)j * 4 + s) * B * n3() * es; }
 
-  // One RK4 step from y (B vectors) to ynext; records stage inputs / demag sums when asked.
-  int step(double* const* y, double* const* ynext, double* const* Yst /*4*B*/, void* const* Sst /*4*B*/) {
+  // One RK4 step from y (B vectors) to ynext; records stage inputs / demag sums when
+  // asked.  Every combination is formed, and packed for its demag pass, by the LL
+  // launch before it (a combination of its own was a launch of 4 us, of 100 for a
+  // step of 128 x 32 x 1).  packed: y has been (by the step before).
+  int step(double* const* y, double* const* ynext, double* const* Yst /*4*B*/, void* const* Sst /*4*B*/, bool packed) {
     const size_t N3 = n3();
     auto W = [&](int k) { return vecs(work + (size_t)k * B * N3, N3); };
     auto k1 = W(0), k2 = W(1), k3 = W(2), k4 = W(3);
@@ -423,25 +500,18 @@ struct Rk4 {
       rc = combine(Yst, Y1.data(), {});
       if (rc) return rc;
     }
-    rc = rhs(Y1.data(), k1.data(), Sst ? Sst : nullptr);
+    rc = rhs(Y1.data(), k1.data(), Sst ? Sst : nullptr, packed, stage(Y2.data(), Y1.data(), {{k1.data(), 0.5 * dt}}));
     if (rc) return rc;
-    // each stage input is packed for its demag pass by the combination that forms it
-    rc = combine(Y2.data(), Y1.data(), {{k1.data(), 0.5 * dt}}, 1.0, true);
+    rc = rhs(Y2.data(), k2.data(), Sst ? Sst + B : nullptr, true,
+             stage(Y3.data(), Y1.data(), {{k2.data(), 0.5 * dt}}));
     if (rc) return rc;
-    rc = rhs(Y2.data(), k2.data(), Sst ? Sst + B : nullptr, true);
+    rc = rhs(Y3.data(), k3.data(), Sst ? Sst + 2 * B : nullptr, true, stage(Y4.data(), Y1.data(), {{k3.data(), dt}}));
     if (rc) return rc;
-    rc = combine(Y3.data(), Y1.data(), {{k2.data(), 0.5 * dt}}, 1.0, true);
-    if (rc) return rc;
-    rc = rhs(Y3.data(), k3.data(), Sst ? Sst + 2 * B : nullptr, true);
-    if (rc) return rc;
-    rc = combine(Y4.data(), Y1.data(), {{k3.data(), dt}}, 1.0, true);
-    if (rc) return rc;
-    rc = rhs(Y4.data(), k4.data(), Sst ? Sst + 3 * B : nullptr, true);
-    if (rc) return rc;
-    // y' = y + h/6 (k1 + 2 k2 + 2 k3 + k4); the kernel reads every operand
-    // element before writing it, so ynext may be y itself
-    return combine(ynext, Y1.data(),
-                   {{k1.data(), dt / 6.0}, {k2.data(), dt / 3.0}, {k3.data(), dt / 3.0}, {k4.data(), dt / 6.0}});
+    // y' = y + h/6 (k1 + 2 k2 + 2 k3 + k4); the launch reads y only at the cell that
+    // it writes, so ynext may be y itself
+    return rhs(Y4.data(), k4.data(), Sst ? Sst + 3 * B : nullptr, true,
+               stage(ynext, Y1.data(),
+                     {{k1.data(), dt / 6.0}, {k2.data(), dt / 3.0}, {k3.data(), dt / 3.0}, {k4.data(), dt / 6.0}}));
   }
 
   int forward(const double* m0_host, double* mT_host) {
@@ -453,7 +523,7 @@ struct Rk4 {
     int rc = combine(cur.data(), ck0.data(), {});
     if (rc) return rc;
     for (long long s = 0; s < nsteps; ++s) {
-      rc = step(cur.data(), nxt.data(), nullptr, nullptr);
+      rc = step(cur.data(), nxt.data(), nullptr, nullptr, s > 0);
       if (rc) return rc;
       std::swap(cur, nxt);
       if ((s + 1) % ck == 0 && (s + 1) < nsteps) {
@@ -470,8 +540,10 @@ struct Rk4 {
     return kOk;
   }
 
-  // mu[b] = vjp of f at stage input Y with cotangent u; accumulates parameter gradients
-  int vjp(double* const* Y, void* const* S, double* const* u, double* const* mu) {
+  // mu[b] = vjp of f at stage input Y with cotangent sum c u; accumulates parameter
+  // gradients.  lam, later: the step's last stage adds mu and the later stages' to lam.
+  int vjp(double* const* Y, void* const* S, const Terms& u, double* const* mu, double* const* lam = nullptr,
+          const std::vector<double* const*>& later = {}) {
     const size_t N3 = n3();
     auto mbar = vecs(work + (size_t)10 * B * N3, N3);
     auto hbar = vecs(work + (size_t)11 * B * N3, N3);
@@ -481,7 +553,10 @@ struct Rk4 {
       std::memset(&d, 0, sizeof(d));  // the padding too: blocks are compared by their bytes
       d.m = Y[b];
       d.S = S[b];
-      d.u = u[b];
+      for (size_t k = 0; k < u.size(); ++k) {
+        d.u[k] = u[k].first[b];
+        d.c[k] = u[k].second;
+      }
       d.mbar = mbar[b];
       d.hbar = hbar[b];
       d.packed = lattice.v.a ? packd : hcol(packd, b);
@@ -494,12 +569,12 @@ struct Rk4 {
       d.alpha = alpha;
       d.gamma = gamma;
     }
-    const VjpDesc* dvd = nullptr;
-    int rc = upload(vd, &dvd, 3);
+    int rc = by_state(vd, 3, [&](auto by_value, const VjpDesc* d, const Inline<VjpDesc>& inl) {
+      constexpr bool V = decltype(by_value)::value;
+      if (fp64) hipLaunchKernelGGL((vjp_kernel<double, V>), dim3(nblocks(), B), dim3(256), 0, stream, grid, d, inl);
+      else hipLaunchKernelGGL((vjp_kernel<float, V>), dim3(nblocks(), B), dim3(256), 0, stream, grid, d, inl);
+    });
     if (rc) return rc;
-    if (fp64) hipLaunchKernelGGL(vjp_kernel<double>, dim3(nblocks(), B), dim3(256), 0, stream, grid, dvd);
-    else hipLaunchKernelGGL(vjp_kernel<float>, dim3(nblocks(), B), dim3(256), 0, stream, grid, dvd);
-    MT_HIP(hipGetLastError());
     rc = demag_pass();
     if (rc) return rc;
     std::vector<FinishDesc> fd(B);
@@ -511,12 +586,29 @@ struct Rk4 {
       fd[b].hbar = hbar[b];
       fd[b].T = hcol(hbuf, b);
       fd[b].mu = mu[b];
+      fd[b].lam = lam ? lam[b] : nullptr;
+      for (size_t k = 0; k < later.size(); ++k) fd[b].later[k] = later[k][b];
     }
-    const FinishDesc* dfd = nullptr;
-    rc = upload(fd, &dfd, 4);
-    if (rc) return rc;
-    if (fp64) hipLaunchKernelGGL(vjp_finish_kernel<double>, dim3(nblocks(), B), dim3(256), 0, stream, grid, dfd);
-    else hipLaunchKernelGGL(vjp_finish_kernel<float>, dim3(nblocks(), B), dim3(256), 0, stream, grid, dfd);
+    return by_state(fd, 4, [&](auto by_value, const FinishDesc* d, const Inline<FinishDesc>& inl) {
+      constexpr bool V = decltype(by_value)::value;
+      const dim3 blocks(nblocks(), B);
+      if (fp64) hipLaunchKernelGGL((vjp_finish_kernel<double, V>), blocks, dim3(256), 0, stream, grid, d, inl);
+      else hipLaunchKernelGGL((vjp_finish_kernel<float, V>), blocks, dim3(256), 0, stream, grid, d, inl);
+    });
+  }
+  // launch(by value?, device descriptors, descriptors by value)
+  template <typename D, typename F>
+  int by_state(const std::vector<D>& v, size_t kind, F&& launch) {
+    Inline<D> inl{};
+    if (B <= kInlineStates) {
+      for (int b = 0; b < B; ++b) inl.d[b] = v[b];
+      launch(std::true_type{}, nullptr, inl);
+    } else {
+      const D* d = nullptr;
+      int rc = upload(v, &d, kind);
+      if (rc) return rc;
+      launch(std::false_type{}, d, inl);
+    }
     MT_HIP(hipGetLastError());
     return kOk;
   }
@@ -531,7 +623,7 @@ struct Rk4 {
     MT_HIP(hipMemsetAsync(hext_part, 0, (size_t)B * nblocks() * 3 * sizeof(double), stream));
     auto lam = vecs(work + (size_t)12 * B * N3, N3);
     auto W = [&](int k) { return vecs(work + (size_t)k * B * N3, N3); };
-    auto kb = W(0), mu4 = W(1), mu3 = W(2), mu2 = W(3), mu1 = W(4);
+    auto mu4 = W(1), mu3 = W(2), mu2 = W(3), mu1 = W(4);
     for (int b = 0; b < B; ++b)
       MT_HIP(hipMemcpyAsync(lam[b], gT_host + (size_t)b * N3, N3 * sizeof(double), hipMemcpyHostToDevice, stream));
     int rc;
@@ -554,7 +646,7 @@ struct Rk4 {
           }
         auto yj = vecs(seg_y(j), N3);
         auto yn = vecs(seg_y(j + 1), N3);
-        rc = step(yj.data(), yn.data(), Yst.data(), Sst.data());
+        rc = step(yj.data(), yn.data(), Yst.data(), Sst.data(), j > 0);
         if (rc) return rc;
       }
       // backward through the segment
@@ -571,23 +663,14 @@ struct Rk4 {
         };
         auto Y1 = st(0), Y2 = st(1), Y3 = st(2), Y4 = st(3);
         auto S1 = sS(0), S2 = sS(1), S3 = sS(2), S4 = sS(3);
-        rc = combine(kb.data(), nullptr, {{lam.data(), dt / 6.0}});
+        rc = vjp(Y4.data(), S4.data(), {{lam.data(), dt / 6.0}}, mu4.data());
         if (rc) return rc;
-        rc = vjp(Y4.data(), S4.data(), kb.data(), mu4.data());
+        rc = vjp(Y3.data(), S3.data(), {{lam.data(), dt / 3.0}, {mu4.data(), dt}}, mu3.data());
         if (rc) return rc;
-        rc = combine(kb.data(), nullptr, {{lam.data(), dt / 3.0}, {mu4.data(), dt}});
+        rc = vjp(Y2.data(), S2.data(), {{lam.data(), dt / 3.0}, {mu3.data(), 0.5 * dt}}, mu2.data());
         if (rc) return rc;
-        rc = vjp(Y3.data(), S3.data(), kb.data(), mu3.data());
-        if (rc) return rc;
-        rc = combine(kb.data(), nullptr, {{lam.data(), dt / 3.0}, {mu3.data(), 0.5 * dt}});
-        if (rc) return rc;
-        rc = vjp(Y2.data(), S2.data(), kb.data(), mu2.data());
-        if (rc) return rc;
-        rc = combine(kb.data(), nullptr, {{lam.data(), dt / 6.0}, {mu2.data(), 0.5 * dt}});
-        if (rc) return rc;
-        rc = vjp(Y1.data(), S1.data(), kb.data(), mu1.data());
-        if (rc) return rc;
-        rc = combine(lam.data(), lam.data(), {{mu1.data(), 1.0}, {mu2.data(), 1.0}, {mu3.data(), 1.0}, {mu4.data(), 1.0}});
+        rc = vjp(Y1.data(), S1.data(), {{lam.data(), dt / 6.0}, {mu2.data(), 0.5 * dt}}, mu1.data(), lam.data(),
+                 {mu2.data(), mu3.data(), mu4.data()});
         if (rc) return rc;
       }
     }
