@@ -16,10 +16,12 @@
 
 namespace mt {
 
-// What the right-hand side of a cell reads, apart from the demag sums.  The
-// kernels issue these reads (and the next stage's, below) before anything waits
-// for another: a launch of a small problem is little more than its round trips
-// to memory.
+// What the right-hand side of a cell reads, apart from the demag sums.  AHEAD: the
+// kernels issue these reads (and the next stage's, below) before anything waits for
+// another, since a launch of a small problem is little more than its round trips to
+// memory.  Otherwise only the vector's values are; the rest is read where it is used
+// (the near-band kernel: 60 registers and eight waves per SIMD, 88 and five with all
+// of it in flight, 117 and 159 us a launch of 64 states at 256 x 64 x 2).
 struct CellReads {
   double c0[3], xm[3], xp[3], ym[3], yp[3], zm[3], zp[3];
   double jf, kf, ms64, aniso[6];  // aniso: xx xy xz yy yz zz
@@ -27,13 +29,14 @@ struct CellReads {
   int kb, ke;
 };
 
+template <bool AHEAD = true>
 __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc& D, int i) {
   CellReads r;
   const int n = g.n;
   const double* m = D.m;
 #pragma unroll
   for (int c = 0; c < 3; ++c) r.c0[c] = m[(size_t)c * n + i];
-  r.jf = g.jfact[i];
+  if (AHEAD) r.jf = g.jfact[i];
   r.kb = r.ke = 0;
   if (g.xs) {
     r.kb = g.xs[i];
@@ -51,8 +54,9 @@ __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc&
       r.xm[c] = v[xm]; r.xp[c] = v[xp];
       r.ym[c] = v[ym]; r.yp[c] = v[yp];
     }
-    if (g.nz > 1) {
-      const int zm = iz > 0 ? i - sz : i, zp = iz < g.nz - 1 ? i + sz : i;
+    if (!AHEAD || g.nz > 1) {
+      const bool z3 = g.nz > 1;
+      const int zm = z3 && iz > 0 ? i - sz : i, zp = z3 && iz < g.nz - 1 ? i + sz : i;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         const double* v = m + (size_t)c * n;
@@ -60,6 +64,7 @@ __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc&
       }
     }
   }
+  if (!AHEAD) return r;
   if (D.hpart64) r.ms64 = g.ms64[i];
   else r.ms32 = g.ms32[i];
   if (g.aniso) {
@@ -74,7 +79,7 @@ __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc&
 // hsum(c) returns the FP32 demag sum S_c = sum of the partials of (K m)_c at i
 // (used unless D.hpart64 holds FP64 sums).  dm: dm/dt, which goes to D.out as
 // well.
-template <typename HS>
+template <bool AHEAD = true, typename HS>
 __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, const CellReads& r, HS hsum,
                                          double (&dm)[3]) {
   const int n = g.n;
@@ -83,44 +88,48 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
   if (g.xs) {
     // loaded operator: alpha = -2 times the row's stored entries in order
     // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
+    const CellReads q = AHEAD ? r : cell_reads<false>(g, D, i);
+    const double jf = AHEAD ? r.jf : g.jfact[i];
     for (int c = 0; c < 3; ++c) {
       const double* v = m + (size_t)c * n;
-      mc[c] = r.c0[c];
+      mc[c] = q.c0[c];
       double sum = 0.0;
-      for (int k = r.kb; k < r.ke; ++k) sum += g.xv[k] * v[g.xc[k]];
-      hj[c] = (-2.0 * sum) * r.jf;
+      for (int k = q.kb; k < q.ke; ++k) sum += g.xv[k] * v[g.xc[k]];
+      hj[c] = (-2.0 * sum) * jf;
     }
   } else {
     // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1)
     const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
+    const CellReads q = AHEAD ? r : cell_reads<false>(g, D, i);
+    const double jf = AHEAD ? r.jf : g.jfact[i];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const double vi = r.c0[c];
+      const double vi = q.c0[c];
       mc[c] = vi;
-      double lx = ix == 0 ? (r.xp[c] - vi) : (ix == g.nx - 1 ? (r.xm[c] - vi) : (r.xm[c] - 2.0 * vi + r.xp[c]));
-      double ly = iy == 0 ? (r.yp[c] - vi) : (iy == g.ny - 1 ? (r.ym[c] - vi) : (r.ym[c] - 2.0 * vi + r.yp[c]));
+      double lx = ix == 0 ? (q.xp[c] - vi) : (ix == g.nx - 1 ? (q.xm[c] - vi) : (q.xm[c] - 2.0 * vi + q.xp[c]));
+      double ly = iy == 0 ? (q.yp[c] - vi) : (iy == g.ny - 1 ? (q.ym[c] - vi) : (q.ym[c] - 2.0 * vi + q.yp[c]));
       double lap = lx * g.idx2 + ly * g.idy2;
       if (g.nz > 1) {
-        double lz = iz == 0 ? (r.zp[c] - vi) : (iz == g.nz - 1 ? (r.zm[c] - vi) : (r.zm[c] - 2.0 * vi + r.zp[c]));
+        double lz = iz == 0 ? (q.zp[c] - vi) : (iz == g.nz - 1 ? (q.zm[c] - vi) : (q.zm[c] - 2.0 * vi + q.zp[c]));
         lap += lz * g.idz2;
       }
-      hj[c] = (-2.0 * lap) * r.jf;
+      hj[c] = (-2.0 * lap) * jf;
     }
   }
   // demag: S = sum_k partial (K m); field = fl32(fl32(-S) * Ms_i)
   if (D.hpart64) {
-    for (int c = 0; c < 3; ++c) hm[c] = (-D.hpart64[(int64_t)c * n + i]) * r.ms64;
+    for (int c = 0; c < 3; ++c) hm[c] = (-D.hpart64[(int64_t)c * n + i]) * (AHEAD ? r.ms64 : g.ms64[i]);
   } else {
     for (int c = 0; c < 3; ++c) {
       const float s = hsum(c);
       if (D.sum_out) D.sum_out[(int64_t)c * n + i] = s;
-      float h = (-s) * r.ms32;
+      float h = (-s) * (AHEAD ? r.ms32 : g.ms32[i]);
       hm[c] = (double)h;
     }
   }
   if (g.aniso) {
-    const double(&A)[6] = r.aniso;
-    double f = -2.0 * r.kf;
+    const double* A = AHEAD ? r.aniso : g.aniso + (size_t)i * 6;  // xx xy xz yy yz zz
+    double f = -2.0 * (AHEAD ? r.kf : g.kfact[i]);
     hk[0] = f * (A[0] * mc[0] + A[1] * mc[1] + A[2] * mc[2]);
     hk[1] = f * (A[1] * mc[0] + A[3] * mc[1] + A[4] * mc[2]);
     hk[2] = f * (A[2] * mc[0] + A[4] * mc[1] + A[5] * mc[2]);
