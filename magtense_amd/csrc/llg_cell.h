@@ -16,12 +16,12 @@
 
 namespace mt {
 
-// What the right-hand side of a cell reads, apart from the demag sums.  AHEAD: the
-// kernels issue these reads (and the next stage's, below) before anything waits for
-// another, since a launch of a small problem is little more than its round trips to
-// memory.  Otherwise only the vector's values are; the rest is read where it is used
-// (the near-band kernel: 60 registers and eight waves per SIMD, 88 and five with all
-// of it in flight, 117 and 159 us a launch of 64 states at 256 x 64 x 2).
+// What the right-hand side of a cell reads, apart from the demag sums.  The
+// kernels issue these reads (and the next stage's, below) before anything waits
+// for another: a launch of a small problem is little more than its round trips
+// to memory.  (The near-band kernel reads each value where it is used: 60 registers
+// and eight waves per SIMD, 88 and five with all of them in flight, 117 and 171 us a
+// launch of 64 states at 256 x 64 x 2.)
 struct CellReads {
   double c0[3], xm[3], xp[3], ym[3], yp[3], zm[3], zp[3];
   double jf, kf, ms64, aniso[6];  // aniso: xx xy xz yy yz zz
@@ -29,14 +29,13 @@ struct CellReads {
   int kb, ke;
 };
 
-template <bool AHEAD = true>
 __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc& D, int i) {
   CellReads r;
   const int n = g.n;
   const double* m = D.m;
 #pragma unroll
   for (int c = 0; c < 3; ++c) r.c0[c] = m[(size_t)c * n + i];
-  if (AHEAD) r.jf = g.jfact[i];
+  r.jf = g.jfact[i];
   r.kb = r.ke = 0;
   if (g.xs) {
     r.kb = g.xs[i];
@@ -54,9 +53,8 @@ __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc&
       r.xm[c] = v[xm]; r.xp[c] = v[xp];
       r.ym[c] = v[ym]; r.yp[c] = v[yp];
     }
-    if (!AHEAD || g.nz > 1) {
-      const bool z3 = g.nz > 1;
-      const int zm = z3 && iz > 0 ? i - sz : i, zp = z3 && iz < g.nz - 1 ? i + sz : i;
+    if (g.nz > 1) {
+      const int zm = iz > 0 ? i - sz : i, zp = iz < g.nz - 1 ? i + sz : i;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         const double* v = m + (size_t)c * n;
@@ -64,7 +62,6 @@ __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc&
       }
     }
   }
-  if (!AHEAD) return r;
   if (D.hpart64) r.ms64 = g.ms64[i];
   else r.ms32 = g.ms32[i];
   if (g.aniso) {
@@ -85,35 +82,81 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
   const int n = g.n;
   const double* m = D.m;
   double mc[3], hj[3], hm[3], hk[3];
-  if (g.xs) {
-    // loaded operator: alpha = -2 times the row's stored entries in order
-    // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
-    const CellReads q = AHEAD ? r : cell_reads<false>(g, D, i);
-    const double jf = AHEAD ? r.jf : g.jfact[i];
-    for (int c = 0; c < 3; ++c) {
-      const double* v = m + (size_t)c * n;
-      mc[c] = q.c0[c];
-      double sum = 0.0;
-      for (int k = q.kb; k < q.ke; ++k) sum += g.xv[k] * v[g.xc[k]];
-      hj[c] = (-2.0 * sum) * jf;
+  if constexpr (AHEAD) {
+    if (g.xs) {
+      // loaded operator: alpha = -2 times the row's stored entries in order
+      // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
+      for (int c = 0; c < 3; ++c) {
+        const double* v = m + (size_t)c * n;
+        mc[c] = r.c0[c];
+        double sum = 0.0;
+        for (int k = r.kb; k < r.ke; ++k) sum += g.xv[k] * v[g.xc[k]];
+        hj[c] = (-2.0 * sum) * r.jf;
+      }
+    } else {
+      // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1)
+      const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double vi = r.c0[c];
+        mc[c] = vi;
+        double lx = ix == 0 ? (r.xp[c] - vi) : (ix == g.nx - 1 ? (r.xm[c] - vi) : (r.xm[c] - 2.0 * vi + r.xp[c]));
+        double ly = iy == 0 ? (r.yp[c] - vi) : (iy == g.ny - 1 ? (r.ym[c] - vi) : (r.ym[c] - 2.0 * vi + r.yp[c]));
+        double lap = lx * g.idx2 + ly * g.idy2;
+        if (g.nz > 1) {
+          double lz = iz == 0 ? (r.zp[c] - vi) : (iz == g.nz - 1 ? (r.zm[c] - vi) : (r.zm[c] - 2.0 * vi + r.zp[c]));
+          lap += lz * g.idz2;
+        }
+        hj[c] = (-2.0 * lap) * r.jf;
+      }
     }
   } else {
-    // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1)
-    const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
-    const CellReads q = AHEAD ? r : cell_reads<false>(g, D, i);
-    const double jf = AHEAD ? r.jf : g.jfact[i];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const double vi = q.c0[c];
-      mc[c] = vi;
-      double lx = ix == 0 ? (q.xp[c] - vi) : (ix == g.nx - 1 ? (q.xm[c] - vi) : (q.xm[c] - 2.0 * vi + q.xp[c]));
-      double ly = iy == 0 ? (q.yp[c] - vi) : (iy == g.ny - 1 ? (q.ym[c] - vi) : (q.ym[c] - 2.0 * vi + q.yp[c]));
-      double lap = lx * g.idx2 + ly * g.idy2;
-      if (g.nz > 1) {
-        double lz = iz == 0 ? (q.zp[c] - vi) : (iz == g.nz - 1 ? (q.zm[c] - vi) : (q.zm[c] - 2.0 * vi + q.zp[c]));
-        lap += lz * g.idz2;
+    const int ix = i % g.nx;
+    const int iy = (i / g.nx) % g.ny;
+    const int iz = i / (g.nx * g.ny);
+    const int sy = g.nx, sz = g.nx * g.ny;
+    if (g.xs) {
+      // loaded operator: alpha = -2 times the row's stored entries in order
+      // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
+      const int kb = g.xs[i], ke = g.xe[i];
+      for (int c = 0; c < 3; ++c) {
+        const double* v = m + (size_t)c * n;
+        mc[c] = v[i];
+        double sum = 0.0;
+        for (int k = kb; k < ke; ++k) sum += g.xv[k] * v[g.xc[k]];
+        hj[c] = (-2.0 * sum) * g.jfact[i];
       }
-      hj[c] = (-2.0 * lap) * jf;
+    } else {
+      // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1).  The
+      // neighbour indices are clamped to the cell itself at a boundary, so every
+      // load is issued unconditionally before the per-row formula is selected.
+      const int xm = ix > 0 ? i - 1 : i, xp = ix < g.nx - 1 ? i + 1 : i;
+      const int ym = iy > 0 ? i - sy : i, yp = iy < g.ny - 1 ? i + sy : i;
+      const bool z3 = g.nz > 1;
+      const int zm = z3 && iz > 0 ? i - sz : i, zp = z3 && iz < g.nz - 1 ? i + sz : i;
+      double c0[3], cxm[3], cxp[3], cym[3], cyp[3], czm[3], czp[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double* v = m + (size_t)c * n;
+        c0[c] = v[i];
+        cxm[c] = v[xm]; cxp[c] = v[xp];
+        cym[c] = v[ym]; cyp[c] = v[yp];
+        czm[c] = v[zm]; czp[c] = v[zp];
+      }
+      const double jf = g.jfact[i];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const double vi = c0[c];
+        mc[c] = vi;
+        double lx = ix == 0 ? (cxp[c] - vi) : (ix == g.nx - 1 ? (cxm[c] - vi) : (cxm[c] - 2.0 * vi + cxp[c]));
+        double ly = iy == 0 ? (cyp[c] - vi) : (iy == g.ny - 1 ? (cym[c] - vi) : (cym[c] - 2.0 * vi + cyp[c]));
+        double lap = lx * g.idx2 + ly * g.idy2;
+        if (z3) {
+          double lz = iz == 0 ? (czp[c] - vi) : (iz == g.nz - 1 ? (czm[c] - vi) : (czm[c] - 2.0 * vi + czp[c]));
+          lap += lz * g.idz2;
+        }
+        hj[c] = (-2.0 * lap) * jf;
+      }
     }
   }
   // demag: S = sum_k partial (K m); field = fl32(fl32(-S) * Ms_i)
@@ -128,11 +171,13 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
     }
   }
   if (g.aniso) {
-    const double* A = AHEAD ? r.aniso : g.aniso + (size_t)i * 6;  // xx xy xz yy yz zz
-    double f = -2.0 * (AHEAD ? r.kf : g.kfact[i]);
-    hk[0] = f * (A[0] * mc[0] + A[1] * mc[1] + A[2] * mc[2]);
-    hk[1] = f * (A[1] * mc[0] + A[3] * mc[1] + A[4] * mc[2]);
-    hk[2] = f * (A[2] * mc[0] + A[4] * mc[1] + A[5] * mc[2]);
+    auto axes = [&](const auto& A, double f) {  // xx xy xz yy yz zz
+      hk[0] = f * (A[0] * mc[0] + A[1] * mc[1] + A[2] * mc[2]);
+      hk[1] = f * (A[1] * mc[0] + A[3] * mc[1] + A[4] * mc[2]);
+      hk[2] = f * (A[2] * mc[0] + A[4] * mc[1] + A[5] * mc[2]);
+    };
+    if constexpr (AHEAD) axes(r.aniso, -2.0 * r.kf);
+    else axes(g.aniso + (size_t)i * 6, -2.0 * g.kfact[i]);
   } else {
     hk[0] = hk[1] = hk[2] = 0.0;
   }
