@@ -39,6 +39,7 @@ MU0 = 4e-7 * np.pi
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0  # dense MFMA, MI355X
 FP32_PEAK_TFLOPS = 157.3  # FP32 matrix, MI355X
+FP32_VALU_TFLOPS = 78.6  # FP32 vector without packed instructions
 
 
 def traffic_from_profile(kind):
@@ -490,7 +491,7 @@ def next_rows(W, reps=5):
         "list_entries": int(ent.value), "stored_fraction_of_dense": 4.0 * ent.value / tiles_all,
         "fragment_bytes": float(nbytes.value), "ksplit": int(ksb.value), "ms_per_product": ms_apply_b,
         "rel_diff_vs_fp32_csr": rel_b,
-        "roofline": {"bound": "hbm", "kernel": "gemm_bf16x2_reg_kernel<4, false, true, false>",
+        "roofline": {"bound": "hbm", "kernel": "gemm_bf16x2_reg_kernel<3, false, true, false, 2>",
                      "achieved": alg_b / (ms_apply_b * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": alg_b / (ms_apply_b * 1e-3) / 1e9 / HBM_PEAK_GBS, "alg_bytes_per_launch": alg_b},
         "note": "wall time per synchronous mt_demag_apply_sparse call (state packing, GEMM over the stored tiles, "
@@ -502,7 +503,7 @@ def next_rows(W, reps=5):
         "workload": out["sparse_demag"]["workload"] + ", kept entries as FP32 32x16 tiles (FP32 MFMAs)",
         "build_s": t_build_f, "list_entries": int(entf.value), "ksplit": int(ksf.value), "ms_per_product": ms_apply_f,
         "speedup_vs_csr": ms_apply / ms_apply_f, "rel_diff_vs_fp32_csr": rel_f,
-        "roofline": {"bound": "mfma", "kernel": "gemm_bf16x2_reg_kernel<4, false, true, true> (FP32 fragments)",
+        "roofline": {"bound": "mfma", "kernel": "gemm_bf16x2_reg_kernel<3, false, true, true, 2> (FP32 fragments)",
                      "achieved": tf_f, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tf_f / FP32_PEAK_TFLOPS,
                      "alg_flops_per_launch": flops_f},
         "note": "wall time per synchronous mt_demag_apply_sparse call; FP32 products with FP32 accumulation "
@@ -641,7 +642,7 @@ def _oracle_run(res, L, m0, hext, t, **kw):
     return time.perf_counter() - t0, st, np.transpose(y[0, -1])
 
 
-def _line(wall, st, timed_st, n, cells_bytes):
+def _line(wall, st, timed_st, n, alg_flops):
     """steps/s, RHS/s and the per-step time split of one GPU run."""
     steps = max(st["steps"], 1)
     out = dict(wall_s=wall, steps=st["steps"], rhs=st["f_calls"], steps_per_s=st["steps"] / wall,
@@ -654,11 +655,12 @@ def _line(wall, st, timed_st, n, cells_bytes):
         out["demag_ms_per_launch"] = timed_st["demag_ms"] / passes
         kern = (timed_st["demag_ms"] + timed_st["llg_ms"] + timed_st["vec_ms"]) / ts
         out["gpu_kernel_frac_of_step"] = kern / out["ms_per_step"]
-        if cells_bytes:
-            gbs = cells_bytes / (out["demag_ms_per_launch"] * 1e-3) / 1e9
-            out["roofline"] = {"bound": "hbm", "kernel": "demag_llg_f32_kernel (FP32 demag rows + LL right-hand side)",
-                               "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS,
-                               "alg_bytes_per_launch": cells_bytes}
+        if alg_flops:
+            tf = alg_flops / (out["demag_ms_per_launch"] * 1e-3) / 1e12
+            out["roofline"] = {"bound": "fp32 valu", "kernel": "lattice_rows_kernel (FP32 demag rows from the "
+                               "grid's distinct tensor entries)",
+                               "achieved": tf, "peak": FP32_VALU_TFLOPS, "unit": "TFLOP/s",
+                               "frac": tf / FP32_VALU_TFLOPS, "alg_flops_per_launch": alg_flops}
     return out
 
 
@@ -695,10 +697,11 @@ def small_configs(no_cpu=False):
     _, st_t, _ = _gpu_run(res, L, m_rel, h_dyn, 1e-9, 200, 2000, timing=True, gamma=2.21e5, **kw)
     c1 = {"workload": "32x8x1 film (15.6x15.6x3 nm), N = 256: relaxation 5 ns (gamma 0) + 1 ns dynamics, FP32 demag",
           "relax": _line(w_rel, st_rel, None, 256, 0), "dynamics": _line(w_dyn, st_dyn, st_t, 256, 0),
-          "note": "the 1.6 MB tensor stays in L2: the step is bound by kernel latency and the host's launch "
-                  "submissions (one launch per right-hand side: stage combination, FP32 demag rows and LL "
-                  "right-hand side in one kernel) and the one host round trip per step of the RKSUITE controller, "
-                  "not by HBM; kernel_ms_per_step.demag includes the stage combination and the LL right-hand side"}
+          "note": "the 1.6 MB tensor stays in L2: the step is bound by the latency of its chain of dependent "
+                  "launches (one per right-hand side: FP32 demag rows, LL right-hand side and the next stage's "
+                  "argument in one kernel) and the one reduction result per step that the RKSUITE controller "
+                  "waits for, not by HBM; kernel_ms_per_step.demag includes the LL right-hand side and the stage "
+                  "arguments"}
     if not no_cpu:
         ht = np.linspace(0, 5e-9, 200)
         hext = np.zeros((200, 4))
@@ -736,7 +739,7 @@ def small_configs(no_cpu=False):
     _, st2t, _ = _gpu_run(res, L, m0, h_c2, 2e-9, 21, 10, timing=True, **kw2)
     c2 = {"workload": f"128x32x1 film (3.9x3.9x3 nm), N = 4096, {mag:.1f} mT in-plane at "
                       f"{np.degrees(theta):.0f} deg, 2 ns from a random start, FP32 demag (402.7 MB tensor)",
-          "run": _line(w2, st2, st2t, n, 6.0 * n * n * 4 + 2 * 3 * n * 4)}
+          "run": _line(w2, st2, st2t, n, 18.0 * n * n)}
     if not no_cpu:
         # two oracle runs of the same problem over 1 ps and 4 ps: both assemble
         # the tensor once, so the difference of their times over the difference
@@ -889,9 +892,10 @@ def main():
         plain_info = dict(steps_per_s=plain, batch_steps=bs2, wall_s=wall2, demag_passes=int(plain_passes),
                           passes_per_batch_step=plain_passes / max(bs2, 1e-9),
                           ms_per_pass=1e3 * wall2 / max(plain_passes, 1),
-                          note="one pass = the 64 per-state FP32 mat-vecs of one right-hand side "
-                               "(demag_llg_f32_kernel: the FP32 rows, 6 N^2 4 B per state, fused with the LL "
-                               "right-hand side)")
+                          note="one pass = the FP32 rows of one right-hand side for all 64 states "
+                               "(lattice_rows_kernel: the uniform grid's distinct tensor entries, several states "
+                               "to a read), summed per state in the order of the one-state product, then the LL "
+                               "kernel")
         log(f"fp32 plain: {args.plain_steps} steps in {wall2:.3f} s = {plain:.4f} steps/s, {plain_passes} passes")
     # ---- batched FP32 MFMA (precision fp32_mfma): the reference's arithmetic class, one tensor pass per RHS
     mfma32 = None
@@ -914,7 +918,7 @@ def main():
         mfma32 = dict(steps_per_s=bs3 / wall3, batch_steps=bs3, wall_s=wall3,
                       passes_per_batch_step=(s31[0].demag_passes - s30[0].demag_passes) / max(bs3, 1e-9),
                       gemm_ms=g3, speedup_vs_plain_fp32=(bs3 / wall3 / plain) if plain else None,
-                      roofline={"bound": "mfma", "kernel": "gemm_bf16x2_reg_kernel<4, false, false, true> (FP32 fragments)",
+                      roofline={"bound": "mfma", "kernel": "gemm_bf16x2_reg_kernel<3, false, false, true, 2> (FP32 fragments)",
                                 "achieved": tf3, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                                 "frac": tf3 / FP32_PEAK_TFLOPS, "alg_flops_per_launch": alg_flops},
                       note="precision fp32_mfma: the FP32 tensor as MFMA fragments, FP32 products and sums, one "
@@ -947,7 +951,7 @@ def main():
         achieved = alg_bytes / (gemm_ms * 1e-3) / 1e9
         roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic_from_profile("dense"),
-                    "kernel": "gemm_bf16x2_reg_kernel<4, false, false, false>", "kernel_ms": gemm_ms,
+                    "kernel": "gemm_bf16x2_reg_kernel<3, false, false, false, 2>", "kernel_ms": gemm_ms,
                     "alg_bytes_per_launch": alg_bytes, "measured_read_peak": rd.value,
                     "frac_of_measured_read_peak": achieved / rd.value,
                     "measured_read_peak_random_bits": rdr.value,
