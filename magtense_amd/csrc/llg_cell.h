@@ -19,8 +19,8 @@ namespace mt {
 // What the right-hand side of a cell reads, apart from the demag sums.  The
 // kernels issue these reads (and the next stage's, below) before anything waits
 // for another: a launch of a small problem is little more than its round trips
-// to memory.  (The near-band kernel reads each value where it is used: 60 registers
-// and eight waves per SIMD, 88 and five with all of them in flight, 117 and 171 us a
+// to memory.  (The near-band kernel reads each value where it is used: 63 registers
+// and eight waves per SIMD, 88 and five with all of them in flight, 123 and 171 us a
 // launch of 64 states at 256 x 64 x 2.)
 struct CellReads {
   double c0[3], xm[3], xp[3], ym[3], yp[3], zm[3], zp[3];

@@ -97,7 +97,7 @@ struct Op {
   VecDesc vec{};      // kVec
   double res[4] = {0, 0, 0, 0};
   double post_res[4] = {0, 0, 0, 0};
-  bool defer_pre = false;  // kEval: the pre-reduction's result may wait for the next synchronising tick
+  VecDesc early{};    // kEval: a reduction whose result may come with post's (rkind may be none), to res
 };
 
 struct Sim {
@@ -336,10 +336,11 @@ struct Solver {
   static constexpr int kMaxLines = 512;                 // of a launch: 32 KiB for the host to read
   static constexpr size_t kMaxLineBytes = 4u << 20;
   // Destination of the reductions of a launch over d (kind 0 vector operations, 1
-  // pre, 2 post), and the note of what the host will find.
-  ResultLines result_lines(int kind, const std::vector<VecDesc>& d) {
+  // pre, 2 post; kinds: 2 for kinds 1 and 2 together), and the note of what the
+  // host will find.
+  ResultLines result_lines(int kind, const std::vector<VecDesc>& d, int kinds = 1) {
     ResultLines l;
-    if (lines_d && (int64_t)d.size() * res_stride <= kMaxLines) {
+    if (lines_d && (int64_t)d.size() * res_stride <= kinds * kMaxLines) {
       if (++res_seq == 0) res_seq = 1;  // 0: a line never written
       l = ResultLines{lines_d + (size_t)kind * B * res_stride, res_stride, res_seq};
     }
@@ -565,7 +566,7 @@ struct Solver {
 
   // ---- operations issued by the per-state coroutines ----------------------
   OpAwait eval(Sim& s, double t, const VecDesc& pre, double* out, const VecDesc& post, double* fields = nullptr,
-               bool defer_pre = false) {
+               const VecDesc& early = blank()) {
     s.op = Op();
     s.op.kind = Op::kEval;
     s.op.pre = pre;
@@ -573,7 +574,7 @@ struct Solver {
     s.op.t = t;
     s.op.out = out;
     s.op.fields = fields;
-    s.op.defer_pre = defer_pre;
+    s.op.early = early;
     return OpAwait{&s};
   }
   OpAwait vec(Sim& s, const VecDesc& d) {
@@ -625,6 +626,7 @@ struct Solver {
         co_await vec(s, w);
       }
       bool restart = false;
+      VecDesc early = blank();
       for (int i = 2; i <= 8; ++i) {
         VecDesc pre = blank();
         // consecutive stage arguments alternate between two vectors: the launch
@@ -636,14 +638,15 @@ struct Solver {
         for (int j = 2; j <= i - 1; ++j)
           if (T.A[i][j] != 0.0) add_term(pre, s.stage[j - 1], htry * T.A[i][j]);
         if (i == 7) {  // stepb (RKSuitef90.f90:1957-1976)
-          pre.rkind = kRedStepB;
-          pre.rn = 5;
-          pre.rsrc[0] = s.yp; pre.rcoef[0] = T.E[1];
-          pre.rsrc[1] = s.stage[2]; pre.rcoef[1] = T.E[3];
-          pre.rsrc[2] = s.stage[3]; pre.rcoef[2] = T.E[4];
-          pre.rsrc[3] = s.stage[4]; pre.rcoef[3] = T.E[5];
-          pre.rsrc[4] = s.stage[5]; pre.rcoef[4] = T.E[6];
-          pre.ra = s.y; pre.rb = s.scratch; pre.thresh = thres;
+          VecDesc& stepb = defer_early ? early : pre;
+          stepb.rkind = kRedStepB;
+          stepb.rn = 5;
+          stepb.rsrc[0] = s.yp; stepb.rcoef[0] = T.E[1];
+          stepb.rsrc[1] = s.stage[2]; stepb.rcoef[1] = T.E[3];
+          stepb.rsrc[2] = s.stage[3]; stepb.rcoef[2] = T.E[4];
+          stepb.rsrc[3] = s.stage[4]; stepb.rcoef[3] = T.E[5];
+          stepb.rsrc[4] = s.stage[5]; stepb.rcoef[4] = T.E[6];
+          stepb.ra = s.y; stepb.rb = s.scratch; stepb.thresh = thres;
         }
         double tstg = tnow + T.Cc[i] * htry;
         if (s.at_t_end && T.Cc[i] == 1.0) tstg = s.t_end;
@@ -666,12 +669,12 @@ struct Solver {
         }
         // Stage 8 is formed from stages 1..7 whatever the early estimate says,
         // so when a right-hand side is cheap next to a host round trip the
-        // estimate is read together with stage 8's: a failed estimate then
-        // rejects the step exactly as before and the extra stage-8
-        // evaluation is discarded uncounted.
-        const bool defer = i == 7 && defer_early;
-        co_await eval(s, tstg, pre, s.stage[i - 1], post, nullptr, defer);
-        if (defer) continue;
+        // estimate is formed and read together with stage 8's (its operands, the
+        // argument of stage 7 in the other vector among them, are still there):
+        // a failed estimate then rejects the step exactly as before and the
+        // extra stage-8 evaluation is discarded uncounted.
+        co_await eval(s, tstg, pre, s.stage[i - 1], post, nullptr, i == 8 ? early : blank());
+        if (i == 7 && defer_early) continue;
         if (i == 7 || (i == 8 && defer_early)) {
           err = std::fabs(s.h) * s.op.res[0];  // stepb scales by |comm%h|
           if (err > s.tol) co_return 0;       // the stage-7 evaluation is not counted
@@ -1278,7 +1281,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
   for (size_t g0 = 0; g0 < evals.size(); g0 += kMaxCols) {
     size_t g1 = std::min(evals.size(), g0 + (size_t)kMaxCols);
     int S = (int)(g1 - g0);
-    std::vector<VecDesc> pre(S), post(S);
+    std::vector<VecDesc> pre(S), post(S), early;
     std::vector<LlgDesc> ld(S);
     bool pre_red = false, post_red = false;
     for (int k = 0; k < S; ++k) {
@@ -1287,12 +1290,15 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
       pre[k].pack_col = k;
       pre[k].rslot = s.id;  // per-state result slots: a deferred result survives later ticks
       if (pre[k].rkind != kRedNone) {
-        pre_red = true;
-        if (!s.op.defer_pre) pre_sync = true;
+        pre_red = pre_sync = true;
       }
       post[k] = s.op.post;
       post[k].rslot = s.id;
       if (post[k].rkind != kRedNone) post_red = true;
+      if (s.op.early.rkind != kRedNone) {
+        early.push_back(s.op.early);
+        early.back().rslot = s.id;
+      }
       LlgDesc& L = ld[k];
       std::memset(&L, 0, sizeof(L));
       L.m = pre[k].dst;
@@ -1325,16 +1331,27 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     for (int k = 0; k < S && late; ++k) late = !ld[k].fields && ld[k].out;
     // the split product's near-band kernel evaluates the LL right-hand side
     const bool llg_in_near = precision == MT_PREC_BF16X2 && near_r > 0 && near_llg;
+    // early estimates go with the reductions after the right-hand side in one
+    // launch, so that stage 7's argument is a plain combination and is formed by
+    // the launch before it: one launch a step less (film of 32 x 8: 11.28 -> 10.29 ms, of
+    // 128 x 32: 28.5 -> 27.2).  In results and lines, state B + id of kind 1 is state id of
+    // kind 2.
+    const bool joined = !early.empty() && (!inl || early.size() + S <= (size_t)kInlineStates);
+    std::vector<VecDesc> reds;
+    if (joined) reds = early;
+    reds.insert(reds.end(), post.begin(), post.end());
+    if (joined)
+      for (size_t k = early.size(); k < reds.size(); ++k) reds[k].rslot += B;
     const VecDesc* dpre = nullptr;
     const LlgDesc* dl = nullptr;
     const VecDesc* dpost = nullptr;
     int rc;
     if (!inl && !(late && formed)) {
-      rc = stage_reserve(3 * 256 + (size_t)S * (2 * sizeof(VecDesc) + sizeof(LlgDesc)));
+      rc = stage_reserve(3 * 256 + (size_t)S * (3 * sizeof(VecDesc) + sizeof(LlgDesc)));
       if (rc) return rc;
       if (!formed) dpre = stage_put(pre);
       if (!late) dl = stage_put(ld);
-      dpost = post_red ? stage_put(post) : nullptr;
+      dpost = post_red ? stage_put(reds) : nullptr;
       rc = stage_flush();
       if (rc) return rc;
     }
@@ -1394,10 +1411,16 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     }
     if (timing) MT_HIP(hipEventRecord(ev[5], stream));
     if (post_red) {
-      double* post_parts = partials + (size_t)2 * B * vec_blocks_per_state((int)N3) * 4;
-      const ResultLines to = result_lines(2, post);
-      rc = inl ? launch_vec_inline(post.data(), S, n, post_parts, res_post, nopack, true, stream, to)
-               : launch_vec(dpost, S, n, post_parts, res_post, nopack, true, stream, to);
+      if (!early.empty() && !joined) {
+        rc = launch_vec_inline(early.data(), (int)early.size(), n, pre_parts, res_pre, nopack, true, stream,
+                               result_lines(1, early));
+        if (rc) return rc;
+      }
+      double* parts = joined ? pre_parts : partials + (size_t)2 * B * vec_blocks_per_state((int)N3) * 4;
+      double* res = joined ? res_pre : res_post;
+      const ResultLines to = result_lines(joined ? 1 : 2, reds, joined ? 2 : 1);
+      rc = inl ? launch_vec_inline(reds.data(), (int)reds.size(), n, parts, res, nopack, true, stream, to)
+               : launch_vec(dpost, (int)reds.size(), n, parts, res, nopack, true, stream, to);
       if (rc) return rc;
     }
     if (timing) {
@@ -1426,7 +1449,8 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
       if (!stage_fused)
         for (const VecDesc& v : pre) vec_bytes += vec_desc_bytes(v, pk.mode);
       if (post_red)
-        for (const VecDesc& v : post) vec_bytes += vec_desc_bytes(v, kPackNone);
+        for (const std::vector<VecDesc>* d : {&early, &post})
+          for (const VecDesc& v : *d) vec_bytes += vec_desc_bytes(v, kPackNone);
     }
     post_reduce_any |= post_red;
   }
@@ -1927,7 +1951,7 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
   }
   // one tick stages at most one vector-only launch over all states and one
   // demag pass of up to 64 states (three descriptor arrays)
-  P.arena_size = std::max((size_t)8 << 20, (size_t)(P.B + 2 * kMaxCols) * sizeof(VecDesc) +
+  P.arena_size = std::max((size_t)8 << 20, (size_t)(P.B + 3 * kMaxCols) * sizeof(VecDesc) +
                                                (size_t)kMaxCols * sizeof(LlgDesc) + 4096);
   MT_HIP(hipHostMalloc(&P.arena_h, P.arena_size, hipHostMallocDefault));
   MT_HIP(hipMalloc(&P.arena_d, P.arena_size));
