@@ -641,17 +641,15 @@ namespace {
 // kHostBlocksKept wait for the next call of any thread.
 constexpr size_t kHostBlock = 2u << 20, kHostBlocksKept = 4;
 std::mutex g_host_mutex;
-std::vector<void*> g_host_blocks;
+void* g_host_blocks[kHostBlocksKept];
+size_t g_host_kept = 0;
 
 class HostBlock {
  public:
   HostBlock() {
     {
       std::lock_guard<std::mutex> lock(g_host_mutex);
-      if (!g_host_blocks.empty()) {
-        p_ = g_host_blocks.back();
-        g_host_blocks.pop_back();
-      }
+      if (g_host_kept > 0) p_ = g_host_blocks[--g_host_kept];
     }
     constexpr unsigned flags = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
     if (!p_ && hipHostMalloc(&p_, kHostBlock, flags) != hipSuccess) {
@@ -668,7 +666,7 @@ class HostBlock {
     if (!p_) return;
     (void)hipStreamSynchronize(nullptr);
     std::lock_guard<std::mutex> lock(g_host_mutex);
-    if (g_host_blocks.size() < kHostBlocksKept) g_host_blocks.push_back(p_);
+    if (g_host_kept < kHostBlocksKept) g_host_blocks[g_host_kept++] = p_;
     else (void)hipHostFree(p_);
   }
   HostBlock(const HostBlock&) = delete;
