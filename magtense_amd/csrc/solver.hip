@@ -1288,7 +1288,7 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
       Sim& s = *evals[g0 + k];
       pre[k] = s.op.pre;
       pre[k].pack_col = k;
-      pre[k].rslot = s.id;  // per-state result slots: a deferred result survives later ticks
+      pre[k].rslot = s.id;  // result slots are per state
       if (pre[k].rkind != kRedNone) {
         pre_red = pre_sync = true;
       }
