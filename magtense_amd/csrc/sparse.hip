@@ -241,7 +241,8 @@ __global__ void __launch_bounds__(256) interleave_kernel(const float* __restrict
 // few states (S <= 8): wave per receiver row, lanes split the entries, h is
 // [S][3n], m the states interleaved by W.  Bound by the gathers of m through L1:
 // a lane takes W states of a source with one load, and the matrix is read once
-// (6 bytes an entry, 8 with 32-bit columns).  @@
+// (6 bytes an entry, 8 with 32-bit columns).  8192 cells, 40 M entries, 3 states: 69 us a call,
+// 92 with a load per state and 32-bit columns; 32761 cells, 1.19 G entries, 8 states: 3.50 ms, 6.57.
 template <int S, int W, typename C>
 __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, const float* __restrict__ m, int64_t ld,
                                                         float pref, float* __restrict__ h) {
