@@ -241,13 +241,17 @@ __global__ void __launch_bounds__(256) interleave_kernel(const float* __restrict
 // few states (S <= 8): wave per receiver row, lanes split the entries, h is
 // [S][3n], m the states interleaved by W.  Bound by the gathers of m through L1:
 // a lane takes W states of a source with one load, and the matrix is read once
-// (6 bytes an entry, 8 with 32-bit columns).  8192 cells, 40 M entries, 3 states: 69 us a call,
-// 92 with a load per state and 32-bit columns; 32761 cells, 1.19 G entries, 8 states: 3.50 ms, 6.57.
+// (6 bytes an entry, 8 with 32-bit columns).  A lane takes
+// four entries at a time and what is left of its row, up to three, at once under
+// a mask: a loop over them one by one is a round trip each, and a component of
+// a row has only some tens of entries a lane.  us a call without and with the mask,
+// 1, 4 and 8 states: 8192 cells, 40 M entries, 44.5 57.1 81.5 and 40.7 53.9 76.2; 32761 cells
+// 502 733 1092 and 458 697 1023 (two entries at a time: 489 691 1094, without the mask 541 781 1181).
 template <int S, int W, typename C>
 __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, const float* __restrict__ m, int64_t ld,
                                                         float pref, float* __restrict__ h) {
   typedef float vecw __attribute__((ext_vector_type(W)));
-  constexpr int G = (S + W - 1) / W;
+  constexpr int G = (S + W - 1) / W, U = 4;
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (i >= n) return;
@@ -260,31 +264,48 @@ __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, con
     const int a = ca[c], b = cb[c];
     const int64_t base = A.coff[c];
     const int64_t q0 = base + A.rowptr[(size_t)c * (n + 1) + i], q1 = base + A.rowptr[(size_t)c * (n + 1) + i + 1];
-    // four iterations unrolled: their loads are issued together (measured 1.19 ms ->
-    // 0.95 ms per one-state product on the 32768-cell film); each lane still sums
-    // its entries in order
-#pragma unroll 4
-    for (int64_t q = q0 + lane; q < q1; q += 64) {
-      const int j = A.cols[q];
-      const float v = A.vals[q];
+    // entries q, q + 64, ... of this lane, in order; TAIL: those below q1 of them
+    int64_t q = q0 + lane;
+    auto group = [&](auto count, auto tail) {
+      constexpr int N = decltype(count)::value;
+      constexpr bool TAIL = decltype(tail)::value;
+      int j[N];
+      float v[N];
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float* f = m + (int64_t)g * 3 * n * W + (int64_t)j * W;
-        if constexpr (W == 1) {
-          acc[a][g] += v * f[(int64_t)b * n];
-          if (a != b) acc[b][g] += v * f[(int64_t)a * n];
-        } else {
-          const vecw x = *reinterpret_cast<const vecw*>(f + (int64_t)b * n * W);
+      for (int u = 0; u < N; ++u) {
+        const int64_t e = TAIL ? min(q + 64 * u, q1 - 1) : q + 64 * u;
+        j[u] = A.cols[e];
+        v[u] = A.vals[e];
+      }
 #pragma unroll
-          for (int s = 0; s < W && g * W + s < S; ++s) acc[a][g * W + s] += v * x[s];
-          if (a != b) {
-            const vecw y = *reinterpret_cast<const vecw*>(f + (int64_t)a * n * W);
+      for (int u = 0; u < N; ++u) {
+        const bool on = !TAIL || q + 64 * u < q1;
+        auto add = [&](float& sum, float x) {
+          const float t = sum + v[u] * x;
+          sum = on ? t : sum;
+        };
 #pragma unroll
-            for (int s = 0; s < W && g * W + s < S; ++s) acc[b][g * W + s] += v * y[s];
+        for (int g = 0; g < G; ++g) {
+          const float* f = m + (int64_t)g * 3 * n * W + (int64_t)j[u] * W;
+          if constexpr (W == 1) {
+            add(acc[a][g], f[(int64_t)b * n]);
+            if (a != b) add(acc[b][g], f[(int64_t)a * n]);
+          } else {
+            const vecw x = *reinterpret_cast<const vecw*>(f + (int64_t)b * n * W);
+#pragma unroll
+            for (int s = 0; s < W && g * W + s < S; ++s) add(acc[a][g * W + s], x[s]);
+            if (a != b) {
+              const vecw y = *reinterpret_cast<const vecw*>(f + (int64_t)a * n * W);
+#pragma unroll
+              for (int s = 0; s < W && g * W + s < S; ++s) add(acc[b][g * W + s], y[s]);
+            }
           }
         }
       }
-    }
+    };
+#pragma unroll 1
+    for (; q + 64 * (U - 1) < q1; q += 64 * U) group(std::integral_constant<int, U>{}, std::false_type{});
+    if (q < q1) group(std::integral_constant<int, U - 1>{}, std::true_type{});
   }
   for (int a = 0; a < 3; ++a)
     for (int s = 0; s < S; ++s) {
@@ -740,8 +761,8 @@ int SparseDemag::apply(const float* m, int64_t ld, int S, float pref, float* h, 
   const int n3 = 3 * n;
   std::lock_guard<std::mutex> lock(launch);
   // up to 16 states: the few-state kernel on groups of at most eight (8192 cells,
-  // 71 M entries: 122 / 145 / 173 / 257 / 497 us for 1 / 2 / 4 / 8 / 16 states; the
-  // many-state kernel takes 1.33 to 1.48 ms)
+  // 40 M entries: 41 / 50 / 54 / 76 / 137 us for 1 / 2 / 4 / 8 / 16 states; the
+  // many-state kernel takes 1.33 to 1.48 ms with 71 M)
   if (S <= 16) {
     for (int s0 = 0; s0 < S;) {
       const int g = std::min(S - s0, 8);
