@@ -253,7 +253,10 @@ __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, con
   typedef float vecw __attribute__((ext_vector_type(W)));
   constexpr int G = (S + W - 1) / W, U = 4;
   const int lane = threadIdx.x & 63;
-  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  // wave-uniform row: its bounds and base addresses are scalars and a lane's place in
+  // it is 32 bits (1, 4 and 8 states at 8192 cells 41.5 54.3 77.4 -> 39.7 51.7 73.0 us; the next
+  // group's entries loaded ahead on top of it: 40.3 52.0 74.4, at 32761 cells 8 % slower)
+  const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (i >= n) return;
   float acc[3][S];
   for (int a = 0; a < 3; ++a)
@@ -264,22 +267,25 @@ __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, con
     const int a = ca[c], b = cb[c];
     const int64_t base = A.coff[c];
     const int64_t q0 = base + A.rowptr[(size_t)c * (n + 1) + i], q1 = base + A.rowptr[(size_t)c * (n + 1) + i + 1];
-    // entries q, q + 64, ... of this lane, in order; TAIL: those below q1 of them
-    int64_t q = q0 + lane;
-    auto group = [&](auto count, auto tail) {
-      constexpr int N = decltype(count)::value;
+    const C* cols = A.cols + q0;
+    const float* vals = A.vals + q0;
+    const int count = (int)(q1 - q0);
+    // entries q, q + 64, ... of this lane, in order; TAIL: those below count of them
+    int q = lane;
+    auto group = [&](auto size, auto tail) {
+      constexpr int N = decltype(size)::value;
       constexpr bool TAIL = decltype(tail)::value;
       int j[N];
       float v[N];
 #pragma unroll
       for (int u = 0; u < N; ++u) {
-        const int64_t e = TAIL ? min(q + 64 * u, q1 - 1) : q + 64 * u;
-        j[u] = A.cols[e];
-        v[u] = A.vals[e];
+        const unsigned e = TAIL ? min(q + 64 * u, count - 1) : q + 64 * u;
+        j[u] = cols[e];
+        v[u] = vals[e];
       }
 #pragma unroll
       for (int u = 0; u < N; ++u) {
-        const bool on = !TAIL || q + 64 * u < q1;
+        const bool on = !TAIL || q + 64 * u < count;
         auto add = [&](float& sum, float x) {
           const float t = sum + v[u] * x;
           sum = on ? t : sum;
@@ -304,8 +310,8 @@ __global__ void __launch_bounds__(256) spmv_rows_kernel(CsrView<C> A, int n, con
       }
     };
 #pragma unroll 1
-    for (; q + 64 * (U - 1) < q1; q += 64 * U) group(std::integral_constant<int, U>{}, std::false_type{});
-    if (q < q1) group(std::integral_constant<int, U - 1>{}, std::true_type{});
+    for (; q + 64 * (U - 1) < count; q += 64 * U) group(std::integral_constant<int, U>{}, std::false_type{});
+    if (q < count) group(std::integral_constant<int, U - 1>{}, std::true_type{});
   }
   for (int a = 0; a < 3; ++a)
     for (int s = 0; s < S; ++s) {
@@ -761,7 +767,7 @@ int SparseDemag::apply(const float* m, int64_t ld, int S, float pref, float* h, 
   const int n3 = 3 * n;
   std::lock_guard<std::mutex> lock(launch);
   // up to 16 states: the few-state kernel on groups of at most eight (8192 cells,
-  // 40 M entries: 41 / 50 / 54 / 76 / 137 us for 1 / 2 / 4 / 8 / 16 states; the
+  // 40 M entries: 40 / 48 / 52 / 73 / 131 us for 1 / 2 / 4 / 8 / 16 states; the
   // many-state kernel takes 1.33 to 1.48 ms with 71 M)
   if (S <= 16) {
     for (int s0 = 0; s0 < S;) {
