@@ -26,6 +26,7 @@ constexpr int kTileRaw = 19;
 int launch_tile_records(const double* raw, int nt, bool vertices, int npt, double* tiles, double* pts,
                         hipStream_t stream);
 // part holds tiles_field_plan(nt, npt).parts x 3 npt doubles (unused with one part), H the field.
+// width: threads of a point; blocks: of a launch, at most; parts: of a point's tiles.
 struct TilesFieldPlan {
   int width, blocks, parts;
 };

@@ -724,7 +724,7 @@ __global__ void __launch_bounds__(256) tiles_tensor_kernel(const double* __restr
 }
 
 // H(p) = sum_i Rinv_i (N_ip (R_i M_i)) (getDotProd, :909-918, and the
-// back-rotation, :721-726).  A block holds 256 / width points; width threads
+// back-rotation, :721-726).  A block holds 256 / width points from `first` on; width threads
 // (a power of two) stride over a point's tiles i = z * width + t, z from
 // blockIdx.y in steps of gridDim.y, and add up in a fixed tree: part z goes to
 // H + z * 3 * npt.  Nin (Fortran-ordered as above) replaces the tensor
@@ -734,11 +734,11 @@ __global__ void __launch_bounds__(256) tiles_tensor_kernel(const double* __restr
 // SIMD), 3.6 with both formulas in one kernel and 24 arctangents per prism.
 template <TileKind KIND>
 __global__ void __launch_bounds__(256, KIND == TileKind::kPrism ? 3 : 1)
-    tiles_field_kernel(const double* __restrict__ tiles, int nt, const double* __restrict__ pts, int npt, int width,
-                       const double* __restrict__ Nin, double* __restrict__ H) {
+    tiles_field_kernel(const double* __restrict__ tiles, int nt, const double* __restrict__ pts, int npt, int first,
+                       int width, const double* __restrict__ Nin, double* __restrict__ H) {
   __shared__ double red[3][256];
   const int t = threadIdx.x % width;
-  const int p = blockIdx.x * (256 / width) + threadIdx.x / width;
+  const int64_t p = first + (int64_t)blockIdx.x * (256 / width) + threadIdx.x / width;
   double acc[3] = {0.0, 0.0, 0.0};
   if (p < npt) {
     const double px = pts[p], py = pts[p + (size_t)npt], pz = pts[p + 2 * (size_t)npt];
@@ -877,12 +877,14 @@ int launch_tiles_tensor(const double* tiles, int nt, TileKind kind, const double
 
 // Threads of a point: the tiles, up to a block.  Parts of a point's tiles: as
 // many as give the chip 2048 blocks (256 CUs, two or three of these blocks on
-// each, several rounds), while every thread keeps a tile.
+// each, several rounds), while every thread keeps a tile.  A grid holds fewer than
+// 2^32 threads: more than 2^23 blocks (256^3 points of over 128 tiles) take several
+// launches.
 TilesFieldPlan tiles_field_plan(int nt, int npt) {
   TilesFieldPlan q;
   q.width = 1;
   while (q.width < 256 && q.width < nt) q.width *= 2;
-  q.blocks = (int)(((int64_t)npt * q.width + 255) / 256);
+  q.blocks = (int)std::min<int64_t>(((int64_t)npt * q.width + 255) / 256, 1 << 23);
   const int64_t most = (nt + q.width - 1) / q.width;
   q.parts = (int)std::max<int64_t>(1, std::min<int64_t>(most, 2048 / std::max(q.blocks, 1)));
   return q;
@@ -893,12 +895,16 @@ int launch_tiles_field(const double* tiles, int nt, TileKind kind, const double*
   if (npt <= 0) return kOk;
   const TilesFieldPlan q = tiles_field_plan(nt, npt);
   double* first = q.parts > 1 ? part : H;
-  const dim3 grid((unsigned)q.blocks, (unsigned)q.parts);
-  by_kind(kind, [&](auto k) {
-    hipLaunchKernelGGL(tiles_field_kernel<decltype(k)::value>, grid, dim3(256), 0, stream, tiles, nt, pts, npt, q.width,
-                       Nin, first);
-  });
-  MT_HIP(hipGetLastError());
+  const int64_t step = (int64_t)q.blocks * (256 / q.width);  // points of a launch
+  for (int64_t p = 0; p < npt; p += step) {
+    const int64_t blocks = std::min<int64_t>(q.blocks, ((npt - p) * q.width + 255) / 256);
+    const dim3 grid((unsigned)blocks, (unsigned)q.parts);
+    by_kind(kind, [&](auto k) {
+      hipLaunchKernelGGL(tiles_field_kernel<decltype(k)::value>, grid, dim3(256), 0, stream, tiles, nt, pts, npt, (int)p,
+                         q.width, Nin, first);
+    });
+    MT_HIP(hipGetLastError());
+  }
   if (q.parts > 1) {
     const int64_t total = (int64_t)3 * npt;
     hipLaunchKernelGGL(tiles_field_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, part,
