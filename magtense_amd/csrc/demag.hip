@@ -1251,8 +1251,8 @@ __global__ void __launch_bounds__(256) near_corr_kernel(const uint32_t* __restri
   if (LLG) {
     const LlgDesc& D = descs[s];
     double dm[3];
-    llg_cell<false>(
-        g, D, (int)i, CellReads{},
+    llg_cell(
+        g, D, (int)i, CellAtUse{g, D, (int)i},
         [&](int c) {
           float v = 0.0f;
           for (int k = 0; k + 1 < D.nsplit; ++k) v += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * n + i];

@@ -16,183 +16,174 @@
 
 namespace mt {
 
-// What the right-hand side of a cell reads, apart from the demag sums.  The
-// kernels issue these reads (and the next stage's, below) before anything waits
-// for another: a launch of a small problem is little more than its round trips
-// to memory.  (The near-band kernel reads each value where it is used: 63 registers
-// and eight waves per SIMD, 88 and five with all of them in flight, 123 and 171 us a
-// launch of 64 states at 256 x 64 x 2.)
-struct CellReads {
+// A cell and its neighbours on the uniform grid.  The neighbour indices are clamped
+// to the cell itself at a boundary, so that every load is issued before the per-row
+// formula is selected.
+struct Stencil {
   double c0[3], xm[3], xp[3], ym[3], yp[3], zm[3], zp[3];
-  double jf, kf, ms64, aniso[6];  // aniso: xx xy xz yy yz zz
+};
+
+__device__ __forceinline__ Stencil stencil_reads(const LlgGrid& g, const LlgDesc& D, int i) {
+  Stencil r;
+  const int n = g.n;
+  const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
+  const int sy = g.nx, sz = g.nx * g.ny;
+  const int xm = ix > 0 ? i - 1 : i, xp = ix < g.nx - 1 ? i + 1 : i;
+  const int ym = iy > 0 ? i - sy : i, yp = iy < g.ny - 1 ? i + sy : i;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double* v = D.m + (size_t)c * n;
+    r.c0[c] = v[i];
+    r.xm[c] = v[xm]; r.xp[c] = v[xp];
+    r.ym[c] = v[ym]; r.yp[c] = v[yp];
+  }
+  if (g.nz > 1) {
+    const int zm = iz > 0 ? i - sz : i, zp = iz < g.nz - 1 ? i + sz : i;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double* v = D.m + (size_t)c * n;
+      r.zm[c] = v[zm]; r.zp[c] = v[zp];
+    }
+  }
+  return r;
+}
+
+// The operands of a cell, apart from the demag sums, read before anything waits
+// for another (and with the next stage's, below): a launch of a small problem is
+// little more than its round trips to memory.
+struct CellReads {
+  Stencil s;  // with a loaded exchange operator only s.c0
+  double jf, kf, ms64, a[6];  // a: xx xy xz yy yz zz
   float ms32;
   int kb, ke;
+  __device__ __forceinline__ const Stencil& stencil() const { return s; }
+  __device__ __forceinline__ double centre(int c) const { return s.c0[c]; }
+  __device__ __forceinline__ int row_begin() const { return kb; }
+  __device__ __forceinline__ int row_end() const { return ke; }
+  __device__ __forceinline__ double jfact() const { return jf; }
+  __device__ __forceinline__ float ms_f32() const { return ms32; }
+  __device__ __forceinline__ double ms_f64() const { return ms64; }
+  __device__ __forceinline__ double kfact() const { return kf; }
+  __device__ __forceinline__ double aniso(int k) const { return a[k]; }
 };
 
 __device__ __forceinline__ CellReads cell_reads(const LlgGrid& g, const LlgDesc& D, int i) {
   CellReads r;
-  const int n = g.n;
-  const double* m = D.m;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) r.c0[c] = m[(size_t)c * n + i];
   r.jf = g.jfact[i];
   r.kb = r.ke = 0;
   if (g.xs) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r.s.c0[c] = D.m[(size_t)c * g.n + i];
     r.kb = g.xs[i];
     r.ke = g.xe[i];
   } else {
-    // the neighbour indices are clamped to the cell itself at a boundary, so
-    // that every load is issued before the per-row formula is selected
-    const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
-    const int sy = g.nx, sz = g.nx * g.ny;
-    const int xm = ix > 0 ? i - 1 : i, xp = ix < g.nx - 1 ? i + 1 : i;
-    const int ym = iy > 0 ? i - sy : i, yp = iy < g.ny - 1 ? i + sy : i;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const double* v = m + (size_t)c * n;
-      r.xm[c] = v[xm]; r.xp[c] = v[xp];
-      r.ym[c] = v[ym]; r.yp[c] = v[yp];
-    }
-    if (g.nz > 1) {
-      const int zm = iz > 0 ? i - sz : i, zp = iz < g.nz - 1 ? i + sz : i;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double* v = m + (size_t)c * n;
-        r.zm[c] = v[zm]; r.zp[c] = v[zp];
-      }
-    }
+    r.s = stencil_reads(g, D, i);
   }
   if (D.hpart64) r.ms64 = g.ms64[i];
   else r.ms32 = g.ms32[i];
   if (g.aniso) {
     r.kf = g.kfact[i];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) r.aniso[k] = g.aniso[(size_t)i * 6 + k];
+    for (int k = 0; k < 6; ++k) r.a[k] = g.aniso[(size_t)i * 6 + k];
   }
   return r;
 }
 
-// LL right-hand side of cell i for the state of descriptor D, from its reads.
-// hsum(c) returns the FP32 demag sum S_c = sum of the partials of (K m)_c at i
-// (used unless D.hpart64 holds FP64 sums).  dm: dm/dt, which goes to D.out as
-// well.
-template <bool AHEAD = true, typename HS>
-__device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, const CellReads& r, HS hsum,
+// The same operands, each read where it is used.  The near-band kernel takes them
+// like this: 62 registers and eight waves per SIMD, 88 and five with all of them in
+// flight, 123 and 171 us a launch of 64 states at 256 x 64 x 2.
+struct CellAtUse {
+  const LlgGrid& g;
+  const LlgDesc& D;
+  int i;
+  __device__ __forceinline__ Stencil stencil() const { return stencil_reads(g, D, i); }
+  __device__ __forceinline__ double centre(int c) const { return D.m[(size_t)c * g.n + i]; }
+  __device__ __forceinline__ int row_begin() const { return g.xs[i]; }
+  __device__ __forceinline__ int row_end() const { return g.xe[i]; }
+  __device__ __forceinline__ double jfact() const { return g.jfact[i]; }
+  __device__ __forceinline__ float ms_f32() const { return g.ms32[i]; }
+  __device__ __forceinline__ double ms_f64() const { return g.ms64[i]; }
+  __device__ __forceinline__ double kfact() const { return g.kfact[i]; }
+  __device__ __forceinline__ double aniso(int k) const { return g.aniso[(size_t)i * 6 + k]; }
+};
+
+// LL right-hand side of cell i for the state of descriptor D, from its operands
+// (CellReads or CellAtUse).  hsum(c) returns the FP32 demag sum S_c = sum of the
+// partials of (K m)_c at i (used unless D.hpart64 holds FP64 sums).  dm: dm/dt,
+// which goes to D.out as well.  Every fused operation is written out, and the
+// compiler fuses none by itself: what it would choose depends on the kernel around
+// the cell, and a state's bits must not.
+template <typename Operands, typename HS>
+__device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int i, const Operands& r, HS hsum,
                                          double (&dm)[3]) {
+#pragma clang fp contract(off)
   const int n = g.n;
   const double* m = D.m;
   double mc[3], hj[3], hm[3], hk[3];
-  if constexpr (AHEAD) {
-    if (g.xs) {
-      // loaded operator: alpha = -2 times the row's stored entries in order
-      // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
-      for (int c = 0; c < 3; ++c) {
-        const double* v = m + (size_t)c * n;
-        mc[c] = r.c0[c];
-        double sum = 0.0;
-        for (int k = r.kb; k < r.ke; ++k) sum += g.xv[k] * v[g.xc[k]];
-        hj[c] = (-2.0 * sum) * r.jf;
-      }
-    } else {
-      // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1)
-      const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double vi = r.c0[c];
-        mc[c] = vi;
-        double lx = ix == 0 ? (r.xp[c] - vi) : (ix == g.nx - 1 ? (r.xm[c] - vi) : (r.xm[c] - 2.0 * vi + r.xp[c]));
-        double ly = iy == 0 ? (r.yp[c] - vi) : (iy == g.ny - 1 ? (r.ym[c] - vi) : (r.ym[c] - 2.0 * vi + r.yp[c]));
-        double lap = lx * g.idx2 + ly * g.idy2;
-        if (g.nz > 1) {
-          double lz = iz == 0 ? (r.zp[c] - vi) : (iz == g.nz - 1 ? (r.zm[c] - vi) : (r.zm[c] - 2.0 * vi + r.zp[c]));
-          lap += lz * g.idz2;
-        }
-        hj[c] = (-2.0 * lap) * r.jf;
-      }
+  if (g.xs) {
+    // loaded operator: alpha = -2 times the row's stored entries in order
+    // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
+    const int kb = r.row_begin(), ke = r.row_end();
+    for (int c = 0; c < 3; ++c) {
+      const double* v = m + (size_t)c * n;
+      mc[c] = r.centre(c);
+      double sum = 0.0;
+      for (int k = kb; k < ke; ++k) sum = __builtin_fma(g.xv[k], v[g.xc[k]], sum);
+      hj[c] = (-2.0 * sum) * r.jfact();
     }
   } else {
-    const int ix = i % g.nx;
-    const int iy = (i / g.nx) % g.ny;
-    const int iz = i / (g.nx * g.ny);
-    const int sy = g.nx, sz = g.nx * g.ny;
-    if (g.xs) {
-      // loaded operator: alpha = -2 times the row's stored entries in order
-      // (updateExchangeTerms, LandauLifshitzEquationSolver.f90:440-474)
-      const int kb = g.xs[i], ke = g.xe[i];
-      for (int c = 0; c < 3; ++c) {
-        const double* v = m + (size_t)c * n;
-        mc[c] = v[i];
-        double sum = 0.0;
-        for (int k = kb; k < ke; ++k) sum += g.xv[k] * v[g.xc[k]];
-        hj[c] = (-2.0 * sum) * g.jfact[i];
-      }
-    } else {
-      // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1).  The
-      // neighbour indices are clamped to the cell itself at a boundary, so every
-      // load is issued unconditionally before the per-row formula is selected.
-      const int xm = ix > 0 ? i - 1 : i, xp = ix < g.nx - 1 ? i + 1 : i;
-      const int ym = iy > 0 ? i - sy : i, yp = iy < g.ny - 1 ? i + sy : i;
-      const bool z3 = g.nz > 1;
-      const int zm = z3 && iz > 0 ? i - sz : i, zp = z3 && iz < g.nz - 1 ? i + sz : i;
-      double c0[3], cxm[3], cxp[3], cym[3], cyp[3], czm[3], czp[3];
+    // Laplacian with the reference's boundary rows: (-1, 1) and (1, -1)
+    const Stencil& x = r.stencil();
+    const double jf = r.jfact();
+    const int ix = i % g.nx, iy = (i / g.nx) % g.ny, iz = i / (g.nx * g.ny);
+    auto row = [](int k, int cells, double low, double mid, double high) {
+      return k == 0 ? high - mid : (k == cells - 1 ? low - mid : __builtin_fma(-2.0, mid, low) + high);
+    };
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double* v = m + (size_t)c * n;
-        c0[c] = v[i];
-        cxm[c] = v[xm]; cxp[c] = v[xp];
-        cym[c] = v[ym]; cyp[c] = v[yp];
-        czm[c] = v[zm]; czp[c] = v[zp];
-      }
-      const double jf = g.jfact[i];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        const double vi = c0[c];
-        mc[c] = vi;
-        double lx = ix == 0 ? (cxp[c] - vi) : (ix == g.nx - 1 ? (cxm[c] - vi) : (cxm[c] - 2.0 * vi + cxp[c]));
-        double ly = iy == 0 ? (cyp[c] - vi) : (iy == g.ny - 1 ? (cym[c] - vi) : (cym[c] - 2.0 * vi + cyp[c]));
-        double lap = lx * g.idx2 + ly * g.idy2;
-        if (z3) {
-          double lz = iz == 0 ? (czp[c] - vi) : (iz == g.nz - 1 ? (czm[c] - vi) : (czm[c] - 2.0 * vi + czp[c]));
-          lap += lz * g.idz2;
-        }
-        hj[c] = (-2.0 * lap) * jf;
-      }
+    for (int c = 0; c < 3; ++c) {
+      const double vi = x.c0[c];
+      mc[c] = vi;
+      const double lx = row(ix, g.nx, x.xm[c], vi, x.xp[c]), ly = row(iy, g.ny, x.ym[c], vi, x.yp[c]);
+      double lap = __builtin_fma(lx, g.idx2, ly * g.idy2);
+      if (g.nz > 1) lap = __builtin_fma(row(iz, g.nz, x.zm[c], vi, x.zp[c]), g.idz2, lap);
+      hj[c] = (-2.0 * lap) * jf;
     }
   }
   // demag: S = sum_k partial (K m); field = fl32(fl32(-S) * Ms_i)
   if (D.hpart64) {
-    for (int c = 0; c < 3; ++c) hm[c] = (-D.hpart64[(int64_t)c * n + i]) * (AHEAD ? r.ms64 : g.ms64[i]);
+    for (int c = 0; c < 3; ++c) hm[c] = (-D.hpart64[(int64_t)c * n + i]) * r.ms_f64();
   } else {
     for (int c = 0; c < 3; ++c) {
       const float s = hsum(c);
       if (D.sum_out) D.sum_out[(int64_t)c * n + i] = s;
-      float h = (-s) * (AHEAD ? r.ms32 : g.ms32[i]);
+      float h = (-s) * r.ms_f32();
       hm[c] = (double)h;
     }
   }
   if (g.aniso) {
-    auto axes = [&](const auto& A, double f) {  // xx xy xz yy yz zz
-      hk[0] = f * (A[0] * mc[0] + A[1] * mc[1] + A[2] * mc[2]);
-      hk[1] = f * (A[1] * mc[0] + A[3] * mc[1] + A[4] * mc[2]);
-      hk[2] = f * (A[2] * mc[0] + A[4] * mc[1] + A[5] * mc[2]);
+    const double f = -2.0 * r.kfact();
+    auto axis = [&](int x, int y, int z) {
+      return f * __builtin_fma(r.aniso(z), mc[2], __builtin_fma(r.aniso(y), mc[1], r.aniso(x) * mc[0]));
     };
-    if constexpr (AHEAD) axes(r.aniso, -2.0 * r.kf);
-    else axes(g.aniso + (size_t)i * 6, -2.0 * g.kfact[i]);
+    hk[0] = axis(0, 1, 2);
+    hk[1] = axis(1, 3, 4);
+    hk[2] = axis(2, 4, 5);
   } else {
     hk[0] = hk[1] = hk[2] = 0.0;
   }
   double hh[3] = {-D.hext[0], -D.hext[1], -D.hext[2]};
   double H[3];
   for (int c = 0; c < 3; ++c) H[c] = hh[c] + hj[c] + hm[c] + hk[c];
-  double cx = -1.0 * (mc[1] * H[2] - mc[2] * H[1]);
-  double cy = -1.0 * (mc[2] * H[0] - mc[0] * H[2]);
-  double cz = -1.0 * (mc[0] * H[1] - mc[1] * H[0]);
-  double dx = mc[1] * cz - mc[2] * cy;
-  double dy = mc[2] * cx - mc[0] * cz;
-  double dz = mc[0] * cy - mc[1] * cx;
-  dm[0] = -D.gamma * cx - D.alpha * dx;
-  dm[1] = -D.gamma * cy - D.alpha * dy;
-  dm[2] = -D.gamma * cz - D.alpha * dz;
+  // t = m x H (the fields are negated: c = -t is m x H of the equation), d = m x c
+  const double tx = __builtin_fma(mc[1], H[2], -(mc[2] * H[1]));
+  const double ty = __builtin_fma(mc[2], H[0], -(mc[0] * H[2]));
+  const double tz = __builtin_fma(mc[0], H[1], -(mc[1] * H[0]));
+  const double dx = __builtin_fma(mc[2], ty, -(mc[1] * tz));
+  const double dy = __builtin_fma(mc[0], tz, -(mc[2] * tx));
+  const double dz = __builtin_fma(mc[1], tx, -(mc[0] * ty));
+  dm[0] = __builtin_fma(D.gamma, tx, -(D.alpha * dx));
+  dm[1] = __builtin_fma(D.gamma, ty, -(D.alpha * dy));
+  dm[2] = __builtin_fma(D.gamma, tz, -(D.alpha * dz));
   if (D.out) {
     D.out[i] = dm[0];
     D.out[n + i] = dm[1];
