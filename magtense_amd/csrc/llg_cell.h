@@ -203,7 +203,8 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
 // The next stage argument at cell i, straight after its right-hand side: the
 // vector kernel's combination (same order, same roundings) over the cell's
 // three components, with dm/dt taken from registers, and its demag input
-// packed into column col.  Only the cell's own values are read, so the launch
+// packed into column col (kPackF32, kPackLattice: the products whose right-hand
+// sides wait for the next stage).  Only the cell's own values are read, so the launch
 // that evaluates dm/dt can write the next stage's argument as long as that is
 // not a vector it reads at other cells.
 struct StageReads {
@@ -249,7 +250,6 @@ __device__ __forceinline__ void next_stage_cell(const StageDesc& S, const LlgDes
     const float f = (float)v[c];
     if (pack.mode == kPackF32) pack.f32[(int64_t)col * pack.col_stride + (int64_t)at[c]] = f;
     else if (pack.mode == kPackLattice) pack.f32[lattice_state_offset(n, (int)pack.col_stride, col, c, i)] = f;
-    else if (pack.mode == kPackF32Frag) *reinterpret_cast<float*>(pack.bf16 + f32_frag_offset(col, c, i)) = f;
     bad |= !(fabsf(f) <= FLT_MAX);
   }
   if (bad && pack.nonfinite) *pack.nonfinite = 1;
