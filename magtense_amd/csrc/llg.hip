@@ -692,6 +692,12 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
   return kOk;
 }
 
+bool next_stage_in_rows_pays(int n, int nstates) {
+  if (n <= kStageFusedMaxCells) return true;
+  if (matvec_group(nstates, n % 4 == 0) == 12 && nstates <= 12) return n <= 3500;
+  return n <= 2000 && nstates >= 2 && nstates <= 4;
+}
+
 static_assert(2 * sizeof(StageDescsInline) + sizeof(LlgDescsInline) + sizeof(LlgGrid) + 256 <= 4096,
               "stage + demag + LL kernel arguments exceed 4 KiB");
 

@@ -1327,7 +1327,8 @@ int Solver::execute_tick(std::vector<Sim*>& evals, std::vector<Sim*>& vecs) {
     // and on small problems forms the stage argument in that kernel as well
     const bool stage_fused = fused && inl && !pre_red && stage_fusion && n <= kStageFusedMaxCells && !formed;
     // nobody waits for these right-hand sides: left to the next tick
-    bool late = (fused || lattice.v.a) && !timing && !post_red && evals.size() <= (size_t)kMaxCols && !pre_sync;
+    bool late = (lattice.v.a || (fused && next_stage_in_rows_pays(n, S))) && !timing && !post_red &&
+                evals.size() <= (size_t)kMaxCols && !pre_sync;
     for (int k = 0; k < S && late; ++k) late = !ld[k].fields && ld[k].out;
     // the split product's near-band kernel evaluates the LL right-hand side
     const bool llg_in_near = precision == MT_PREC_BF16X2 && near_r > 0 && near_llg;
