@@ -663,7 +663,7 @@ int launch_matvec_f32(const float* K, int n, const float* m, int64_t m_stride, f
                          stream, K, n, ms, m_stride, o, out_stride, pref, nstates - s0, groups);
     };
     auto by_groups = [&](auto v4) { groups == 1 ? kernel(v4, std::true_type{}) : kernel(v4, std::false_type{}); };
-    if constexpr (S == 12) by_groups(std::false_type{});  // matvec_group: single columns
+    if constexpr (S == 12) kernel(std::false_type{}, std::true_type{});  // matvec_group: single columns, one group
     else vec4 ? by_groups(std::true_type{}) : by_groups(std::false_type{});
   };
   for (int s0 = 0; s0 < nstates;) {

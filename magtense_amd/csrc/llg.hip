@@ -655,6 +655,7 @@ int launch_demag_llg_s(const float* K, const LlgGrid& g, const LlgDesc* d_descs,
   const std::true_type yes;
   const std::false_type no;
   auto by_columns = [&](auto v4) {
+    if constexpr (S == 12) return go(no, v4, yes);  // matvec_group: one group
     if constexpr (S <= kInlineStates) {
       if (!d_descs) return go(yes, v4, yes);  // by value: one group
     }
@@ -694,7 +695,7 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
 
 bool next_stage_in_rows_pays(int n, int nstates) {
   if (n <= kStageFusedMaxCells) return true;
-  if (matvec_group(nstates, n % 4 == 0) == 12 && nstates <= 12) return n <= 3500;
+  if (matvec_group(nstates, n % 4 == 0) == 12) return n <= 3500;
   return n <= 2000 && nstates >= 2 && nstates <= 4;
 }
 

@@ -210,9 +210,13 @@ inline unsigned matvec_blocks(int row_blocks, int G) {
 // States per block for the next `left` states: the narrowest kernel that takes
 // them in one pass, some of its states idle (90 x 70 cells: 1 / 2 / 4 / 8 states
 // 0.164 / 0.170 / 0.182 / 0.227 ms a pass, HBM up to four).  With single columns
-// (n % 4 != 0) a thread holds a quarter of the values, and twelve states fit.
+// (n % 4 != 0) a thread holds a quarter of the values, and twelve states fit: one pass
+// for nine to twelve, where eights take two.  Beyond, groups of eight in one launch are
+// as good or better.  us a right-hand side by twelves / by eights, 9, 12, 13, 16, 20, 24,
+// 32, 64 states: 45 x 17 x 2: 38/46 39/46 54/51 56/43 60/55 55/57 72/63 130/118; 77 x 33:
+// 68/80 74/87 100/93 109/81 117/108 112/110 148/130 263/233.
 inline int matvec_group(int left, bool vec4) {
-  if (left > 8 && !vec4) return 12;
+  if (left > 8 && left <= 12 && !vec4) return 12;
   return left > 4 ? 8 : (left > 2 ? 4 : left);
 }
 // Groups of S states of one launch.
