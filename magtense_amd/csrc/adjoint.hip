@@ -746,14 +746,12 @@ int mt_rk4_create(const mt_micromag_problem* q, double dt, long long nsteps, int
     for (int i = 0; i < P.nz; ++i) axes[2].push_back(axis(P.nz, q->Lz, dz, i));
   }
   bool lattice = false;
-  if (!P.fp64 && !q->K_in && lattice_pays(n, P.B)) {
-    size_t free_b = 0, total_b = 0;
-    MT_HIP(hipMemGetInfo(&free_b, &total_b));
+  if (!P.fp64 && !q->K_in) {
+    int rc = lattice_wanted(P.nx, P.ny, P.nz, P.B, &lattice);
+    if (rc) return rc;
     const double d[3] = {dx, dy, dz};
-    if (6.0 * nn * sizeof(float) < (double)total_b) {  // a problem too large for the device stays refused
-      int rc = P.lattice.build(P.nx, P.ny, P.nz, axes[0], axes[1], axes[2], d, P.stream, &lattice);
-      if (rc) return rc;
-    }
+    if (lattice) rc = P.lattice.build(P.nx, P.ny, P.nz, axes[0], axes[1], axes[2], d, P.stream, &lattice);
+    if (rc) return rc;
   }
   if (lattice) {
     P.nsplit = lattice_nsplit(n);

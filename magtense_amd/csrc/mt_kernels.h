@@ -189,19 +189,11 @@ struct LatticeTable {
   void release();
   ~LatticeTable() { release(); }
 };
-// Whether the product from the table and the LL kernel (7 us) beat the one launch
-// over the dense tensor.  us per right-hand side, table + LL / dense:
-//   one state  32 x 40: 20 / 14, 44 x 40: 20 / 17, 96 x 24: 22 / 27, 64 x 64: 25 / 71
-//   8 states   30 x 30 x 2: 41 / 33, 44 x 40: 34 / 28, 96 x 24: 43 / 39
-//   12         32 x 40: 33 / 30, 64 x 30: 40 / 51
-//   16         32 x 16: 21 / 15, 20 x 20 x 2 (24 states): 40 / 27
-// With n % 4 != 0 a chain's four columns lie in four places of the grid:
-//   one state  45 x 17 x 2: 30 / 16, 77 x 33: 48 / 30, 63 x 67: 47 / 84, 91 x 71: 93 / 184
-//   8 or more  45 x 17 x 2 (12): 60 / 30, 77 x 33 (12): 110 / 66, 63 x 67: 114 / 123
-inline bool lattice_pays(int n, int nstates) {
-  if (n % 4) return n > 3500;
-  return n > 2000 || (n > 1024 && nstates > 8);
-}
+// Whether the table is the faster form for so many states.
+bool lattice_pays(int nx, int ny, int nz, int nstates);
+// Whether to build it: where it pays, or the device has no room for the dense tensor
+// at the moment.
+int lattice_wanted(int nx, int ny, int nz, int nstates, bool* wanted);
 int lattice_nsplit(int n);  // partial-sum slots of launch_lattice_rows
 // Layout of its states, cols of them (a multiple of 4): the columns in steps of
 // 1024, of which chain T of the row sums takes four, 4 T + q, or T + 256 q

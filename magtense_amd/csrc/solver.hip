@@ -1668,14 +1668,12 @@ int mt_solver_create(const mt_micromag_problem* q, mt_solver** out) {
   // gives it or asks for it, or on grids that the kernel does not take
   bool lattice = false;
   if (P.precision == MT_PREC_FP32 && approx == MT_DEMAG_DENSE && !unstructured && !q->K_in && !q->K_out &&
-      !q->keep_fp32_tensor && lattice_pays(n, P.B)) {
-    size_t free_b = 0, total_b = 0;
-    MT_HIP(hipMemGetInfo(&free_b, &total_b));
+      !q->keep_fp32_tensor) {
+    int rc = lattice_wanted(P.nx, P.ny, P.nz, P.B, &lattice);
+    if (rc) return rc;
     const double d[3] = {P.dx, P.dy, P.dz};
-    if (6.0 * nn * sizeof(float) < (double)total_b) {  // a problem too large for the device stays refused
-      int rc = P.lattice.build(P.nx, P.ny, P.nz, xs, ys, zs, d, P.stream, &lattice);
-      if (rc) return rc;
-    }
+    if (lattice) rc = P.lattice.build(P.nx, P.ny, P.nz, xs, ys, zs, d, P.stream, &lattice);
+    if (rc) return rc;
   }
   if (use_toep) {
     MT_HIP(hipMalloc(&P.Ktab, (size_t)toeplitz_tensor_bytes(P.nx, P.ny, P.nz)));
