@@ -210,17 +210,20 @@ inline unsigned matvec_blocks(int row_blocks, int G) {
 // States per block for the next `left` states: the narrowest kernel that takes
 // them in one pass, some of its states idle (90 x 70 cells: 1 / 2 / 4 / 8 states
 // 0.164 / 0.170 / 0.182 / 0.227 ms a pass, HBM up to four).  With single columns
-// (n % 4 != 0) a thread holds a quarter of the values, and twelve states fit: one pass
-// for nine to twelve, where eights take two.  Beyond, groups of eight in one launch are
-// as good or better.  us a right-hand side by twelves / by eights, 9, 12, 13, 16, 20, 24,
-// 32, 64 states: 45 x 17 x 2: 38/46 39/46 54/51 56/43 60/55 55/57 72/63 130/118; 77 x 33:
-// 68/80 74/87 100/93 109/81 117/108 112/110 148/130 263/233.
+// (n % 4 != 0) a thread holds a quarter of the values, and twelve states fit in one pass,
+// which reads a large tensor once for nine to twelve.  us by twelves / by eights: twelve
+// states 1530 cells 38/34 a product, 38/40 a right-hand side, 2001 46/48 a product, 3465
+// 122/124 a right-hand side, 6461 348/386 a product; beyond twelve states eights are as
+// good or better (13 16 24 64 states, 6461 cells: 534/386 557/386 598/509 1575/1185).
 inline int matvec_group(int left, bool vec4) {
   if (left > 8 && left <= 12 && !vec4) return 12;
   return left > 4 ? 8 : (left > 2 ? 4 : left);
 }
-// Groups of S states of one launch.
-inline int matvec_groups(int left, int S) { return S >= 8 ? std::max(1, std::min(left / S, 64)) : 1; }
+// Groups of S states of one launch, the last of them partly idle: its tensor rows come
+// from L2, where a launch of its own for the states left over reads them from HBM (6300
+// cells, 9 / 13 / 17 / 30 states 380 / 426 / 484 / 629 -> 306 / 327 / 414 / 540 us a
+// product), and a launch takes 3 us (64 cells, 9 states 20 -> 17).
+inline int matvec_groups(int left, int S) { return S == 8 ? std::min((left + 7) / 8, 64) : 1; }
 // Receiver rows of its blocks: a value of a state is read from L2 once per block,
 // so that more rows are less traffic, until the sums take a wave's registers.
 // One state, 402.7 MB tensor: 2 / 4 / 8 rows -> 72.2 / 66.8 / 114.4 us per launch;

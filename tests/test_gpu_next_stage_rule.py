@@ -28,7 +28,8 @@ def test_rule(n, states, pays):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("res,states", [([36, 30, 1], 3), ([45, 17, 2], 12), ([45, 25, 1], 2), ([11, 33, 5], 4),
-                                        ([12, 14, 13], 9), ([9, 41, 9], 12)])
+                                        ([12, 14, 13], 9), ([9, 41, 9], 12), ([12, 14, 13], 17),
+                                        ([8, 8, 8], 30), ([33, 31, 1], 13), ([2, 2, 1], 10)])
 def test_batch_equals_single_states(res, states):
     from magtense.micromag import MicromagProblem
 
