@@ -517,33 +517,36 @@ int launch_rows(const LatticeView& v, const float* m, int cols, float* out, int6
 // Whether the product from the table and the LL kernel behind it beat the launch over
 // the dense tensor.  Time of the table's right-hand side over the dense one's:
 //   n % 4 == 0, one plane, states      1     4     8     12    16    24    48
-//     32 x 40   (1280 cells)          1.27  1.46  1.32  0.81  1.18  1.13  1.08
-//     44 x 40   (1760)                0.94  1.16  1.10  0.84  1.18  1.32  1.34
-//     64 x 30   (1920)                0.83  1.02  0.80  0.73  0.91  0.97  1.01
-//     96 x 24   (2304)                0.67  0.81  0.99  0.75  1.15  1.20  1.23
-//     20 x 110  (2200)                0.76  0.85  1.06  0.70  1.10  1.13  1.17
-//     128 x 20  (2560)                0.59  0.75  0.81  0.61  0.93  0.96  1.00
-//     50 x 82   (4100)                0.53  0.78  0.91  0.72  1.10  1.18  1.30
-//     128 x 64  (8192)                            0.53  0.47  0.64  0.73
+//     36 x 30   (1080 cells)          1.17  1.28  1.15  1.18  1.18  1.19  1.29
+//     64 x 17   (1088)                1.12  1.26  1.13  0.90  1.05  0.96  0.98
+//     44 x 40   (1760)                0.93  1.16  1.11  1.05  1.20  1.34  1.36
+//     64 x 30   (1920)                0.82  1.02  0.82  0.97  0.96  0.99  1.05
+//     20 x 110  (2200)                0.76  0.85  1.05  0.95  1.13  1.16  1.18
+//     96 x 24   (2304)                0.67  0.82  0.99  1.03  1.17  1.21  1.26
+//     128 x 20  (2560)                0.59  0.75  0.83  0.83  0.96  0.99  1.02
+//     50 x 82   (4100)                0.53  0.73  0.83  0.78  1.01  1.08  1.18
+//     128 x 64  (8192)                0.19  0.35  0.52  0.54        0.75
 //   several planes, where (xz, yz) cost a second LDS read a pair
-//     30 x 30 x 2   (1800)            1.26  1.59  1.21  1.17  1.50  1.65  1.77
-//     32 x 33 x 2   (2112)            0.94  1.04  1.36  0.87  1.42  1.40  1.41
-//     48 x 16 x 4   (3072)            0.58  0.88  1.21  1.00  1.60  1.76  1.84
-//     50 x 37 x 2   (3700)            0.70  1.19  1.50  1.20  1.67  1.82  2.01
-//     64 x 16 x 4   (4096)            0.36  0.68  0.87  0.74  1.04  1.18  1.34
-//     100 x 30 x 2  (6000)            0.41  0.72  1.05  0.91  1.29  1.45  1.60
+//     30 x 30 x 2   (1800)            1.25  1.52  1.15  1.47  1.46  1.59  1.72
+//     32 x 33 x 2   (2112)            0.94  1.03  1.29  1.12  1.35  1.37  1.38
+//     64 x 12 x 3   (2304)            0.79  0.98  1.25  1.13  1.38  1.36  1.35
+//     48 x 16 x 4   (3072)            0.58  0.81  1.08  1.20  1.49  1.60  1.67
+//     50 x 37 x 2   (3700)            0.69  1.13  1.42  1.31  1.57  1.70  1.88
+//     64 x 16 x 4   (4096)            0.37  0.60  0.75  0.73  0.91  1.04  1.17
+//     100 x 30 x 2  (6000)            0.41  0.66  0.96  0.96  1.20  1.34  1.48
 //   n % 4 != 0: a chain's four columns lie in four places of the grid
-//     77 x 33   (2541)                1.21  1.59  1.88  1.53  2.03  2.06  2.21
-//     91 x 41   (3731)                0.67  0.91  1.11  1.03  1.29  1.41  1.53
-//     63 x 57   (3591, lanes 0.98)    0.47  0.62  0.85  0.82  1.00  1.15  1.22
-//     63 x 101  (6363, lanes 0.98)    0.35  0.56  0.82  0.73  0.98  1.03  1.12
-//     91 x 71   (6461)                0.47  0.75  1.03  1.01  1.24  1.38  1.51
-//     45 x 41 x 2   (3690)            1.51  1.68  1.99  1.88  2.48  2.68  2.92
-//     17 x 17 x 13  (3757)            1.57  1.77  2.10  1.97  2.27  2.46  2.71
-//     45 x 47 x 3   (6345)            1.19  (45 x 45 x 3, 2 to 24 states: 1.9 1.5 2.1 2.1 2.6)
-//     65 x 49 x 3   (9555)            1.23
-//     45 x 79 x 3   (10665)           0.97  1.28  1.97
-//     49 x 49 x 5   (12005)           0.90  1.10  1.79  1.95        2.40
+//     77 x 33   (2541)                1.19  1.58  1.88  1.53  2.09  2.09  2.23
+//     91 x 41   (3731, lanes 0.71)    0.67  0.91  1.12  1.03  1.30  1.46  1.56
+//     63 x 57   (3591, lanes 0.98)    0.47  0.62  0.86  0.82  1.02  1.19  1.24
+//     63 x 101  (6363, lanes 0.98)    0.35  0.56  0.82  0.73  0.98  1.07  1.14
+//     91 x 71   (6461, lanes 0.71)    0.47  0.75  1.03  1.00  1.25  1.40  1.52
+//     45 x 41 x 2   (3690)            1.40  1.57  1.99  1.88  2.50  2.74  2.94
+//     17 x 17 x 13  (3757)            1.57  1.77  2.08  1.94  2.29  2.46  2.69
+//     45 x 45 x 3   (6075)            1.18  1.48  2.06  2.08        2.60
+//     65 x 49 x 3   (9555)            1.45  1.70  2.67  2.75        3.73
+//     45 x 79 x 3   (10665)           1.00  1.25  1.91  2.06        2.59
+//     49 x 49 x 5   (12005)           0.87  1.12  1.71  1.97        2.45
+// (4096 cells of 128 x 32, one state: 22 us against 74.)
 // From 8192 cells on, where the dense tensor takes 1.6 GB and its assembly 4 ms, the
 // table is kept at any number of states except on odd layered grids, whose dense rows
 // are twice as fast.
@@ -554,9 +557,9 @@ bool lattice_pays(int nx, int ny, int nz, int nstates) {
   if (n % 4 && nz > 1) return n > 10000 && nstates == 1 && !wide;
   if (n >= 8192) return true;
   if (n % 4) return n > 3500 && (nstates <= 4 || (nstates <= 12 && full));
-  if (nz > 1) return n > 2000 && (nstates <= 4 || (nstates <= 12 && (wide || (full && nstates > 8))));
-  if (nstates <= 12) return n > 2000 || (n > 1024 && nstates > 8);
-  return n > 1024 && wide && full;
+  if (nz > 1) return nstates <= 4 ? n > 2000 : n > 4000 && wide && (nstates <= 8 || (nstates <= 12 && full));
+  if (nstates <= 12 && n > 2000) return true;
+  return n > 1024 && nstates > 8 && wide && full;
 }
 
 int lattice_wanted(int nx, int ny, int nz, int nstates, bool* wanted) {

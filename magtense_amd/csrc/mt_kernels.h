@@ -465,15 +465,14 @@ int launch_demag_llg_f32(const float* K, const LlgGrid& g, const LlgDesc* d_desc
 // well, or a vector launch after it.  It saves that launch, but its registers (180 for
 // 88 to 126 with one state) leave the rows two waves per SIMD for four or five.  us a
 // right-hand side with the next stage in the launch / in its own:
-//   cells            1 state    2        4        8        12       24 states
-//   1023 (33 x 31)   11 / 14    14 / 16  18 / 26  22 / 22  26 / 27  35 / 35
-//   1080 (36 x 30)   17 / 15    16 / 17  19 / 20  24 / 24  41 / 40  43 / 42
-//   1530 (45x17x2)   21 / 18    19 / 19  21 / 22  30 / 30  38 / 39  54 / 52
-//   1760 (44 x 40)   22 / 20    21 / 22  24 / 25  36 / 35  53 / 52  60 / 55
-//   1925 (77 x 25)   25 / 22    23 / 24  25 / 26  33 / 34  42 / 44  74 / 72
-//   2304 (96 x 24)   36 / 30    34 / 32  41 / 40  47 / 45  84 / 79  81 / 74
-//   2541 (77 x 33)   38 / 32    36 / 34  40 / 38  53 / 45  73 / 76  111 / 108
-//   3465 (63 x 55)   72 / 58    62 / 61  69 / 68  91 / 88  122 / 125  194 / 188
+//   cells            1 state    2        4        8        12       16       24 states
+//   1080 (36 x 30)   17 / 15    16 / 17  19 / 20  24 / 24  30 / 32  31 / 32  42 / 41
+//   1530 (45x17x2)   21 / 18    19 / 19  22 / 22  30 / 30  38 / 40  41 / 38  56 / 48
+//   1760 (44 x 40)   22 / 20    21 / 22  24 / 25  36 / 35  42 / 41  44 / 44  58 / 53
+//   1925 (77 x 25)   25 / 22    23 / 24  25 / 26  33 / 34  42 / 44  51 / 49  71 / 61
+//   2304 (96 x 24)   36 / 30    34 / 32  41 / 40  48 / 45  59 / 57  61 / 58  79 / 72
+//   2541 (77 x 33)   38 / 33    36 / 34  40 / 38  53 / 45  73 / 76  77 / 67  107 / 89
+//   3465 (63 x 55)   72 / 58    62 / 61  70 / 68  91 / 88  122 / 125  140 / 124  192 / 163
 //   16425 (75x73x3)  1214 / 1146  1189 / 1191  1299 / 1294
 // (up to 1024 cells one to four states are formed whole in the launch before, and twelve
 // states to a pass are rows of single columns).

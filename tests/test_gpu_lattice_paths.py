@@ -60,15 +60,13 @@ def _problem(res, m0, path):
 
 def _both(res, m0, held, tmp_path):
     """Fields and magnetizations of the batch m0 by the table and by the dense tensor."""
-    n, out = int(np.prod(res)), []
+    n, out, used = int(np.prod(res)), [], []
     h = np.linspace(-0.03, 0.03, len(m0))[:, None] * np.array([1.0, 0.3, 0.0]) / MU0
     for path in ("t", str(tmp_path / "tensor.bin")):
         out.append(_problem(res, m0, path).run_simulation_batch(
             2e-13, 2, [lambda t, v=v: np.ones((len(t), 1)) * v for v in h], 4, m0, return_fields=True))
-        if path == "t":
-            assert held["bytes"] < 12 * n * n, "this grid is not taken by the table"
-        else:
-            assert held["bytes"] >= 24 * n * n
+        used.append(held["bytes"])
+    assert used[1] >= 24 * n * n and used[0] < used[1] - 12 * n * n, "this grid is not taken by the table"
     return out
 
 
@@ -79,9 +77,9 @@ def _unit(rng, states, n):
 
 # measured with both forms (lattice.hip); the listed lines of the rule
 @pytest.mark.parametrize("res,states,pays", [
-    ((32, 32, 1), 64, False), ((32, 40, 1), 8, False), ((32, 40, 1), 9, True), ((32, 40, 1), 16, False),
+    ((32, 32, 1), 64, False), ((32, 40, 1), 8, False), ((32, 40, 1), 9, False), ((64, 17, 1), 9, True),
     ((64, 30, 1), 16, True), ((96, 24, 1), 8, True), ((96, 24, 1), 16, False), ((128, 32, 1), 1, True),
-    ((128, 32, 1), 64, True), ((32, 33, 2), 4, True), ((32, 33, 2), 8, False), ((32, 33, 2), 12, True),
+    ((128, 32, 1), 64, True), ((32, 33, 2), 4, True), ((32, 33, 2), 8, False), ((32, 33, 2), 12, False), ((64, 12, 3), 9, False), ((64, 16, 4), 12, True),
     ((48, 16, 4), 8, False), ((64, 16, 4), 8, True), ((64, 16, 4), 24, False), ((256, 64, 2), 64, True),
     ((77, 33, 1), 1, False), ((91, 41, 1), 4, True), ((91, 41, 1), 8, False), ((63, 57, 1), 12, True),
     ((63, 57, 1), 24, False), ((45, 41, 2), 1, False), ((67, 19, 3), 2, False), ((65, 49, 3), 1, False),
@@ -98,8 +96,9 @@ def test_rule(res, states, pays):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("res,states", [([91, 71, 1], 1), ([77, 47, 1], 3), ([99, 37, 1], 2), ([63, 57, 1], 9),
-                                        ([32, 33, 2], 3), ([20, 20, 6], 4), ([16, 9, 16], 2), ([90, 14, 2], 3),
-                                        ([64, 12, 3], 9), ([130, 6, 3], 1), ([32, 33, 2], 9)])
+                                        ([90, 30, 1], 5), ([20, 110, 1], 6), ([64, 18, 1], 9), ([32, 33, 2], 3),
+                                        ([20, 20, 6], 4), ([16, 9, 16], 2), ([90, 14, 2], 3), ([130, 6, 3], 1),
+                                        ([64, 22, 3], 9), ([128, 17, 2], 12)])
 def test_table_equals_dense(res, states, held, tmp_path):
     m0 = _unit(np.random.default_rng(4), states, int(np.prod(res)))
     got, ref = _both(res, m0, held, tmp_path)
@@ -146,7 +145,7 @@ def test_state_beyond_fp32_in_a_solver(res, component, held, tmp_path):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("where", ["m0", "stage", "cotangent"])
-@pytest.mark.parametrize("res,states,alone", [([32, 35, 1], 9, "dense"), ([32, 33, 2], 5, "table")])
+@pytest.mark.parametrize("res,states,alone", [([64, 18, 1], 9, "dense"), ([32, 33, 2], 5, "table")])
 def test_non_finite_state_in_a_gradient(res, states, alone, where, held):
     """A state of the batch and the state alone, one of them on the table and one on the
     dense tensor.  m0: 1e39; stage: finite in FP32 at first, beyond it in the second
