@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(256) interleave_kernel(const float* __restrict
 }
 
 // few states (S <= 8): wave per receiver row, lanes split the entries, h is
-// [S][3n], m the states interleaved by W.  Bound by the gathers of m through L1:
+// [S][3n], m the states interleaved by W (W = 1: [S][3n] as well).  Bound by the gathers of m through L1:
 // a lane takes W states of a source with one load, and the matrix is read once
 // (6 bytes an entry, 8 with 32-bit columns).  A lane takes
 // four entries at a time and what is left of its row, up to three, at once under
@@ -774,7 +774,13 @@ int SparseDemag::apply(const float* m, int64_t ld, int S, float pref, float* h, 
       const int g = std::min(S - s0, 8);
       const float* mg = m + (int64_t)s0 * ld;
       float* hg = h + (int64_t)s0 * ld;
-      if (g > 1) {
+      // few states of a small matrix gather one by one from [S][3n]: the launch that
+      // interleaves them takes 3 us.  us one by one / interleaved: 1000 cells, 0.17 M
+      // entries, 2 3 4 states 17/20 18/21 19/22; 512, 1.1 M 21/22 23/23 26/24; 2049, 0.58 M
+      // 18/21 20/22 24/23; 1500, 1.5 M 21/21 25/23 28/24; 4096, 1.5 M 25/25 35/27 43/28
+      const int64_t gathers = (nnz[0] + nnz[1] + nnz[2] + nnz[3] + nnz[4] + nnz[5]) * (g - 1);
+      const bool direct = g <= 4 && ld == n3 && gathers < std::min<int64_t>(1500000, (int64_t)2200 * n);
+      if (g > 1 && !direct) {
         int rc = scratch();
         if (rc) return rc;
         const unsigned eb = (unsigned)((n3 + 255) / 256);
@@ -791,6 +797,12 @@ int SparseDemag::apply(const float* m, int64_t ld, int S, float pref, float* h, 
         const CsrView<C> A{rowptr, coff, c, vals};
         auto go = [&](auto w) {
           constexpr int G = decltype(w)::value, W = G < 3 ? G : 4;
+          if constexpr (G > 1 && G <= 4) {
+            if (direct) {
+              hipLaunchKernelGGL((spmv_rows_kernel<G, 1, C>), dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg);
+              return;
+            }
+          }
           hipLaunchKernelGGL((spmv_rows_kernel<G, W, C>), dim3(blocks), dim3(256), 0, st, A, n, mg, ld, pref, hg);
         };
         switch (g) {
