@@ -77,6 +77,7 @@ __global__ void __launch_bounds__(256) llg_kernel(const LlgGrid g, const LlgDesc
         for (int k = 0; k < kAhead; ++k)
           if (k < D.nsplit) s += part[k][c];
         for (int k = kAhead; k < D.nsplit; ++k) s += D.hpart[(int64_t)k * D.split_stride + (int64_t)c * g.n + i];
+        if (D.sum_out) D.sum_out[(int64_t)c * g.n + i] = s;
         return s;
       },
       dm);

@@ -153,10 +153,9 @@ __device__ __forceinline__ void llg_cell(const LlgGrid& g, const LlgDesc& D, int
   if (D.hpart64) {
     for (int c = 0; c < 3; ++c) hm[c] = (-D.hpart64[(int64_t)c * n + i]) * r.ms_f64();
   } else {
+    const float ms = r.ms_f32();
     for (int c = 0; c < 3; ++c) {
-      const float s = hsum(c);
-      if (D.sum_out) D.sum_out[(int64_t)c * n + i] = s;
-      float h = (-s) * r.ms_f32();
+      float h = (-hsum(c)) * ms;
       hm[c] = (double)h;
     }
   }
