@@ -854,7 +854,10 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
     const int jy = (wy - r + gny) % gny, jz = (wz - sp + gnz) % gnz;
     return (jz * gny + jy) * cpr + x1c;
   };
-  // full false: without the xz and yz fragments (4, 5, 8, 9)
+  // full false: without the xz and yz fragments (4, 5, 8, 9).  The states' three
+  // transfers behind one M0 set-up pay beside those eight only (192 x 100 x 1: 745 us a
+  // launch, 865 with three set-ups); beside twelve they hold the wave (160 x 50 x 3: 1850
+  // us, 1655 with three; 64 x 64 x 4: 845 and 787).
   auto issue = [&](auto full, int v, int slot) {
     const int J = chunk_of(v);
     const int jrow = J / cpr;
@@ -866,7 +869,14 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
     for (int q = 0; q < 12; ++q)
       if (full || q < 4 || q == 6 || q == 7 || q > 9)
         lds_dma16(Kt + (base + q) * 64 + lane, lds_addr(&smem[slot][wave * 12 + q][0]));
-    lds_dma16x3(Mp + ((int64_t)J * 12 + wave * 3) * 64 + lane, lds_addr(&smem[slot][48 + wave * 3][0]));
+    const uint4* ms = Mp + ((int64_t)J * 12 + wave * 3) * 64 + lane;
+    const uint32_t ml = lds_addr(&smem[slot][48 + wave * 3][0]);
+    if constexpr (decltype(full)::value) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) lds_dma16(ms + q * 64, ml + q * kFragBytes);
+    } else {
+      lds_dma16x3(ms, ml);
+    }
   };
   floatx16 acc[2][3];
 #pragma unroll
