@@ -978,7 +978,9 @@ __global__ void __launch_bounds__(256, 2) gemm_bf16x2_t4s_kernel(const uint4* __
 // Bound by the matrix cores at the clock that their power leaves.  256 x 64 x
 // 2, 64 states, per call: 3.04 ms with the barrier at the step's start, 2.93
 // with it inside, 2.63 with the in-plane half of the chunks at 30 MFMAs
-// instead of 54 (nx x 2 planes; a single plane takes 30 throughout).
+// instead of 54 (nx x 2 planes; a single plane takes 30 throughout).  The launch
+// alone: 2.10 ms, 589 TFLOP/s of 18 n^2 flop a state, matrix pipe busy 61 % at 2.15
+// GHz (table_block).
 __global__ void __launch_bounds__(256, 1) gemm_bf16x2_tw_kernel(const uint4* __restrict__ Kt,
                                                                 const uint4* __restrict__ Mp, int ksplit,
                                                                 float* __restrict__ out, int n, int64_t col_stride,

@@ -5,9 +5,12 @@
 // cell offsets, and the rounding of the cell centres gives each of them a few
 // FP64 values (4 on average on a 128-cell axis).  LatticeTable stores the
 // tensor once per distinct triple of differences, evaluated from the same FP64
-// arguments as the dense assembly, and index maps from cell pairs to entries:
-// the same FP32 entries in 4.4 MB instead of 402.7 MB for 128 x 32 x 1, 72 MB
-// instead of 25.8 GB for 256 x 64 x 2.
+// arguments as the dense assembly, and index maps from cell pairs to entries.
+// An entry takes 16 bytes in one plane (xx, xy, yy, zz), 24 in several, and
+// columns of equal entries are stored once: the same FP32 entries in about 1 MB
+// instead of 402.7 MB for 128 x 32 x 1 (326 columns of 183 entries in a film of
+// 500 x 125 nm), 105 MB instead of 25.8 GB for 256 x 64 x 2 cells of 4 nm, where
+// next to nothing is equal.
 //
 // Product: the sums of matvec_rows_f32 (matvec_rows.h), bit for bit.  There a
 // receiver row is summed by 256 threads, thread T taking the column quads
@@ -104,9 +107,9 @@ __host__ __device__ inline LatLds lat_lds(const LatticeView& v, int qc, int nbuf
 // 0.6 of the launch's) and by what a wave waits for between them.  The next sums'
 // reads are issued after the last ones have arrived, the x map's values of a step
 // before its barrier, and a step's place in the grid is kept up by addition.
-// Before, with a wait per read, us a launch: one state 128 x 32 x 1 16.7 (17.7), 90
-// x 70 x 1 70 (81), 91 x 71 x 1 86 (119), 256 x 64 x 2 896 (1024), there four
-// states 1770 (1867).
+// Kernel alone, us a launch (in parentheses with a wait per read): one state 128 x 32
+// x 1 14 (15), 90 x 70 x 1 68 (79), 91 x 71 x 1 84 (116), 256 x 64 x 2 893 (1023),
+// there four states 1879 (1985).
 template <int QC, bool HASB, bool ALIGNED, int SB>
 __global__ void __launch_bounds__(kLatThreads)
     lattice_rows_kernel(const LatticeView v, const float* __restrict__ m, int cols, float* __restrict__ out,
@@ -636,7 +639,8 @@ int LatticeTable::build(int nx, int ny, int nz, const std::vector<double>& cx, c
   int rc = entries_of(val[0]);
   if (rc) return rc;
   // x differences whose entries all equal those of their offset's commonest
-  // one are the same column of the table: 997 -> 316 columns at 128 x 32 x 1
+  // one are the same column of the table: 997 -> 326 columns at 128 x 32 x 1
+  // (500 x 125 nm)
   std::vector<int> owner(std::max(extra, 1), 0), same(std::max(extra, 1), 1);
   for (int j = 0; j < nx; ++j)
     for (int i = 0; i < nx; ++i) {

@@ -128,7 +128,9 @@ constexpr int kRowThreads = 256;  // of matvec_rows_f32
 // further waves of the block meet by themselves.  States from `have` on
 // repeat the last one.
 // NT: non-temporal tensor loads, for a tensor that the launch reads once, so that
-// it does not displace the state vectors from L2.
+// it does not displace the state vectors from L2.  Where the tensor fits in L2 they
+// cost nothing (32 x 8 cells, one state: 8.6 us a launch either way; 32 x 32: 10.1
+// either way; 44 x 40: 21.8, cached loads 22.5).
 template <int RB, bool VEC4, int S, bool NT = true>
 __device__ __forceinline__ void matvec_rows_f32(const float* __restrict__ K, int n, const float* __restrict__ m,
                                        int64_t m_stride, int have, int i0, float (&red)[4][RB * S * 3],
@@ -226,7 +228,9 @@ inline int matvec_group(int left, bool vec4) {
 inline int matvec_groups(int left, int S) { return S == 8 ? std::min((left + 7) / 8, 64) : 1; }
 // Receiver rows of its blocks: a value of a state is read from L2 once per block,
 // so that more rows are less traffic, until the sums take a wave's registers.
-// One state, 402.7 MB tensor: 2 / 4 / 8 rows -> 72.2 / 66.8 / 114.4 us per launch;
+// One state, 2 / 4 rows, us a launch: 32 x 8 8.2 / 8.6, 30 x 18 12.3 / 9.4, 32 x 32
+// 14.1 / 10.1, 44 x 40 29.2 / 21.8, 77 x 33 44.2 / 38.5 (a tensor of 402.7 MB 72.2 /
+// 66.8, 8 rows 114.4);
 // 8 states of 90 x 70: 2 / 3 rows -> 0.254 / 0.234 ms (4: 299 registers, one wave
 // per SIMD).
 constexpr int matvec_block_rows(int S, bool vec4) { return S >= 8 && vec4 ? 3 : 4; }

@@ -36,10 +36,14 @@ constexpr double kSclH = 1.0001, kSclL = 0.9999;
 
 __device__ inline double sq(double v) { return v * v; }
 
-// a / b and sqrt(a), rounded to nearest as the operators give them, without the
-// scaling and the special cases around the same Newton steps (8 operations for
-// 11, 13 for 19): for arguments and results in FP64's normal range, which the
-// unit of length of prism_k6 sees to; root(0) = 0.
+// a / b and sqrt(a), rounded to nearest as the operators give them, for arguments
+// and results in FP64's normal range, which the unit of length of prism_k6 sees to;
+// root(0) = 0.  quotient: two Newton-Raphson steps of the hardware's reciprocal,
+// then the quotient corrected once by its residual a - b q (Markstein, IBM J. Res.
+// Dev. 34, 1990).  root: Goldschmidt's coupled iteration for sqrt(a) and 1 / (2
+// sqrt(a)) from the hardware's reciprocal root, then two residual corrections.
+// Without the scaling and the special cases of the operators: 8 operations for 11,
+// 13 for 19.
 __device__ inline double quotient(double a, double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = fma(y, fma(-b, y, 1.0), y);
